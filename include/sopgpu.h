@@ -175,10 +175,10 @@ typedef struct sop_tuning {
     int verlet_chunk; /* 64-entry chunks of a possible-list row in flight in the LDS Verlet build: 4 or 8 */
     int sort_every;   /* Verlet rows re-sorted by length at every k-th Verlet rebuild */
     int split_rows;   /* 4, 8 or 16: the jobs of at most 5120 beads are stepped with each bead's force terms
-                         spread over a 1024-thread workgroup of that many beads (for a few small jobs; the
-                         same results); 0: one bead per lane */
-    int split_global; /* the same for the jobs above 5120 beads (partners gathered from global memory): 4, 8
-                         or 16 beads per workgroup, 0: one bead per lane */
+                         spread over the lanes of a wavefront, that many beads per wavefront, and their lists
+                         built one wavefront per bead (the same results); 0: one bead per lane.  Until a shape
+                         is set or tuned, the engine chooses by the beads it steps. */
+    int split_global; /* the same step for the jobs above 5120 beads (partners gathered from global memory) */
 } sop_tuning;
 int sop_engine_get_shape(sop_engine* e, sop_tuning* out);
 int sop_engine_set_shape(sop_engine* e, const sop_tuning* shape);

@@ -166,6 +166,7 @@ Engine::~Engine() {
     for (auto& j : jobs_)
         for (void* b : j.blocks) arena_.release(b);
     (void)hipFree(d_jobs_);
+    (void)hipFree(d_descs_);
     (void)hipFree(d_state_);
     (void)hipFree(d_tiles_);
     (void)hipFree(d_tiles1_);
@@ -780,19 +781,24 @@ int Engine::sync_tables() {
     if (nj > cap_jobs_) {
         int cap = std::max(16, nj * 2);
         (void)hipFree(d_jobs_);
+        (void)hipFree(d_descs_);
         (void)hipFree(d_state_);
         d_jobs_ = nullptr;
+        d_descs_ = nullptr;
         d_state_ = nullptr;
         if (int rc = check(hipMalloc(&d_jobs_, cap * sizeof(DevJob)), "job table")) return rc;
+        if (int rc = check(hipMalloc(&d_descs_, cap * sizeof(StepDesc)), "step table")) return rc;
         if (int rc = check(hipMalloc(&d_state_, cap * sizeof(DevJobState)), "state table")) return rc;
         cap_jobs_ = cap;
     }
     std::vector<DevJob> dj(nj);
+    std::vector<StepDesc> sd(nj);
     std::vector<DevJobState> ds(nj);
     std::vector<int2> tiles;
     int g = 0;
     for (int k = 0; k < nj; ++k) {
         dj[k] = jobs_[k].dj;
+        sd[k] = step_desc(jobs_[k].dj);
         ds[k] = jobs_[k].st0;
         ds[k].step = jobs_[k].step;
         jobs_[k].tile0 = (int)tiles.size();
@@ -828,6 +834,9 @@ int Engine::sync_tables() {
         if (int rc = check(hipMemcpyAsync(d_jobs_, dj.data(), nj * sizeof(DevJob), hipMemcpyHostToDevice, stream_),
                            "job table upload"))
             return rc;
+        if (int rc = check(hipMemcpyAsync(d_descs_, sd.data(), nj * sizeof(StepDesc), hipMemcpyHostToDevice, stream_),
+                           "step table upload"))
+            return rc;
         if (int rc = check(hipMemcpyAsync(d_state_, ds.data(), nj * sizeof(DevJobState), hipMemcpyHostToDevice, stream_),
                            "state upload"))
             return rc;
@@ -841,8 +850,11 @@ int Engine::sync_tables() {
     std::vector<int2> units;
     lds_beads_ = 0;
     any_global_ = 0;
+    long long lds_rows = 0, global_rows = 0, short_rows = 0;
     for (int k = 0; k < nj; ++k) {
         const DevJob& J = jobs_[k].dj;
+        (J.lds_step ? lds_rows : global_rows) += J.n;
+        if (J.n <= kRowsShort) short_rows += J.n;
         if (!J.lds_step) {
             any_global_ = 1;
             continue;
@@ -863,6 +875,7 @@ int Engine::sync_tables() {
                            "unit upload"))
             return rc;
     }
+    eff_ = effective_shape(lds_rows, global_rows, short_rows);
     // LDS step plan
     std::vector<int2> su;
     std::vector<int4> sg;
@@ -874,6 +887,43 @@ int Engine::sync_tables() {
     tables_dirty_ = false;
     synced_jobs_ = nj;
     return 0;
+}
+
+// The launch shape for so many rows (Verlet rows: beads) of LDS-step jobs and
+// of the others, short_rows of them of jobs of at most kRowsShort beads: the
+// one set by set_shape or autotune, else the spread step (k_step_rows) up to
+// kRowsMaxLds and kRowsMaxGlobal rows and one bead per lane above.
+//
+// Rows per wavefront, measured per step launch with R = 2 / 4 / 8 / 16 and
+// one bead per lane (us):
+//   1,000 rows of one chain        7.7 / 8.5 /  11 /  15,  31
+//   3,186 of three chains          8.6 / 9.0 /  12 /  17
+//   9,558 of nine chains            16 /  11 /  13 /  17,  34
+//   18,000 of an assembly           23 /  17 /  16 /  19,  58 (above the LDS limit)
+//   32,000 of 32 chains             31 /  18 /  16 /  17,  34
+//   64,000 of 64 chains             62 /  34 /  29 /  25,  35
+//   100,000 of a capsid            101 /  66 /  50 /  47,  71 (above the LDS limit)
+//   120,000 of 24 chains             - /  71 /  58 /  52,  48
+//   300,000 of a shell               - / 223 / 163 / 151, 139 (above the LDS limit)
+//   7,700 of peptides (22 beads)    11 /  10 / 7.9 / 7.8,  21
+// Few rows want many wavefronts; many rows want few instructions per row.
+// Lists as short as the peptides' leave most of a 4-row wavefront's positions
+// empty.
+StepShape Engine::effective_shape(long long lds_rows, long long global_rows, long long short_rows) const {
+    StepShape e = shape_;
+    const bool set = shape_set_;
+    const bool l = lds_rows > 0 && (set ? e.split_rows > 0 : lds_rows <= kRowsMaxLds);
+    const bool g = global_rows > 0 && (set ? e.split_global > 0 : global_rows <= kRowsMaxGlobal);
+    const long long rows = (l ? lds_rows : 0) + (g ? global_rows : 0);  // both classes in one launch
+    const bool shorts = 2 * short_rows > rows, two = rows <= kRowsTwo && !shorts;
+    auto rows_per_wave = [&](int asked) {
+        if (set) return asked == 4 && two ? 2 : asked;
+        if (rows <= kRowsFour) return shorts ? 8 : two ? 2 : 4;
+        return rows <= kRowsEight ? 8 : 16;
+    };
+    if (l) e.split_rows = rows_per_wave(e.split_rows);
+    if (g) e.split_global = rows_per_wave(e.split_global);
+    return e;
 }
 
 // The LDS step plan of the LDS-step jobs: each whole block of unit_rows
@@ -1047,12 +1097,14 @@ std::vector<long long> Engine::block_key() const {
 // slot_only >= 0 runs that job alone with its own stride (plain mode).
 int Engine::launch_block(int slot_only) {
     const DevJob* jobs = d_jobs_;
+    const StepDesc* descs = d_descs_;
     DevJobState* st = d_state_;
     const int2* tiles = d_tiles_;
     int nj = (int)jobs_.size(), nt = ntiles_, L = L_;
     if (slot_only >= 0) {
         if (int rc = tiles_for_slot(slot_only, &nt)) return rc;
         jobs = d_jobs_ + slot_only;
+        descs = d_descs_ + slot_only;
         st = d_state_ + slot_only;
         tiles = d_tiles1_;
         nj = 1;
@@ -1066,9 +1118,9 @@ int Engine::launch_block(int slot_only) {
                 ? launch_possible(jobs, st, tiles, nt, nj, cell_words_of(jobs_[slot_only].dj),
                                   !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
                                   jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, 0, stream_,
-                                  shape_)
+                                  eff1_)
                 : launch_possible(jobs, st, tiles, nt, nj, cell_words_, any_global_, d_sunits_, d_segs_, nsunits_,
-                                  lds_beads_, 0, stream_, shape_);
+                                  lds_beads_, 0, stream_, eff_);
         if (int rc = check(e, "possible pairs")) return rc;
     }
     if (due & 2) {
@@ -1080,9 +1132,9 @@ int Engine::launch_block(int slot_only) {
                                 sort && jobs_[slot_only].dj.sort_rows ? (jobs_[slot_only].n + kLdsUnit - 1) / kLdsUnit
                                                                       : 0,
                                 d_sunits1_, d_segs1_, jobs_[slot_only].dj.lds_step ? nsunits1_ : 0,
-                                jobs_[slot_only].n, 0, stream_, shape_)
+                                jobs_[slot_only].n, 0, stream_, eff1_)
                 : launch_verlet(jobs, st, tiles, nt, any_idx32_, any_global_, d_units_, sort ? nunits_ : 0,
-                                d_sunits_, d_segs_, nsunits_, lds_beads_, 0, stream_, shape_);
+                                d_sunits_, d_segs_, nsunits_, lds_beads_, 0, stream_, eff_);
         if (int rc = check(e, "verlet")) return rc;
     }
     const bool tea = slot_only >= 0 ? ((jobs_[slot_only].dj.flags & JF_HI) && !(jobs_[slot_only].dj.flags & JF_HI_EXACT))
@@ -1113,11 +1165,11 @@ int Engine::launch_block(int slot_only) {
             (void)hipEventRecord(ev_pool_[ev_used_].first, stream_);
         }
         if (int rc = check(slot_only >= 0
-                               ? launch_step(jobs, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
+                               ? launch_step(jobs, descs, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
                                              jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, k,
-                                             max_blocks_, stream_, shape_)
-                               : launch_step(jobs, st, tiles, nt, any_global_, d_sunits_, d_segs_, nsunits_, lds_beads_,
-                                             k, max_blocks_, stream_, shape_),
+                                             max_blocks_, stream_, eff1_)
+                               : launch_step(jobs, descs, st, tiles, nt, any_global_, d_sunits_, d_segs_, nsunits_, lds_beads_,
+                                             k, max_blocks_, stream_, eff_),
                            "step"))
             return rc;
         if (prof_end) {
@@ -1155,6 +1207,8 @@ int Engine::tiles_for_slot(int slot, int* nt) {
     const int n = jobs_[slot].n;
     const int need = (n + 63) / 64;
     *nt = need;
+    const bool lds = jobs_[slot].dj.lds_step != 0;
+    eff1_ = effective_shape(lds ? n : 0, lds ? 0 : n, n <= kRowsShort ? n : 0);
     if (tiles1_n_ == n && tiles1_rows_ == shape_.unit_rows) return 0;
     if (need > cap_tiles1_) {
         (void)hipFree(d_tiles1_);
@@ -1205,13 +1259,13 @@ int Engine::stage_possible() {
     if (int rc = sync_tables()) return rc;
     return check(launch_possible(d_jobs_, d_state_, d_tiles_, ntiles_, (int)jobs_.size(), cell_words_, any_global_,
                                  d_sunits_,
-                                 d_segs_, nsunits_, lds_beads_, 0, stream_, shape_),
+                                 d_segs_, nsunits_, lds_beads_, 0, stream_, eff_),
                  "possible pairs");
 }
 int Engine::stage_verlet() {
     if (int rc = sync_tables()) return rc;
     return check(launch_verlet(d_jobs_, d_state_, d_tiles_, ntiles_, any_idx32_, any_global_, d_units_, nunits_,
-                               d_sunits_, d_segs_, nsunits_, lds_beads_, 0, stream_, shape_),
+                               d_sunits_, d_segs_, nsunits_, lds_beads_, 0, stream_, eff_),
                  "verlet");
 }
 int Engine::stage_tea_update() {
@@ -1222,8 +1276,8 @@ int Engine::stage_tea_update() {
 }
 int Engine::stage_step(int k) {
     if (int rc = sync_tables()) return rc;
-    if (int rc = check(launch_step(d_jobs_, d_state_, d_tiles_, ntiles_, any_global_, d_sunits_, d_segs_, nsunits_,
-                                   lds_beads_, k, max_blocks_, stream_, shape_),
+    if (int rc = check(launch_step(d_jobs_, d_descs_, d_state_, d_tiles_, ntiles_, any_global_, d_sunits_, d_segs_, nsunits_,
+                                   lds_beads_, k, max_blocks_, stream_, eff_),
                        "step"))
         return rc;
     if (any_tea_)
@@ -1504,8 +1558,8 @@ int Engine::compute_forces(int id, float* out4) {
     int nt = 0;
     if (int rc = tiles_for_slot(slot, &nt)) return rc;
     const bool lds = hj.dj.lds_step != 0;
-    if (int rc = check(launch_forces(d_jobs_ + slot, d_state_ + slot, d_tiles1_, nt, !lds, d_sunits1_, d_segs1_,
-                                     lds ? nsunits1_ : 0, hj.n, d_scratch4_, stream_, shape_),
+    if (int rc = check(launch_forces(d_jobs_ + slot, d_descs_ + slot, d_state_ + slot, d_tiles1_, nt, !lds, d_sunits1_, d_segs1_,
+                                     lds ? nsunits1_ : 0, hj.n, d_scratch4_, stream_, eff1_),
                        "forces"))
         return rc;
     if (int rc = synchronize()) return rc;
@@ -1548,7 +1602,7 @@ int Engine::rebuild_lists(int id, int mask) {
                                            cell_words_of(jobs_[slot].dj), !jobs_[slot].dj.lds_step, d_sunits1_,
                                            d_segs1_,
                                            jobs_[slot].dj.lds_step ? nsunits1_ : 0, jobs_[slot].n, 1, stream_,
-                                           shape_),
+                                           eff1_),
                            "possible pairs"))
             return rc;
     if (mask & 2)
@@ -1557,7 +1611,7 @@ int Engine::rebuild_lists(int id, int mask) {
                                          d_units1_,
                                          jobs_[slot].dj.sort_rows ? (jobs_[slot].n + kLdsUnit - 1) / kLdsUnit : 0,
                                          d_sunits1_, d_segs1_, jobs_[slot].dj.lds_step ? nsunits1_ : 0,
-                                         jobs_[slot].n, 1, stream_, shape_),
+                                         jobs_[slot].n, 1, stream_, eff1_),
                            "verlet"))
             return rc;
     return synchronize();
@@ -1601,6 +1655,7 @@ int Engine::set_shape(const Tuning& t) {
     shape_.split_rows = t.split_rows;
     shape_.split_global = t.split_global;
     shared_units_ = t.shared_units != 0;
+    shape_set_ = true;
     tables_dirty_ = true;  // the unit plan depends on unit_rows and shared_units
     tiles1_n_ = -1;
     drop_graph();
@@ -1691,10 +1746,15 @@ int Engine::time_blocks(int nblocks, double* ms) {
 int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int* trials_out) {
     if (hipSetDevice(device_) != hipSuccess) return fail(SOP_E_HIP, "hipSetDevice failed");
     if (int rc = sync_tables()) return rc;
-    const Tuning start = tuning();
+    const bool was_set = shape_set_;
+    Tuning start = tuning();
     if (best_out) *best_out = start;
     if (trials_out) *trials_out = 0;
     if (jobs_.empty()) return 0;
+    if (!was_set) {  // the shape the jobs run in now (four rows per wavefront stand for two, too)
+        start.split_rows = eff_.split_rows == 2 ? 4 : eff_.split_rows;
+        start.split_global = eff_.split_global == 2 ? 4 : eff_.split_global;
+    }
     bool lds = false;
     long long window = L_;
     for (auto& j : jobs_) {
@@ -1734,7 +1794,11 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
             best_ms = ms;
         }
     };
-    if (lds) {
+    // each bead's terms spread over a wavefront, or one bead per lane
+    if (lds && ntiles_ <= kSplitMaxTiles)
+        for (int v : {0, 16, 8, 4})
+            if (v != best.split_rows) { Tuning t = best; t.split_rows = v; consider(t); }
+    if (lds && !best.split_rows) {
         // smaller units spread a few small jobs over more CUs
         for (int v : {1024, 768, 512, 256, 128})
             if (v != best.unit_rows) { Tuning t = best; t.unit_rows = v; consider(t); }
@@ -1744,19 +1808,16 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
         { Tuning t = best; t.verlet_chunk = best.verlet_chunk == 8 ? 4 : 8; consider(t); }
         for (int v : {10, 40})
             if (v != best.sort_every) { Tuning t = best; t.sort_every = v; consider(t); }
-        // a few small jobs: each bead's terms spread over a workgroup
-        if (ntiles_ <= kSplitMaxTiles)
-            for (int v : {16, 8, 4})
-                if (v != best.split_rows) { Tuning t = best; t.split_rows = v; consider(t); }
     }
     if (any_global_) {
-        const int full = (ntiles_ + 3) / 4;
-        for (int b : {256, 1024, 4096})
-            if (b < full && b != best.max_blocks) { Tuning t = best; t.max_blocks = b; consider(t); }
-        if (best.max_blocks != 0) { Tuning t = best; t.max_blocks = 0; consider(t); }
-        // each bead's terms spread over a workgroup: more wavefronts to hide the gathers
-        for (int v : {16, 8, 4})
+        for (int v : {0, 16, 8, 4})
             if (v != best.split_global) { Tuning t = best; t.split_global = v; consider(t); }
+        const int full = (ntiles_ + 3) / 4;
+        if (!best.split_global) {
+            for (int b : {256, 1024, 4096})
+                if (b < full && b != best.max_blocks) { Tuning t = best; t.max_blocks = b; consider(t); }
+            if (best.max_blocks != 0) { Tuning t = best; t.max_blocks = 0; consider(t); }
+        }
     }
     // the jobs as they were, under the chosen shape
     const int rc2 = set_shape(rc ? start : best);
@@ -1764,6 +1825,10 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
     (void)hipFree(snap);
     use_graph_ = saved_graph;
     profiling_ = saved_prof;
+    if (rc && !was_set) {  // as it was: the shape follows the rows again
+        shape_.split_rows = shape_.split_global = 0;
+        shape_set_ = false;
+    }
     if (rc) return rc;
     if (rc2) return rc2;
     if (rc3) return rc3;

@@ -77,8 +77,8 @@ struct Tuning {
     int pair_batch;    // Verlet entries fetched ahead per lane in the LDS step
     int verlet_chunk;  // 64-entry chunks in flight per row in the LDS Verlet build
     int sort_every;    // Verlet rows re-sorted at every k-th Verlet rebuild
-    int split_rows;    // 4, 8 or 16: LDS-step jobs stepped by k_step_split, that many rows per workgroup (0: off)
-    int split_global;  // the same for the jobs above the LDS limit (gathers from global memory)
+    int split_rows;    // 4, 8 or 16: LDS-step jobs stepped by k_step_rows, that many rows per wavefront (0: off)
+    int split_global;  // the same for the jobs above the LDS limit
 };
 
 class Engine {
@@ -172,6 +172,7 @@ class Engine {
     int next_id_ = 1;
     // device tables
     DevJob* d_jobs_ = nullptr;
+    StepDesc* d_descs_ = nullptr;
     DevJobState* d_state_ = nullptr;
     int2* d_tiles_ = nullptr;
     int cap_jobs_ = 0, cap_tiles_ = 0, ntiles_ = 0;
@@ -206,6 +207,9 @@ class Engine {
     int cap_sunits1_ = 0, cap_segs1_ = 0, nsunits1_ = 0;
     int tiles1_rows_ = 0;  // unit rows the single-job plan was built for
     StepShape shape_;
+    bool shape_set_ = false;  // by set_shape or autotune; else the spread step follows the rows (effective_shape)
+    StepShape eff_, eff1_;    // the shapes launched: of the admitted jobs, and of the single-job path's job
+    StepShape effective_shape(long long lds_rows, long long global_rows, long long short_rows) const;
     bool shared_units_ = true;
     // autotuner snapshot of the jobs' device arrays and state table
     int snapshot(void** buf);

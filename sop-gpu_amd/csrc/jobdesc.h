@@ -124,6 +124,41 @@ struct DevJob {
     int hi_eps_freq, hi_capricious, hi_chol_freq;
 };
 
+// What a step reads of a job, in one piece, for k_step_rows: its wavefronts
+// are too few to hide one scalar load of the descriptor after another, so it
+// reads this record at once.  The same fields as DevJob, with the bonded lists
+// the step uses (row order or bead order, 16- or 32-bit) already chosen; filled
+// by the engine whenever the job table is.
+struct StepDesc {
+    float4* coord[2];
+    int* perm;         // rows' beads; null where row r is bead r
+    int* pair_cnt;
+    void* pair_j;
+    int* b_cnt;        // per row: covalent | native << 16 (null: cov_cnt and nat_cnt, per bead)
+    void* cov_j;       // bonded entries at [k*b_ld + col], col the row (b_cnt) or the bead
+    float* cov_r0;
+    void* nat_j;
+    float2* nat_par;
+    int* cov_cnt;
+    int* nat_cnt;
+    uint4* rng;
+    float* T;
+    unsigned char* bflag;
+    float4* fextra;
+    int n, flags, idx16, lds_step;
+    int pair_ld, pair_cap, b_ld;
+    float ks, R2, a2, m6, rc2;
+    float hOverZeta, tempNorm;
+    int stride, nav;
+    long long end_step;
+    // not read by every job's step
+    float4* ext;
+    float4* tipF;
+    float4* rforce;
+    float4* mforce;
+    float tipR, tipAp, tipBp, surfAp, surfBp, micaN[3];
+};
+
 struct DevJobState {
     long long step;   // local step at the start of the current block
     float var;        // sqrt(2 T zeta / h)
@@ -140,6 +175,62 @@ struct DevJobState {
     float cell_inv;     // 1 / cell edge
     int cell_dim[3];
 };
+
+inline StepDesc step_desc(const DevJob& J) {
+    StepDesc d{};
+    d.coord[0] = J.coord[0];
+    d.coord[1] = J.coord[1];
+    d.perm = J.rb_cnt ? J.perm : nullptr;  // only such jobs' rows were ever sorted
+    d.pair_cnt = J.pair_cnt;
+    d.pair_j = J.pair_j;
+    d.cov_cnt = J.cov_cnt;
+    d.nat_cnt = J.nat_cnt;
+    if (J.sort_rows) {
+        d.b_cnt = J.rb_cnt;
+        d.cov_j = J.rb_cov_j;
+        d.cov_r0 = J.rb_cov_r0;
+        d.nat_j = J.rb_nat_j;
+        d.nat_par = J.rb_nat_par;
+        d.b_ld = J.pair_ld;
+    } else {
+        d.cov_j = J.idx16 ? (void*)J.cov_j16 : (void*)J.cov_j;
+        d.cov_r0 = J.cov_r0;
+        d.nat_j = J.idx16 ? (void*)J.nat_j16 : (void*)J.nat_j;
+        d.nat_par = J.nat_par;
+        d.b_ld = J.n;
+    }
+    d.rng = J.rng;
+    d.T = J.T;
+    d.bflag = J.bflag;
+    d.fextra = J.fextra;
+    d.n = J.n;
+    d.flags = J.flags;
+    d.idx16 = J.idx16;
+    d.lds_step = J.lds_step;
+    d.pair_ld = J.pair_ld;
+    d.pair_cap = J.pair_cap;
+    d.ks = J.ks;
+    d.R2 = J.R2;
+    d.a2 = J.a2;
+    d.m6 = J.m6;
+    d.rc2 = J.rc2;
+    d.hOverZeta = J.hOverZeta;
+    d.tempNorm = J.tempNorm;
+    d.stride = J.stride;
+    d.nav = J.nav;
+    d.end_step = J.end_step;
+    d.ext = J.ext;
+    d.tipF = J.tipF;
+    d.rforce = J.rforce;
+    d.mforce = J.mforce;
+    d.tipR = J.tipR;
+    d.tipAp = J.tipAp;
+    d.tipBp = J.tipBp;
+    d.surfAp = J.surfAp;
+    d.surfBp = J.surfBp;
+    for (int k = 0; k < 3; ++k) d.micaN[k] = J.micaN[k];
+    return d;
+}
 
 // Jobs of this many beads and more build their possible-pairs list from a
 // cell grid instead of the all-pairs scan (same list, same order).

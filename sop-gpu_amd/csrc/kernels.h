@@ -11,10 +11,9 @@ namespace sop {
 // rows), Verlet entries fetched ahead per lane in the step, 64-entry chunks
 // in flight per row in the Verlet build, and the row-sort cadence (every
 // k-th Verlet rebuild).  split_rows (4, 8 or 16; 0: off) steps the LDS-step
-// jobs by k_step_split instead, one workgroup per split_rows rows with each
-// row's force terms spread over the workgroup (for a few small jobs), and
-// builds their lists one wavefront per row; split_global does the same for
-// the jobs above the LDS limit (gathers from global memory).
+// jobs by k_step_rows instead, that many rows per wavefront (two instead of
+// four in the smallest launches) with each row's force terms spread over its lanes, and builds their lists one wavefront
+// per row; split_global steps the jobs above the LDS limit the same way.
 struct StepShape {
     int unit_rows = kLdsUnit;
     int pair_batch = 6;
@@ -23,9 +22,16 @@ struct StepShape {
     int split_rows = 0;
     int split_global = 0;
 };
-// The autotuner tries split_rows only where the launch has at most this
-// many 64-row tiles (the spread pays where one bead per lane leaves CUs idle).
-constexpr int kSplitMaxTiles = 128;
+// The rule for the spread step where no shape was set (measurements at
+// Engine::effective_shape): rows of the launch up to which a wavefront takes
+// two, four and eight rows (sixteen above), the rows of LDS-step jobs and of the
+// others up to which they are spread at all, and the beads of a job whose lists
+// are too short for less than eight rows per wavefront.
+constexpr int kRowsTwo = 4500, kRowsFour = 17000, kRowsEight = 34000, kRowsMaxLds = 90000, kRowsMaxGlobal = 220000;
+constexpr int kRowsShort = 28;
+// The autotuner tries split_rows only where the launch has at most this many
+// 64-row tiles.
+constexpr int kSplitMaxTiles = 1536;
 
 // One Langevin step (local step = state.step + kstep) of every job that owns
 // a tile.  max_blocks caps the persistent grid (0 = one block per 4 tiles).
@@ -33,8 +39,9 @@ constexpr int kSplitMaxTiles = 128;
 // segment, segment count) of `segs` (job slot, first row, rows, LDS offset
 // in float4; lds_beads = the largest LDS use of a unit), the others by the
 // tile kernel (launched when any_global is set).  With shape.split_rows set
-// the LDS-step jobs are stepped by k_step_split over the tiles instead.
-hipError_t launch_step(const DevJob* jobs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
+// (split_global) the LDS-step (other) jobs are stepped by k_step_rows over the
+// tiles instead, from the step records `descs`.
+hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
                        const int2* units, const int4* segs, int nunits, int lds_beads, int kstep, int max_blocks,
                        hipStream_t stream, const StepShape& shape);
 // List rebuilds for jobs whose cadence is due (force != 0: rebuild all).
@@ -64,7 +71,7 @@ hipError_t launch_job_advance(const DevJob* jobs, DevJobState* st, int njobs, in
 hipError_t launch_energies(const DevJob* jobs, const DevJobState* st, int job, int n, hipStream_t stream);
 // Forces only (the step kernels' force terms, no state change) of the jobs
 // of the given tiles / LDS plan, into out[bead] (one job per launch).
-hipError_t launch_forces(const DevJob* jobs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
+hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
                          const int2* units, const int4* segs, int nunits, int lds_beads, float4* out,
                          hipStream_t stream, const StepShape& shape);
 hipError_t launch_rng_probe(uint4* state, int n, int count, int gaussian, float* out, hipStream_t stream);

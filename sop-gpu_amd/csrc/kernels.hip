@@ -197,7 +197,8 @@ __device__ __forceinline__ void pair_loop(const __attribute__((address_space(1))
 // langevin_kernel.cu:43-50): a fixed bead's force is zeroed, a pulled bead's
 // gets the cantilever force.  The one-byte flag is read for every bead, the
 // 16-byte force record only for pulled beads.
-__device__ __forceinline__ void ext_rules_flag(const DevJob& J, int i, int f, float& fx, float& fy, float& fz) {
+template <typename D>
+__device__ __forceinline__ void ext_rules_flag(const D& J, int i, int f, float& fx, float& fy, float& fz) {
     if (f == 1) {
         fx = 0.0f; fy = 0.0f; fz = 0.0f;
     } else if (f == 2) {
@@ -293,28 +294,22 @@ __device__ __forceinline__ void step_head(const DevJob& J, int i, int r, int n, 
     }
 }
 
-// The per-bead state the tail reads (RNG state, temperature accumulator,
-// fixed/pulled flag), loaded ahead by a caller with latency to hide.
+// The per-bead state the tail reads and its noise, formed ahead by a caller
+// with latency to hide (which then also writes the RNG state back): the
+// Gaussian triple, the temperature accumulator and the fixed/pulled flag.
 struct TailPre {
-    uint4 rng;
+    float3 g;
     float T;
     int flag;
 };
-__device__ __forceinline__ TailPre tail_prefetch(const DevJob& J, int i) {
-    TailPre t;
-    t.rng = J.rng[i];
-    t.T = J.T[i];
-    t.flag = (J.flags & JF_PULLING) ? (int)J.bflag[i] : 0;
-    return t;
-}
 
 // The rest of a bead's step, after the repulsive pairs: indentation walls,
-// then (FO) the forces written to cout, or the noise, the fixed/pulled rules
-// and the Euler update written to `cout` in global memory.  Hydrodynamic
+// then (FO) the forces written to cout, or the noise (of amplitude var), the
+// fixed/pulled rules and the Euler update written to `cout` in global memory.  Hydrodynamic
 // jobs stop after the forces.  pre: the state loaded ahead (null: loaded
 // here).
-template <bool FO>
-__device__ __forceinline__ void step_tail(const DevJob& J, const DevJobState& S, long long s, int i, const float4 c,
+template <bool FO, typename D>
+__device__ __forceinline__ void step_tail(const D& J, const DevJobState& S, float var, long long s, int i, const float4 c,
                                           float fx, float fy, float fz, float4* __restrict__ cout,
                                           const TailPre* pre = nullptr) {
     // indentation tip and substrate plane (indentation_kernel.cu:71-128)
@@ -354,10 +349,9 @@ __device__ __forceinline__ void step_tail(const DevJob& J, const DevJobState& S,
     // (integrateTea_prepare, bdhitea_kernel.cu:33-65); the update itself
     // runs in hi.hip once every bead's forces are known
     if (J.flags & JF_HI) {
-        uint4 rs = pre ? pre->rng : J.rng[i];
-        const float var = S.var;
-        const float3 g = gauss3(rs);
-        J.rng[i] = rs;
+        uint4 rs = pre ? make_uint4(0, 0, 0, 0) : J.rng[i];
+        const float3 g = pre ? pre->g : gauss3(rs);
+        if (!pre) J.rng[i] = rs;
         J.rforce[i] = make_float4(g.x * var, g.y * var, g.z * var, 0.0f);
         if (J.flags & JF_PULLING) ext_rules_flag(J, i, pre ? pre->flag : (int)J.bflag[i], fx, fy, fz);
         J.mforce[i] = make_float4(fx, fy, fz, 0.0f);
@@ -365,10 +359,9 @@ __device__ __forceinline__ void step_tail(const DevJob& J, const DevJobState& S,
     }
     // Langevin step (langevin_kernel.cu:24-56)
     if (!(J.flags & JF_MINIMIZATION)) {
-        uint4 rs = pre ? pre->rng : J.rng[i];
-        const float var = S.var;
-        const float3 g = gauss3(rs);
-        J.rng[i] = rs;
+        uint4 rs = pre ? make_uint4(0, 0, 0, 0) : J.rng[i];
+        const float3 g = pre ? pre->g : gauss3(rs);
+        if (!pre) J.rng[i] = rs;
         fx += g.x * var;
         fy += g.y * var;
         fz += g.z * var;
@@ -409,7 +402,7 @@ __device__ __forceinline__ void step_bead(const DevJob& J, const DevJobState& S,
     else
         pair_loop<PB, int, TAILB>(gmem(static_cast<const int*>(J.pair_j)) + r, np, J.pair_ld, cin, c, J.rc2, J.a2,
                                   J.m6, fx, fy, fz);
-    step_tail<FO>(J, S, s, i, c, fx, fy, fz, cout);
+    step_tail<FO>(J, S, S.var, s, i, c, fx, fy, fz, cout);
 }
 
 // FO: forces only, into fout (bead-indexed), for every job of the tiles
@@ -482,208 +475,326 @@ __global__ __launch_bounds__(1024, PB <= 6 ? 8 : 4) void k_step_lds(const DevJob
     }
 }
 
-// The step with each bead's force terms spread over a workgroup, for jobs
-// whose rows are too few to fill the GPU one row per lane (a single chain of
-// a thousand beads fills 16 wavefronts).  One 1024-thread workgroup steps R
-// Verlet rows of an LDS-step job, with the job's coordinates staged in LDS.
-// A row's terms form one stream in the order the one-lane step adds them:
-// FENE (nc), native (nn), then the Verlet entries (np).  Thirteen
-// wavefronts evaluate the stream in chunks of kSplitK(R) positions (a lane
-// per row and position, 64 / R positions of R rows per wavefront), each
-// term written to LDS as its three components (-0.0 where a pair lies
-// beyond the cut-off or the row has no term at that position: x + (-0.0)
-// is x for every float x).  Three owner wavefronts, one per component, add
-// a chunk's terms in stream order while the next chunk is evaluated
-// (double buffer), starting from the extra force record.  The sums are the
-// one-lane step's sums, rounded the same way term by term, so the step is
-// bit-identical to k_step_lds.  Wavefront 0 then runs the walls, noise and
-// update for the R rows.
-constexpr int kSplitOwners = 3;
-constexpr int kSplitWorkers = 16 - kSplitOwners;
+// The step with each bead's force terms spread over a wavefront, for launches
+// whose rows, one per lane, would leave most of the GPU idle or the lanes
+// walking their ~150 terms at the latency of one gather after another.
+// A wavefront steps R Verlet rows: lane q + R p evaluates, of row q, the terms
+// at positions p, p + P, p + 2P ... (P = 64 / R) of a chunk of K = P U terms
+// and writes their three components to the wavefront's own LDS rows; lanes
+// p < 3 then add component p of row q in stream order -- FENE, native, the
+// Verlet entries -- while the next chunk's partners are on their way.
+// Positions without a term hold -0.0 (x + (-0.0) is x for every float x), so
+// the sums are the one-lane step's, rounded term by term, and the step is
+// bit-identical.  Nothing is shared between wavefronts: no barrier, and a
+// launch of any number of rows.  Partners are gathered from global memory
+// (the coordinates of a job stay in L1/L2), so jobs on either side of the
+// LDS limit are stepped by the same launch.  Bound by the latency of its
+// dependent reads (tile, record, lists, partners) where rows are few, by VALU
+// issue from about 30,000 rows on; measured at Engine::effective_shape (18,000
+// beads: 58 us one bead per lane, 16 us here).
 template <int R>
-constexpr int split_k() { return kSplitWorkers * (64 / R); }
-// row stride of the term buffers: K, or K + 4 where K / 4 is even, so that
-// the owners' 16-byte reads of R rows fall in distinct bank groups
-template <int R>
-constexpr int split_kp() { return (split_k<R>() / 4) % 2 ? split_k<R>() : split_k<R>() + 4; }
+struct RowsShape {
+    static constexpr int P = 64 / R;              // positions of a row evaluated at a time
+    static constexpr int U = R <= 4 ? 4 : 8;      // terms per lane and chunk
+    static constexpr int K = P * U;               // terms of a row per chunk
+    // row stride of the LDS rows: the R rows' P consecutive words (writes) and
+    // 16-byte reads fall in distinct banks
+    static constexpr int KP = K + 64 / R;
+};
 
-// Term p of the stream of Verlet row r (bead i, nc + nn + np terms), in two
-// parts so that the list reads of a chunk go out ahead of its evaluation:
-// split_fetch reads the partner and the pair's parameters (type 0 FENE with
-// par.x = r0, 1 native, 2 repulsive, 3 no term), split_eval gathers the
-// partner from the staged coordinates and forms (tx, ty, tz), -0.0 each where
-// nothing is added.
-struct SplitSrc {
+// p[off bytes on] in global memory: base in scalar registers, a 32-bit offset
+// per lane.
+template <typename T>
+__device__ __forceinline__ T ldg_off(const T* p, unsigned off) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) T*>(
+        reinterpret_cast<const __attribute__((address_space(1))) char*>(gmem(p)) + off);
+}
+// Coordinates of bead j (jobs hold far fewer than 2^28 beads).
+__device__ __forceinline__ float4 ldg_coord(const float4* p, int j) {
+    const f32x4_g v = ldg_off(reinterpret_cast<const f32x4_g*>(p), (unsigned)j << 4);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// A FENE (type 0, par.x = r0) or native (type 1) term of a row, fetched ahead
+// of its evaluation; type 3: no term at this position.
+struct BondedSrc {
     int j, type;
     float2 par;
 };
-__device__ __forceinline__ SplitSrc split_fetch(const DevJob& J, int p, int r, int i, int nc, int nn, int np) {
-    SplitSrc f;
-    f.j = 0;
+// Term t of the bonded stream (nc FENE, then nn native) of column col of the
+// job's bonded lists; i: the row's bead (a partner for positions without a term).
+template <typename IdxT>
+__device__ __forceinline__ BondedSrc bonded_fetch(const StepDesc& D, int t, int col, int i, int nc, int nn) {
+    BondedSrc f;
+    f.j = i;
     f.type = 3;
     f.par = make_float2(0.0f, 0.0f);
-    if (p < nc) {
+    if (t < nc) {
+        const size_t e = (size_t)t * D.b_ld + col;
         f.type = 0;
-        if (J.sort_rows) {
-            f.j = gmem(J.rb_cov_j)[(size_t)p * J.pair_ld + r];
-            f.par.x = gmem(J.rb_cov_r0)[(size_t)p * J.pair_ld + r];
-        } else {
-            f.j = J.nat_j16 ? (int)gmem(J.cov_j16)[(size_t)p * J.n + i] : gmem(J.cov_j)[(size_t)p * J.n + i];
-            f.par.x = gmem(J.cov_r0)[(size_t)p * J.n + i];
-        }
-    } else if (p < nc + nn) {
-        const int k = p - nc;
+        f.j = (int)gmem(static_cast<const IdxT*>(D.cov_j))[e];
+        f.par.x = gmem(D.cov_r0)[e];
+    } else if (t < nc + nn) {
+        const size_t e = (size_t)(t - nc) * D.b_ld + col;
         f.type = 1;
-        if (J.sort_rows) {
-            f.j = gmem(J.rb_nat_j)[(size_t)k * J.pair_ld + r];
-            f.par = J.rb_nat_par[(size_t)k * J.pair_ld + r];
-        } else {
-            f.j = J.nat_j16 ? (int)gmem(J.nat_j16)[(size_t)k * J.n + i] : gmem(J.nat_j)[(size_t)k * J.n + i];
-            f.par = J.nat_par[(size_t)k * J.n + i];
-        }
-    } else if (p < nc + nn + np) {
-        const size_t e = (size_t)(p - nc - nn) * J.pair_ld + r;
-        f.type = 2;
-        f.j = J.idx16 ? (int)__builtin_nontemporal_load(gmem(static_cast<const unsigned short*>(J.pair_j)) + e)
-                      : __builtin_nontemporal_load(gmem(static_cast<const int*>(J.pair_j)) + e);
+        f.j = (int)gmem(static_cast<const IdxT*>(D.nat_j))[e];
+        f.par = ldg2(D.nat_par, e);
     }
     return f;
 }
-template <typename CP>
-__device__ __forceinline__ void split_eval(const DevJob& J, const SplitSrc& f, CP cin, const float4 c, bool fast,
-                                           float& tx, float& ty, float& tz) {
-    tx = -0.0f, ty = -0.0f, tz = -0.0f;
-    if (f.type == 3) return;
-    const float4 o = cin[f.j];
-    const float x = o.x - c.x, y = o.y - c.y, z = o.z - c.z;
-    if (f.type == 0) {
-        const float w = fene_w(J.ks, J.R2, x, y, z, f.par.x);
-        tx = w * x;
-        ty = w * y;
-        tz = w * z;
-    } else if (f.type == 1) {
-        const float q = native_q(x, y, z, f.par);
-        tx = x * q;
-        ty = y * q;
-        tz = z * q;
-    } else {
-        const float d2 = x * x + y * y + z * z;
-        if (d2 < J.rc2) {
-            const float q = pair_q(d2, J.a2, J.m6, fast);
-            tx = x * q;
-            ty = y * q;
-            tz = z * q;
+
+// Orders a wavefront's LDS writes before its own reads of other lanes' words
+// (and those before the next writes): the LDS executes a wavefront's
+// operations in order, so only the compiler has to be held.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Adds the first m positions (up to the next multiple of 4) of a row's LDS
+// words to acc, in order; 32 at a time with their reads in flight together.
+__device__ __forceinline__ void rows_add(const float* __restrict__ t, int m, float& acc) {
+    const float4* __restrict__ t4 = reinterpret_cast<const float4*>(t);
+    for (; m > 28; m -= 32, t4 += 8) {
+        float4 v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = t4[k];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            acc += v[k].x;
+            acc += v[k].y;
+            acc += v[k].z;
+            acc += v[k].w;
         }
+    }
+    for (; m > 0; m -= 4, ++t4) {
+        const float4 v = *t4;
+        acc += v.x;
+        acc += v.y;
+        acc += v.z;
+        acc += v.w;
     }
 }
 
-// Grid: ntiles * (64 / R) workgroups; workgroup b steps rows
-// 64 * tile + R * (b % (64 / R)) .. + R - 1 of tile b / (64 / R) when the
-// tile's job is an LDS-step job (G: a job above the LDS limit, whose
-// partners are gathered from global memory, L2-resident; the other jobs are
-// stepped by the other kernels).  Every lane works for row lane % R: it
-// reads that row's bead and counts itself, and a worker reads its first two
-// chunks' list entries, while the coordinates are staged; wavefront 0 also
-// reads the extra force record and the state its tail needs.
-template <bool FO, int R, bool G>
-__global__ __launch_bounds__(1024) void k_step_split(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
-                                                     const int2* __restrict__ tiles, int ntiles, int kstep,
-                                                     float4* __restrict__ fout) {
-    constexpr int K = split_k<R>(), KP = split_kp<R>(), S = 64 / R;
-    extern __shared__ float4 lds_coord[];
-    __shared__ __align__(16) float term[2][3][R][KP];
-    __shared__ float fsum[3][R];
-    const int tile = blockIdx.x / S;
-    if (tile >= ntiles) return;
-    const int2 td = tiles[tile];
-    const DevJob& J = jobs[td.x];
-    if (G ? J.lds_step : !J.lds_step) return;
-    const long long s = st[td.x].step + kstep;
-    if (!FO && s >= J.end_step) return;
-    const int n = J.n;
-    const int row0 = td.y + R * (blockIdx.x % S);
-    if (row0 >= n) return;  // every exit above is uniform over the workgroup
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    if constexpr (!G) {
-        const float4* __restrict__ g = J.coord[s & 1];
-        for (int k = tid; k < n; k += 1024) lds_coord[k] = g[k];
+// The rows of k_step_rows: R rows of one job by one wavefront, lists of IdxT.
+template <bool FO, int R, typename IdxT>
+__device__ __forceinline__ void step_rows(const StepDesc& D, const DevJobState& S, float var, long long s, int row0,
+                                          float (*term)[R][RowsShape<R>::KP], float4* __restrict__ fout) {
+    constexpr int P = RowsShape<R>::P, U = RowsShape<R>::U, K = RowsShape<R>::K;
+    const int lane = threadIdx.x & 63;
+    const int n = D.n;
+    const float4* const cin = (s & 1) ? D.coord[1] : D.coord[0];
+    // this lane's row (loads from the job's last row where the tile ends
+    // early; such lanes have no terms)
+    const int q = lane % R, p = lane / R, r = row0 + q, rc = min(r, n - 1);
+    // the first chunk's Verlet entries, before the counts are known: slots
+    // of the list whether filled or not (the unfilled are not used)
+    const IdxT* const pj = static_cast<const IdxT*>(D.pair_j);
+    const size_t ld = D.pair_ld;
+    const unsigned off = ((unsigned)p * (unsigned)D.pair_ld + (unsigned)rc) * (unsigned)sizeof(IdxT);
+    IdxT jn[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int k = min(u * P + p, D.pair_cap - 1);
+        jn[u] = gmem(pj)[(size_t)k * ld + rc];
     }
-    const float4* __restrict__ cin = G ? J.coord[s & 1] : lds_coord;
-    const bool owner = w < kSplitOwners;
-    // this lane's row (loads from a clamped row where the tile ends early)
-    const int q = lane % R, r = row0 + q, rc = min(r, n - 1);
-    const int i = gmem(J.perm)[rc];
+    int np = gmem(D.pair_cnt)[rc];
+    int i = rc;
+    if (D.perm) i = gmem(D.perm)[rc];
     int nc, nn;
-    if (J.sort_rows) {
-        const int cnt = gmem(J.rb_cnt)[rc];
+    if (D.b_cnt) {
+        const int cnt = gmem(D.b_cnt)[rc];
         nc = cnt & 0xffff;
         nn = cnt >> 16;
     } else {
-        nc = gmem(J.cov_cnt)[i];
-        nn = gmem(J.nat_cnt)[i];
+        nc = gmem(D.cov_cnt)[i];
+        nn = gmem(D.nat_cnt)[i];
     }
-    const int np = gmem(J.pair_cnt)[rc];
-    const int len = r < n ? nc + nn + np : 0;
-    // the longest row: lanes 0 .. R-1 of each wavefront hold every row
-    int lmax = len;
-#pragma unroll
-    for (int o = R / 2; o > 0; o >>= 1) lmax = max(lmax, __shfl_xor(lmax, o));
-    lmax = __shfl(lmax, 0);
-    const int nch = (lmax + K - 1) / K;
-    // a worker evaluates position pos of every chunk
-    const int pos = (w - kSplitOwners) * S + lane / R;
-    SplitSrc f0, f1;
-    if (!owner) {
-        f0 = split_fetch(J, pos < len ? pos : INT_MAX, r, i, nc, nn, np);
-        f1 = split_fetch(J, K + pos < len ? K + pos : INT_MAX, r, i, nc, nn, np);
+    const int col = D.b_cnt ? rc : i;
+    const float4 c = ldg_coord(cin, i);
+    const bool noise = !FO && !(D.flags & JF_MINIMIZATION);
+    TailPre pre;
+    uint4 rng = make_uint4(0, 0, 0, 0);
+    if constexpr (!FO) {
+        rng = D.rng[i];
+        pre.T = gmem(D.T)[i];
+        pre.flag = 0;
+        if (D.flags & JF_PULLING) pre.flag = (int)gmem(D.bflag)[i];
     }
     float acc = 0.0f;
-    TailPre pre;
-    if (owner && lane < R && r < n) {
-        if (J.flags & JF_EXTRA_FORCE) {
-            const float4 e = J.fextra[i];
-            acc = w == 0 ? e.x : w == 1 ? e.y : e.z;
+    if (D.flags & JF_EXTRA_FORCE) {
+        float4 e = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (p == 0 && r < n) {
+            e = D.fextra[i];
+            if constexpr (!FO) D.fextra[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
-        if (w == 0 && !FO) pre = tail_prefetch(J, i);
+        const float ex = __shfl(e.x, q), ey = __shfl(e.y, q), ez = __shfl(e.z, q);
+        acc = p == 0 ? ex : p == 1 ? ey : ez;
     }
-    __syncthreads();  // coordinates staged; extra forces read by all three owners
-    if constexpr (!FO) {
-        if (w == 0 && lane < R && r < n && (J.flags & JF_EXTRA_FORCE))
-            J.fextra[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (r >= n) nc = nn = np = 0;
+    int nbm = nc + nn, npm = np;  // the longest rows (every set of R lanes holds all rows)
+#pragma unroll
+    for (int o = R / 2; o > 0; o >>= 1) {
+        nbm = max(nbm, __shfl_xor(nbm, o));
+        npm = max(npm, __shfl_xor(npm, o));
     }
-    const bool fast = div_fast_numerator(J.a2) && J.rc2 <= kDivFastMaxB;
-    const float4 c = cin[i];
-    for (int ch = 0; ch <= nch; ++ch) {
-        if (!owner && ch < nch) {
-            float tx, ty, tz;
-            split_eval(J, f0, cin, c, fast, tx, ty, tz);
-            f0 = f1;
-            const int p = (ch + 2) * K + pos;
-            if (ch + 2 < nch) f1 = split_fetch(J, p < len ? p : INT_MAX, r, i, nc, nn, np);
-            term[ch & 1][0][q][pos] = tx;
-            term[ch & 1][1][q][pos] = ty;
-            term[ch & 1][2][q][pos] = tz;
-        }
-        if (owner && ch > 0 && lane < R) {
-            // chunk ch - 1 in stream order; positions up to the next multiple
-            // of 4 past the longest row hold -0.0
-            const float* __restrict__ t = &term[(ch - 1) & 1][w][lane][0];
-            const int m = min(K, lmax - (ch - 1) * K);
-            for (int k = 0; k < m; k += 4) {
-                const float4 v = *reinterpret_cast<const float4*>(t + k);
-                acc += v.x;
-                acc += v.y;
-                acc += v.z;
-                acc += v.w;
+    nbm = __builtin_amdgcn_readfirstlane(nbm);
+    npm = __builtin_amdgcn_readfirstlane(npm);
+    // partners of the first chunk of pairs, the entries of the second, and
+    // the first bonded terms: all on their way during the noise
+    // (loads without branches, so that each can be waited for by itself:
+    // positions without an entry read slot min(.., npm - 1) of the job's first
+    // row and gather the row's own bead)
+    float4 o[U];
+    auto gather = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) o[u] = ldg_coord(cin, b + u * P + p < np ? (int)jn[u] : i);
+    };
+    auto fetch = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            jn[u] = ldg_off(pj + (size_t)min(b + u * P, npm - 1) * ld, b + u * P + p < np ? off : 0u);
+    };
+    constexpr int UB = R <= 4 ? 1 : R / 4;  // bonded terms per lane and chunk: 16 of a row (32 for R = 2)
+    BondedSrc f[UB];
+    auto bonded = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < UB; ++u)
+            if (b + u * P < nbm) f[u] = bonded_fetch<IdxT>(D, b + u * P + p, col, i, nc, nn);
+    };
+    bonded(0);
+    if (npm > 0) gather(0);
+    if (npm > K) fetch(K);
+    // lanes p = 0 and 1 draw the step's four numbers and form one Box-Muller
+    // pair each (gauss3's order; the second's cosine is not used)
+    if (noise) {
+        const uint32_t u0 = hybrid_taus(rng);
+        const uint32_t u1 = hybrid_taus(rng);
+        const uint32_t u2 = hybrid_taus(rng);
+        const uint32_t u3 = hybrid_taus(rng);
+        if (p == 0 && r < n) D.rng[i] = rng;
+        float sn, cs;
+        const float rr = sqrtf(-2.0f * logf_series(uint_to_unit(p == 0 ? u0 : u2)));
+        const float th = (float)(6.283185307179586 * (double)uint_to_unit(p == 0 ? u1 : u3));
+        sincosf_series(th, sn, cs);
+        const float gs = rr * sn;
+        pre.g = make_float3(gs, rr * cs, __shfl(gs, (lane + R) & 63));
+    }
+    // FENE and native terms
+    for (int b = 0; b < nbm; b += P * UB) {
+        if (b > 0) bonded(b);
+#pragma unroll
+        for (int u = 0; u < UB; ++u)
+            if (b + u * P < nbm) {
+                const float4 w = ldg_coord(cin, f[u].j);
+                const float x = w.x - c.x, y = w.y - c.y, z = w.z - c.z;
+                float tx = -0.0f, ty = -0.0f, tz = -0.0f;
+                if (f[u].type == 0) {
+                    const float v = fene_w(D.ks, D.R2, x, y, z, f[u].par.x);
+                    tx = v * x;
+                    ty = v * y;
+                    tz = v * z;
+                } else if (f[u].type == 1) {
+                    const float v = native_q(x, y, z, f[u].par);
+                    tx = x * v;
+                    ty = y * v;
+                    tz = z * v;
+                }
+                term[0][q][u * P + p] = tx;
+                term[1][q][u * P + p] = ty;
+                term[2][q][u * P + p] = tz;
+            }
+        wave_lds_order();
+        if (p < 3) rows_add(&term[p][q][0], min(P * UB, nbm - b), acc);
+        wave_lds_order();
+    }
+    // repulsive pairs: the next chunk's partners and the entries of the one
+    // after it are in flight while a chunk is added
+    const float rc2 = D.rc2, a2 = D.a2, m6 = D.m6;
+    const bool fast = div_fast_numerator(a2) && rc2 <= kDivFastMaxB;
+    // term u of the chunk from b into LDS; its factor by the short division,
+    // or (SLOW) by whichever the divisor admits
+    auto put = [&](int u, bool ok, float x, float y, float z, float w) {
+        term[0][q][u * P + p] = ok ? x * w : -0.0f;
+        term[1][q][u * P + p] = ok ? y * w : -0.0f;
+        term[2][q][u * P + p] = ok ? z * w : -0.0f;
+    };
+    for (int b = 0; b < npm; b += K) {
+        // straight-line code over the chunk's terms, so that their latencies
+        // overlap; a divisor outside the short division's range (beads almost
+        // on top of each other) sends the chunk through the general one
+        bool bad = !fast;
+#pragma unroll
+        for (int h = 0; h < U; h += 4)
+            if (b + h * P < npm) {
+#pragma unroll
+                for (int u = h; u < h + 4; ++u) {
+                    const float x = o[u].x - c.x, y = o[u].y - c.y, z = o[u].z - c.z;
+                    const float d2 = x * x + y * y + z * z;
+                    const bool ok = (b + u * P + p < np) & (d2 < rc2);
+                    bad = bad | (ok & !(d2 >= kDivFastMinB));
+                    float w = div_rn_fast(a2, d2);
+                    w = w * w;
+                    put(u, ok, x, y, z, m6 * w * w);
+                }
+            }
+        if (__builtin_amdgcn_ballot_w64(bad)) {
+            for (int u = 0; u < U && b + u * P < npm; ++u) {
+                float4 w = o[0];  // the partner of term u (o is indexed by constants only)
+#pragma unroll
+                for (int v = 1; v < U; ++v)
+                    if (v == u) w = o[v];
+                const float x = w.x - c.x, y = w.y - c.y, z = w.z - c.z;
+                const float d2 = x * x + y * y + z * z;
+                const bool ok = (b + u * P + p < np) & (d2 < rc2);
+                put(u, ok, x, y, z, ok ? pair_q(d2, a2, m6, fast) : 0.0f);
             }
         }
-        __syncthreads();
+        if (b + K < npm) gather(b + K);
+        if (b + 2 * K < npm) fetch(b + 2 * K);
+        wave_lds_order();
+        if (p < 3) rows_add(&term[p][q][0], min(K, npm - b), acc);
+        wave_lds_order();
     }
-    if (owner && lane < R) fsum[w][lane] = acc;
-    __syncthreads();
-    if (w == 0 && lane < R && r < n)
-        step_tail<FO>(J, st[td.x], s, i, c, fsum[0][lane], fsum[1][lane], fsum[2][lane],
-                      FO ? fout : J.coord[(s + 1) & 1], FO ? nullptr : &pre);
+    const float fy = __shfl(acc, (lane + R) & 63), fz = __shfl(acc, (lane + 2 * R) & 63);
+    if (p == 0 && r < n) {
+        float4* const cout = FO ? fout : (s & 1) ? D.coord[0] : D.coord[1];
+        step_tail<FO>(D, S, var, s, i, c, acc, fy, fz, cout, FO ? nullptr : &pre);
+    }
+}
+
+// Grid: one wavefront per R rows, four per workgroup; workgroups of one XCD
+// take consecutive tiles.  classes: 1 the LDS-step jobs, 2 the others.  FO:
+// forces only, into fout.
+template <bool FO, int R>
+__global__ __launch_bounds__(256, 4) void k_step_rows(const StepDesc* __restrict__ descs,
+                                                      const DevJobState* __restrict__ st,
+                                                      const int2* __restrict__ tiles, int ntiles, int kstep,
+                                                      int classes, float4* __restrict__ fout) {
+    constexpr int P = RowsShape<R>::P;
+    __shared__ __align__(16) float terms[4][3][R][RowsShape<R>::KP];
+    const int w = wave_id();
+    const int nb = gridDim.x, nxcd = nb >= 8 ? 8 : 1;  // the grid is a multiple of 8 from 8 on
+    const int gw = ((blockIdx.x % nxcd) * (nb / nxcd) + blockIdx.x / nxcd) * 4 + w;
+    const int tile = gw / P;
+    if (tile >= ntiles) return;
+    const int2 td = tiles[tile];
+    const StepDesc D = descs[td.x];
+    const long long step0 = st[td.x].step;
+    const float var = st[td.x].var;
+    // the record's loads are all issued here, not each at its first use
+    asm volatile("" ::"s"(D.coord[0]), "s"(D.coord[1]), "s"(D.perm), "s"(D.pair_cnt), "s"(D.pair_j), "s"(D.b_cnt),
+                 "s"(D.cov_j), "s"(D.cov_r0), "s"(D.nat_j), "s"(D.nat_par), "s"(D.rng), "s"(D.T), "s"(D.bflag));
+    asm volatile("" ::"s"(D.flags), "s"(D.a2), "s"(D.hOverZeta), "s"(D.nav), "s"(D.end_step), "s"(step0), "s"(var));
+    if (!(classes & (D.lds_step ? 1 : 2))) return;
+    const long long s = step0 + kstep;
+    if (!FO && s >= D.end_step) return;
+    const int row0 = td.y + R * (gw % P);
+    if (row0 >= D.n) return;
+    if (D.idx16)
+        step_rows<FO, R, unsigned short>(D, st[td.x], var, s, row0, terms[w], fout);
+    else
+        step_rows<FO, R, int>(D, st[td.x], var, s, row0, terms[w], fout);
 }
 
 // ---------------------------------------------------------------------------
@@ -1816,34 +1927,36 @@ static int grid_for(int ntiles, int max_blocks) {
     return b < 1 ? 1 : b;
 }
 
-// k_step_split over every tile (its workgroups of other jobs exit at once);
-// G: the jobs above the LDS limit, gathering from global memory.
-template <bool FO, bool G>
-static void launch_split(int R, const DevJob* jobs, const DevJobState* st, const int2* tiles, int ntiles,
-                         int lds_beads, int kstep, float4* out, hipStream_t stream) {
-    const size_t lds = G ? 0 : (size_t)lds_beads * sizeof(float4);
-    if (R == 4)
-        hipLaunchKernelGGL((k_step_split<FO, 4, G>), dim3(ntiles * 16), dim3(1024), lds, stream, jobs, st, tiles,
-                           ntiles, kstep, out);
+// k_step_rows over every tile for the job classes given (1 LDS-step jobs, 2
+// the others), R rows per wavefront.
+template <bool FO>
+static void launch_rows(int R, int classes, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles,
+                        int kstep, float4* out, hipStream_t stream) {
+    int blocks = (ntiles * (64 / R) + 3) / 4;
+    if (blocks >= 8) blocks = (blocks + 7) / 8 * 8;
+    const dim3 g(blocks), b(256);
+    if (R == 2)
+        hipLaunchKernelGGL((k_step_rows<FO, 2>), g, b, 0, stream, descs, st, tiles, ntiles, kstep, classes, out);
+    else if (R == 4)
+        hipLaunchKernelGGL((k_step_rows<FO, 4>), g, b, 0, stream, descs, st, tiles, ntiles, kstep, classes, out);
     else if (R == 8)
-        hipLaunchKernelGGL((k_step_split<FO, 8, G>), dim3(ntiles * 8), dim3(1024), lds, stream, jobs, st, tiles,
-                           ntiles, kstep, out);
+        hipLaunchKernelGGL((k_step_rows<FO, 8>), g, b, 0, stream, descs, st, tiles, ntiles, kstep, classes, out);
     else
-        hipLaunchKernelGGL((k_step_split<FO, 16, G>), dim3(ntiles * 4), dim3(1024), lds, stream, jobs, st, tiles,
-                           ntiles, kstep, out);
+        hipLaunchKernelGGL((k_step_rows<FO, 16>), g, b, 0, stream, descs, st, tiles, ntiles, kstep, classes, out);
 }
 
-hipError_t launch_step(const DevJob* jobs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
+hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
                        const int2* units, const int4* segs, int nunits, int lds_beads, int kstep, int max_blocks,
                        hipStream_t stream, const StepShape& shape) {
     if (ntiles <= 0) return hipSuccess;
-    if (any_global && shape.split_global)
-        launch_split<false, true>(shape.split_global, jobs, st, tiles, ntiles, 0, kstep, nullptr, stream);
+    const int rl = nunits > 0 ? shape.split_rows : 0, rg = any_global ? shape.split_global : 0;
+    if (rg)  // with the LDS-step jobs where both classes take the same shape
+        launch_rows<false>(rg, rl == rg ? 3 : 2, descs, st, tiles, ntiles, kstep, nullptr, stream);
     else if (any_global)
         hipLaunchKernelGGL(k_step<false>, dim3(grid_for(ntiles, max_blocks)), dim3(256), 0, stream, jobs, st, tiles,
                            ntiles, kstep, nullptr);
-    if (nunits > 0 && shape.split_rows) {
-        launch_split<false, false>(shape.split_rows, jobs, st, tiles, ntiles, lds_beads, kstep, nullptr, stream);
+    if (rl) {
+        if (rl != rg) launch_rows<false>(rl, 1, descs, st, tiles, ntiles, kstep, nullptr, stream);
     } else if (nunits > 0) {
         const dim3 g(nunits), b(shape.unit_rows);
         const size_t lds = (size_t)lds_beads * sizeof(float4);
@@ -1857,17 +1970,17 @@ hipError_t launch_step(const DevJob* jobs, const DevJobState* st, const int2* ti
     return hipGetLastError();
 }
 
-hipError_t launch_forces(const DevJob* jobs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
+hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
                          const int2* units, const int4* segs, int nunits, int lds_beads, float4* out,
                          hipStream_t stream, const StepShape& shape) {
     if (ntiles <= 0) return hipSuccess;
     if (any_global && shape.split_global)
-        launch_split<true, true>(shape.split_global, jobs, st, tiles, ntiles, 0, 0, out, stream);
+        launch_rows<true>(shape.split_global, 2, descs, st, tiles, ntiles, 0, out, stream);
     else if (any_global)
         hipLaunchKernelGGL(k_step<true>, dim3(grid_for(ntiles, 0)), dim3(256), 0, stream, jobs, st, tiles, ntiles, 0,
                            out);
     if (nunits > 0 && shape.split_rows)
-        launch_split<true, false>(shape.split_rows, jobs, st, tiles, ntiles, lds_beads, 0, out, stream);
+        launch_rows<true>(shape.split_rows, 1, descs, st, tiles, ntiles, 0, out, stream);
     else if (nunits > 0)
         hipLaunchKernelGGL((k_step_lds<true, 6>), dim3(nunits), dim3(kLdsUnit), (size_t)lds_beads * sizeof(float4),
                            stream, jobs, st, units, segs, nunits, 0, out);
