@@ -48,6 +48,26 @@ __device__ __forceinline__ float div_rn_fast(float a, float b) {
     const float q = a * y;
     return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
+// RN(1/b) as div_rn_fast forms it, and RN(a/b) from it, for several quotients
+// with one divisor.
+__device__ __forceinline__ float recip_rn_fast(float b) {
+    const float y0 = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y0, 1.0f), y0, y0);
+}
+__device__ __forceinline__ float quot_rn_fast(float a, float b, float y) {
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+// sqrt(x) correctly rounded for x in [kDivFastMinB, kDivFastMaxB]: the
+// hardware estimate of 1/sqrt(x) times x, and one Newton step whose residual
+// is formed in an FMA (x from 2^-100 on keeps it clear of underflow).  That
+// this rounds correctly for every such x is a property of the hardware
+// estimate, checked over all of them by sop_check_division.
+__device__ __forceinline__ float sqrt_rn_fast(float x) {
+    const float r = __builtin_amdgcn_rsqf(x);
+    const float g = x * r;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * r, g);
+}
 // The IEEE division, kept on its own rare branch: the divisor passes
 // through an empty asm, so the compiler cannot compute the quotient ahead of
 // the branch for every lane.
@@ -58,6 +78,14 @@ __device__ __forceinline__ float div_ieee(float a, float b) {
 // a can take the fast division (a wave-uniform test, made once per bead).
 __device__ __forceinline__ bool div_fast_numerator(float a) {
     return a == 0.0f || (a >= kDivFastMinA && a <= kDivFastMaxA);
+}
+
+// Orders a wavefront's LDS writes before its own reads of other lanes' words
+// (and those before the next writes): the LDS executes a wavefront's
+// operations in order, so only the compiler has to be held.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // Mantissa bits into [1,2), minus one; an exact zero becomes 1e-8.

@@ -113,6 +113,44 @@ __device__ __forceinline__ float4 unit_sep(const float4 a, const float4 b) {
     return dr;
 }
 
+// rpy(unit_sep(..)) for the separation (x, y, z) of squared length d2, in
+// about half the operations, where pair_short_ok holds: every quotient and the
+// square root correctly rounded by the short sequences (one reciprocal per
+// divisor; 2/ra is twice the rounded 1/ra), so the same bits.  ya = RN(1/a).
+// The close form (ra <= 2) is evaluated only where some lane needs it.
+__device__ __forceinline__ bool pair_short_ok(float x, float y, float z, float d2) {
+    return (fminf(fminf(fabsf(x), fabsf(y)), fabsf(z)) >= 0x1p-32f) & (d2 <= kDivFastMaxB);
+}
+// a: w / a stays within the short division's range for every w = sqrt(d2) above
+__device__ __forceinline__ bool pair_short_radius(float a) { return a >= 0x1p-20f && a <= 0x1p20f; }
+__device__ __forceinline__ F6 rpy_short(float x, float y, float z, float d2, float a, float ya) {
+    constexpr float two_thirds = 2.f / 3.f;
+    const float w = sqrt_rn_fast(d2);
+    const float yw = recip_rn_fast(w);
+    x = quot_rn_fast(x, w, yw);
+    y = quot_rn_fast(y, w, yw);
+    z = quot_rn_fast(z, w, yw);
+    const float ra = quot_rn_fast(w, a, ya);
+    const float yr = recip_rn_fast(ra);
+    const float q0 = quot_rn_fast(0.75f, ra, yr), q2 = quot_rn_fast(2.f * yr, ra, yr);
+    const float q4 = quot_rn_fast(quot_rn_fast(two_thirds, ra, yr), ra, yr);
+    float crr = q0 * (1.f - q2);
+    float cii = q0 * (1.f + q4);
+    if (__builtin_amdgcn_ballot_w64(!(ra > 2.f))) {
+        asm volatile("");  // a branch, not a select: few chunks hold a close pair
+        crr = ra > 2.f ? crr : 3.f * ra / 32.f;
+        cii = ra > 2.f ? cii : 1.f - 9.f * ra / 32.f;
+    }
+    F6 d;
+    d.xx = x * x * crr + cii;
+    d.xy = x * y * crr;
+    d.xz = x * z * crr;
+    d.yy = y * y * crr + cii;
+    d.yz = y * z * crr;
+    d.zz = z * z * crr + cii;
+    return d;
+}
+
 __device__ __forceinline__ int wave_of() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 // tile loop shared with kernels.hip's layout (64-bead tiles, 4 per block)
@@ -153,44 +191,89 @@ __device__ __forceinline__ void eps_add(const float4 c1, const float4 c2, float 
     sum.w += p.w;
 }
 
-// The all-pairs HI sums (epsilon, TEA step, exact D.F) run kHiSplit
-// 1024-thread workgroups per 64-bead tile, 16 beads each, so that one job
-// of a few thousand beads fills the chip.
-constexpr int kHiSplit = 4;
+// The all-pairs HI sums (epsilon, TEA step, exact D.F): workgroups of B beads,
+// B wavefronts, 64 / B workgroups per 64-bead tile, taking the partners in
+// chunks of C.  hi_config chooses (B, C) by the beads of the launch.  Measured
+// on TEA runs, us per step of the whole run, with (4, 256) / (8, 256) /
+// (16, 256) / (8, 128):
+//   4,096 beads of one chain          72 / 68 / 66 / 70
+//   9,558 beads of nine chains        58 / 56 / 71 / 51
+// One workgroup per CU (16 wavefronts hide the latencies): the largest B that
+// still gives every CU one, 256 partners between barriers.  More beads than 16
+// per CU: small workgroups, several on a CU, whose last round leaves less of
+// the chip idle.
+struct HiConfig {
+    int beads, chunk;
+};
+static HiConfig hi_config(long long beads) {
+    constexpr int kCus = 256;
+    if (beads <= 4 * kCus) return {4, 256};
+    if (beads <= 8 * kCus) return {8, 256};
+    if (beads <= 16 * kCus) return {16, 256};
+    return {8, 128};
+}
 
-// Ordered all-pairs sums of a workgroup's 16 beads.  Wavefront w owns bead
-// dbase + w: for each chunk of kHiChunk partners its lanes form the NC
-// components of the (bead, partner) terms -- partner j = base + lane + 64u
-// -- into an LDS buffer, and after the chunk's barrier lanes 16c + b of
-// wavefront 0 add component c of bead dbase + b in partner order, four
-// terms per LDS read, while the other wavefronts already form the next
-// chunk into the second buffer.  Terms that the sequential loop skips (the
-// bead itself, partners past n) are -0.0f, which leaves every sum unchanged
-// (x + -0 = x for every x), so each sum is the same sequence of additions
-// as the reference's bead-by-bead loop.  `term(j, v)` fills the wavefront's
-// term for partner j; `acc` enters as the summing lane's starting value and
-// leaves as its sum.
-constexpr int kHiChunk = 256, kHiRow = kHiChunk + 4;
-template <int NC, typename Term>
-__device__ __forceinline__ void hi_ordered_sums(float (*buf)[NC][16][kHiRow], int n, Term term, float& acc) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int sc = lane >> 4, sb = lane & 15;
+// Ordered all-pairs sums of a workgroup's B beads.  Each chunk of C
+// partners: wavefront w forms the NC components of the terms of beads
+// dbase + 2 (w % (B/2)) and the next one with one half of the chunk (a partner
+// per lane, its data loaded once for both beads) into an LDS buffer, and
+// after the chunk's barrier lanes B c + b of wavefront 0 add component c of
+// bead dbase + b in partner order, four terms per LDS read, while the other
+// wavefronts already form the next chunk into the second buffer.  Terms that
+// the sequential loop skips (the bead itself, partners past n) are -0.0f,
+// which leaves every sum unchanged (x + -0 = x for every x), so each sum is
+// the same sequence of additions as the reference's bead-by-bead loop.
+// `acc` enters as the summing lane's starting value and leaves as its sum.
+// `pair` holds the two beads' data: pair.load(j) reads a partner's,
+// pair.sep(k, s, ..) its separation from bead k, pair.term(k, s, D, v) fills
+// the terms from the RPY block, and pair.general(k, s) gives the block where
+// the short evaluation is not admitted.
+// Bound by VALU issue: per pair about 90 instructions with the short square
+// root and shared reciprocals (150 before: the general square root, range
+// checks per quotient and a reciprocal per quotient).
+template <int B, int C, int NC, typename Pair>
+__device__ __forceinline__ void hi_ordered_sums(float (*buf)[NC][B][C + 4], int n, const int (&b)[2], Pair pair,
+                                                float& acc) {
+    const int lane = threadIdx.x & 63, w = wave_of();
+    const int sc = lane / B, sb = lane % B;
+    const int row = 2 * (w % (B / 2)), half = w / (B / 2);
+    const float a = pair.a, ya = 1.0f / a;
+    const bool radius = pair_short_radius(a);
     int c = 0;
-    for (int base = 0; base < n; base += kHiChunk, ++c) {
-        float(*tb)[16][kHiRow] = buf[c & 1];
+    for (int base = 0; base < n; base += C, ++c) {
+        float(*tb)[B][C + 4] = buf[c & 1];
 #pragma unroll
-        for (int u = 0; u < kHiChunk / 64; ++u) {
-            float v[NC];
-            term(base + lane + 64 * u, v);
+        for (int u = 0; u < C / 128; ++u) {
+            const int at = half * (C / 2) + 64 * u, j0 = base + at, j = j0 + lane;
+            const auto src = pair.load(min(j, n - 1));
 #pragma unroll
-            for (int k = 0; k < NC; ++k) tb[k][w][lane + 64 * u] = v[k];
+            for (int k = 0; k < 2; ++k) {
+                // the chunk's 64 partners hold the bead itself or pass n
+                const bool edge = j0 + 64 > n || (b[k] >= j0 && b[k] < j0 + 64);
+                const bool valid = j < n && j != b[k];
+                float x, y, z, v[NC];
+                pair.sep(k, src, x, y, z);
+                const float d2 = x * x + y * y + z * z;
+                const bool ok = radius & pair_short_ok(x, y, z, d2);
+                pair.term(k, src, rpy_short(x, y, z, d2, a, ya), v);
+                const bool bad = edge ? valid & !ok : !ok;
+                if (__builtin_amdgcn_ballot_w64(bad)) {
+                    if (bad) pair.term(k, src, pair.general(k, src), v);
+                }
+#pragma unroll
+                for (int q = 0; q < NC; ++q) tb[q][row + k][at + lane] = v[q];
+                if (edge && !valid) {
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) tb[q][row + k][at + lane] = -0.f;
+                }
+            }
         }
         __syncthreads();
         if (w == 0 && sc < NC) {
-            const float4* __restrict__ row = reinterpret_cast<const float4*>(&tb[sc][sb][0]);
+            const float4* __restrict__ r4 = reinterpret_cast<const float4*>(&tb[sc][sb][0]);
 #pragma unroll 8
-            for (int k = 0; k < kHiChunk / 4; ++k) {
-                const float4 q = row[k];
+            for (int k = 0; k < C / 4; ++k) {
+                const float4 q = r4[k];
                 acc += q.x;
                 acc += q.y;
                 acc += q.z;
@@ -200,32 +283,108 @@ __device__ __forceinline__ void hi_ordered_sums(float (*buf)[NC][16][kHiRow], in
     }
 }
 
+// The two beads (clamped to the last one) of wavefront w and their pairs.
+struct HiPairBase {
+    const float4* __restrict__ cur;
+    float4 c[2];
+    float a;
+    struct Src {
+        float4 r;
+    };
+    __device__ __forceinline__ void sep(int k, const float4 r, float& x, float& y, float& z) const {
+        x = r.x - c[k].x;
+        y = r.y - c[k].y;
+        z = r.z - c[k].z;
+    }
+};
+__device__ __forceinline__ float4 ld4(const float4* p, int j) {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    const v4 v = *reinterpret_cast<const __attribute__((address_space(1))) v4*>(
+        reinterpret_cast<const __attribute__((address_space(1))) char*>(
+            (const __attribute__((address_space(1))) float4*)p) +
+        ((unsigned)j << 4));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+// epsilon: the sums of the RPY block's squares and of its entries
+struct HiPairEps : HiPairBase {
+    __device__ __forceinline__ float4 load(int j) const { return ld4(cur, j); }
+    __device__ __forceinline__ F6 general(int k, const float4 r) const { return rpy(unit_sep(c[k], r), a); }
+    __device__ __forceinline__ void term(int, const float4, const F6 d, float (&v)[4]) const {
+        v[3] = d.xx + 2 * d.xy + 2 * d.xz + d.yy + 2 * d.yz + d.zz;
+        v[0] = d.xx * d.xx + d.xy * d.xy + d.xz * d.xz;
+        v[1] = d.xy * d.xy + d.yy * d.yy + d.yz * d.yz;
+        v[2] = d.xz * d.xz + d.yz * d.yz + d.zz * d.zz;
+    }
+};
+// D F of the exact path
+struct HiPairD : HiPairBase {
+    const float4* __restrict__ mforce;
+    struct Src {
+        float4 r, f;
+    };
+    __device__ __forceinline__ Src load(int j) const { return Src{ld4(cur, j), ld4(mforce, j)}; }
+    __device__ __forceinline__ void sep(int k, const Src& s, float& x, float& y, float& z) const {
+        HiPairBase::sep(k, s.r, x, y, z);
+    }
+    __device__ __forceinline__ F6 general(int k, const Src& s) const { return rpy(unit_sep(c[k], s.r), a); }
+    __device__ __forceinline__ void term(int, const Src& s, const F6 D, float (&v)[3]) const {
+        v[0] = D.xx * s.f.x + D.xy * s.f.y + D.xz * s.f.z;
+        v[1] = D.xy * s.f.x + D.yy * s.f.y + D.yz * s.f.z;
+        v[2] = D.xz * s.f.x + D.yz * s.f.y + D.zz * s.f.z;
+    }
+};
+// the TEA step: D (F_j + C_i rho_j)
+struct HiPairTea : HiPairBase {
+    const float4* __restrict__ mforce;
+    const float4* __restrict__ rforce;
+    float ci[2][3];
+    struct Src {
+        float4 r, f, g;
+    };
+    __device__ __forceinline__ Src load(int j) const { return Src{ld4(cur, j), ld4(mforce, j), ld4(rforce, j)}; }
+    __device__ __forceinline__ void sep(int k, const Src& s, float& x, float& y, float& z) const {
+        HiPairBase::sep(k, s.r, x, y, z);
+    }
+    __device__ __forceinline__ F6 general(int k, const Src& s) const { return rpy(unit_sep(c[k], s.r), a); }
+    __device__ __forceinline__ void term(int k, const Src& s, const F6 D, float (&v)[3]) const {
+        const float gx = s.f.x + s.g.x * ci[k][0], gy = s.f.y + s.g.y * ci[k][1], gz = s.f.z + s.g.z * ci[k][2];
+        v[0] = D.xx * gx + D.xy * gy + D.xz * gz;
+        v[1] = D.xy * gx + D.yy * gy + D.yz * gz;
+        v[2] = D.xz * gx + D.yz * gy + D.zz * gz;
+    }
+};
+// the beads of this wavefront, of the workgroup's B from dbase
+template <int B>
+__device__ __forceinline__ void hi_beads(int dbase, int n, int (&b)[2]) {
+    const int row = 2 * (wave_of() % (B / 2));
+    b[0] = min(dbase + row, n - 1);
+    b[1] = min(dbase + row + 1, n - 1);
+}
+
 // Per-bead sums of the TEA epsilon (bdhitea_kernel.cu:212-249): without
 // lists, the ordered chunk sums of hi_ordered_sums (the same bits as the
 // bead-by-bead loop); with lists, wavefront 0 of the tile's first
 // workgroup walks bead i's lists.
-__global__ __launch_bounds__(1024) void k_hi_eps(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
+template <int B, int C>
+__global__ __launch_bounds__(64 * B) void k_hi_eps(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
                                                  const int2* __restrict__ tiles, int ntiles) {
-    __shared__ __attribute__((aligned(16))) float eterm[2][4][16][kHiRow];
+    __shared__ __attribute__((aligned(16))) float eterm[2][4][B][C + 4];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int2 td = tiles[blockIdx.x / kHiSplit];
-    const int q = blockIdx.x % kHiSplit;
+    const int2 td = tiles[blockIdx.x / (64 / B)];
+    const int q = blockIdx.x % (64 / B);
     const DevJob& J = jobs[td.x];
     if (!(J.flags & JF_HI) || (J.flags & JF_HI_EXACT)) return;
     const long long s = st[td.x].step;
     if (!(s < J.end_step && s % J.stride == 0 && s % J.hi_eps_freq == 0)) return;
     const bool listed = (J.flags & JF_HI_LISTED) != 0;
-    if (listed && (q != 0 || w != 0)) return;
-    // listed: lane = bead of the 64-bead tile; unlisted: t & 15 = bead of
-    // this workgroup's 16, t >> 4 = partner of the chunk
-    const int d = listed ? td.y + lane : td.y + 16 * q + (t & 15);
     const int n = J.n;
     const float4* __restrict__ cur = J.coord[s & 1];
-    const float4 c = d < n ? cur[d] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float a = J.hi_a;
-    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (listed) {
-        if (d >= n) return;
+    if (listed) {  // lane = bead of the 64-bead tile
+        const int d = td.y + lane;
+        if (q != 0 || w != 0 || d >= n) return;
+        const float4 c = cur[d];
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
         for (int k = 0; k < J.cov_cnt[d]; ++k) eps_add(c, cur[J.cov_j[(size_t)k * n + d]], a, sum);
         for (int k = 0; k < J.nat_cnt[d]; ++k) eps_add(c, cur[J.nat_j[(size_t)k * n + d]], a, sum);
         for (int k = 0; k < J.pair_cnt[d]; ++k)
@@ -234,36 +393,38 @@ __global__ __launch_bounds__(1024) void k_hi_eps(const DevJob* __restrict__ jobs
         J.eps[d] = sum.w;
         return;
     }
-    // unlisted: wavefront w serves bead dbase + w (c and d above were the
-    // listed path's); lanes 16c + b of wavefront 0 sum component c of bead dbase + b
-    const int dbase = td.y + 16 * q, dw = dbase + w;
-    const float4 cw = dw < n ? cur[dw] : make_float4(0.f, 0.f, 0.f, 0.f);
+    // unlisted: lanes 16c + b of wavefront 0 sum component c of bead dbase + b
+    const int dbase = td.y + B * q;
+    int bb[2];
+    hi_beads<B>(dbase, n, bb);
+    HiPairEps pair;
+    pair.cur = cur;
+    pair.a = a;
+    pair.c[0] = ld4(cur, bb[0]);
+    pair.c[1] = ld4(cur, bb[1]);
     float acc = 0.f;
-    hi_ordered_sums<4>(eterm, n,
-                       [&](int i, float(&v)[4]) {
-                           float4 z = make_float4(-0.f, -0.f, -0.f, -0.f);
-                           if (i < n && i != dw && dw < n) {
-                               z = make_float4(0.f, 0.f, 0.f, 0.f);
-                               eps_add(cw, cur[i], a, z);
-                           }
-                           v[0] = z.x, v[1] = z.y, v[2] = z.z, v[3] = z.w;
-                       },
-                       acc);
+    hi_ordered_sums<B, C, 4>(eterm, n, bb, pair, acc);
     // component c of bead dbase + b is in lane 16c + b of wavefront 0
-    const float sy = __shfl(acc, lane + 16), sz = __shfl(acc, lane + 32), sw = __shfl(acc, lane + 48);
-    if (w == 0 && lane < 16 && dbase + lane < n) {
+    const float sy = __shfl(acc, lane + B), sz = __shfl(acc, lane + 2 * B), sw = __shfl(acc, (lane + 3 * B) & 63);
+    if (w == 0 && lane < B && dbase + lane < n) {
         J.ci[dbase + lane] = make_float4(acc, sy, sz, sw);
         J.eps[dbase + lane] = sw;
     }
 }
 
-// TeaUpdater::update (bdhitea.cu:133-176): epsilon and beta' in FP64.  One
-// wavefront per job: the per-bead values are staged in LDS 256 at a time and
-// added in bead order by every lane (the reference's sequential double sum,
-// the same bits; the lanes' sums are equal).
-__global__ __launch_bounds__(64) void k_hi_beta(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
-                                                int njobs) {
-    const int jb = blockIdx.x, lane = threadIdx.x;
+// TeaUpdater::update (bdhitea.cu:133-176): epsilon and beta' in FP64, one
+// 256-thread workgroup per job.  The reference adds the per-bead values in
+// bead order into a double.  Where the values' exponents span few enough bits
+// that every partial sum, in any order, is a multiple of the smallest value's
+// last place below 2^53 of them, each addition is exact and the order does
+// not matter: the workgroup adds them in parallel (4,096 values: 56 -> 8 us,
+// the chain of dependent additions).  Otherwise (values apart by more than
+// about 2^18, infinities, NaN) wavefront 0 adds them one by one, staged in
+// LDS kBetaChunk at a time.
+constexpr int kBetaThreads = 256;
+__global__ __launch_bounds__(kBetaThreads) void k_hi_beta(const DevJob* __restrict__ jobs,
+                                                          DevJobState* __restrict__ st, int njobs) {
+    const int jb = blockIdx.x, t = threadIdx.x, lane = t & 63;
     if (jb >= njobs) return;
     const DevJob& J = jobs[jb];
     if (!(J.flags & JF_HI) || (J.flags & JF_HI_EXACT)) return;
@@ -271,33 +432,67 @@ __global__ __launch_bounds__(64) void k_hi_beta(const DevJob* __restrict__ jobs,
     const long long s = S.step;
     if (!(s < J.end_step && s % J.stride == 0 && s % J.hi_eps_freq == 0)) return;
     const int N = J.n;
-    // the values staged kBetaChunk at a time, all of a chunk's loads in flight
-    // together, then added in bead order
     constexpr int kBetaChunk = 4096;
     __shared__ __attribute__((aligned(16))) float chunk[kBetaChunk];
+    __shared__ double psum[kBetaThreads / 64];
+    __shared__ int pmax[kBetaThreads / 64], pmin[kBetaThreads / 64];
+    // biased exponents: the largest of all values, the smallest of the nonzero
+    double part = 0.0;
+    int emax = 0, emin = 255;
+#pragma unroll 4
+    for (int i = t; i < N; i += kBetaThreads) {
+        const float v = J.eps[i];
+        const int e = (int)((__float_as_uint(v) >> 23) & 0xffu);
+        part += (double)v;
+        emax = max(emax, e);
+        if (v != 0.0f) emin = min(emin, max(e, 1));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        part += __shfl_xor(part, o);
+        emax = max(emax, __shfl_xor(emax, o));
+        emin = min(emin, __shfl_xor(emin, o));
+    }
+    if (lane == 0) {
+        psum[t >> 6] = part;
+        pmax[t >> 6] = emax;
+        pmin[t >> 6] = emin;
+    }
+    __syncthreads();
     double epsilon = 0.0;
-    for (int base = 0; base < N; base += kBetaChunk) {
-        float v[kBetaChunk / 64];
+    for (int k = 0; k < kBetaThreads / 64; ++k) {
+        epsilon += psum[k];
+        emax = max(emax, pmax[k]);
+        emin = min(emin, pmin[k]);
+    }
+    if (t >= 64) return;
+    // |partial sum| < N 2^(emax+1), a multiple of 2^(emin-23)
+    const int bits = 32 - __builtin_clz((unsigned)N) + emax + 1 - (emin - 23);
+    if (emax == 255 || (emax > 0 && bits > 53)) {
+        epsilon = 0.0;
+        for (int base = 0; base < N; base += kBetaChunk) {
+            float v[kBetaChunk / 64];
 #pragma unroll
-        for (int u = 0; u < kBetaChunk / 64; ++u) {
-            const int i = base + 64 * u + lane;
-            v[u] = i < N ? J.eps[i] : 0.f;
-        }
+            for (int u = 0; u < kBetaChunk / 64; ++u) {
+                const int i = base + 64 * u + lane;
+                v[u] = i < N ? J.eps[i] : 0.f;
+            }
 #pragma unroll
-        for (int u = 0; u < kBetaChunk / 64; ++u) chunk[64 * u + lane] = v[u];
-        __syncthreads();
-        const int m = min(kBetaChunk, N - base);
-        const float4* __restrict__ c4 = reinterpret_cast<const float4*>(chunk);
-        int k = 0;
-        for (; k + 4 <= m; k += 4) {
-            const float4 q = c4[k >> 2];
-            epsilon += (double)q.x;
-            epsilon += (double)q.y;
-            epsilon += (double)q.z;
-            epsilon += (double)q.w;
+            for (int u = 0; u < kBetaChunk / 64; ++u) chunk[64 * u + lane] = v[u];
+            wave_lds_order();
+            const int m = min(kBetaChunk, N - base);
+            const float4* __restrict__ c4 = reinterpret_cast<const float4*>(chunk);
+            int k = 0;
+            for (; k + 4 <= m; k += 4) {
+                const float4 q = c4[k >> 2];
+                epsilon += (double)q.x;
+                epsilon += (double)q.y;
+                epsilon += (double)q.z;
+                epsilon += (double)q.w;
+            }
+            for (; k < m; ++k) epsilon += (double)chunk[k];
+            wave_lds_order();
         }
-        for (; k < m; ++k) epsilon += (double)chunk[k];
-        __syncthreads();
     }
     if (lane != 0) return;  // the sum is uniform; one lane updates the state
     if (N > 1) epsilon /= 3. * N * (3. * N - 3.);
@@ -330,55 +525,45 @@ __device__ __forceinline__ void tea_force(const float4 c1, const float4 c2, cons
     fz += D.xz * gx + D.yz * gy + D.zz * gz;
 }
 
-// The TEA step (bdhitea_kernel.cu:364-515).  Unlisted: kHiSplit 1024-thread
-// workgroups per 64-bead tile of a TEA job, each serving 16 beads, so a
-// single job of a few thousand beads still fills the chip; the terms are
+// The TEA step (bdhitea_kernel.cu:364-515).  Unlisted: the terms are
 // added in partner order, the order of the reference's sequential loop, by
 // hi_ordered_sums.  Listed: wavefront 0 of the tile's first workgroup walks
 // the lists.
-__global__ __launch_bounds__(1024) void k_hi_tea(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
+template <int B, int C>
+__global__ __launch_bounds__(64 * B) void k_hi_tea(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
                                                  const int2* __restrict__ tiles, int ntiles, int kstep) {
-    __shared__ __attribute__((aligned(16))) float tterm[2][3][16][kHiRow];
+    __shared__ __attribute__((aligned(16))) float tterm[2][3][B][C + 4];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int2 td = tiles[blockIdx.x / kHiSplit];
-    const int q = blockIdx.x % kHiSplit;
+    const int2 td = tiles[blockIdx.x / (64 / B)];
+    const int q = blockIdx.x % (64 / B);
     const DevJob& J = jobs[td.x];
     if (!(J.flags & JF_HI) || (J.flags & JF_HI_EXACT)) return;
     const DevJobState& S = st[td.x];
     const long long s = S.step + kstep;
     if (s >= J.end_step) return;
     const bool listed = (J.flags & JF_HI_LISTED) != 0;
-    if (listed && (q != 0 || w != 0)) return;
-    // listed: lane = bead of the 64-bead tile; unlisted: t & 15 = bead of
-    // this workgroup's 16, t >> 4 = partner of the chunk
-    const int d = listed ? td.y + lane : td.y + 16 * q + (t & 15);
     const int n = J.n;
-    const bool own = d < n;
     const float4* __restrict__ cur = J.coord[s & 1];
-    float ci0 = 0.f, ci1 = 0.f, ci2 = 0.f, fx = 0.f, fy = 0.f, fz = 0.f;
-    float4 coord = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (own) {
+    const float a = J.hi_a;
+    if (listed) {  // lane = bead of the 64-bead tile
+        const int d = td.y + lane;
+        if (q != 0 || w != 0 || d >= n) return;
         float4 cs = J.ci[d];
         const float4 f0 = J.mforce[d];
         const float4 df = J.rforce[d];
         const float beta = S.beta;
         cs.w = beta * beta;
-        ci0 = 1.f / sqrtf(1.f + cs.w * cs.x);
-        ci1 = 1.f / sqrtf(1.f + cs.w * cs.y);
-        ci2 = 1.f / sqrtf(1.f + cs.w * cs.z);
-        coord = cur[d];
-        fx = f0.x, fy = f0.y, fz = f0.z;
+        float ci0 = 1.f / sqrtf(1.f + cs.w * cs.x);
+        float ci1 = 1.f / sqrtf(1.f + cs.w * cs.y);
+        float ci2 = 1.f / sqrtf(1.f + cs.w * cs.z);
+        const float4 coord = cur[d];
+        float fx = f0.x, fy = f0.y, fz = f0.z, tx, ty, tz;
         fx += df.x * ci0;
         fy += df.y * ci1;
         fz += df.z * ci2;
         ci0 *= beta;
         ci1 *= beta;
         ci2 *= beta;
-    }
-    const float a = J.hi_a;
-    float tx, ty, tz;
-    if (listed) {
-        if (!own) return;
         for (int k = 0; k < J.cov_cnt[d]; ++k) {
             const int i = J.cov_j[(size_t)k * n + d];
             tx = 0.f; ty = 0.f; tz = 0.f;
@@ -400,90 +585,78 @@ __global__ __launch_bounds__(1024) void k_hi_tea(const DevJob* __restrict__ jobs
         hi_finish(J, d, s, fx, fy, fz, coord);
         return;
     }
-    // unlisted: wavefront w serves bead dbase + w with that bead's ci
-    // (uniform over the wavefront); lanes 16c + b of wavefront 0 sum
-    // component c of bead dbase + b from its starting value
-    const int dbase = td.y + 16 * q, dw = dbase + w, ds = dbase + (lane & 15);
-    const bool ownw = dw < n;
-    float wi0 = 0.f, wi1 = 0.f, wi2 = 0.f;
-    float4 cw = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (ownw) {
-        const float4 cs = J.ci[dw];
+    // unlisted: the wavefront's two beads with their ci (uniform over the
+    // wavefront); lanes 16c + b of wavefront 0 sum component c of bead dbase + b
+    // from its starting value
+    const int dbase = td.y + B * q, ds = dbase + lane % B;
+    int bd[2];
+    hi_beads<B>(dbase, n, bd);
+    HiPairTea pair;
+    pair.cur = cur;
+    pair.mforce = J.mforce;
+    pair.rforce = J.rforce;
+    pair.a = a;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const float4 cs = ld4(J.ci, bd[k]);
         const float bb = S.beta * S.beta;
-        wi0 = 1.f / sqrtf(1.f + bb * cs.x) * S.beta;
-        wi1 = 1.f / sqrtf(1.f + bb * cs.y) * S.beta;
-        wi2 = 1.f / sqrtf(1.f + bb * cs.z) * S.beta;
-        cw = cur[dw];
+        pair.ci[k][0] = 1.f / sqrtf(1.f + bb * cs.x) * S.beta;
+        pair.ci[k][1] = 1.f / sqrtf(1.f + bb * cs.y) * S.beta;
+        pair.ci[k][2] = 1.f / sqrtf(1.f + bb * cs.z) * S.beta;
+        pair.c[k] = ld4(cur, bd[k]);
     }
     float acc = 0.f;
-    if (w == 0 && lane < 48 && ds < n) {  // the bead's starting value, component lane / 16
+    if (w == 0 && lane < 3 * B && ds < n) {  // the bead's starting value, component lane / 16
         const float4 cs = J.ci[ds], f0 = J.mforce[ds], df = J.rforce[ds];
         const float bb = S.beta * S.beta;
-        const int k = lane >> 4;
+        const int k = lane / B;
         const float cc = k == 0 ? cs.x : (k == 1 ? cs.y : cs.z);
         const float f = k == 0 ? f0.x : (k == 1 ? f0.y : f0.z), g = k == 0 ? df.x : (k == 1 ? df.y : df.z);
         acc = f;
         acc += g * (1.f / sqrtf(1.f + bb * cc));
     }
-    hi_ordered_sums<3>(tterm, n,
-                       [&](int i, float(&v)[3]) {
-                           float x = -0.f, y = -0.f, z = -0.f;
-                           if (i < n && i != dw && ownw) {
-                               x = 0.f, y = 0.f, z = 0.f;
-                               tea_force(cw, cur[i], J.mforce[i], J.rforce[i], wi0, wi1, wi2, a, x, y, z);
-                           }
-                           v[0] = x, v[1] = y, v[2] = z;
-                       },
-                       acc);
-    const float sy = __shfl(acc, lane + 16), sz = __shfl(acc, lane + 32);
-    if (w == 0 && lane < 16 && ds < n) hi_finish(J, ds, s, acc, sy, sz, cur[ds]);
+    hi_ordered_sums<B, C, 3>(tterm, n, bd, pair, acc);
+    const float sy = __shfl(acc, lane + B), sz = __shfl(acc, lane + 2 * B);
+    if (w == 0 && lane < B && ds < n) hi_finish(J, ds, s, acc, sy, sz, cur[ds]);
 }
 
 // ---------------------------------------------------------------------------
 // exact path
 // ---------------------------------------------------------------------------
 
-// F_i + sum_j D_ij F_j into fdf, summed in bead order.  kHiSplit 1024-thread
-// workgroups per 64-bead tile of the (single) exact-HI job of the launch,
-// 16 beads each, wavefront w forming bead dbase + w's terms D_ij F_j (the
-// three row sums, written exactly as the sequential loop writes them) and
-// wavefront 0 adding them in j order (hi_ordered_sums), so every sum is the
-// same bits as the bead-by-bead loop.
-__global__ __launch_bounds__(1024) void k_chol_D(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
+// F_i + sum_j D_ij F_j into fdf, summed in bead order (hi_ordered_sums), for
+// the (single) exact-HI job of the launch: the terms D_ij F_j are the three
+// row sums, written exactly as the sequential loop writes them, so every sum
+// is the same bits as the bead-by-bead loop.
+template <int B, int C>
+__global__ __launch_bounds__(64 * B) void k_chol_D(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
                                                  const int2* __restrict__ tiles, int ntiles, int kstep) {
-    __shared__ __attribute__((aligned(16))) float dterm[2][3][16][kHiRow];
+    __shared__ __attribute__((aligned(16))) float dterm[2][3][B][C + 4];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int2 td = tiles[blockIdx.x / kHiSplit];
+    const int2 td = tiles[blockIdx.x / (64 / B)];
     const DevJob& J = jobs[td.x];
     if (!(J.flags & JF_HI_EXACT)) return;  // one job per launch: uniform
     const long long s = st[td.x].step + kstep;
     if (s >= J.end_step) return;
     const int n = J.n;
-    const int dbase = td.y + 16 * (blockIdx.x % kHiSplit), dw = dbase + w, ds = dbase + (lane & 15);
+    const int dbase = td.y + B * (blockIdx.x % (64 / B)), ds = dbase + lane % B;
     const float4* __restrict__ cur = J.coord[s & 1];
-    const float4 c = dw < n ? cur[dw] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float a = J.hi_a;
+    int bd[2];
+    hi_beads<B>(dbase, n, bd);
+    HiPairD pair;
+    pair.cur = cur;
+    pair.mforce = J.mforce;
+    pair.a = J.hi_a;
+    pair.c[0] = ld4(cur, bd[0]);
+    pair.c[1] = ld4(cur, bd[1]);
     float acc = 0.f;
-    if (w == 0 && lane < 48 && ds < n) {
+    if (w == 0 && lane < 3 * B && ds < n) {
         const float4 f0 = J.mforce[ds];
-        acc = lane < 16 ? f0.x : (lane < 32 ? f0.y : f0.z);
+        acc = lane < B ? f0.x : (lane < 2 * B ? f0.y : f0.z);
     }
-    hi_ordered_sums<3>(dterm, n,
-                       [&](int j, float(&v)[3]) {
-                           float tx = -0.f, ty = -0.f, tz = -0.f;
-                           if (j < n && j != dw && dw < n) {
-                               const float4 dr = unit_sep(c, cur[j]);
-                               const F6 D = rpy(dr, a);
-                               const float4 g = J.mforce[j];
-                               tx = D.xx * g.x + D.xy * g.y + D.xz * g.z;
-                               ty = D.xy * g.x + D.yy * g.y + D.yz * g.z;
-                               tz = D.xz * g.x + D.yz * g.y + D.zz * g.z;
-                           }
-                           v[0] = tx, v[1] = ty, v[2] = tz;
-                       },
-                       acc);
-    const float sy = __shfl(acc, lane + 16), sz = __shfl(acc, lane + 32);
-    if (w == 0 && lane < 16 && ds < n) J.fdf[ds] = make_float4(acc, sy, sz, 0.0f);
+    hi_ordered_sums<B, C, 3>(dterm, n, bd, pair, acc);
+    const float sy = __shfl(acc, lane + B), sz = __shfl(acc, lane + 2 * B);
+    if (w == 0 && lane < B && ds < n) J.fdf[ds] = make_float4(acc, sy, sz, 0.0f);
 }
 
 // D/D_ii lower block triangle into M on refactorisation steps: block
@@ -1556,18 +1729,28 @@ __global__ __launch_bounds__(256) void k_chol_step(CholStep a) {
 // launchers
 // ---------------------------------------------------------------------------
 
+// The kernel for (B, C) = cfg over `ntiles` tiles.
+#define SOP_HI_LAUNCH(kernel, cfg, ntiles, stream, ...)                                                             \
+    do {                                                                                                            \
+        const dim3 g((ntiles) * (64 / (cfg).beads)), b(64 * (cfg).beads);                                           \
+        if ((cfg).beads == 4) hipLaunchKernelGGL((kernel<4, 256>), g, b, 0, stream, __VA_ARGS__);                   \
+        else if ((cfg).beads == 16) hipLaunchKernelGGL((kernel<16, 256>), g, b, 0, stream, __VA_ARGS__);            \
+        else if ((cfg).chunk == 256) hipLaunchKernelGGL((kernel<8, 256>), g, b, 0, stream, __VA_ARGS__);            \
+        else hipLaunchKernelGGL((kernel<8, 128>), g, b, 0, stream, __VA_ARGS__);                                    \
+    } while (0)
+
 hipError_t launch_hi_tea_update(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int njobs,
                                 hipStream_t stream) {
-    if (ntiles > 0)
-        hipLaunchKernelGGL(k_hi_eps, dim3(ntiles * kHiSplit), dim3(1024), 0, stream, jobs, st, tiles, ntiles);
-    hipLaunchKernelGGL(k_hi_beta, dim3(njobs), dim3(64), 0, stream, jobs, st, njobs);
+    const HiConfig cfg = hi_config(64ll * ntiles);
+    if (ntiles > 0) SOP_HI_LAUNCH(k_hi_eps, cfg, ntiles, stream, jobs, st, tiles, ntiles);
+    hipLaunchKernelGGL(k_hi_beta, dim3(njobs), dim3(kBetaThreads), 0, stream, jobs, st, njobs);
     return hipGetLastError();
 }
 
 hipError_t launch_hi_tea_step(const DevJob* jobs, const DevJobState* st, const int2* tiles, int ntiles, int kstep,
                               hipStream_t stream) {
-    if (ntiles > 0)
-        hipLaunchKernelGGL(k_hi_tea, dim3(ntiles * kHiSplit), dim3(1024), 0, stream, jobs, st, tiles, ntiles, kstep);
+    const HiConfig cfg = hi_config(64ll * ntiles);
+    if (ntiles > 0) SOP_HI_LAUNCH(k_hi_tea, cfg, ntiles, stream, jobs, st, tiles, ntiles, kstep);
     return hipGetLastError();
 }
 
@@ -1653,7 +1836,8 @@ hipError_t launch_chol_factor(float* M, size_t ld, int mp, int mode, const CholW
 
 hipError_t launch_chol_step(const DevJob* jobs, const DevJobState* st, const int2* tiles, int ntiles, int kstep,
                             const HiExactWork* w, hipStream_t stream) {
-    hipLaunchKernelGGL(k_chol_D, dim3(ntiles * kHiSplit), dim3(1024), 0, stream, jobs, st, tiles, ntiles, kstep);
+    const HiConfig cfg = hi_config(64ll * ntiles);
+    SOP_HI_LAUNCH(k_chol_D, cfg, ntiles, stream, jobs, st, tiles, ntiles, kstep);
     if (w) {
         hipLaunchKernelGGL(k_chol_build, dim3(ntiles, ntiles), dim3(256), 0, stream, jobs, st, tiles, kstep);
         // the factorisation's error covers the event record/wait pairs that

@@ -543,14 +543,6 @@ __device__ __forceinline__ BondedSrc bonded_fetch(const StepDesc& D, int t, int 
     return f;
 }
 
-// Orders a wavefront's LDS writes before its own reads of other lanes' words
-// (and those before the next writes): the LDS executes a wavefront's
-// operations in order, so only the compiler has to be held.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Adds the first m positions (up to the next multiple of 4) of a row's LDS
 // words to acc, in order; 32 at a time with their reads in flight together.
 __device__ __forceinline__ void rows_add(const float* __restrict__ t, int m, float& acc) {
@@ -1868,12 +1860,14 @@ __global__ __launch_bounds__(256) void k_energies(const DevJob* __restrict__ job
 
 // Self-check of div_rn_fast against the IEEE division: every float bit
 // pattern b in [lo, hi) (inside the fast range) with each numerator a[k];
-// counts the results that differ.
+// counts the results that differ, and the b whose sqrt_rn_fast is not the
+// IEEE square root.
 __global__ void k_division_check(unsigned lo, unsigned hi, const float* __restrict__ a, int na,
                                  unsigned long long* __restrict__ bad) {
     unsigned long long mine = 0;
     for (unsigned u = lo + blockIdx.x * blockDim.x + threadIdx.x; u < hi; u += gridDim.x * blockDim.x) {
         const float b = __uint_as_float(u);
+        mine += __float_as_uint(sqrt_rn_fast(b)) != __float_as_uint(sqrtf(b)) ? 1ull : 0ull;
         for (int k = 0; k < na; ++k)
             mine += __float_as_uint(div_rn_fast(a[k], b)) != __float_as_uint(a[k] / b) ? 1ull : 0ull;
     }
