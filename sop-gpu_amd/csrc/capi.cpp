@@ -295,8 +295,8 @@ int sop_chol_factor(int device, int n, const float* A, int mode, float* L, int r
     if (err == hipSuccess) err = hipMalloc(&dM, mp * mp * 4);
     if (err == hipSuccess) err = hipMalloc(&w.linv, sop::kCholLinvBytes);
     if (err == hipSuccess) err = hipMalloc(&w.bbuf, sop::chol_bbuf_bytes(mp));
-    if (err == hipSuccess) err = hipMalloc(&w.phi, sop::chol_panel_bytes(mp));
-    if (err == hipSuccess) err = hipMalloc(&w.plo, sop::chol_panel_bytes(mp));
+    if (err == hipSuccess) err = hipMalloc(&w.pan[0], sop::chol_panel_bytes(mp));
+    if (err == hipSuccess) err = hipMalloc(&w.pan[1], sop::chol_panel_bytes(mp));
     if (err == hipSuccess) err = hipEventCreate(&e0);
     if (err == hipSuccess) err = hipEventCreate(&e1);
     if (err == hipSuccess) err = hipMemcpy(dA, h.data(), mp * mp * 4, hipMemcpyHostToDevice);
@@ -328,8 +328,8 @@ int sop_chol_factor(int device, int n, const float* A, int mode, float* L, int r
     (void)hipFree(dM);
     (void)hipFree(w.linv);
     (void)hipFree(w.bbuf);
-    (void)hipFree(w.phi);
-    (void)hipFree(w.plo);
+    (void)hipFree(w.pan[0]);
+    (void)hipFree(w.pan[1]);
     if (s) (void)hipStreamDestroy(s);
     return rc;
 }

@@ -613,8 +613,8 @@ int Engine::add_job(const sop_params& p, const sop_system& s, long long numsteps
             hw.mode = exact_mode_;
             hw.work.linv = (double*)A(kCholLinvBytes);
             hw.work.bbuf = (float*)A(chol_bbuf_bytes(mp));
-            hw.work.phi = (unsigned short*)A(chol_panel_bytes(mp));
-            hw.work.plo = (unsigned short*)A(chol_panel_bytes(mp));
+            hw.work.pan[0] = (char*)A(chol_panel_bytes(mp));
+            hw.work.pan[1] = (char*)A(chol_panel_bytes(mp));
             hw.chol_freq = J.hi_chol_freq;
             if (!aux_stream_) {  // the factorisation's lookahead stream, shared by the exact-HI jobs
                 if (hipStreamCreateWithFlags(&aux_stream_, hipStreamNonBlocking) != hipSuccess ||

@@ -8,11 +8,11 @@ namespace sop {
 
 enum { SOP_CHOL_BF16X3 = 0, SOP_CHOL_F32 = 1 };
 
-// Width of the factorisation's outer panel: the split-BF16 panel buffers
-// hold two panels of mp x kCholPanel elements each (consecutive panels
-// alternate: a panel's trailing update, and the next panel's steps, still
-// read its copy while the next panel is factored).
-constexpr int kCholPanel = 512;
+// Width of the factorisation's outer panel, and the bytes of a panel copy's
+// record (32 columns of a row, panel_rec in hi.hip).  Consecutive panels
+// alternate between two copies: a panel's trailing update, and the next
+// panel's steps, still read its copy while the next panel is factored.
+constexpr int kCholPanel = 512, kCholRecord = 128;
 // Step buffers of the 64-column steps: the inverses of two consecutive 64x64
 // diagonal blocks (FP64, or FP32 in the first half of the slot in the
 // split-BF16 mode), then two FP32 64x64 blocks that carry a diagonal block,
@@ -20,15 +20,14 @@ constexpr int kCholPanel = 512;
 constexpr size_t kCholLinvBytes = (size_t)2 * 64 * 64 * sizeof(double) + (size_t)2 * 64 * 64 * sizeof(float);
 // Column blocks left for the next step (two consecutive steps): mp x 64 FP32 each.
 inline size_t chol_bbuf_bytes(size_t mp) { return (size_t)2 * mp * 64 * sizeof(float); }
-// One split-BF16 half (hi or lo) of the two panel buffers.
-inline size_t chol_panel_bytes(size_t mp) { return (size_t)2 * mp * kCholPanel * sizeof(unsigned short); }
+// One panel copy: 4 bytes per element (FP32, or split-BF16 hi and lo).
+inline size_t chol_panel_bytes(size_t mp) { return mp * (kCholPanel / 32) * kCholRecord; }
 
 // Device workspace of one blocked factorisation.
 struct CholWork {
     double* linv;          // kCholLinvBytes: two inverse slots (FP64-sized), then two FP32 diagonal blocks
     float* bbuf;           // chol_bbuf_bytes(mp)
-    unsigned short* phi;   // chol_panel_bytes(mp): split-BF16 hi of the outer panels
-    unsigned short* plo;   // chol_panel_bytes(mp): lo
+    char* pan[2];          // chol_panel_bytes(mp) each: the panel copies
 };
 
 // Device workspace of one exact-HI job's blocked factorisation.

@@ -17,18 +17,19 @@
 // kCholPanel columns, each factored by 64-column steps (k_chol_step), one
 // launch per step over the 64-row blocks from the step's diagonal down:
 //   the previous step's column block is solved against the inverse of its
-//   diagonal block (X = B Li^T on FP64 MFMA) and emitted in FP32 and as
-//   split-BF16 pairs (hi = bf16(x), lo = bf16(x - hi));
-//   the step's column block is updated by the columns to its left that no
-//   trailing update has applied yet (the previous panel's and this
-//   panel's), on MFMA -- split-BF16 with three products (hi*hi + hi*lo +
-//   lo*hi, FP32 accumulate) or FP32 -- with the K range split over the
-//   workgroup's four wavefronts;
-//   the diagonal workgroup factors its block in FP64 (16-column passes in
-//   registers, rank-16 updates and the inverse's off-diagonal blocks on FP64
-//   MFMA) and forms the inverse the next step solves with.
-// The rest of the trailing matrix is updated once per outer panel by wide
-// MFMA kernels on a second stream, overlapped with the next panel's steps.
+//   diagonal block (X = B Li^T on MFMA) and emitted in FP32, and into the
+//   panel copy that the updates read (FP32, or split-BF16 pairs hi = bf16(x),
+//   lo = bf16(x - hi));
+//   the step's column block is updated by the panel's columns to its left on
+//   MFMA -- split-BF16 with three products (hi*hi + hi*lo + lo*hi, FP32
+//   accumulate) or FP32 -- with the K range split over the workgroup's
+//   wavefronts;
+//   the diagonal workgroup factors its block (FP64 in the FP32 mode, FP32 in
+//   the split-BF16 mode; 16-column passes in registers, rank-16 updates and
+//   the inverse's off-diagonal blocks on MFMA) and forms the inverse the
+//   next step solves with.
+// Wide MFMA kernels then update the next panel's columns and, on a second
+// stream beside the next panel's steps, the rest of the trailing matrix.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -47,7 +48,6 @@ namespace sop {
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 struct F6 {
     float xx, xy, xz, yy, yz, zz;
@@ -762,6 +762,17 @@ __global__ __launch_bounds__(256) void k_chol_L(const DevJob* __restrict__ jobs,
 static constexpr int NB = 64;    // inner block: diagonal factor, panel solve
 static constexpr int NB2 = kCholPanel;  // outer panel: depth of the trailing update
 
+// The panel copy that the updates read: for every 32 columns of a panel and
+// every row one 128-byte record (a cache line), the rows of a chunk one after
+// another -- 32 floats (FP32), or 32 bf16 hi parts followed by the 32 lo
+// parts (split-BF16).  A wavefront that reads 16 rows of a chunk reads 2 KB on
+// end; from rows a kilobyte or a matrix row apart the same operands came from
+// a few L2 channels at a quarter of the rate (the row blocks' update of 960
+// columns: 19 us).
+__device__ __forceinline__ size_t panel_rec(size_t mp, int chunk, size_t row) {
+    return ((size_t)chunk * mp + row) * kCholRecord;
+}
+
 __device__ __forceinline__ unsigned short f2bf(float x) {  // round to nearest even
     unsigned int u = __float_as_uint(x);
     u += 0x7fffu + ((u >> 16) & 1u);
@@ -817,57 +828,98 @@ __device__ __forceinline__ int drow(int lk, int v) {
     return std::is_same<R, double>::value ? lk + 4 * v : 4 * lk + v;
 }
 
-// 16-column steps of the diagonal factorisation, run by one wavefront on
-// registers: lanes 0..15 hold the rows of the 16x16 diagonal sub-block,
-// lanes 16..63 the rows below it.  Step J (a template parameter, so every
-// register index is a constant) scales column J by 1/L[J][J] and subtracts
-// L[r][J] L[c][J] from the columns c > J, with L[c][J] read from lane c
-// (readlane, no LDS round trip): for lanes below the sub-block this is the
-// forward substitution of the panel solve, so both run as one pass.  Lanes
-// 0..15 accumulate scratch above their diagonal, which is never written
-// back.  y[J] receives 1/L[J][J] (uniform).
-template <int J, typename R>
+// Four columns (4B .. 4B+3) of the diagonal factorisation, run by one
+// wavefront on registers: lanes 0..15 hold the rows of the 16x16 diagonal
+// sub-block, lanes 16..63 the rows below it.  The 4x4 block on the diagonal
+// is read into every lane (readlane) and factored there, so that one pivot
+// waits for a reciprocal square root and two multiply-adds and not for a
+// round trip through the columns; then each lane substitutes its row's four
+// values, and the columns to the right take the four products, with L[c][k]
+// read from lane c.  The same operations, in the same order, as one column
+// after another (four passes: 8 -> 4 us of a 64x64 block in FP32).  For lanes
+// below the sub-block this is the forward substitution of the panel solve, so
+// both run as one pass.  Lanes 0..15 accumulate scratch above their diagonal,
+// which is never written back.  y[4B + k] receives 1/L[4B+k][4B+k] (uniform).
+template <int B, typename R>
 __device__ __forceinline__ void chol16_step(R (&v)[16], R (&y)[16]) {
-    y[J] = rsqrt_r(readlane_r(v[J], J));
-    v[J] *= y[J];  // lane J: L[J][J] = p / sqrt(p); below: a[r][J] / L[J][J]
-    if constexpr (J + 1 < 16) {
+    constexpr int J = 4 * B;
+    R d[4][4];
 #pragma unroll
-        for (int c = J + 1; c < 16; ++c) v[c] = fma(-v[J], readlane_r(v[J], c), v[c]);
-        chol16_step<J + 1>(v, y);
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int k = 0; k <= i; ++k) d[i][k] = readlane_r(v[J + k], J + i);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        y[J + k] = rsqrt_r(d[k][k]);
+#pragma unroll
+        for (int i = k + 1; i < 4; ++i) d[i][k] *= y[J + k];
+#pragma unroll
+        for (int i = k + 1; i < 4; ++i)
+#pragma unroll
+            for (int q = k + 1; q <= i; ++q) d[i][q] = fma(-d[i][k], d[q][k], d[i][q]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+        for (int q = 0; q < k; ++q) v[J + k] = fma(-v[J + q], d[k][q], v[J + k]);
+        v[J + k] *= y[J + k];  // lane J+k: L[J+k][J+k] = p / sqrt(p)
+    }
+    if constexpr (B + 1 < 4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            // all of a column's L[c][k] read before they are used: read and
+            // used one by one, each product would wait for its own read
+            R lc[12];
+#pragma unroll
+            for (int c = J + 4; c < 16; ++c) lc[c - 4] = readlane_r(v[J + k], c);
+#pragma unroll
+            for (int c = J + 4; c < 16; ++c) asm volatile("" : "+s"(lc[c - 4]));
+#pragma unroll
+            for (int c = J + 4; c < 16; ++c) v[c] = fma(-v[J + k], lc[c - 4], v[c]);
+        }
+        chol16_step<B + 1>(v, y);
     }
 }
 
+static constexpr int kCholThreads = 512;  // a step's workgroup: eight wavefronts, two per SIMD
 static constexpr int LDS_ROW = NB + 1;  // row stride of the block being factored
-// row stride of the transposed blocks (Li^T): 16-byte rows, and for FP32 the
-// four row groups of an MFMA operand read in distinct bank ranges
-template <typename R>
-constexpr int ldt() { return std::is_same<R, double>::value ? NB + 2 : NB + 16; }
+// Row stride of the transposed blocks (Li^T): 16-byte rows, and the four row
+// groups of an MFMA operand, four rows apart (load_solve_rows), read in
+// distinct bank ranges, in either type.
+static constexpr int LDT = NB + 4;
 
-// Column block K of the 64x64 block s (rows 16K..63) factored by
-// wavefront 0 in registers: lane r holds row 16K + r (lanes 0..15 the
-// diagonal sub-block, the others the rows below, forward-substituted in
-// the same pass).  Lanes past row 63 read a clamped row and keep zeros;
-// lanes 0..15 write their scratch above the diagonal back, where nothing
-// reads it.  dinv receives the reciprocals of the sub-block's diagonal.
+// Column block K of the 64x64 block s (rows 16K..63), factored in registers
+// by wavefront 0: lane r holds row 16K + r (lanes 0..15 the diagonal sub-block,
+// the others the rows below, forward-substituted in the same pass; lanes past
+// row 63 keep zeros).  Wavefront 1 runs the same pass with the rows of the
+// identity in lanes 16..31: forward-substituted, e_i becomes row i of the
+// transposed inverse of the sub-block, so the inverse comes with the factor
+// (a substitution of its own took longer than the pass).  pass_load reads the
+// registers; a barrier later, pass_store follows the factorisation.  Lanes
+// 0..15 write their scratch above the diagonal back, where nothing reads it.
 template <typename R>
-__device__ __forceinline__ void chol_pass(R (*s)[LDS_ROW], R* __restrict__ dinv, int K) {
-    const int r = threadIdx.x & 63, q0 = 16 * K, row = q0 + r;
-    const bool live = row < NB;
-    const int rr = live ? row : NB - 1;
-    R v[16], y[16];
+__device__ __forceinline__ void pass_load(const R (*s)[LDS_ROW], R (&v)[16], int K) {
+    const int r = threadIdx.x & 63, w = wave_of();
+    const int q0 = 16 * K;
+    const bool row = r < (w == 0 ? NB - q0 : 16);
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
-        const R e = s[rr][q0 + c];
-        v[c] = live && (r >= 16 || c <= r) ? e : R(0);
+        const R e = s[row ? q0 + r : q0][q0 + c];
+        v[c] = row && (r >= 16 || c <= r) ? e : w != 0 && r - 16 == c ? R(1) : R(0);
     }
-    chol16_step<0>(v, y);
-    if (live) {
+}
+template <typename R>
+__device__ __forceinline__ void pass_store(R (*s)[LDS_ROW], R* __restrict__ LiT, const R (&v)[16], int K) {
+    const int r = threadIdx.x & 63, w = wave_of();
+    const int q0 = 16 * K;
+    if (w == 0) {
+        if (r < NB - q0) {
 #pragma unroll
-        for (int c = 0; c < 16; ++c) s[row][q0 + c] = v[c];
-    }
-    if (r == 0) {
+            for (int c = 0; c < 16; ++c) s[q0 + r][q0 + c] = v[c];
+        }
+    } else if (r >= 16 && r < 32) {
 #pragma unroll
-        for (int c = 0; c < 16; ++c) dinv[q0 + c] = y[c];
+        for (int c = 0; c < 16; ++c) LiT[(q0 + r - 16) * LDT + q0 + c] = v[c];
     }
 }
 
@@ -885,30 +937,6 @@ __device__ __forceinline__ void rank16_tile(R (*s)[LDS_ROW], int I, int J, int K
     for (int v = 0; v < 4; ++v) s[16 * I + drow<R>(lk, v)][16 * J + lr] = acc[v];
 }
 
-// Column c (lane c < 16) of inv(L_KK) by forward substitution, y_t =
-// (e_c - sum_{u<t} L_tu y_u) / L_tt with the sums accumulated right-looking
-// so each y_t waits for one product; written transposed to LiT (LiT[a*LDT
-// + b] = Li[b][a]).
-template <typename R>
-__device__ __forceinline__ void inv_diag16(const R (*s)[LDS_ROW], R* __restrict__ LiT, const R* __restrict__ dinv,
-                                           int K) {
-    constexpr int LDT = ldt<R>();
-    const int c = threadIdx.x & 63, q0 = 16 * K;
-    if (c < 16) {
-        R acc[16], y[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = R(0);
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            y[t] = t < c ? R(0) : (t == c ? dinv[q0 + t] : -acc[t] * dinv[q0 + t]);
-#pragma unroll
-            for (int r = t + 1; r < 16; ++r) acc[r] = fma(s[q0 + r][q0 + t], y[t], acc[r]);
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) LiT[(q0 + c) * LDT + q0 + r] = y[r];
-    }
-}
-
 // Off-diagonal 16x16 block (I, J) of the inverse, J < I, on MFMA by one
 // wavefront, in two halves: T = sum_{J<=K<I} L_IK Li_KJ into the
 // wavefront's LDS tile (needs the rows J..I-1 of the inverse), then
@@ -916,7 +944,6 @@ __device__ __forceinline__ void inv_diag16(const R (*s)[LDS_ROW], R* __restrict_
 template <typename R>
 __device__ __forceinline__ void inv_sum16(const R (*s)[LDS_ROW], const R* __restrict__ LiT, R (*T)[17], int I,
                                           int J) {
-    constexpr int LDT = ldt<R>();
     const int l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
     R4<R> acc = {R(0), R(0), R(0), R(0)};
     for (int k0 = 0; k0 < 16 * (I - J); k0 += 4)
@@ -926,7 +953,6 @@ __device__ __forceinline__ void inv_sum16(const R (*s)[LDS_ROW], const R* __rest
 }
 template <typename R>
 __device__ __forceinline__ void inv_apply16(R* __restrict__ LiT, const R (*T)[17], int I, int J) {
-    constexpr int LDT = ldt<R>();
     const int l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
     R4<R> li = {R(0), R(0), R(0), R(0)};
 #pragma unroll
@@ -937,396 +963,211 @@ __device__ __forceinline__ void inv_apply16(R* __restrict__ LiT, const R (*T)[17
 
 // Factor the 64x64 block s (lower triangle, row-major) in place and form
 // the inverse of the factor, transposed, in LiT (zero above its diagonal),
-// with 256 threads.  The factor runs in four rounds, one per 16-column
-// block K: wavefront 0 applies the previous block's rank-16 update to block
-// K's tiles, then factors block K in registers; meanwhile wavefronts 2 and
-// 3 apply that update to the tiles right of block K, and wavefront 1 forms
-// row K-1 of the inverse (its diagonal block by substitution, the blocks
-// left of it on MFMA) -- so the inverse trails the factor by one round
-// instead of following it.  The inverse's last row is formed after the
-// last round.  dinv receives the reciprocals of the factor's diagonal.
+// with the workgroup's eight wavefronts, in a round per 16-column block K:
+// the previous block's rank-16 update of the tiles right of it, a tile per
+// wavefront, beside the products that complete row K-1 of the inverse; then
+// the factorisation of block K with its diagonal block's inverse (wavefronts 0
+// and 1, see pass_load), beside the sums of row K's blocks left of the
+// diagonal.  So the inverse trails the factor by one product.
 template <typename R>
-__device__ __forceinline__ void potrf_inv64(R (*s)[LDS_ROW], R* __restrict__ LiT, R (*T)[16][17],
-                                            R* __restrict__ dinv) {
-    constexpr int LDT = ldt<R>();
-    const int tid = threadIdx.x, w = wave_of();
-    if (w == 0)
-        chol_pass(s, dinv, 0);
-    else
-        for (int e = tid - 64; e < NB * LDT; e += 192) LiT[e] = R(0);
-    __syncthreads();
+__device__ __forceinline__ void potrf_inv64(R (*s)[LDS_ROW], R* __restrict__ LiT, R (*T)[16][17]) {
+    const int w = wave_of();
+    for (int e = threadIdx.x; e < NB * LDT; e += kCholThreads) LiT[e] = R(0);
 #pragma unroll 1
-    for (int K = 1; K < NB / 16; ++K) {
-        const int k = K - 1;  // the block factored in the previous round
-        if (w == 0) {
-            for (int I = K; I < NB / 16; ++I) rank16_tile(s, I, K, k);
-            chol_pass(s, dinv, K);
-        } else if (w == 1) {
-            inv_diag16(s, LiT, dinv, k);
-            for (int J = 0; J < k; ++J) {
-                inv_sum16(s, LiT, T[0], k, J);
-                inv_apply16(LiT, T[0], k, J);
-            }
-        } else {
-            // tiles (I, J), K < J <= I, dealt to wavefronts 2 and 3 in turn
-            int t = 0;
-            for (int J = K + 1; J < NB / 16; ++J)
-                for (int I = J; I < NB / 16; ++I, ++t)
-                    if ((t & 1) == w - 2) rank16_tile(s, I, J, k);
+    for (int K = 0; K < NB / 16; ++K) {  // one copy of the code: its first pass fetches it
+        if (K > 0) {
+            // tiles (I, J), K <= J <= I, from the last: (3,3), (3,2), (2,2),
+            // (3,1), (2,1), (1,1)
+            if (w < (4 - K) * (5 - K) / 2)
+                rank16_tile(s, (0x123233 >> (4 * w)) & 15, (0x111223 >> (4 * w)) & 15, K - 1);
+            else if (w >= 6 && w - 6 < K - 1)  // row K-1 of the inverse, left of its diagonal
+                inv_apply16(LiT, T[w - 6], K - 1, w - 6);
+            __syncthreads();
+        }
+        R v[16];
+        if (w < 2) pass_load(s, v, K);
+        __syncthreads();
+        if (w < 2) {
+            R y[16];
+            chol16_step<0>(v, y);
+            pass_store(s, LiT, v, K);
+        } else if (w - 2 < K) {
+            inv_sum16(s, LiT, T[w - 2], K, w - 2);
         }
         __syncthreads();
     }
-    // row 3 of the inverse: its diagonal block (wavefront 0) beside the sums
-    // of the blocks left of it (wavefronts 1..3), then the products
-    constexpr int RL = NB / 16 - 1;
-    if (w == 0)
-        inv_diag16(s, LiT, dinv, RL);
-    else
-        inv_sum16(s, LiT, T[w - 1], RL, w - 1);
-    __syncthreads();
-    if (w != 0) inv_apply16(LiT, T[w - 1], RL, w - 1);
+    constexpr int RL = NB / 16 - 1;  // the inverse's last row
+    if (w < RL) inv_apply16(LiT, T[w], RL, w);
     __syncthreads();
 }
 
-// Trailing update after an outer panel: C_IJ -= P_I P_J^T over the panel's
-// K = kw columns, on 128x128 tiles of the lower triangle from row/column
-// s0 on.  Wave w computes the 64x64 quarter (w>>1, w&1) as 4x4 MFMA blocks;
-// operands are staged through LDS in K-chunks.  Rows at or beyond mp are
-// read as zero and not written.
-static constexpr int GT = 128;   // trailing tile edge
-static constexpr int KCB = 32;   // K-chunk of the split-BF16 update (bf16 elements)
-static constexpr int KCF = 16;   // K-chunk of the FP32 update (floats)
-static constexpr int LPB = KCB + 8;  // padded LDS row (bf16 elements)
-static constexpr int LPF = KCF + 4;  // padded LDS row (floats)
-
-// Tile (blockIdx.x, blockIdx.y) of the update region: rows and columns
-// [s, mp).  Tiles wholly above the diagonal have nothing to do.
-__device__ __forceinline__ bool big_tile(int s, size_t& r0, size_t& c0) {
-    r0 = (size_t)s + (size_t)blockIdx.x * GT;
-    c0 = (size_t)s + (size_t)blockIdx.y * GT;
-    return c0 < r0 + GT;
+// M[row][col] -= v over the lower triangle, rows and columns below mp, for N
+// elements of a lane.  All loads are issued, from clamped addresses, before
+// the first store: each behind its own condition, they ran one memory round
+// trip after another (64 of them took 25 of a 128x128 tile's 40 us, 128 took
+// 80 of a 256x256 tile's 118).
+template <int N>
+__device__ __forceinline__ void sub_store(float* __restrict__ M, size_t ld, int mp, const int (&row)[N],
+                                          const int (&col)[N], const float (&v)[N]) {
+    float c[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) c[q] = M[(size_t)min(row[q], mp - 1) * ld + min(col[q], mp - 1)];
+#pragma unroll
+    for (int q = 0; q < N; ++q) c[q] -= v[q];
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+        if (row[q] < mp && col[q] < mp && col[q] <= row[q]) M[(size_t)row[q] * ld + col[q]] = c[q];
 }
 
-__device__ __forceinline__ void big_store(float* __restrict__ M, size_t ld, int mp, int ce, size_t r0, size_t c0,
-                                          const f32x4 (&acc)[4][4]) {
-    const int l = threadIdx.x & 63, w = wave_of();
-    const size_t rb = r0 + 64 * (w >> 1), cb = c0 + 64 * (w & 1);
+// Update after an outer panel: C -= P_r P_c^T over the panel copy's kw columns
+// for one TM x TN tile of the lower triangle (rows from r0, columns from c0;
+// rows at or beyond mp are computed from a clamped row and not written), by
+// WM x WN wavefronts of 64 rows each.  Per 32-column chunk the tile's row and
+// column records (128 bytes a row, panel_rec) are staged in LDS -- 144 bytes
+// apart, so that the 16 rows of an MFMA operand fall in distinct banks -- and
+// multiplied from there: split-BF16 hi hi + hi lo + lo hi on 16x16x32 MFMA,
+// FP32 on 16x16x4.  Two LDS buffers and D chunks in registers: while chunk k
+// is multiplied, chunk k+1 is written to the other buffer and chunks k+2 ..
+// k+1+D are on their way; one barrier per chunk.  Bound by the operands: a CU's
+// vector loads bring 37 GB/s from L2 or beyond, a 256x256 tile's 1 MB 28 us,
+// its split-BF16 products 23 us (one buffer, two barriers and the next chunk
+// only took 59 us).
+static constexpr int kLdsRec = kCholRecord + 16;
+template <int MODE, int TM, int TN, int WM, int WN, int D>
+__device__ __forceinline__ void update_tile(float* __restrict__ M, size_t ld, int mp, int kw,
+                                            const char* __restrict__ pan, int r0, int c0, char* __restrict__ lds) {
+    constexpr int TH = 64 * WM * WN, BUF = (TM + TN) * kLdsRec;
+    constexpr int UN = (TM + TN) * (kCholRecord / 16) / TH;  // 16-byte units per thread and chunk
+    constexpr int NI = TM / WM / 16, NJ = TN / WN / 16;      // 16x16 tiles per wavefront
+    static_assert(UN * TH * 16 == (TM + TN) * kCholRecord, "the threads divide a chunk evenly");
+    using V = typename std::conditional<MODE == SOP_CHOL_BF16X3, bf16x8, f32x4>::type;
+    const int tid = threadIdx.x, l = tid & 63, w = wave_of(), wr = (w / WN) * (TM / WM), wc = (w % WN) * (TN / WN);
+    const int lr = l & 15, lk = l >> 4;
+    // the thread's units: row (of the row, then the column operand) and 16-byte unit
+    unsigned src[UN], dst[UN];
 #pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const size_t row = rb + 16 * bi + 4 * (l >> 4) + q;
-                const size_t col = cb + 16 * bj + (l & 15);
-                if (row >= (size_t)mp || col >= (size_t)ce || col > row) continue;
-                M[row * ld + col] -= acc[bi][bj][q];
-            }
-}
-
-// Operands of the next K-chunk are loaded into registers while the MFMAs of
-// the current chunk run from LDS; they are stored to LDS after the chunk.
-__global__ __launch_bounds__(256) void k_gemm_bf16x3(float* __restrict__ M, size_t ld, int s, int mp, int kw,
-                                                     const unsigned short* __restrict__ phi,
-                                                     const unsigned short* __restrict__ plo) {
-    __shared__ __attribute__((aligned(16))) unsigned short sa[2][GT][LPB];  // hi, lo of the row tile
-    __shared__ __attribute__((aligned(16))) unsigned short sb[2][GT][LPB];  // hi, lo of the column tile
-    const int ce = mp;
-    size_t r0, c0;
-    if (!big_tile(s, r0, c0)) return;
-    const int tid = threadIdx.x, l = tid & 63, w = wave_of();
-    const int lr = l & 15, lk = (l >> 4) * 8;
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // loader: thread t moves 16 bf16 (two 16-byte words) of row t/2 per array
-    const int ldr = tid >> 1, ldk = (tid & 1) * 16;
-    const size_t ga = r0 + ldr, gb = c0 + ldr;
-    const bool va = ga < (size_t)mp, vb = gb < (size_t)ce;
-    uint4 v[8];
-    auto fetch = [&](int kc) {
-        const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-        if (va) {
-            const uint4* ph = reinterpret_cast<const uint4*>(phi + ga * NB2 + kc + ldk);
-            const uint4* pl = reinterpret_cast<const uint4*>(plo + ga * NB2 + kc + ldk);
-            v[0] = ph[0], v[1] = ph[1], v[2] = pl[0], v[3] = pl[1];
-        } else {
-            v[0] = v[1] = v[2] = v[3] = z;
-        }
-        if (vb) {
-            const uint4* ph = reinterpret_cast<const uint4*>(phi + gb * NB2 + kc + ldk);
-            const uint4* pl = reinterpret_cast<const uint4*>(plo + gb * NB2 + kc + ldk);
-            v[4] = ph[0], v[5] = ph[1], v[6] = pl[0], v[7] = pl[1];
-        } else {
-            v[4] = v[5] = v[6] = v[7] = z;
-        }
-    };
-    auto stash = [&]() {
-        *reinterpret_cast<uint4*>(&sa[0][ldr][ldk]) = v[0];
-        *reinterpret_cast<uint4*>(&sa[0][ldr][ldk + 8]) = v[1];
-        *reinterpret_cast<uint4*>(&sa[1][ldr][ldk]) = v[2];
-        *reinterpret_cast<uint4*>(&sa[1][ldr][ldk + 8]) = v[3];
-        *reinterpret_cast<uint4*>(&sb[0][ldr][ldk]) = v[4];
-        *reinterpret_cast<uint4*>(&sb[0][ldr][ldk + 8]) = v[5];
-        *reinterpret_cast<uint4*>(&sb[1][ldr][ldk]) = v[6];
-        *reinterpret_cast<uint4*>(&sb[1][ldr][ldk + 8]) = v[7];
-    };
-    fetch(0);
-    stash();
-    __syncthreads();
-    const int ra = 64 * (w >> 1) + lr, rbb = 64 * (w & 1) + lr;
-    for (int kc = 0; kc < kw; kc += KCB) {
-        const bool more = kc + KCB < kw;
-        if (more) fetch(kc + KCB);
-        bf16x8 ah[4], al[4], bh[4], bl[4];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            ah[b] = *reinterpret_cast<const bf16x8*>(&sa[0][ra + 16 * b][lk]);
-            al[b] = *reinterpret_cast<const bf16x8*>(&sa[1][ra + 16 * b][lk]);
-            bh[b] = *reinterpret_cast<const bf16x8*>(&sb[0][rbb + 16 * b][lk]);
-            bl[b] = *reinterpret_cast<const bf16x8*>(&sb[1][rbb + 16 * b][lk]);
-        }
-        // the three products in separate sweeps over the sixteen accumulators,
-        // so consecutive MFMAs never wait on each other's results
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[bi], bh[bj], acc[bi][bj], 0, 0, 0);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[bi], bl[bj], acc[bi][bj], 0, 0, 0);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[bi], bh[bj], acc[bi][bj], 0, 0, 0);
-        if (more) {
-            __syncthreads();  // every wave has read this chunk's operands
-            stash();
-            __syncthreads();
-        }
+    for (int i = 0; i < UN; ++i) {
+        const int e = tid + TH * i, r = e / 8, u = e % 8;
+        const int g = min(r < TM ? r0 + r : c0 + r - TM, mp - 1);
+        src[i] = (unsigned)g * kCholRecord + 16 * u;
+        dst[i] = r * kLdsRec + 16 * u;
     }
-    big_store(M, ld, mp, ce, r0, c0, acc);
+    typedef const __attribute__((address_space(1))) char* gptr;
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const int nch = kw / 32;
+    u32x4 v[D][UN];
+    auto fetch = [&](u32x4 (&x)[UN], int k) {
+        const gptr p = (gptr)pan + (size_t)min(k, nch - 1) * mp * kCholRecord;
+#pragma unroll
+        for (int i = 0; i < UN; ++i) x[i] = *reinterpret_cast<const __attribute__((address_space(1))) u32x4*>(p + src[i]);
+    };
+    auto stash = [&](const u32x4 (&x)[UN], int buf) {
+#pragma unroll
+        for (int i = 0; i < UN; ++i) *reinterpret_cast<u32x4*>(lds + buf * BUF + dst[i]) = x[i];
+    };
+    f32x4 acc[NI][NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    fetch(v[0], 0);
+    stash(v[0], 0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) fetch(v[d], 1 + d);
+    __syncthreads();
+    auto at = [&](int buf, int r, int half) {
+        return *reinterpret_cast<const V*>(lds + buf * BUF + r * kLdsRec + (kCholRecord / 2) * half + 16 * lk);
+    };
+    auto chunk = [&](int k, u32x4 (&x)[UN]) {
+        stash(x, (k + 1) & 1);
+        fetch(x, k + 1 + D);
+        __builtin_amdgcn_sched_barrier(0);
+        const int buf = k & 1;
+        V a0[NI], a1[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            a0[i] = at(buf, wr + 16 * i + lr, 0);
+            a1[i] = at(buf, wr + 16 * i + lr, 1);
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const V b0 = at(buf, TM + wc + 16 * j + lr, 0), b1 = at(buf, TM + wc + 16 * j + lr, 1);
+            if constexpr (MODE == SOP_CHOL_BF16X3) {
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[i], b0, acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[i], b1, acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], b0, acc[i][j], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int i = 0; i < NI; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[i][c], b0[c], acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int i = 0; i < NI; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[i][c], b1[c], acc[i][j], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    };
+    // kw is a multiple of 64: an even number of chunks
+    for (int k = 0; k < nch; k += 2) {
+        chunk(k, v[0]);
+        chunk(k + 1, v[D - 1]);
+    }
+    // C -= acc: D rows 4(l/16) + q, column l%16 of each 16x16 tile
+    constexpr int NB_ = 32;  // elements of a lane at a time
+#pragma unroll
+    for (int h = 0; h < NI * NJ * 4; h += NB_) {
+        int row[NB_], col[NB_];
+        float x[NB_];
+#pragma unroll
+        for (int e = 0; e < NB_; ++e) {
+            const int t = (h + e) / 4, i = t / NJ, j = t % NJ, q = e % 4;
+            row[e] = r0 + wr + 16 * i + 4 * lk + q;
+            col[e] = c0 + wc + 16 * j + lr;
+            x[e] = acc[i][j][q];
+        }
+        sub_store(M, ld, mp, row, col, x);
+    }
 }
 
-// Split-BF16 trailing update on 256x256 tiles for the large trailing
-// regions: four times the MFMA work of a 128x128 tile per operand byte
-// staged, half the operand traffic per flop.  One workgroup of eight
-// wavefronts per CU (two per SIMD); wavefront w forms the 64x128 block
-// (w>>1, w&1) as 2x4 tiles of 32x32 on v_mfma_f32_32x32x16_bf16 (lane l:
-// A[i=l%32][k=8(l/32)..+7], B[k=8(l/32)..+7][j=l%32], D row
-// 8(q/4)+4(l/32)+q%4, column l%32 in accumulator register q).  Per
-// 32-column chunk the hi and lo halves of the tile's 256 panel rows and 256
-// panel columns (64 KB) are staged in LDS in 16-byte units, unit u of row r
-// stored at u ^ ((r >> 1) & 3) so that the eight lanes of each read phase
-// hit distinct banks; the next chunk is loaded into registers while the
-// current one is multiplied.  Tiles are numbered over the lower triangle
-// row by row and dealt to the XCDs in contiguous ranges (workgroup i runs
-// on XCD i % 8), so the tiles an XCD holds at once share their row panels
-// in its L2.
-static constexpr int BT = 256;  // tile edge
-static constexpr int BK = 32;   // K chunk (bf16 elements): four 16-byte units per row
-constexpr int kXcds = 8;        // MI355X: workgroup i is dispatched to XCD i % 8
-
-__device__ __forceinline__ int swz(int r, int u) { return u ^ ((r >> 1) & 3); }
-
-// The loader of k_trail_bf16x3: thread t moves unit t%4 of rows t/4 and
-// t/4 + 128, hi and lo, of the row panel (rows from r0) and of the column
-// panel (rows from c0) -- eight 16-byte loads, zeros past row mp -- into v,
-// and v into LDS.  Written as macros: the same code as helper functions or
-// lambdas makes this compiler (ROCm 7.2 clang) crash in its machine copy
-// propagation pass.
-#define TRAIL_FETCH(KC)                                                                       \
-    for (int pnl = 0; pnl < 2; ++pnl)                                                         \
-        for (int q = 0; q < 2; ++q) {                                                         \
-            const size_t g = (pnl ? c0 : r0) + (size_t)(lrow + 128 * q);                      \
-            if (g < (size_t)mp) {                                                             \
-                const size_t off = g * NB2 + (size_t)(KC) + 8 * lu;                           \
-                v[pnl][0][q] = *reinterpret_cast<const uint4*>(phi + off);                    \
-                v[pnl][1][q] = *reinterpret_cast<const uint4*>(plo + off);                    \
-            } else {                                                                          \
-                v[pnl][0][q] = v[pnl][1][q] = make_uint4(0u, 0u, 0u, 0u);                     \
-            }                                                                                 \
-        }
-#define TRAIL_STASH()                                                                         \
-    for (int pnl = 0; pnl < 2; ++pnl)                                                         \
-        for (int h = 0; h < 2; ++h)                                                           \
-            for (int q = 0; q < 2; ++q) {                                                     \
-                const int r = lrow + 128 * q;                                                 \
-                sm[pnl][h][r][swz(r, lu)] = v[pnl][h][q];                                     \
-            }
-
-__global__ __launch_bounds__(512) void k_trail_bf16x3(float* __restrict__ M, size_t ld, int s, int mp, int kw,
-                                                      int ntr, const unsigned short* __restrict__ phi,
-                                                      const unsigned short* __restrict__ plo) {
-    __shared__ uint4 sm[2][2][BT][BK / 8];  // [row panel, column panel][hi, lo][row][unit]: 64 KB
+// Regions [s, mp) x [s, mp): 256x256 tiles by eight wavefronts, one workgroup
+// per CU, numbered over the lower triangle row by row and dealt to the XCDs in
+// contiguous ranges (workgroup i runs on XCD i % 8), so the tiles an XCD holds
+// at once share their row panels in its L2.
+static constexpr int BT = 256;
+constexpr int kXcds = 8;
+template <int MODE>
+__global__ __launch_bounds__(512) void k_update_big(float* __restrict__ M, size_t ld, int s, int mp, int kw, int ntr,
+                                                    const char* __restrict__ pan) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * 2 * BT * kLdsRec];
     const int ntile = ntr * (ntr + 1) / 2, per = (ntile + kXcds - 1) / kXcds;
     const int t = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
-    if (t >= ntile) return;
+    if ((int)(blockIdx.x / kXcds) >= per || t >= ntile) return;
     int bi = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
     while (bi * (bi + 1) / 2 > t) --bi;
     while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
     const int bj = t - bi * (bi + 1) / 2;
-    const size_t r0 = (size_t)s + (size_t)BT * bi, c0 = (size_t)s + (size_t)BT * bj;
-    const int tid = threadIdx.x, l = tid & 63, w = wave_of();
-    // loader: thread t moves unit t%4 of rows t/4 and t/4 + 128, hi and lo,
-    // of the row panel and of the column panel: eight 16-byte loads
-    const int lu = tid & 3, lrow = tid >> 2;
-    uint4 v[2][2][2];
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x16{};
-    TRAIL_FETCH(0);
-    TRAIL_STASH();
-    __syncthreads();
-    const int wr = 64 * (w >> 1), wc = 128 * (w & 1), li = l & 31, lk = l >> 5;
-    for (int kc = 0; kc < kw; kc += BK) {
-        const bool more = kc + BK < kw;
-        if (more) { TRAIL_FETCH(kc + BK); }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {  // two K = 16 substeps per chunk
-            const int u = 2 * ks + lk;
-            bf16x8 ah[2], al[2], bh[4], bl[4];
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int ra = wr + 32 * b + li;
-                const uint4 xa = sm[0][0][ra][swz(ra, u)], ya = sm[0][1][ra][swz(ra, u)];
-                ah[b] = *reinterpret_cast<const bf16x8*>(&xa);
-                al[b] = *reinterpret_cast<const bf16x8*>(&ya);
-            }
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const int rb = wc + 32 * b + li;
-                const uint4 xb = sm[1][0][rb][swz(rb, u)], yb = sm[1][1][rb][swz(rb, u)];
-                bh[b] = *reinterpret_cast<const bf16x8*>(&xb);
-                bl[b] = *reinterpret_cast<const bf16x8*>(&yb);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) {
-            __syncthreads();  // every wave has read this chunk
-            TRAIL_STASH();
-            __syncthreads();
-        }
-    }
-    // C -= acc over the lower triangle of the tile, rows below mp
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const size_t row = r0 + wr + 32 * i + 8 * (q >> 2) + 4 * lk + (q & 3);
-                const size_t col = c0 + wc + 32 * j + li;
-                if (row >= (size_t)mp || col > row) continue;
-                M[row * ld + col] -= acc[i][j][q];
-            }
+    update_tile<MODE, BT, BT, 4, 2, 1>(M, ld, mp, kw, pan, s + BT * bi, s + BT * bj, lds);
 }
-#undef TRAIL_FETCH
-#undef TRAIL_STASH
 
-// FP32 trailing update: operands are the panel columns [pc, pc+kw) of M.
-// LDS rows hold a K-chunk of 16 permuted so that lane group g = l/16 reads
-// k = g, g+4, g+8, g+12 (its four MFMA steps) as one float4.  The next
-// chunk is loaded into registers during the current chunk's MFMAs.
-__global__ __launch_bounds__(256) void k_gemm_f32(float* __restrict__ M, size_t ld, int s, int mp, int pc, int kw) {
-    __shared__ __attribute__((aligned(16))) float sa[GT][LPF];
-    __shared__ __attribute__((aligned(16))) float sb[GT][LPF];
-    const int ce = mp;
-    size_t r0, c0;
-    if (!big_tile(s, r0, c0)) return;
-    const int tid = threadIdx.x, l = tid & 63, w = wave_of();
-    const int lr = l & 15, lg = l >> 4;
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 4; ++bj) acc[bi][bj] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // loader: thread t moves 8 floats (two float4, k = 8h..8h+7) of row t/2
-    const int ldr = tid >> 1, h = tid & 1;
-    const size_t ga = r0 + ldr, gb = c0 + ldr;
-    const bool va = ga < (size_t)mp, vb = gb < (size_t)ce;
-    float4 a0, a1, b0, b1;
-    auto fetch = [&](int kc) {
-        a0 = a1 = b0 = b1 = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (va) {
-            const float4* pa = reinterpret_cast<const float4*>(M + ga * ld + pc + kc + 8 * h);
-            a0 = pa[0], a1 = pa[1];
-        }
-        if (vb) {
-            const float4* pb = reinterpret_cast<const float4*>(M + gb * ld + pc + kc + 8 * h);
-            b0 = pb[0], b1 = pb[1];
-        }
-    };
-    // element k (0..15) goes to position (k%4)*4 + k/4
-    auto stash = [&]() {
-        const int q0 = 2 * h, q1 = 2 * h + 1;  // k/4 of a0 and a1
-        sa[ldr][0 + q0] = a0.x, sa[ldr][4 + q0] = a0.y, sa[ldr][8 + q0] = a0.z, sa[ldr][12 + q0] = a0.w;
-        sa[ldr][0 + q1] = a1.x, sa[ldr][4 + q1] = a1.y, sa[ldr][8 + q1] = a1.z, sa[ldr][12 + q1] = a1.w;
-        sb[ldr][0 + q0] = b0.x, sb[ldr][4 + q0] = b0.y, sb[ldr][8 + q0] = b0.z, sb[ldr][12 + q0] = b0.w;
-        sb[ldr][0 + q1] = b1.x, sb[ldr][4 + q1] = b1.y, sb[ldr][8 + q1] = b1.z, sb[ldr][12 + q1] = b1.w;
-    };
-    fetch(0);
-    stash();
-    __syncthreads();
-    const int ra = 64 * (w >> 1) + lr, rbb = 64 * (w & 1) + lr;
-    for (int kc = 0; kc < kw; kc += KCF) {
-        const bool more = kc + KCF < kw;
-        if (more) fetch(kc + KCF);
-        float4 av[4], bv[4];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            av[b] = *reinterpret_cast<const float4*>(&sa[ra + 16 * b][4 * lg]);
-            bv[b] = *reinterpret_cast<const float4*>(&sb[rbb + 16 * b][4 * lg]);
-        }
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[bi].x, bv[bj].x, acc[bi][bj], 0, 0, 0);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[bi].y, bv[bj].y, acc[bi][bj], 0, 0, 0);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[bi].z, bv[bj].z, acc[bi][bj], 0, 0, 0);
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-                acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[bi].w, bv[bj].w, acc[bi][bj], 0, 0, 0);
-        if (more) {
-            __syncthreads();
-            stash();
-            __syncthreads();
-        }
-    }
-    big_store(M, ld, mp, ce, r0, c0, acc);
+// Tile (blockIdx.x, blockIdx.y) of the lower triangle from row and column s
+// on: TM x TN tiles by four wavefronts.
+template <int MODE, int TM, int TN>
+__global__ __launch_bounds__(256, 2) void k_update(float* __restrict__ M, size_t ld, int s, int mp, int kw,
+                                                   const char* __restrict__ pan) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * (TM + TN) * kLdsRec];
+    const int r0 = s + (int)blockIdx.x * TM, c0 = s + (int)blockIdx.y * TN;
+    if (c0 >= r0 + TM || c0 >= mp) return;  // wholly above the diagonal, or past the last column
+    update_tile<MODE, TM, TN, 2, 2, 2>(M, ld, mp, kw, pan, r0, c0, lds);
 }
 
 // ---- the factorisation by fused 64-column steps -----------------------------
@@ -1339,9 +1180,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(float* __restrict__ M, size_t 
 //      Li^T the inverse of L_{j-1,j-1} (FP64 accumulation), written to M and,
 //      split-BF16 mode, to the panel copy;
 //  (2) for j < nb, column block j of each row block minus the products of
-//      every column to its left that no trailing update has applied: the
-//      previous outer panel's columns (its lookahead update, folded in here)
-//      and this panel's columns 0 .. 64j-1, on MFMA:
+//      this panel's columns 0 .. 64j-1, on MFMA:
 //      B_g = A_gj - sum_k X_gk X_dk^T.  Workgroup 0 (g = d) factors B in
 //      FP64 into L_jj and its inverse; the others store B for step j+1.
 // Every workgroup forms X_d for (2) itself (the diagonal row block's solve,
@@ -1354,8 +1193,12 @@ __global__ __launch_bounds__(256) void k_gemm_f32(float* __restrict__ M, size_t 
 // diagonal workgroup then only subtracts X_d,j-1 X_d,j-1^T (64 columns)
 // before it factors.  The panel's first step has no such block and forms
 // the whole sum.
-// The trailing matrix beyond the next panel is updated by the wide MFMA
-// kernels on the second stream, one pass per outer panel.
+// A finished panel's update of the next panel's columns runs between the two
+// panels' steps, that of the rest of the trailing matrix on the second stream
+// beside the next panel's steps, both by the wide MFMA kernels.  (Folded into
+// the next panel's steps, the former made each of them read 128 KB of panel
+// columns per row block again: at the 37 GB/s a CU's vector loads reach, the
+// row blocks took 20-26 us a step and not the diagonal workgroup's 14.)
 static constexpr int XS = NB + 4;  // row stride of the FP32 X blocks in LDS (16-byte rows)
 
 struct CholStep {
@@ -1363,7 +1206,6 @@ struct CholStep {
     size_t ld;
     int mp;
     int c0, kw;                      // this outer panel
-    int pc, pkw;                     // the previous outer panel (pkw = 0: none)
     int j;                           // step 0 .. nb
     const void* li_in;               // Li^T of column block j-1 (64 x 64 CholReal, row a = column a of Li)
     void* li_out;                    // Li^T of column block j
@@ -1372,175 +1214,172 @@ struct CholStep {
     const float* p_in;               // the diagonal block's P formed by the previous step (j >= 1)
     float* p_out;                    // the next diagonal block's P (when look)
     int look;                        // 1: an extra workgroup forms P for step j+1
-    unsigned short *phi, *plo;       // this panel's split-BF16 copy, mp x NB2
-    const unsigned short *pphi, *pplo;  // the previous panel's copy
+    char* pan;                       // this panel's copy (panel_rec)
 };
 
-// The 64 values of B a lane feeds the solve's MFMAs: B[16w + l%16][4s + l/16]
-// for s = 0..15 (B is 64 x 64 FP32, rows r0.. of a row-major mp x 64 buffer).
-__device__ __forceinline__ void load_solve_rows(const float* __restrict__ b, size_t r0, float (&bv)[16]) {
-    const int l = threadIdx.x & 63, w = wave_of();
-    const float* __restrict__ row = b + (r0 + 16 * w + (l & 15)) * NB + (l >> 4);
+// The 64 values of B a lane feeds the solve's MFMAs, four 16-byte loads: in
+// step 4m + i of the sum over t, lane group l/16 takes t = 16m + 4(l/16) + i
+// (B[16(w%4) + l%16][t]; B is 64 x 64 FP32, rows r0.. of a row-major mp x 64
+// buffer).
+__device__ __forceinline__ void load_solve_rows(const float* __restrict__ b, size_t r0, float4 (&bv)[4]) {
+    const int l = threadIdx.x & 63, w = wave_of() & 3;
+    const float* __restrict__ row = b + (r0 + 16 * w + (l & 15)) * NB + 4 * (l >> 4);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) bv[q] = row[4 * q];
+    for (int m = 0; m < 4; ++m) bv[m] = *reinterpret_cast<const float4*>(row + 16 * m);
 }
 
 // X = B Li^T for one 64x64 block on MFMA in CholReal (B from
 // load_solve_rows, LiT[t*LDT + c] = Li[c][t], zero for t > c), to Xs (LDS,
 // row stride XS) and, when `out`, to M (rows r0.., columns col0..) and the
-// panel copy (columns pcol0..).  Wave w forms rows 16w..16w+15; output
-// block jb (columns 16jb..) sums t < 16(jb+1) only, where Li^T is not zero.
-template <int MODE>
-__device__ __forceinline__ void solve_block(const float (&bv)[16], const CholReal<MODE>* __restrict__ LiT,
+// panel copy (columns pcol0.. of the panel).  Wavefront w forms rows 16(w%4) .. +15 of the
+// output blocks jb (columns 16jb..) in JBS (a bit each); block jb sums
+// t < 16(jb+1) only, where Li^T is not zero.
+template <int MODE, int JBS>
+__device__ __forceinline__ void solve_block(const float4 (&bv)[4], const CholReal<MODE>* __restrict__ LiT,
                                             float* __restrict__ Xs, bool out, float* __restrict__ M, size_t ld,
-                                            size_t r0, size_t col0, unsigned short* __restrict__ phi,
-                                            unsigned short* __restrict__ plo, int pcol0) {
+                                            size_t mp, size_t r0, size_t col0, char* __restrict__ pan,
+                                            int pcol0) {
     using R = CholReal<MODE>;
-    constexpr int LDT = ldt<R>();
-    const int l = threadIdx.x & 63, w = wave_of(), lr = l & 15, lk = l >> 4;
+    const int l = threadIdx.x & 63, w = wave_of() & 3, lr = l & 15, lk = l >> 4;
     R4<R> acc[4];
 #pragma unroll
     for (int jb = 0; jb < 4; ++jb) acc[jb] = R4<R>{R(0), R(0), R(0), R(0)};
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int t0 = 4 * q;
-        const R a = (R)bv[q];
+    for (int m = 0; m < 4; ++m) {
+        const float av[4] = {bv[m].x, bv[m].y, bv[m].z, bv[m].w};
 #pragma unroll
-        for (int jb = 0; jb < 4; ++jb)
-            if (t0 < 16 * (jb + 1)) acc[jb] = mfma16(a, LiT[(t0 + lk) * LDT + 16 * jb + lr], acc[jb]);
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int jb = 0; jb < 4; ++jb)
+                if (((JBS >> jb) & 1) && m <= jb)
+                    acc[jb] = mfma16((R)av[i], LiT[(16 * m + 4 * lk + i) * LDT + 16 * jb + lr], acc[jb]);
     }
 #pragma unroll
     for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
+            if (!((JBS >> jb) & 1)) continue;
             const int row = 16 * w + drow<R>(lk, v), c = 16 * jb + lr;
             const float x = (float)acc[jb][v];
             Xs[row * XS + c] = x;
             if (!out) continue;
             M[(r0 + row) * ld + col0 + c] = x;
+            char* const rec = pan + panel_rec(mp, (pcol0 + 16 * jb) / 32, r0 + row);
+            const int e = 16 * (jb & 1) + lr;
             if constexpr (MODE == SOP_CHOL_BF16X3) {
                 const unsigned short h = f2bf(x);
-                phi[(r0 + row) * NB2 + pcol0 + c] = h;
-                plo[(r0 + row) * NB2 + pcol0 + c] = f2bf(x - bf2f(h));
+                reinterpret_cast<unsigned short*>(rec)[e] = h;
+                reinterpret_cast<unsigned short*>(rec)[32 + e] = f2bf(x - bf2f(h));
+            } else {
+                reinterpret_cast<float*>(rec)[e] = x;
             }
         }
 }
 
-// acc += X_g X_d^T (the full 64x64 block, 4x4 MFMA tiles) over this
-// wavefront's share of the columns left of column block j-1 that no
-// trailing update has applied: the previous panel's pkw columns, then this
-// panel's first 64(j-1).  Those columns are cut into chunks (32 columns
-// split-BF16, 16 FP32) dealt to the four wavefronts in turn; each keeps one
-// chunk's operands in flight while the MFMAs of the previous one run.
-// SYM (the diagonal block, g = d): the rows are loaded once and only the
-// tiles on and below the diagonal are formed (the factorisation reads the
-// lower triangle); each of them sums the same products in the same order.
-template <int MODE, bool SYM>
-__device__ __forceinline__ void mfma_split(f32x4 (&acc)[4][4], const CholStep& a, size_t rg, size_t rd) {
-    const int l = threadIdx.x & 63, w = wave_of(), lr = l & 15;
-    constexpr int CW = MODE == SOP_CHOL_BF16X3 ? 32 : 16;
-    const int n1 = a.pkw / CW, n = n1 + (a.j >= 2 ? NB * (a.j - 1) : 0) / CW;
-    if constexpr (MODE == SOP_CHOL_BF16X3) {
-        const int lk = (l >> 4) * 8;
-        struct Ops {
-            bf16x8 ah[4], al[4], bh[4], bl[4];
-        };
-        auto load = [&](Ops& o, int c) {
-            const unsigned short* __restrict__ ph = c < n1 ? a.pphi : a.phi;
-            const unsigned short* __restrict__ pl = c < n1 ? a.pplo : a.plo;
-            const int col = (c < n1 ? c : c - n1) * CW + lk;
+// acc += X_g X_d^T over this wavefront's share of the panel's columns left of
+// column block j-1, 64(j-1) of them.  Wavefront w forms the half
+// h = w/4 of the 64x64 block (rows 0..63, columns 32h .. 32h+31: 4x2 MFMA
+// tiles) from the 32-column chunks w%4, w%4 + 4, .., the next chunk's operands
+// in flight while one is multiplied.
+template <int MODE>
+__device__ __forceinline__ void mfma_split(f32x4 (&acc)[4][2], const CholStep& a, size_t rg, size_t rd) {
+    const int l = threadIdx.x & 63, w = wave_of(), kq = w & 3, h = w >> 2, lr = l & 15, lk = l >> 4;
+    const int n = (a.j >= 2 ? NB * (a.j - 1) : 0) / 32;
+    typedef const __attribute__((address_space(1))) char* gptr;
+    // byte offsets of the lane's rows within a chunk (128 bytes a row: 32 bits
+    // hold 33 million rows); lane group l/16 reads 16 bytes of each half record
+    unsigned ao[4], bo[2];
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const size_t ao = (rg + 16 * b + lr) * NB2 + col, bo = (rd + 16 * b + lr) * NB2 + col;
-                o.ah[b] = *reinterpret_cast<const bf16x8*>(ph + ao);
-                o.al[b] = *reinterpret_cast<const bf16x8*>(pl + ao);
-                if constexpr (!SYM) {
-                    o.bh[b] = *reinterpret_cast<const bf16x8*>(ph + bo);
-                    o.bl[b] = *reinterpret_cast<const bf16x8*>(pl + bo);
-                }
-            }
-        };
-        auto mma = [&](const Ops& o) {
-            const bf16x8(&bh)[4] = SYM ? o.ah : o.bh;
-            const bf16x8(&bl)[4] = SYM ? o.al : o.bl;
+    for (int b = 0; b < 4; ++b) ao[b] = (unsigned)(rg + 16 * b + lr) * kCholRecord + 16 * lk;
 #pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
+    for (int b = 0; b < 2; ++b) bo[b] = (unsigned)(rd + 32 * h + 16 * b + lr) * kCholRecord + 16 * lk;
+    auto chunk = [&](int c) { return (gptr)a.pan + (size_t)c * a.mp * kCholRecord; };
+    // the two halves of a record: split-BF16 hi and lo of k = 8(l/16) .. +7;
+    // FP32 k = 4(l/16) .. +3 and 16 further on, MFMA step i taking component i
+    using V = typename std::conditional<MODE == SOP_CHOL_BF16X3, bf16x8, f32x4>::type;
+    auto at = [](gptr p, unsigned off) {
+        return *reinterpret_cast<const __attribute__((address_space(1))) V*>(p + off);
+    };
+    struct Ops {
+        V a0[4], a1[4], b0[2], b1[2];
+    };
+    auto load = [&](Ops& o, int c) {
+        const gptr p = chunk(c);
 #pragma unroll
-                for (int bj = 0; bj < 4; ++bj)
-                    if (!SYM || bj <= bi)
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.ah[bi], bh[bj], acc[bi][bj], 0, 0, 0);
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-                for (int bj = 0; bj < 4; ++bj)
-                    if (!SYM || bj <= bi)
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.ah[bi], bl[bj], acc[bi][bj], 0, 0, 0);
-#pragma unroll
-            for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-                for (int bj = 0; bj < 4; ++bj)
-                    if (!SYM || bj <= bi)
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.al[bi], bh[bj], acc[bi][bj], 0, 0, 0);
-        };
-        Ops o0, o1;
-        if (w < n) load(o0, w);
-        for (int c = w; c < n; c += 8) {
-            if (c + 4 < n) load(o1, c + 4);
-            mma(o0);
-            if (c + 4 >= n) break;
-            if (c + 8 < n) load(o0, c + 8);
-            mma(o1);
+        for (int b = 0; b < 4; ++b) {
+            o.a0[b] = at(p, ao[b]);
+            o.a1[b] = at(p + kCholRecord / 2, ao[b]);
         }
-    } else {
-        // lane group g = l/16 holds k = 4g .. 4g+3 of a 16-column chunk (one
-        // 16-byte load); MFMA step i takes component i
-        const int lg = l >> 4;
-        struct Ops {
-            float4 a[4], b[4];
-        };
-        auto load = [&](Ops& o, int c) {
-            const size_t col = (c < n1 ? (size_t)a.pc + (size_t)c * CW : (size_t)a.c0 + (size_t)(c - n1) * CW) + 4 * lg;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                o.a[b] = *reinterpret_cast<const float4*>(a.M + (rg + 16 * b + lr) * a.ld + col);
-                if constexpr (!SYM) o.b[b] = *reinterpret_cast<const float4*>(a.M + (rd + 16 * b + lr) * a.ld + col);
-            }
-        };
-        auto mma = [&](const Ops& o) {
-            const float4(&ob)[4] = SYM ? o.a : o.b;
+        for (int b = 0; b < 2; ++b) {
+            o.b0[b] = at(p, bo[b]);
+            o.b1[b] = at(p + kCholRecord / 2, bo[b]);
+        }
+    };
+    auto mma = [&](const Ops& o) {
+        if constexpr (MODE == SOP_CHOL_BF16X3) {
 #pragma unroll
             for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
-                for (int bj = 0; bj < 4; ++bj)
-                    if (!SYM || bj <= bi) {
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[bi].x, ob[bj].x, acc[bi][bj], 0, 0, 0);
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[bi].y, ob[bj].y, acc[bi][bj], 0, 0, 0);
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[bi].z, ob[bj].z, acc[bi][bj], 0, 0, 0);
-                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[bi].w, ob[bj].w, acc[bi][bj], 0, 0, 0);
-                    }
-        };
-        Ops o0, o1;
-        if (w < n) load(o0, w);
-        for (int c = w; c < n; c += 8) {
-            if (c + 4 < n) load(o1, c + 4);
-            mma(o0);
-            if (c + 4 >= n) break;
-            if (c + 8 < n) load(o0, c + 8);
-            mma(o1);
+                for (int bj = 0; bj < 2; ++bj)
+                    acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a0[bi], o.b0[bj], acc[bi][bj], 0, 0, 0);
+#pragma unroll
+            for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+                for (int bj = 0; bj < 2; ++bj)
+                    acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a0[bi], o.b1[bj], acc[bi][bj], 0, 0, 0);
+#pragma unroll
+            for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+                for (int bj = 0; bj < 2; ++bj)
+                    acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.a1[bi], o.b0[bj], acc[bi][bj], 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+                    for (int bj = 0; bj < 2; ++bj)
+                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a0[bi][i], o.b0[bj][i], acc[bi][bj], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int bi = 0; bi < 4; ++bi)
+#pragma unroll
+                    for (int bj = 0; bj < 2; ++bj)
+                        acc[bi][bj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a1[bi][i], o.b1[bj][i], acc[bi][bj], 0, 0, 0);
         }
+    };
+    // loads without branches (a last chunk again past the end) and held in
+    // place: moved or merged by the compiler, the products of one chunk waited
+    // for the next one's operands
+    if (kq >= n) return;
+    Ops o0, o1;
+    load(o0, kq);
+    for (int c = kq; c < n; c += 8) {
+        load(o1, min(c + 4, n - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        mma(o0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + 4 >= n) break;
+        load(o0, min(c + 8, n - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        mma(o1);
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
 // The same over the 64 columns of the X blocks just solved, from LDS; in
-// split-BF16 mode each value is split as the panel copy holds it.
+// split-BF16 mode each value is split as the panel copy holds it.  Wavefront w
+// forms tiles 2(w/4) and the next one of tile row w%4.
 template <int MODE>
-__device__ __forceinline__ void mfma_lds(f32x4 (&acc)[4], const float* __restrict__ Xg, const float* __restrict__ Xd) {
-    const int l = threadIdx.x & 63, w = wave_of(), lr = l & 15;
+__device__ __forceinline__ void mfma_lds(f32x4 (&acc)[2], const float* __restrict__ Xg, const float* __restrict__ Xd) {
+    const int l = threadIdx.x & 63, w = wave_of() & 3, t0 = 2 * (wave_of() >> 2), lr = l & 15;
     if constexpr (MODE == SOP_CHOL_BF16X3) {
         const int lk = (l >> 4) * 8;
 #pragma unroll
         for (int kc = 0; kc < NB; kc += 32) {
-            bf16x8 ah, al, bh[4], bl[4];
+            bf16x8 ah, al, bh[2], bl[2];
             const float* a = Xg + (16 * w + lr) * XS + kc + lk;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -1549,8 +1388,8 @@ __device__ __forceinline__ void mfma_lds(f32x4 (&acc)[4], const float* __restric
                 al[e] = (short)f2bf(a[e] - bf2f(h));
             }
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const float* b = Xd + (16 * t + lr) * XS + kc + lk;
+            for (int t = 0; t < 2; ++t) {
+                const float* b = Xd + (16 * (t0 + t) + lr) * XS + kc + lk;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const unsigned short h = f2bf(b[e]);
@@ -1559,49 +1398,50 @@ __device__ __forceinline__ void mfma_lds(f32x4 (&acc)[4], const float* __restric
                 }
             }
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[t], acc[t], 0, 0, 0);
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[t], acc[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[t], acc[t], 0, 0, 0);
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[t], acc[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[t], acc[t], 0, 0, 0);
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[t], acc[t], 0, 0, 0);
         }
     } else {
         const int lg = l >> 4;  // k = kc+4g .. kc+4g+3, as in mfma_rows
 #pragma unroll
         for (int kc = 0; kc < NB; kc += 16) {
             const float4 a = *reinterpret_cast<const float4*>(Xg + (16 * w + lr) * XS + kc + 4 * lg);
-            float4 b[4];
+            float4 b[2];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) b[t] = *reinterpret_cast<const float4*>(Xd + (16 * t + lr) * XS + kc + 4 * lg);
+            for (int t = 0; t < 2; ++t) b[t] = *reinterpret_cast<const float4*>(Xd + (16 * (t0 + t) + lr) * XS + kc + 4 * lg);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[t].x, acc[t], 0, 0, 0);
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b[t].x, acc[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[t].y, acc[t], 0, 0, 0);
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b[t].y, acc[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[t].z, acc[t], 0, 0, 0);
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b[t].z, acc[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[t].w, acc[t], 0, 0, 0);
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b[t].w, acc[t], 0, 0, 0);
         }
     }
 }
 
+// Eight wavefronts: with four, one per SIMD, the row blocks' long update (up
+// to 960 columns) waited for its operands and outlasted the diagonal
+// workgroup's chain (row blocks 20-25 us a step, the diagonal 18).
 template <int MODE>
-__global__ __launch_bounds__(256) void k_chol_step(CholStep a) {
+__global__ __launch_bounds__(kCholThreads) void k_chol_step(CholStep a) {
     using R = CholReal<MODE>;
-    constexpr int LDT = ldt<R>();
     // SA: the block factored (R, row stride LDS_ROW), and the partial sums of
     // the update (FP32); LiT: Li^T in, then the new inverse (R, stride LDT),
     // and partial sums; both sized for the larger use
-    constexpr int kSA = NB * (NB + 2);  // doubles
+    constexpr int kSA = NB * LDT;  // doubles
     __shared__ __attribute__((aligned(16))) double SA[kSA];
     __shared__ __attribute__((aligned(16))) double LiTraw[kSA];
     __shared__ __attribute__((aligned(16))) float Xg[NB * XS];
     __shared__ __attribute__((aligned(16))) float Xd[NB * XS];
     __shared__ R T[3][16][17];
-    __shared__ R dinv[NB];
     R* const LiT = reinterpret_cast<R*>(LiTraw);
-    static_assert(NB * ldt<R>() * sizeof(R) <= sizeof(LiTraw), "Li^T fits its buffer");
     static_assert(NB * LDS_ROW * sizeof(R) <= sizeof(SA), "the factored block fits its buffer");
+    static_assert(2 * NB * NB * sizeof(float) <= sizeof(SA), "two wavefronts' partial blocks fit a buffer");
     const int tid = threadIdx.x;
     const int nb = a.kw / NB, j = a.j;
     // workgroup 0: the diagonal block; 1 (when a.look): the lookahead, which
@@ -1612,88 +1452,94 @@ __global__ __launch_bounds__(256) void k_chol_step(CholStep a) {
     const size_t rg = rd + (size_t)NB * x;             // first row of this workgroup's block g
     const bool update = j < nb;
     const bool diag_p = x == 0 && j >= 1;              // the diagonal block arrives as P
-    const int l = tid & 63, w = wave_of();
+    const bool need_d = update && x != 0 && !look;     // X_d too
+    const int l = tid & 63, w = wave_of(), w4 = w & 3, half = w >> 2;
     // the block this workgroup updates: column block j (rows rg), or for the
     // lookahead the next diagonal block (rows and columns rg)
     const size_t cj = look ? rg : rd;
     // every global read first, so their latencies overlap: this row block of
-    // column block j (or P), the B rows of the solves, the inverse Li^T
-    float mblk[4][4], bg[16], bd[16];
+    // column block j (or P), the B rows of the solves, the inverse Li^T.
+    // Wavefront w holds tiles t = 2(w/4), 2(w/4)+1 of tile row w%4.
+    float mblk[2][4];
+    float4 bv[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int row = 16 * w + 4 * (l >> 4) + q, c = 16 * t + (l & 15);
+            const int row = 16 * w4 + 4 * (l >> 4) + q, c = 16 * (2 * half + t) + (l & 15);
             mblk[t][q] = !update ? 0.f : diag_p ? a.p_in[row * NB + c] : a.M[(rg + row) * a.ld + cj + c];
         }
     if (j >= 1) {
-        load_solve_rows(a.b_in, rg, bg);
-        if (update && x != 0 && !look) load_solve_rows(a.b_in, rd, bd);
+        load_solve_rows(a.b_in, need_d && half ? rd : rg, bv);
         {  // Li^T: 16-byte loads, all in flight before the LDS stores
             using V = typename std::conditional<std::is_same<R, double>::value, double2, float4>::type;
-            constexpr int EPV = 16 / sizeof(R), NV = NB * NB / (256 * EPV);
+            constexpr int EPV = 16 / sizeof(R), NV = NB * NB / (kCholThreads * EPV);
             const V* __restrict__ src = reinterpret_cast<const V*>(a.li_in);
             V lv[NV];
 #pragma unroll
-            for (int k = 0; k < NV; ++k) lv[k] = src[tid + 256 * k];
+            for (int k = 0; k < NV; ++k) lv[k] = src[tid + kCholThreads * k];
 #pragma unroll
             for (int k = 0; k < NV; ++k) {
-                const int e = EPV * (tid + 256 * k);  // e .. e+EPV-1 in the same row
+                const int e = EPV * (tid + kCholThreads * k);  // e .. e+EPV-1 in the same row
                 *reinterpret_cast<V*>(LiT + (e >> 6) * LDT + (e & 63)) = lv[k];
             }
         }
         __syncthreads();
         const int pcol = NB * (j - 1);  // column block j-1 within the panel
-        if (update && x != 0 && !look)  // X_d, for the update only
-            solve_block<MODE>(bd, LiT, Xd, false, a.M, a.ld, rd, a.c0 + pcol, a.phi, a.plo, pcol);
-        // the lookahead's rows are written by the workgroup that serves them
-        solve_block<MODE>(bg, LiT, Xg, !look, a.M, a.ld, rg, a.c0 + pcol, a.phi, a.plo, pcol);
+        // with X_d to form as well, half the wavefronts solve each; else the
+        // halves share the output blocks (1 + 4 and 2 + 3 sixteenths of work).
+        // The lookahead's rows are written by the workgroup that serves them.
+        if (need_d) {
+            if (half)
+                solve_block<MODE, 15>(bv, LiT, Xd, false, a.M, a.ld, a.mp, rd, a.c0 + pcol, a.pan, pcol);
+            else
+                solve_block<MODE, 15>(bv, LiT, Xg, true, a.M, a.ld, a.mp, rg, a.c0 + pcol, a.pan, pcol);
+        } else if (half) {
+            solve_block<MODE, 6>(bv, LiT, Xg, !look, a.M, a.ld, a.mp, rg, a.c0 + pcol, a.pan, pcol);
+        } else {
+            solve_block<MODE, 9>(bv, LiT, Xg, !look, a.M, a.ld, a.mp, rg, a.c0 + pcol, a.pan, pcol);
+        }
     }
     if (!update) return;
     __syncthreads();  // X blocks complete; SA and LiT are free
-    f32x4 acc[4];
+    f32x4 acc[2];
     if (diag_p) {
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < 2; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     } else {
-        // the columns left of j-1, K split over the wavefronts; the four
-        // partial blocks are summed through LDS in wavefront order
-        f32x4 part[4][4];
+        // the columns left of j-1, K split over the wavefronts: the partial
+        // blocks are summed through LDS in wavefront order
+        f32x4 part[4][2];
 #pragma unroll
         for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
-            for (int bj = 0; bj < 4; ++bj) part[bi][bj] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (x == 0 || look)
-            mfma_split<MODE, true>(part, a, rg, rg);
-        else
-            mfma_split<MODE, false>(part, a, rg, rd);
-        constexpr int PS = NB + 1;
-        float* const P = (w < 2 ? reinterpret_cast<float*>(SA) : reinterpret_cast<float*>(LiTraw)) + (w & 1) * NB * PS;
+            for (int bj = 0; bj < 2; ++bj) part[bi][bj] = f32x4{0.f, 0.f, 0.f, 0.f};
+        mfma_split<MODE>(part, a, rg, cj);
+        // partial block of wavefronts (kq, half): half a 64x64 block, tile by
+        // tile with a lane's four values together
+        auto at = [&](int kq, int tile) {
+            float* const buf = kq < 2 ? reinterpret_cast<float*>(SA) : reinterpret_cast<float*>(LiTraw);
+            return reinterpret_cast<f32x4*>(buf) + (size_t)((kq & 1) * 2 + half) * 512 + 64 * tile + l;
+        };
 #pragma unroll
         for (int bi = 0; bi < 4; ++bi)
 #pragma unroll
-            for (int bj = 0; bj < 4; ++bj)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) P[(16 * bi + 4 * (l >> 4) + q) * PS + 16 * bj + (l & 15)] = part[bi][bj][q];
+            for (int bj = 0; bj < 2; ++bj) *at(w4, 2 * bi + bj) = part[bi][bj];
         __syncthreads();
-        const float* const P0 = reinterpret_cast<const float*>(SA);
-        const float* const P2 = reinterpret_cast<const float*>(LiTraw);
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int e = (16 * w + 4 * (l >> 4) + q) * PS + 16 * t + (l & 15);
-                acc[t][q] = ((P0[e] + P0[NB * PS + e]) + P2[e]) + P2[NB * PS + e];
-            }
+        for (int t = 0; t < 2; ++t) {
+            const int e = 2 * w4 + t;
+            acc[t] = ((*at(0, e) + *at(1, e)) + *at(2, e)) + *at(3, e);
+        }
         __syncthreads();  // SA and LiT are reused below
     }
     if (j >= 1) mfma_lds<MODE>(acc, Xg, x == 0 || look ? Xg : Xd);
     R(*S)[LDS_ROW] = reinterpret_cast<R(*)[LDS_ROW]>(SA);
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int row = 16 * w + 4 * (l >> 4) + q, c = 16 * t + (l & 15);
+            const int row = 16 * w4 + 4 * (l >> 4) + q, c = 16 * (2 * half + t) + (l & 15);
             const float b = mblk[t][q] - acc[t][q];
             if (look)
                 a.p_out[row * NB + c] = b;
@@ -1704,24 +1550,24 @@ __global__ __launch_bounds__(256) void k_chol_step(CholStep a) {
         }
     if (x != 0 || look) return;
     __syncthreads();
-    potrf_inv64(S, LiT, T, dinv);
+    potrf_inv64(S, LiT, T);
 #pragma unroll
-    for (int k = 0; k < NB * NB / 256; ++k) {
-        const int e = tid + 256 * k, r = e / NB, c = e % NB;
+    for (int k = 0; k < NB * NB / kCholThreads; ++k) {
+        const int e = tid + kCholThreads * k, r = e / NB, c = e % NB;
         if (c <= r) a.M[(rd + r) * a.ld + rd + c] = (float)S[r][c];
     }
     {  // 16-byte LDS reads, then the stores
         using V = typename std::conditional<std::is_same<R, double>::value, double2, float4>::type;
-        constexpr int EPV = 16 / sizeof(R), NV = NB * NB / (256 * EPV);
+        constexpr int EPV = 16 / sizeof(R), NV = NB * NB / (kCholThreads * EPV);
         V lv[NV];
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            const int e = EPV * (tid + 256 * k);
+            const int e = EPV * (tid + kCholThreads * k);
             lv[k] = *reinterpret_cast<const V*>(LiT + (e >> 6) * LDT + (e & 63));
         }
         V* __restrict__ dst = reinterpret_cast<V*>(a.li_out);
 #pragma unroll
-        for (int k = 0; k < NV; ++k) dst[tid + 256 * k] = lv[k];
+        for (int k = 0; k < NV; ++k) dst[tid + kCholThreads * k] = lv[k];
     }
 }
 
@@ -1754,33 +1600,35 @@ hipError_t launch_hi_tea_step(const DevJob* jobs, const DevJobState* st, const i
     return hipGetLastError();
 }
 
-// Rows [rs, mp) x columns [cs, ce) of the trailing matrix minus the outer
-// panel (columns [pc, pc+kw)) times its transpose.
-// Regions whose 256x256 tiles would leave most CUs idle take 128x128 tiles.
+// The lower triangle's rows from s on, columns [s, s + cols) (cols < 0: all),
+// minus the panel copy's kw columns times their transpose.  The next panel's
+// columns (cols = 512): 128x64 tiles, which put 3,700 rows on 232 CUs, or
+// 128x128 from 8,000 rows on, where those fill two rounds of CUs.  Regions of
+// at least a round of 256x256 tiles take those, smaller ones 128x128.
 static constexpr int kTrailBigMinTiles = 256;
-
-static void trailing_update(float* M, size_t ld, int s, int mp, int pc, int kw, int mode, const unsigned short* phi,
-                            const unsigned short* plo, hipStream_t stream) {
+template <int MODE>
+static void trailing_update(float* M, size_t ld, int s, int mp, int cols, int kw, const char* pan,
+                            hipStream_t stream) {
     if (s >= mp) return;
-    const int nr = (mp - s + GT - 1) / GT;
-    const dim3 g(nr, nr);
+    const int nr = (mp - s + 127) / 128;
     const int ntr = (mp - s + BT - 1) / BT, ntile = ntr * (ntr + 1) / 2;
-    if (mode == SOP_CHOL_F32)
-        hipLaunchKernelGGL(k_gemm_f32, g, dim3(256), 0, stream, M, ld, s, mp, pc, kw);
-    else if (ntile >= kTrailBigMinTiles)
-        hipLaunchKernelGGL(k_trail_bf16x3, dim3((ntile + kXcds - 1) / kXcds * kXcds), dim3(512), 0, stream, M, ld, s,
-                           mp, kw, ntr, phi, plo);
+    if (cols >= 0 && nr <= 62)
+        hipLaunchKernelGGL((k_update<MODE, 128, 64>), dim3(nr, cols / 64), dim3(256), 0, stream, M, ld, s, mp, kw, pan);
+    else if (cols < 0 && ntile >= kTrailBigMinTiles)
+        hipLaunchKernelGGL((k_update_big<MODE>), dim3((ntile + kXcds - 1) / kXcds * kXcds), dim3(512), 0, stream, M, ld,
+                           s, mp, kw, ntr, pan);
     else
-        hipLaunchKernelGGL(k_gemm_bf16x3, g, dim3(256), 0, stream, M, ld, s, mp, kw, phi, plo);
+        hipLaunchKernelGGL((k_update<MODE, 128, 128>), dim3(nr, cols < 0 ? nr : cols / 128), dim3(256), 0, stream, M, ld,
+                           s, mp, kw, pan);
 }
 
 // Blocked factorisation over outer panels of NB2 columns, each factored by
-// fused 64-column steps (k_chol_step).  A panel's columns receive the
-// previous panel's update inside its own steps; the rest of the trailing
-// matrix (from the panel after the next one on) is updated by the wide MFMA
-// kernels on `aux`, overlapped with the next panel.  Panel p waits for the
-// trailing update of panel p-2, which wrote its columns and read the copy
-// buffer panel p writes.  With aux == nullptr everything runs on `stream`.
+// fused 64-column steps (k_chol_step).  A panel's update of the next panel's
+// columns follows its steps; the rest of the trailing matrix (from the panel
+// after the next one on) is updated on `aux`, overlapped with the next panel.
+// Panel p's update of the next panel's columns waits for the trailing update
+// of panel p-1, which writes them too and reads the copy that panel p+1
+// writes.  With aux == nullptr everything runs on `stream`.
 hipError_t launch_chol_factor(float* M, size_t ld, int mp, int mode, const CholWork& w, hipStream_t stream,
                               hipStream_t aux, hipEvent_t ev_f, hipEvent_t ev_t2a, hipEvent_t ev_t2b) {
     const bool two = aux != nullptr && ev_f != nullptr && ev_t2a != nullptr && ev_t2b != nullptr;
@@ -1789,45 +1637,44 @@ hipError_t launch_chol_factor(float* M, size_t ld, int mp, int mode, const CholW
     hipError_t e = hipSuccess;
     const int nblk = mp / NB;
     float* const pbuf = reinterpret_cast<float*>(w.linv + (size_t)2 * NB * NB);  // after the two inverses
-    int pc = 0, pkw = 0;
+    auto update = [&](int s, int cols, int kw, const char* pan, hipStream_t on) {
+        if (mode == SOP_CHOL_F32) trailing_update<SOP_CHOL_F32>(M, ld, s, mp, cols, kw, pan, on);
+        else trailing_update<SOP_CHOL_BF16X3>(M, ld, s, mp, cols, kw, pan, on);
+    };
     for (int c0 = 0, p = 0; c0 < mp; c0 += NB2, ++p) {
         const int kw = mp - c0 < NB2 ? mp - c0 : NB2, nb = kw / NB;
-        unsigned short* const ph = w.phi + (size_t)(p & 1) * mp * NB2;
-        unsigned short* const pl = w.plo + (size_t)(p & 1) * mp * NB2;
-        const unsigned short* const qh = w.phi + (size_t)((p + 1) & 1) * mp * NB2;
-        const unsigned short* const ql = w.plo + (size_t)((p + 1) & 1) * mp * NB2;
-        if (two && pending[p & 1]) {
-            if ((e = hipStreamWaitEvent(stream, ev_t2[p & 1], 0)) != hipSuccess) return e;
-            pending[p & 1] = false;
-        }
+        char* const pan = w.pan[p & 1];
         for (int j = 0; j <= nb; ++j) {
             const int nwg = nblk - (c0 / NB + j);
             if (nwg <= 0) continue;
             const int look = j + 1 < nb ? 1 : 0;  // a next diagonal block in this panel
-            const CholStep a{M, ld, mp, c0, kw, pc, pkw, j,
+            const CholStep a{M, ld, mp, c0, kw, j,
                              w.linv + (size_t)((j + 1) & 1) * NB * NB, w.linv + (size_t)(j & 1) * NB * NB,
                              w.bbuf + (size_t)((j + 1) & 1) * mp * NB, w.bbuf + (size_t)(j & 1) * mp * NB,
                              pbuf + (size_t)(j & 1) * NB * NB, pbuf + (size_t)((j + 1) & 1) * NB * NB, look,
-                             ph, pl, qh, ql};
+                             pan};
             if (mode == SOP_CHOL_F32)
-                hipLaunchKernelGGL(k_chol_step<SOP_CHOL_F32>, dim3(nwg + look), dim3(256), 0, stream, a);
+                hipLaunchKernelGGL(k_chol_step<SOP_CHOL_F32>, dim3(nwg + look), dim3(kCholThreads), 0, stream, a);
             else
-                hipLaunchKernelGGL(k_chol_step<SOP_CHOL_BF16X3>, dim3(nwg + look), dim3(256), 0, stream, a);
+                hipLaunchKernelGGL(k_chol_step<SOP_CHOL_BF16X3>, dim3(nwg + look), dim3(kCholThreads), 0, stream, a);
         }
-        const int s1 = c0 + kw + NB2;  // the first column the next panel does not fold in
-        if (s1 < mp) {
-            if (two) {
-                if ((e = hipEventRecord(ev_f, stream)) != hipSuccess) return e;
-                if ((e = hipStreamWaitEvent(aux, ev_f, 0)) != hipSuccess) return e;
-                trailing_update(M, ld, s1, mp, c0, kw, mode, ph, pl, aux);
-                if ((e = hipEventRecord(ev_t2[p & 1], aux)) != hipSuccess) return e;
-                pending[p & 1] = true;
-            } else {
-                trailing_update(M, ld, s1, mp, c0, kw, mode, ph, pl, stream);
-            }
+        const int s0 = c0 + kw, s1 = s0 + NB2;  // the next panel, and what follows it
+        // the panel before this one updates the next panel's columns on aux,
+        // reading the copy that the next panel writes: done with both first
+        if (pending[(p + 1) & 1]) {
+            if ((e = hipStreamWaitEvent(stream, ev_t2[(p + 1) & 1], 0)) != hipSuccess) return e;
+            pending[(p + 1) & 1] = false;
         }
-        pc = c0;
-        pkw = kw;
+        if (s0 < mp) update(s0, NB2, kw, pan, stream);
+        if (s1 < mp && two) {
+            if ((e = hipEventRecord(ev_f, stream)) != hipSuccess) return e;
+            if ((e = hipStreamWaitEvent(aux, ev_f, 0)) != hipSuccess) return e;
+            update(s1, -1, kw, pan, aux);
+            if ((e = hipEventRecord(ev_t2[p & 1], aux)) != hipSuccess) return e;
+            pending[p & 1] = true;
+        } else if (s1 < mp) {
+            update(s1, -1, kw, pan, stream);
+        }
     }
     for (int q = 0; q < 2; ++q)
         if (pending[q] && (e = hipStreamWaitEvent(stream, ev_t2[q], 0)) != hipSuccess) return e;
@@ -1855,8 +1702,8 @@ hipError_t launch_chol_step(const DevJob* jobs, const DevJobState* st, const int
 // ---------------------------------------------------------------------------
 // Factorisation on caller-owned device memory with nothing allocated
 // (sop_chol_factor_noalloc): the workspace of launch_chol_factor -- the FP64
-// inverses of a panel's diagonal blocks and the two split-BF16 panel
-// buffers -- sized for matrices up to kNoAllocMaxOrder, lives in one static
+// inverses of a panel's diagonal blocks and the two panel copies
+// -- sized for matrices up to kNoAllocMaxOrder, lives in one static
 // device array that every GPU the library runs on holds until the process
 // ends.  Its device address is taken once per device with
 // hipGetSymbolAddress; the array's name is never used as an address on the
@@ -1866,8 +1713,8 @@ namespace sop {
 
 constexpr int kNoAllocMaxOrder = 12288;  // 3N for N = 4,096 beads
 constexpr size_t kNoAllocBBytes = (size_t)2 * kNoAllocMaxOrder * 64 * sizeof(float);  // chol_bbuf_bytes
-constexpr size_t kNoAllocPanelBytes = (size_t)2 * kNoAllocMaxOrder * kCholPanel * sizeof(unsigned short);
-constexpr size_t kNoAllocScratchBytes = kCholLinvBytes + kNoAllocBBytes + 2 * kNoAllocPanelBytes;  // linv|bbuf|phi|plo
+constexpr size_t kNoAllocPanelBytes = (size_t)kNoAllocMaxOrder * kCholPanel * 4;  // chol_panel_bytes
+constexpr size_t kNoAllocScratchBytes = kCholLinvBytes + kNoAllocBBytes + 2 * kNoAllocPanelBytes;  // linv|bbuf|pan0|pan1
 static_assert(kCholLinvBytes % 256 == 0 && kNoAllocBBytes % 256 == 0 && kNoAllocPanelBytes % 256 == 0,
               "scratch sections stay 256-byte aligned");
 
@@ -1932,8 +1779,8 @@ extern "C" int sop_chol_factor_noalloc(int device, int n, float* M, unsigned lon
     CholWork w{};
     w.linv = reinterpret_cast<double*>(base);
     w.bbuf = reinterpret_cast<float*>(base + kCholLinvBytes);
-    w.phi = reinterpret_cast<unsigned short*>(base + kCholLinvBytes + kNoAllocBBytes);
-    w.plo = reinterpret_cast<unsigned short*>(base + kCholLinvBytes + kNoAllocBBytes + kNoAllocPanelBytes);
+    w.pan[0] = reinterpret_cast<char*>(base + kCholLinvBytes + kNoAllocBBytes);
+    w.pan[1] = w.pan[0] + kNoAllocPanelBytes;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (mp > n) hipLaunchKernelGGL(k_chol_pad, dim3((mp + 255) / 256, mp - n), dim3(256), 0, s, M, (size_t)ld, n, mp);
     e = hipGetLastError();
