@@ -315,8 +315,8 @@ def capsid_phase(S, steps=2000):
     """Continuous indentation of a 100,000-bead capsid-like shell (200 chains
     x 500 beads on a sphere of R = 140 A), tip R = 50 A moving at 1 um/s,
     Verlet/possible rebuilds every 10/100 steps: stepping rate with the
-    cell-binned possible-pairs build, and one possible-pairs rebuild with
-    cells vs the all-pairs scan."""
+    possible-pairs build by tile boxes, and one possible-pairs rebuild with
+    the boxes vs the all-pairs scan."""
     sysm = S.synth_shell(200, 500, seed=2026, radius=140.0)
     c = sysm.coords[:, :3]
     top, bot = float(c[:, 2].max()), float(c[:, 2].min())

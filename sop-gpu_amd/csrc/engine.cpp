@@ -509,8 +509,7 @@ static unsigned long long built_bytes(const BuiltJob& b, bool pulling, bool inde
     t += round_up(std::max<size_t>(1, b.pulled.size()) * 4);
     t += round_up(n * 12);                // energies
     if (b.dj.flags & JF_EXTRA_FORCE) t += round_up(n * 16);  // forces of host potentials
-    if (n >= (unsigned long long)kCellMinBeads && n <= 64ull * kMaxCellWords)
-        t += round_up((n + 64) * 4) + round_up((n + 65) * 4) + 3 * round_up(n * 4);  // cell grid
+    if (n >= (unsigned long long)kBoxMinBeads) t += round_up((n + 63) / 64 * 32);  // tile boxes
     if (b.dj.flags & JF_HI) {
         t += 3 * round_up(n * 16) + round_up(n * 4);  // rforce, mforce, ci, eps
         if (b.dj.flags & JF_HI_EXACT) {
@@ -588,14 +587,7 @@ int Engine::add_job(const sop_params& p, const sop_system& s, long long numsteps
     J.energies = (float*)A(n * 12);
     J.lds_step = use_lds_step_ && n <= (size_t)kLdsStepBeads ? 1 : 0;
     J.sort_rows = J.lds_step && J.rb_cnt ? 1 : 0;
-    if (uses_cells(n)) {
-        J.cell_cap = (int)n + 64;
-        J.cell_cnt = (int*)A((size_t)J.cell_cap * 4);
-        J.cell_start = (int*)A((size_t)(J.cell_cap + 1) * 4);
-        J.cell_beads = (int*)A(n * 4);
-        J.bead_cell = (int*)A(n * 4);
-        J.bead_slot = (int*)A(n * 4);
-    }
+    if (uses_boxes(n)) J.tile_box = (float4*)A((n + 63) / 64 * 32);
     HiExactWork hw{};
     if (J.flags & JF_HI) {
         J.rforce = (float4*)A(n * 16);
@@ -808,12 +800,12 @@ int Engine::sync_tables() {
     }
     L_ = g > 0 ? g : 1;
     any_tea_ = any_exact_ = false;
-    cell_words_ = 0;
+    any_boxes_ = 0;
     any_idx32_ = 0;
     std::vector<int2> tea_tiles;  // the tiles of the TEA jobs
     for (auto& j : jobs_) {
         if (!j.dj.idx16) any_idx32_ = 1;
-        cell_words_ = std::max(cell_words_, cell_words_of(j.dj));
+        any_boxes_ |= boxes_of(j.dj);
         if ((j.dj.flags & JF_HI) && !(j.dj.flags & JF_HI_EXACT)) {
             any_tea_ = true;
             tea_tiles.insert(tea_tiles.end(), tiles.begin() + j.tile0, tiles.begin() + j.tile0 + j.ntile);
@@ -996,15 +988,13 @@ void Engine::drop_graph() {
     graphs_.clear();
 }
 
-bool Engine::uses_cells(size_t n) const {
-    return cell_min_ > 0 && n >= (size_t)cell_min_ && n <= (size_t)64 * kMaxCellWords;
-}
+bool Engine::uses_boxes(size_t n) const { return box_min_ > 0 && n >= (size_t)box_min_; }
 
-int Engine::cell_words_of(const DevJob& J) const { return (use_cells_ && J.cell_cnt) ? (J.n + 63) / 64 : 0; }
+int Engine::boxes_of(const DevJob& J) const { return use_boxes_ && J.tile_box; }
 
 void Engine::set_cells(int min_beads, int enabled) {
-    if (min_beads != 0) cell_min_ = min_beads;
-    use_cells_ = enabled != 0;
+    if (min_beads != 0) box_min_ = min_beads;
+    use_boxes_ = enabled != 0;
     tables_dirty_ = true;
     drop_graph();
 }
@@ -1115,11 +1105,11 @@ int Engine::launch_block(int slot_only) {
     if (due & 1) {
         const hipError_t e =
             slot_only >= 0
-                ? launch_possible(jobs, st, tiles, nt, nj, cell_words_of(jobs_[slot_only].dj),
+                ? launch_possible(jobs, st, tiles, nt, boxes_of(jobs_[slot_only].dj),
                                   !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
                                   jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, 0, stream_,
                                   eff1_)
-                : launch_possible(jobs, st, tiles, nt, nj, cell_words_, any_global_, d_sunits_, d_segs_, nsunits_,
+                : launch_possible(jobs, st, tiles, nt, any_boxes_, any_global_, d_sunits_, d_segs_, nsunits_,
                                   lds_beads_, 0, stream_, eff_);
         if (int rc = check(e, "possible pairs")) return rc;
     }
@@ -1257,9 +1247,8 @@ int Engine::stage_job_update(int mask) {
 }
 int Engine::stage_possible() {
     if (int rc = sync_tables()) return rc;
-    return check(launch_possible(d_jobs_, d_state_, d_tiles_, ntiles_, (int)jobs_.size(), cell_words_, any_global_,
-                                 d_sunits_,
-                                 d_segs_, nsunits_, lds_beads_, 0, stream_, eff_),
+    return check(launch_possible(d_jobs_, d_state_, d_tiles_, ntiles_, any_boxes_, any_global_, d_sunits_, d_segs_,
+                                 nsunits_, lds_beads_, 0, stream_, eff_),
                  "possible pairs");
 }
 int Engine::stage_verlet() {
@@ -1598,8 +1587,7 @@ int Engine::rebuild_lists(int id, int mask) {
     int nt = 0;
     if (int rc = tiles_for_slot(slot, &nt)) return rc;
     if (mask & 1)
-        if (int rc = check(launch_possible(d_jobs_ + slot, d_state_ + slot, d_tiles1_, nt, 1,
-                                           cell_words_of(jobs_[slot].dj), !jobs_[slot].dj.lds_step, d_sunits1_,
+        if (int rc = check(launch_possible(d_jobs_ + slot, d_state_ + slot, d_tiles1_, nt, boxes_of(jobs_[slot].dj), !jobs_[slot].dj.lds_step, d_sunits1_,
                                            d_segs1_,
                                            jobs_[slot].dj.lds_step ? nsunits1_ : 0, jobs_[slot].n, 1, stream_,
                                            eff1_),

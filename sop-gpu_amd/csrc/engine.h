@@ -129,8 +129,8 @@ class Engine {
     int read_state_of(int id, DevJobState* out);
 
     void set_tuning(int max_blocks, int use_graph);
-    // Possible-pairs cell grid: jobs of min_beads beads and more admitted
-    // from now on get one (0 keeps the threshold, < 0 gives none); enabled = 0
+    // Possible-pairs tile boxes: jobs of min_beads beads and more admitted
+    // from now on get them (0 keeps the threshold, < 0 gives none); enabled = 0
     // builds every list by the all-pairs scan.
     void set_cells(int min_beads, int enabled);
     // Step jobs of at most kLdsStepBeads beads with their coordinates in
@@ -186,9 +186,9 @@ class Engine {
     int plan_lds_units(std::vector<int2>& units, std::vector<int4>& segs) const;
     // tuning
     int max_blocks_ = 0;
-    int cell_min_ = kCellMinBeads;
-    bool use_cells_ = true;
-    int cell_words_ = 0;
+    int box_min_ = kBoxMinBeads;
+    bool use_boxes_ = true;
+    int any_boxes_ = 0;
     int any_idx32_ = 0;  // some job stores int32 list entries
     bool use_lds_step_ = true;
     int2* d_units_ = nullptr;  // row-sort units (job slot, first row) per kLdsUnit rows of LDS-step jobs
@@ -215,8 +215,8 @@ class Engine {
     int snapshot(void** buf);
     int restore(void* buf, const std::vector<long long>& steps);
     int time_blocks(int nblocks, double* ms);
-    bool uses_cells(size_t n) const;
-    int cell_words_of(const DevJob& J) const;
+    bool uses_boxes(size_t n) const;
+    int boxes_of(const DevJob& J) const;
     int exact_mode_ = SOP_CHOL_BF16X3;
     bool any_tea_ = false, any_exact_ = false;
     bool use_graph_ = true;

@@ -70,15 +70,9 @@ struct DevJob {
     void* pp_j;     // bead-major: entry k of bead i at [i*pp_ld + k]
     int* excl_cnt;  // sorted covalent+native partners (possible-pair exclusions)
     int* excl_j;
-    // cell grid of the possible-pairs build, for jobs of kCellMinBeads
-    // beads and more (null otherwise): per-cell counts and exclusive starts,
-    // the beads grouped by cell, each bead's cell and slot within it
-    int* cell_cnt;
-    int* cell_start;
-    int* cell_beads;
-    int* bead_cell;
-    int* bead_slot;
-    int cell_cap;
+    // bounding boxes (lo, hi) of the tiles for the possible-pairs build, for
+    // jobs of kBoxMinBeads beads and more (null otherwise)
+    float4* tile_box;
     int lds_step;   // stepped by k_step_lds (coordinates staged in LDS)
     int* pulled;    // bead indices of pulled beads
     float* energies; // 3n per-bead energies (output cadence)
@@ -171,9 +165,6 @@ struct DevJobState {
     float tipDr;      // |chip - tip| of the last tip update, before the tip moved
     float beta;       // TEA beta' (bdhitea.cu:162-170)
     double eps_traj;  // TEA epsilon of the last update
-    float cell_org[3];  // possible-pairs cell grid of the last rebuild
-    float cell_inv;     // 1 / cell edge
-    int cell_dim[3];
 };
 
 inline StepDesc step_desc(const DevJob& J) {
@@ -232,9 +223,10 @@ inline StepDesc step_desc(const DevJob& J) {
     return d;
 }
 
-// Jobs of this many beads and more build their possible-pairs list from a
-// cell grid instead of the all-pairs scan (same list, same order).
-constexpr int kCellMinBeads = 8192;
+// Jobs of this many beads and more build their possible-pairs list from the
+// tiles whose boxes are near instead of the all-pairs scan (same list, same
+// order).
+constexpr int kBoxMinBeads = 8192;
 // Jobs of at most this many beads are stepped with their coordinates staged
 // in LDS (16 bytes per bead: 80 KB, two workgroups per CU).
 constexpr int kLdsStepBeads = 5120;

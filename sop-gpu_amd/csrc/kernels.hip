@@ -9,7 +9,7 @@
 //              beads in LDS.  Reference bodies: src/Potentials/covalent_kernel.cu:28-51,
 //              native_kernel.cu:27-52, pairs_kernel.cu:33-59,
 //              indentation_kernel.cu:71-128, src/Integrators/langevin_kernel.cu:17-58.
-// k_possible, k_possible_lds, k_possible_cells
+// k_possible, k_possible_lds, k_possible_boxes
 //              possible-pairs list: same-job beads j != i, ascending j, with
 //              sqrtf(d^2) < threshold, excluding covalent and native partners
 //              (src/Updaters/possiblepairlist_kernel.cu:18-71).
@@ -811,13 +811,13 @@ __device__ __forceinline__ unsigned long long lanes_below(int lane) {
 // is evaluated as d^2 <= pp_d2 (the same set of floats).
 __global__ __launch_bounds__(256) void k_possible(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
                                                   const int2* __restrict__ tiles, int ntiles, int force,
-                                                  int use_cells, int skip_lds) {
+                                                  int use_boxes, int skip_lds) {
     const int lane = threadIdx.x & 63;
     const TileRange tr = xcd_tiles(ntiles);
     for (int t = tr.begin; t < tr.end; t += tr.step) {
         const int2 td = tiles[t];
         const DevJob& J = jobs[td.x];
-        if (use_cells && J.cell_cnt) continue;  // built by k_possible_cells
+        if (use_boxes && J.tile_box) continue;  // built by k_possible_boxes
         if (skip_lds && J.lds_step && J.idx16) continue;  // built by k_possible_lds
         const long long s = st[td.x].step;
         if (!force && !due(J, s, J.pp_freq)) continue;
@@ -973,13 +973,13 @@ __device__ __forceinline__ void possible_rows(const DevJob& J, const float4* __r
     }
 }
 
-__device__ __forceinline__ bool possible_lds_wanted(const DevJob& J, long long s, int force, int use_cells) {
-    return J.lds_step && J.idx16 && !(use_cells && J.cell_cnt) && (force || due(J, s, J.pp_freq));
+__device__ __forceinline__ bool possible_lds_wanted(const DevJob& J, long long s, int force, int use_boxes) {
+    return J.lds_step && J.idx16 && !(use_boxes && J.tile_box) && (force || due(J, s, J.pp_freq));
 }
 
 __global__ __launch_bounds__(1024) void k_possible_lds(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
                                                        const int2* __restrict__ units, const int4* __restrict__ segs,
-                                                       int nunits, int force, int use_cells) {
+                                                       int nunits, int force, int use_boxes) {
     extern __shared__ float4 lds_coord[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int u = blockIdx.x; u < nunits; u += gridDim.x) {
@@ -990,7 +990,7 @@ __global__ __launch_bounds__(1024) void k_possible_lds(const DevJob* __restrict_
             const int4 sg = segs[ud.x + q];
             const DevJob& J = jobs[sg.x];
             const long long s = st[sg.x].step;
-            if (!possible_lds_wanted(J, s, force, use_cells)) continue;
+            if (!possible_lds_wanted(J, s, force, use_boxes)) continue;
             any = true;
             const float4* __restrict__ g = J.coord[s & 1];
             for (int k = threadIdx.x; k < J.n; k += blockDim.x) lds_coord[sg.w + k] = g[k];
@@ -1008,7 +1008,7 @@ __global__ __launch_bounds__(1024) void k_possible_lds(const DevJob* __restrict_
         }
         if (q == ud.y) continue;
         const DevJob& J = jobs[sg.x];
-        if (!possible_lds_wanted(J, st[sg.x].step, force, use_cells)) continue;
+        if (!possible_lds_wanted(J, st[sg.x].step, force, use_boxes)) continue;
         possible_rows(J, lds_coord + sg.w, sg.y + t, sg.y + min(t + 64, sg.z), &st[sg.x].overflow);
     }
 }
@@ -1018,14 +1018,14 @@ __global__ __launch_bounds__(1024) void k_possible_lds(const DevJob* __restrict_
 // row, from the job's coordinates staged in LDS.  Grid: ntiles * 4.
 __global__ __launch_bounds__(1024) void k_possible_split(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
                                                          const int2* __restrict__ tiles, int ntiles, int force,
-                                                         int use_cells) {
+                                                         int use_boxes) {
     extern __shared__ float4 lds_coord[];
     const int tile = blockIdx.x >> 2, quarter = blockIdx.x & 3;
     if (tile >= ntiles) return;
     const int2 td = tiles[tile];
     const DevJob& J = jobs[td.x];
     const long long s = st[td.x].step;
-    if (!possible_lds_wanted(J, s, force, use_cells)) return;
+    if (!possible_lds_wanted(J, s, force, use_boxes)) return;
     const int n = J.n, row0 = td.y + 16 * quarter;
     if (row0 >= n) return;  // every exit above is uniform over the workgroup
     {
@@ -1038,318 +1038,204 @@ __global__ __launch_bounds__(1024) void k_possible_split(const DevJob* __restric
 }
 
 // ---------------------------------------------------------------------------
-// cell-binned possible pairs (large jobs)
+// possible pairs by bounding boxes (large jobs)
 // ---------------------------------------------------------------------------
 // The list of k_possible -- the same predicate on the same operands, the
-// same ascending-j order -- from the candidates in the 27 cells around the
-// bead instead of the whole job.  Cells are cubes of edge thr*(1+1e-4) +
-// 0.01 A: a pair with sqrtf(d^2) < thr has every |coordinate difference|
-// within thr*(1 + 2^-21), and the cell index (x - x0) / edge is computed
-// with an error far below the margin, so such a pair always lies in
-// adjacent cells.  Accepted j are set in a per-wave LDS bitmap over the
-// job's beads, the bead's exclusions cleared, and the bitmap read back in
-// index order with a wave prefix sum of popcounts.
+// same ascending-j order -- without the tiles of 64 consecutive beads that no
+// bead of a group can reach.  With lo and hi a tile's least and greatest
+// coordinates, rounded subtraction, multiplication and addition are monotone,
+// so max(lo.x - x, x - hi.x, 0) is at most |r_j.x - x| for each bead j of
+// the tile, and the sum of the squares, formed in the order of the predicate,
+// at most the predicate's: a tile that fails it holds no accepted bead.
 
-__device__ __forceinline__ int cell_axis(float x, float org, float inv, int dim) {
-    const float q = (x - org) * inv;
-    if (!(q >= 0.0f)) return 0;  // below the grid, or NaN
-    if (q >= (float)dim) return dim - 1;
-    return min((int)q, dim - 1);
-}
-
-__device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
-    return v;
-}
-__device__ __forceinline__ int wave_max(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-    return v;
-}
-__device__ __forceinline__ int wave_inclusive_sum(int v, int lane) {
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(v, o);
-        if (lane >= o) v += u;
-    }
-    return v;
-}
-
-// Per job (one 1024-thread block each): bounding box of the coordinates,
-// the grid (edge grown until the cell count fits cell_cap), zeroed counts.
-__global__ __launch_bounds__(1024) void k_cells_setup(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
-                                                      int njobs, int force) {
-    const int jb = blockIdx.x;
-    if (jb >= njobs) return;
-    const DevJob& J = jobs[jb];
-    if (!J.cell_cnt) return;
-    DevJobState& S = st[jb];
-    const long long s = S.step;
-    if (!force && !due(J, s, J.pp_freq)) return;
-    const float4* __restrict__ cur = J.coord[s & 1];
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int i = threadIdx.x; i < J.n; i += blockDim.x) {
-        const float4 r = cur[i];
-        lo[0] = fminf(lo[0], r.x), hi[0] = fmaxf(hi[0], r.x);
-        lo[1] = fminf(lo[1], r.y), hi[1] = fmaxf(hi[1], r.y);
-        lo[2] = fminf(lo[2], r.z), hi[2] = fmaxf(hi[2], r.z);
-    }
-    __shared__ float red[6][16];
-    __shared__ int dims[4];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        float a = lo[d], b = hi[d];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            a = fminf(a, __shfl_xor(a, o));
-            b = fmaxf(b, __shfl_xor(b, o));
-        }
-        if (lane == 0) {
-            red[d][w] = a;
-            red[3 + d][w] = b;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int nw = blockDim.x >> 6;
-        float org[3], ext[3];
-        for (int d = 0; d < 3; ++d) {
-            float a = red[d][0], b = red[3 + d][0];
-            for (int k = 1; k < nw; ++k) a = fminf(a, red[d][k]), b = fmaxf(b, red[3 + d][k]);
-            org[d] = a;
-            ext[d] = b - a;
-        }
-        float edge = J.pp_thr * 1.0001f + 0.01f;
-        int dm[3] = {1, 1, 1};
-        const bool finite = isfinite(ext[0]) && isfinite(ext[1]) && isfinite(ext[2]);
-        if (finite) {
-            for (int it = 0; it < 200; ++it) {
-                double cells = 1.0;
-                for (int d = 0; d < 3; ++d) cells *= floor((double)ext[d] / edge) + 1.0;
-                if (cells <= (double)J.cell_cap) break;
-                edge *= 1.1f;
-            }
-            for (int d = 0; d < 3; ++d) dm[d] = (int)floor((double)ext[d] / edge) + 1;
-            if ((long long)dm[0] * dm[1] * dm[2] > J.cell_cap) dm[0] = dm[1] = dm[2] = 1;
-        } else {
-            org[0] = org[1] = org[2] = 0.0f;
-        }
-        for (int d = 0; d < 3; ++d) {
-            S.cell_org[d] = org[d];
-            S.cell_dim[d] = dm[d];
-        }
-        S.cell_inv = 1.0f / edge;
-        dims[0] = dm[0] * dm[1] * dm[2];
-    }
-    __syncthreads();
-    const int nc = dims[0];
-    for (int c = threadIdx.x; c < nc; c += blockDim.x) J.cell_cnt[c] = 0;
-}
-
-// Each bead's cell and its slot there (the order within a cell is free:
-// the bitmap restores index order).
-__global__ __launch_bounds__(256) void k_cells_count(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
-                                                     const int2* __restrict__ tiles, int ntiles, int force) {
-    const int lane = threadIdx.x & 63;
-    const TileRange tr = xcd_tiles(ntiles);
-    for (int t = tr.begin; t < tr.end; t += tr.step) {
-        const int2 td = tiles[t];
-        const DevJob& J = jobs[td.x];
-        if (!J.cell_cnt) continue;
-        const DevJobState& S = st[td.x];
-        const long long s = S.step;
-        if (!force && !due(J, s, J.pp_freq)) continue;
-        const int i = td.y + lane;
-        if (i >= J.n) continue;
-        const float4 r = J.coord[s & 1][i];
-        const int cx = cell_axis(r.x, S.cell_org[0], S.cell_inv, S.cell_dim[0]);
-        const int cy = cell_axis(r.y, S.cell_org[1], S.cell_inv, S.cell_dim[1]);
-        const int cz = cell_axis(r.z, S.cell_org[2], S.cell_inv, S.cell_dim[2]);
-        const int c = (cz * S.cell_dim[1] + cy) * S.cell_dim[0] + cx;
-        J.bead_cell[i] = c;
-        J.bead_slot[i] = atomicAdd(&J.cell_cnt[c], 1);
-    }
-}
-
-// Exclusive scan of the cell counts (one 1024-thread block per job).
-__global__ __launch_bounds__(1024) void k_cells_scan(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
-                                                     int njobs, int force) {
-    const int jb = blockIdx.x;
-    if (jb >= njobs) return;
-    const DevJob& J = jobs[jb];
-    if (!J.cell_cnt) return;
-    const DevJobState& S = st[jb];
-    if (!force && !due(J, S.step, J.pp_freq)) return;
-    const int nc = S.cell_dim[0] * S.cell_dim[1] * S.cell_dim[2];
-    const int per = (nc + blockDim.x - 1) / blockDim.x;
-    const int b = threadIdx.x * per, e = min(b + per, nc);
-    int sum = 0;
-    for (int c = b; c < e; ++c) sum += J.cell_cnt[c];
-    __shared__ int part[1024];
-    part[threadIdx.x] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int k = 0; k < (int)blockDim.x; ++k) {
-            const int v = part[k];
-            part[k] = acc;
-            acc += v;
-        }
-    }
-    __syncthreads();
-    int acc = part[threadIdx.x];
-    for (int c = b; c < e; ++c) {
-        J.cell_start[c] = acc;
-        acc += J.cell_cnt[c];
-    }
-    if (threadIdx.x == 0) J.cell_start[nc] = J.n;
-}
-
-__global__ __launch_bounds__(256) void k_cells_fill(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
+// A tile's box, one wavefront each: J.tile_box[2t] = lo, [2t + 1] = hi.
+// A coordinate that is not a number is left out (it is never accepted).
+__global__ __launch_bounds__(256) void k_tile_boxes(const DevJob* __restrict__ jobs,
+                                                    const DevJobState* __restrict__ st,
                                                     const int2* __restrict__ tiles, int ntiles, int force) {
     const int lane = threadIdx.x & 63;
     const TileRange tr = xcd_tiles(ntiles);
     for (int t = tr.begin; t < tr.end; t += tr.step) {
         const int2 td = tiles[t];
         const DevJob& J = jobs[td.x];
-        if (!J.cell_cnt) continue;
-        if (!force && !due(J, st[td.x].step, J.pp_freq)) continue;
-        const int i = td.y + lane;
-        if (i >= J.n) continue;
-        J.cell_beads[J.cell_start[J.bead_cell[i]] + J.bead_slot[i]] = i;
+        if (!J.tile_box) continue;
+        const long long s = st[td.x].step;
+        if (!force && !due(J, s, J.pp_freq)) continue;
+        const CoordGlobal cur{J.coord[s & 1]};
+        float4 lo = cur[min(td.y + lane, J.n - 1)], hi = lo;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            lo.x = fminf(lo.x, __shfl_xor(lo.x, o));
+            lo.y = fminf(lo.y, __shfl_xor(lo.y, o));
+            lo.z = fminf(lo.z, __shfl_xor(lo.z, o));
+            hi.x = fmaxf(hi.x, __shfl_xor(hi.x, o));
+            hi.y = fmaxf(hi.y, __shfl_xor(hi.y, o));
+            hi.z = fmaxf(hi.z, __shfl_xor(hi.z, o));
+        }
+        if (lane < 2) J.tile_box[2 * (td.y >> 6) + lane] = lane ? hi : lo;
     }
 }
 
-// One 64-thread workgroup (one wavefront) per tile; dynamic LDS holds the
-// bitmap of ceil(n/64) words for the largest cell-binned job.
-// One wavefront per half tile (32 beads), its beads one after another.  A bead's
-// candidates (the 3 x 3 rows of three x-adjacent cells, each row one
-// contiguous range of cell_beads) are read eight 64-entry chunks at a time,
-// all index loads and then all coordinate gathers in flight together; the
-// next bead's coordinates and first 64 exclusions are loaded while this one
-// is scanned.  Accepted j set bit j of the LDS bitmap bm and bit j / 64 of
-// bm2, so the read-back in index order visits only the 64-word blocks of bm
-// that hold an entry.
-constexpr int kCellChunks = 8;
-__global__ __launch_bounds__(64) void k_possible_cells(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
-                                                       const int2* __restrict__ tiles, int ntiles, int force,
-                                                       int cell_words) {
-    extern __shared__ unsigned long long bm[];
-    unsigned long long* const bm2 = bm + cell_words;  // one bit per word of bm
-    const int lane = threadIdx.x;
+// One wavefront per kBoxBeads consecutive beads.  The boxes are tested 64 at
+// a time, one per lane, against each of the beads; the tiles that some bead
+// reaches collect in LDS with a mask of those beads, and each such tile's
+// coordinates (one contiguous 1 KB load, four tiles ahead) are tested for the
+// beads in its mask: ballot, exclusions out, compaction in ascending order.
+// What bounds it is the pair tests themselves, ~18 vector instructions per
+// bead and near tile.  Four beads a wavefront: 76 us for 18,000 beads of a
+// capsid shell (32 A threshold, ~1,000 entries a bead) and 340 us for 100,000;
+// eight take 108 and 345 (too few wavefronts for the smaller), two 76 and 380.
+// Taking the candidates bead by bead from a cell grid and sorting the accepted
+// ones through a bitmap of the job's beads took 947 and 2,283 us.  Beads in no
+// spatial order along the chain would make every box span the job: the scan
+// is then k_possible's.
+constexpr int kBoxBeads = 4;
+constexpr int kBoxAhead = 4;
+constexpr int kBoxList = 256;  // collected tiles before they are worked off
+__global__ __launch_bounds__(256) void k_possible_boxes(const DevJob* __restrict__ jobs,
+                                                        DevJobState* __restrict__ st,
+                                                        const int2* __restrict__ tiles, int ntiles, int force) {
+    __shared__ unsigned near_tiles[4][kBoxList + 64];  // tile << 8 | beads
+    const int lane = threadIdx.x & 63, wv = wave_id();
+    volatile unsigned* const list = near_tiles[wv];
+    constexpr int kUnits = 64 / kBoxBeads;  // per tile
+    const int nunits = kUnits * ntiles;
     const int nb = gridDim.x, nxcd = nb >= 8 ? 8 : 1;
-    const int nhalf = 2 * ntiles;  // work units: the two halves of every tile
-    const int slice = (nhalf + nxcd - 1) / nxcd;
+    const int slice = (nunits + nxcd - 1) / nxcd;
     const int xcd = blockIdx.x % nxcd;
-    const int hend = min((xcd + 1) * slice, nhalf);
-    for (int h = xcd * slice + blockIdx.x / nxcd; h < hend; h += nb / nxcd) {
-        const int2 td = tiles[h >> 1];
+    const int hend = min((xcd + 1) * slice, nunits);
+    for (int h = xcd * slice + 4 * (int)(blockIdx.x / nxcd) + wv; h < hend; h += 4 * (nb / nxcd)) {
+        const int2 td = tiles[h / kUnits];
         const DevJob& J = jobs[td.x];
-        if (!J.cell_cnt) continue;
-        const DevJobState& S = st[td.x];
-        const long long s = S.step;
+        if (!J.tile_box) continue;
+        const long long s = st[td.x].step;
         if (!force && !due(J, s, J.pp_freq)) continue;
-        const int n = J.n;
-        const int i0 = td.y + 32 * (h & 1);
+        const int n = J.n, nt = (n + 63) >> 6;
+        const int i0 = td.y + kBoxBeads * (h % kUnits);
         if (i0 >= n) continue;
-        const int nwords = (n + 63) >> 6;
-        for (int w = lane; w < nwords; w += 64) bm[w] = 0ull;
-        for (int w = lane; w < (nwords + 63) >> 6; w += 64) bm2[w] = 0ull;
-        __syncthreads();
-        const CoordGlobal cur{J.coord[s & 1]};
-        const auto cbeads = gmem(J.cell_beads);
-        const auto cstart = gmem(J.cell_start);
-        const auto ecnt = gmem(J.excl_cnt);
+        const int nbead = min(kBoxBeads, n - i0);
+        const CoordGlobal cur{J.coord[s & 1]}, box{J.tile_box};
         const auto ej = gmem(J.excl_j);
         const float d2max = J.pp_d2;
-        const int cap = J.pp_cap, ecap = J.excl_cap;
-        const int dx = S.cell_dim[0], dy = S.cell_dim[1], dz = S.cell_dim[2];
-        const int iend = min(i0 + 32, n);
-        float4 r1n = cur[i0];
-        int nen = ecnt[i0];
-        int evn = ej[(size_t)min(lane, ecap - 1) * n + i0];
-        for (int i = i0; i < iend; ++i) {
-            const float4 r1 = r1n;
-            const int ne = nen, ev = evn;
-            if (i + 1 < iend) {
-                r1n = cur[i + 1];
-                nen = ecnt[i + 1];
-                evn = ej[(size_t)min(lane, ecap - 1) * n + i + 1];
-            }
-            const int cx = cell_axis(r1.x, S.cell_org[0], S.cell_inv, dx);
-            const int cy = cell_axis(r1.y, S.cell_org[1], S.cell_inv, dy);
-            const int cz = cell_axis(r1.z, S.cell_org[2], S.cell_inv, dz);
-            int jlo = INT_MAX, jhi = -1;
-            for (int z = max(cz - 1, 0); z <= min(cz + 1, dz - 1); ++z)
-                for (int y = max(cy - 1, 0); y <= min(cy + 1, dy - 1); ++y) {
-                    const int row = (z * dy + y) * dx;
-                    // the cells x-1..x+1 of one row are contiguous in cell_beads
-                    const int b = cstart[row + max(cx - 1, 0)];
-                    const int e = cstart[row + min(cx + 1, dx - 1) + 1];
-                    for (int k0 = b; k0 < e; k0 += 64 * kCellChunks) {
-                        int jj[kCellChunks];
+        const int cap = J.pp_cap, ecap = J.excl_cap, idx16 = J.idx16, ld = J.pp_ld;
+        void* const pp = J.pp_j;
+        // lanes' beads: coordinates and exclusion counts of i0 + lane % kBoxBeads
+        const int il = min(i0 + lane % kBoxBeads, n - 1);
+        const float4 rl = cur[il];
+        const int nel = gmem(J.excl_cnt)[il];
+        float4 lo = box[2 * min(lane, nt - 1)], hi = box[2 * min(lane, nt - 1) + 1];
+        int ev[kBoxBeads];  // lane k: the bead's k-th exclusion, -1 past the last
 #pragma unroll
-                        for (int u = 0; u < kCellChunks; ++u) {
-                            const int k = k0 + 64 * u + lane;
-                            jj[u] = k < e ? cbeads[k] : i;  // past the range: the bead itself, skipped
+        for (int b = 0; b < kBoxBeads; ++b) ev[b] = ej[(size_t)min(lane, ecap - 1) * n + min(i0 + b, n - 1)];
+        float px[kBoxBeads], py[kBoxBeads], pz[kBoxBeads];
+        int ne[kBoxBeads], cnt[kBoxBeads];
+        int most = 0;
+#pragma unroll
+        for (int b = 0; b < kBoxBeads; ++b) {
+            px[b] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rl.x), b));
+            py[b] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rl.y), b));
+            pz[b] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rl.z), b));
+            ne[b] = __builtin_amdgcn_readlane(nel, b);
+            ev[b] = lane < ne[b] ? ev[b] : -1;
+            cnt[b] = 0;
+            most = max(most, ne[b]);
+        }
+        // candidates of tile e >> 8 (coordinates c) for the beads in e
+        auto scan = [&](unsigned e, float4 c) {
+            const int base = (int)(e >> 8) << 6;
+            if (base + 64 > n && base + lane >= n) c.x = __builtin_nanf("");
+#pragma unroll
+            for (int b = 0; b < kBoxBeads; ++b) {
+                if (!((e >> b) & 1u)) continue;
+                const float x = c.x - px[b], y = c.y - py[b], z = c.z - pz[b];
+                bool acc = x * x + y * y + z * z <= d2max;
+                unsigned long long m = __builtin_amdgcn_ballot_w64(acc);
+                unsigned long long hit = __builtin_amdgcn_ballot_w64((unsigned)(ev[b] ^ base) < 64u);
+                if (hit | (unsigned long long)(base == td.y) | (unsigned long long)(most > 64)) {
+                    unsigned long long drop = base == td.y ? 1ull << (i0 + b - base) : 0ull;
+                    while (hit) {
+                        const int q = __builtin_ctzll(hit);
+                        hit &= hit - 1ull;
+                        drop |= 1ull << (__builtin_amdgcn_readlane(ev[b], q) & 63);
+                    }
+                    for (int g = 64; g < ne[b]; g += 64) {  // exclusions past the 64th
+                        const int v = g + lane < ne[b] ? ej[(size_t)(g + lane) * n + i0 + b] : -1;
+                        unsigned long long far = __builtin_amdgcn_ballot_w64((unsigned)(v ^ base) < 64u);
+                        while (far) {
+                            const int q = __builtin_ctzll(far);
+                            far &= far - 1ull;
+                            drop |= 1ull << (__builtin_amdgcn_readlane(v, q) & 63);
                         }
-                        float4 r2[kCellChunks];
-#pragma unroll
-                        for (int u = 0; u < kCellChunks; ++u) r2[u] = cur[jj[u]];
-#pragma unroll
-                        for (int u = 0; u < kCellChunks; ++u) {
-                            const int j = jj[u];
-                            const float x = r2[u].x - r1.x, y2 = r2[u].y - r1.y, z2 = r2[u].z - r1.z;
-                            if (j != i && x * x + y2 * y2 + z2 * z2 <= d2max) {
-                                atomicOr(&bm[j >> 6], 1ull << (j & 63));
-                                atomicOr(&bm2[j >> 12], 1ull << ((j >> 6) & 63));
-                                jlo = min(jlo, j);
-                                jhi = max(jhi, j);
-                            }
-                        }
+                    }
+                    m &= ~drop;
+                    acc = acc && !((drop >> lane) & 1ull);
+                }
+                if (acc) {
+                    const int pos = (int)__builtin_amdgcn_mbcnt_hi(
+                        (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)cnt[b]));
+                    if (pos < cap) {
+                        if (idx16)
+                            (gmem(static_cast<unsigned short*>(pp)) + (size_t)(i0 + b) * ld)[pos] =
+                                (unsigned short)(base + lane);
+                        else
+                            (gmem(static_cast<int*>(pp)) + (size_t)(i0 + b) * ld)[pos] = base + lane;
                     }
                 }
-            __syncthreads();
-            for (int k = lane; k < ne; k += 64) {
-                const int e = k < 64 ? ev : ej[(size_t)k * n + i];
-                atomicAnd(&bm[e >> 6], ~(1ull << (e & 63)));
+                cnt[b] += __popcll(m);
             }
-            __syncthreads();
-            jlo = wave_min(jlo);
-            jhi = wave_max(jhi);
-            int cnt = 0;
-            const size_t rowp = (size_t)i * J.pp_ld;
-            if (jhi >= 0) {
-                const int wlo = jlo >> 6, whi = jhi >> 6;
-                for (int wb = wlo & ~63; wb <= whi; wb += 64) {
-                    const unsigned long long m2 = bm2[wb >> 6];
-                    if (m2 == 0ull) continue;  // no entry in these 64 words
-                    const int w = wb + lane;
-                    unsigned long long word = 0ull;
-                    if ((m2 >> lane) & 1ull) {
-                        word = bm[w];
-                        bm[w] = 0ull;
-                    }
-                    const int pc = __popcll(word);
-                    const int incl = wave_inclusive_sum(pc, lane);
-                    int pos = cnt + incl - pc;
-                    while (word) {
-                        const int j = (w << 6) + __builtin_ctzll(word);
-                        if (pos < cap) list_put(J.pp_j, J.idx16, rowp + pos, j);
-                        ++pos;
-                        word &= word - 1ull;
-                    }
-                    cnt += __shfl(incl, 63);
-                    if (lane == 0) bm2[wb >> 6] = 0ull;
+        };
+        int m = 0;  // collected tiles
+        for (int c0 = 0; c0 < nt; c0 += 64) {
+            const int cn = min(c0 + 64 + lane, nt - 1);
+            const float4 lon = box[2 * cn], hin = box[2 * cn + 1];
+            unsigned mask = 0u;
+#pragma unroll
+            for (int b = 0; b < kBoxBeads; ++b) {
+                const float x = fmaxf(fmaxf(lo.x - px[b], px[b] - hi.x), 0.0f);
+                const float y = fmaxf(fmaxf(lo.y - py[b], py[b] - hi.y), 0.0f);
+                const float z = fmaxf(fmaxf(lo.z - pz[b], pz[b] - hi.z), 0.0f);
+                mask |= x * x + y * y + z * z <= d2max ? 1u << b : 0u;
+            }
+            mask &= c0 + lane < nt ? (1u << nbead) - 1u : 0u;
+            const unsigned long long some = __builtin_amdgcn_ballot_w64(mask != 0u);
+            if (mask)
+                list[__builtin_amdgcn_mbcnt_hi((unsigned)(some >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((unsigned)some, (unsigned)m))] =
+                    (unsigned)(c0 + lane) << 8 | mask;
+            m += __popcll(some);
+            lo = lon;
+            hi = hin;
+            if (m == 0 || (m < kBoxList && c0 + 64 < nt)) continue;
+            wave_lds_order();
+            unsigned e[kBoxAhead];
+            float4 c[kBoxAhead];
+            auto load = [&](int q) {
+#pragma unroll
+                for (int u = 0; u < kBoxAhead; ++u) {
+                    e[u] = __builtin_amdgcn_readfirstlane(list[min(q + u, m - 1)]);
+                    c[u] = cur[min(((int)(e[u] >> 8) << 6) + lane, n - 1)];
                 }
+            };
+            load(0);
+            for (int q = 0; q < m; q += kBoxAhead) {
+                unsigned eq[kBoxAhead];
+                float4 cq[kBoxAhead];
+#pragma unroll
+                for (int u = 0; u < kBoxAhead; ++u) eq[u] = e[u], cq[u] = c[u];
+                load(q + kBoxAhead);
+#pragma unroll
+                for (int u = 0; u < kBoxAhead; ++u)
+                    if (q + u < m) scan(eq[u], cq[u]);
             }
-            __syncthreads();
-            if (lane == 0) {
-                J.pp_cnt[i] = cnt < cap ? cnt : cap;
-                if (cnt > cap) atomicOr(&st[td.x].overflow, 1);
-            }
+            wave_lds_order();
+            m = 0;
+        }
+        int total = cnt[0];
+#pragma unroll
+        for (int b = 1; b < kBoxBeads; ++b) total = lane == b ? cnt[b] : total;
+        if (lane < nbead) {
+            J.pp_cnt[i0 + lane] = min(total, cap);
+            if (total > cap) atomicOr(&st[td.x].overflow, 1);
         }
     }
 }
@@ -1981,31 +1867,24 @@ hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const DevJob
     return hipGetLastError();
 }
 
-hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int njobs,
-                           int cell_words, int any_global, const int2* sunits, const int4* segs, int nsunits,
+hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int use_boxes,
+                           int any_global, const int2* sunits, const int4* segs, int nsunits,
                            int lds_beads, int force, hipStream_t stream, const StepShape& shape) {
     if (ntiles <= 0) return hipSuccess;
-    const int use_cells = cell_words > 0;
     if (any_global || nsunits <= 0)
         hipLaunchKernelGGL(k_possible, dim3(grid_for(ntiles, 0)), dim3(256), 0, stream, jobs, st, tiles, ntiles,
-                           force, use_cells, nsunits > 0);
+                           force, use_boxes, nsunits > 0);
     if (nsunits > 0 && shape.split_rows)
         hipLaunchKernelGGL(k_possible_split, dim3(ntiles * 4), dim3(1024), (size_t)lds_beads * sizeof(float4), stream,
-                           jobs, st, tiles, ntiles, force, use_cells);
+                           jobs, st, tiles, ntiles, force, use_boxes);
     else if (nsunits > 0)
         hipLaunchKernelGGL(k_possible_lds, dim3(nsunits), dim3(kLdsUnit), (size_t)lds_beads * sizeof(float4), stream,
-                           jobs, st, sunits, segs, nsunits, force, use_cells);
-    if (use_cells) {
-        hipLaunchKernelGGL(k_cells_setup, dim3(njobs), dim3(1024), 0, stream, jobs, st, njobs, force);
-        hipLaunchKernelGGL(k_cells_count, dim3(grid_for(ntiles, 0)), dim3(256), 0, stream, jobs, st, tiles, ntiles,
-                           force);
-        hipLaunchKernelGGL(k_cells_scan, dim3(njobs), dim3(1024), 0, stream, jobs, st, njobs, force);
-        hipLaunchKernelGGL(k_cells_fill, dim3(grid_for(ntiles, 0)), dim3(256), 0, stream, jobs, st, tiles, ntiles,
-                           force);
-        int blocks = 2 * ntiles;  // one wavefront per half tile
+                           jobs, st, sunits, segs, nsunits, force, use_boxes);
+    if (use_boxes) {
+        hipLaunchKernelGGL(k_tile_boxes, dim3(grid_for(ntiles, 0)), dim3(256), 0, stream, jobs, st, tiles, ntiles, force);
+        int blocks = 64 / kBoxBeads / 4 * ntiles;
         if (blocks >= 8) blocks = (blocks + 7) / 8 * 8;
-        hipLaunchKernelGGL(k_possible_cells, dim3(blocks), dim3(64), (size_t)(cell_words + (cell_words + 63) / 64) * 8,
-                           stream, jobs, st, tiles, ntiles, force, cell_words);
+        hipLaunchKernelGGL(k_possible_boxes, dim3(blocks), dim3(256), 0, stream, jobs, st, tiles, ntiles, force);
     }
     return hipGetLastError();
 }
