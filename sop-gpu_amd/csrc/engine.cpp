@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -153,6 +154,13 @@ Engine::Engine(int device, size_t budget) : device_(device), arena_(budget) {
     if (hipSetDevice(device) != hipSuccess) throw Error{SOP_E_HIP, "hipSetDevice failed"};
     if (hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking) != hipSuccess)
         throw Error{SOP_E_HIP, "hipStreamCreate failed"};
+    // without it get_coords copies from the device buffer
+    if (hipHostMalloc((void**)&stage_, (kStageBeads + 1) * sizeof(float4), hipHostMallocCoherent) == hipSuccess) {
+        std::memset(stage_ + kStageBeads, 0, sizeof(float4));
+    } else {
+        stage_ = nullptr;
+        (void)hipGetLastError();
+    }
 }
 
 Engine::~Engine() {
@@ -165,6 +173,7 @@ Engine::~Engine() {
     }
     for (auto& j : jobs_)
         for (void* b : j.blocks) arena_.release(b);
+    (void)hipHostFree(stage_);
     (void)hipFree(d_jobs_);
     (void)hipFree(d_descs_);
     (void)hipFree(d_state_);
@@ -1390,9 +1399,28 @@ int Engine::get_indentation(int id, float* out) {
 int Engine::get_coords(int id, float* out4) {
     int slot = slot_of(id);
     if (slot < 0) return fail(SOP_E_ARG, "no such job");
+    const HostJob& hj = jobs_[slot];
+    if (stage_ && hj.n <= kStageBeads) {
+        if (int rc = sync_tables()) return rc;
+        if (hipSetDevice(device_) != hipSuccess) return fail(SOP_E_HIP, "hipSetDevice failed");
+        // the coordinates are awaited by the ticket behind them for a short
+        // while (no runtime call), then by the stream
+        unsigned* const done = reinterpret_cast<unsigned*>(stage_ + kStageBeads);
+        const unsigned ticket = ++ticket_;
+        if (int rc = check(launch_read_coords(d_jobs_ + slot, d_state_ + slot, hj.n, stage_, done, ticket, stream_),
+                           "coords read"))
+            return rc;
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(100);
+        while (__atomic_load_n(done, __ATOMIC_ACQUIRE) != ticket)
+            if (std::chrono::steady_clock::now() > until) {
+                if (int rc = check(hipStreamSynchronize(stream_), "coords read")) return rc;
+                break;
+            }
+        std::memcpy(out4, stage_, (size_t)hj.n * 16);
+        return 0;
+    }
     DevJobState s;
     if (int rc = read_state(slot, &s)) return rc;
-    const HostJob& hj = jobs_[slot];
     return check(hipMemcpy(out4, hj.dj.coord[s.step & 1], (size_t)hj.n * 16, hipMemcpyDeviceToHost), "coords read");
 }
 

@@ -189,6 +189,8 @@ class Engine {
     int box_min_ = kBoxMinBeads;
     bool use_boxes_ = true;
     int any_boxes_ = 0;
+    float4* stage_ = nullptr;  // pinned host memory that k_read_coords writes: kStageBeads entries, its ticket
+    unsigned ticket_ = 0;
     int any_idx32_ = 0;  // some job stores int32 list entries
     bool use_lds_step_ = true;
     int2* d_units_ = nullptr;  // row-sort units (job slot, first row) per kLdsUnit rows of LDS-step jobs

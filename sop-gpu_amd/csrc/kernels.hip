@@ -1087,8 +1087,9 @@ __global__ __launch_bounds__(256) void k_tile_boxes(const DevJob* __restrict__ j
 // eight take 108 and 345 (too few wavefronts for the smaller), two 76 and 380.
 // Taking the candidates bead by bead from a cell grid and sorting the accepted
 // ones through a bitmap of the job's beads took 947 and 2,283 us.  Beads in no
-// spatial order along the chain would make every box span the job: the scan
-// is then k_possible's.
+// spatial order along the chain make every box span the job and the scan
+// k_possible's (a rebuild of 18,000: 313 us, 621 by the grid; of 100,000: 5,386
+// and 2,342).
 constexpr int kBoxBeads = 4;
 constexpr int kBoxAhead = 4;
 constexpr int kBoxList = 256;  // collected tiles before they are worked off
@@ -1692,6 +1693,17 @@ __global__ void k_job_advance(const DevJob* __restrict__ jobs, DevJobState* __re
     st[jb].step = s < jobs[jb].end_step ? s : jobs[jb].end_step;
 }
 
+// One workgroup; `done` gets `ticket` once every coordinate is in host memory.
+__global__ __launch_bounds__(1024) void k_read_coords(const DevJob* __restrict__ job,
+                                                      const DevJobState* __restrict__ st, int n,
+                                                      float4* __restrict__ host, unsigned* done, unsigned ticket) {
+    const float4* const cur = job->coord[st->step & 1];
+    for (int i = threadIdx.x; i < n; i += 1024) host[i] = cur[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(done, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---------------------------------------------------------------------------
 // energies (output cadence only)
 // ---------------------------------------------------------------------------
@@ -1927,6 +1939,12 @@ hipError_t launch_job_update(const DevJob* jobs, DevJobState* st, int njobs, hip
 hipError_t launch_job_advance(const DevJob* jobs, DevJobState* st, int njobs, int nsteps, hipStream_t stream) {
     if (njobs <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_job_advance, dim3((njobs + 63) / 64), dim3(64), 0, stream, jobs, st, njobs, nsteps);
+    return hipGetLastError();
+}
+
+hipError_t launch_read_coords(const DevJob* job, const DevJobState* st, int n, float4* host, unsigned* done,
+                              unsigned ticket, hipStream_t stream) {
+    hipLaunchKernelGGL(k_read_coords, dim3(1), dim3(1024), 0, stream, job, st, n, host, done, ticket);
     return hipGetLastError();
 }
 
