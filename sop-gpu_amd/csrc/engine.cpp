@@ -927,6 +927,30 @@ StepShape Engine::effective_shape(long long lds_rows, long long global_rows, lon
     return e;
 }
 
+// Rows per wavefront of k_block_rows for jobs first .. first + count - 1, 0 where
+// their steps take a launch each: a shape that was set, a job past kBlockBeads
+// or with hydrodynamics, or few jobs whose rows the spread step divides over
+// more CUs than they have workgroups here.  Measured, us per step of a block of
+// 10, a launch per step | R = 8, 16 (the larger R where rows are many):
+//   beads x jobs   22 x 1      64        256       512        1,000       6,000
+//                  6.7 | 5.0  7.1 | 5.1  8.1 | 5.8  10.2 | 7.4  17.0 | 10.4  64 | 55, 50
+//   100 x          7.3 | 8.3  8.3 | 8.8  14.7 | 10.9, 12.1  20.0 | 19.9, 16.3  45 | 40, 32
+//   150 x 8        7.6 | -, 11.1   128: 13.4 | -, 12.8   512: 32.7 | -, 26.9
+//   250 x 32       9.5 | -, 15.2   128: 17.6 | -, 17.5   512: 59.4 | -, 41.5
+int Engine::block_rows(int first, int count, int* beads) const {
+    long long rows = 0;
+    int most = 0;
+    for (int k = first; k < first + count; ++k) {
+        const DevJob& J = jobs_[k].dj;
+        if (!J.lds_step || (J.flags & JF_HI) || J.n > kBlockBeads) return 0;
+        rows += J.n;
+        most = std::max(most, J.n);
+    }
+    *beads = most;
+    if (shape_set_ || (most > kBlockShort && rows < (long long)kBlockJobs * most)) return 0;
+    return most <= 128 && rows <= kRowsEight ? 8 : 16;
+}
+
 // The LDS step plan of the LDS-step jobs: each whole block of unit_rows
 // rows of a job is a unit; the rows left over (or a whole small job) are
 // packed, largest first, into units of at most unit_rows threads (segments
@@ -1147,6 +1171,8 @@ int Engine::launch_block(int slot_only) {
     // profiling: HIP events around the step launches; when nothing else is
     // launched between them, one pair spans the block's L launches
     const bool span = !tea && !exact;
+    int beads = 0;
+    const int block = slot_only >= 0 ? block_rows(slot_only, 1, &beads) : block_rows(0, nj, &beads);
     for (int k = 0; k < L; ++k) {
         const bool prof = profiling_ && (!span || k == 0);
         const bool prof_end = profiling_ && (!span || k == L - 1);
@@ -1163,14 +1189,17 @@ int Engine::launch_block(int slot_only) {
             }
             (void)hipEventRecord(ev_pool_[ev_used_].first, stream_);
         }
-        if (int rc = check(slot_only >= 0
-                               ? launch_step(jobs, descs, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
-                                             jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, k,
-                                             max_blocks_, stream_, eff1_)
-                               : launch_step(jobs, descs, st, tiles, nt, any_global_, d_sunits_, d_segs_, nsunits_, lds_beads_,
-                                             k, max_blocks_, stream_, eff_),
-                           "step"))
-            return rc;
+        const hipError_t e =
+            block && k % kBlockSteps ? hipSuccess  // in the launch before
+            : block ? launch_block_rows(descs, st, nj, beads, block, k, std::min(L - k, kBlockSteps),
+                                      k + kBlockSteps >= L ? L : 0, stream_)
+            : slot_only >= 0
+                ? launch_step(jobs, descs, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
+                              jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, k, max_blocks_, stream_,
+                              eff1_)
+                : launch_step(jobs, descs, st, tiles, nt, any_global_, d_sunits_, d_segs_, nsunits_, lds_beads_, k,
+                              max_blocks_, stream_, eff_);
+        if (int rc = check(e, "step")) return rc;
         if (prof_end) {
             (void)hipEventRecord(ev_pool_[ev_used_].second, stream_);
             ev_launches_[ev_used_] = span ? L : 1;
@@ -1197,8 +1226,8 @@ int Engine::launch_block(int slot_only) {
             }
         }
     }
-    if (int rc = check(launch_job_advance(jobs, st, nj, L, stream_), "advance")) return rc;
-    return 0;
+    if (block) return 0;  // advanced by its last launch
+    return check(launch_job_advance(jobs, st, nj, L, stream_), "advance");
 }
 
 // Tile list of one job (job index 0 relative to its slot), cached.
@@ -1256,13 +1285,17 @@ int Engine::stage_job_update(int mask) {
 }
 int Engine::stage_possible() {
     if (int rc = sync_tables()) return rc;
+    if (!(lists_due(-1) & 1)) return 0;
     return check(launch_possible(d_jobs_, d_state_, d_tiles_, ntiles_, any_boxes_, any_global_, d_sunits_, d_segs_,
                                  nsunits_, lds_beads_, 0, stream_, eff_),
                  "possible pairs");
 }
 int Engine::stage_verlet() {
     if (int rc = sync_tables()) return rc;
-    return check(launch_verlet(d_jobs_, d_state_, d_tiles_, ntiles_, any_idx32_, any_global_, d_units_, nunits_,
+    const int due = lists_due(-1);
+    if (!(due & 2)) return 0;
+    return check(launch_verlet(d_jobs_, d_state_, d_tiles_, ntiles_, any_idx32_, any_global_, d_units_,
+                               due & 4 ? nunits_ : 0,
                                d_sunits_, d_segs_, nsunits_, lds_beads_, 0, stream_, eff_),
                  "verlet");
 }
@@ -1290,6 +1323,18 @@ int Engine::stage_step(int k) {
                                "Cholesky step"))
                 return rc;
         }
+    return 0;
+}
+int Engine::stage_steps(int n) {
+    if (int rc = sync_tables()) return rc;
+    int beads = 0;
+    const int block = block_rows(0, (int)jobs_.size(), &beads);
+    for (int k = 0; k < n; k += block ? kBlockSteps : 1)
+        if (int rc = block ? check(launch_block_rows(d_descs_, d_state_, (int)jobs_.size(), beads, block, k,
+                                                     std::min(n - k, kBlockSteps), 0, stream_),
+                                   "steps")
+                           : stage_step(k))
+            return rc;
     return 0;
 }
 int Engine::stage_advance(int nsteps) {
@@ -1788,8 +1833,17 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
     void* snap = nullptr;
     if (int rc = snapshot(&snap)) return rc;
     int trials = 0;
+    auto unset = [&] {  // the shape follows the rows again
+        shape_.split_rows = shape_.split_global = 0;
+        shape_set_ = false;
+    };
+    // a block in one launch is taken only where no shape is set: measured as
+    // such, and left so unless a set shape is faster
+    int beads = 0;
+    bool block = block_rows(0, (int)jobs_.size(), &beads) > 0;
     auto trial = [&](const Tuning& t, double* per_step) -> int {
         if (int rc = set_shape(t)) return rc;
+        if (block && trials == 0) unset();
         if (int rc = restore(snap, steps)) return rc;
         double ms = 0.0;
         if (int rc = time_blocks(nblocks, &ms)) return rc;
@@ -1808,6 +1862,7 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
         if (!rc && ms < best_ms * 0.995) {  // a real gain, beyond run-to-run noise
             best = t;
             best_ms = ms;
+            block = false;
         }
     };
     // each bead's terms spread over a wavefront, or one bead per lane
@@ -1837,14 +1892,11 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
     }
     // the jobs as they were, under the chosen shape
     const int rc2 = set_shape(rc ? start : best);
+    if (block || (rc && !was_set)) unset();
     const int rc3 = restore(snap, steps);
     (void)hipFree(snap);
     use_graph_ = saved_graph;
     profiling_ = saved_prof;
-    if (rc && !was_set) {  // as it was: the shape follows the rows again
-        shape_.split_rows = shape_.split_global = 0;
-        shape_set_ = false;
-    }
     if (rc) return rc;
     if (rc2) return rc2;
     if (rc3) return rc3;

@@ -125,6 +125,7 @@ class Engine {
     int stage_verlet();
     int stage_tea_update();
     int stage_step(int kstep);
+    int stage_steps(int n);  // steps 0 .. n - 1 of the block
     int stage_advance(int nsteps);
     int read_state_of(int id, DevJobState* out);
 
@@ -219,6 +220,7 @@ class Engine {
     int time_blocks(int nblocks, double* ms);
     bool uses_boxes(size_t n) const;
     int boxes_of(const DevJob& J) const;
+    int block_rows(int first, int count, int* beads) const;
     int exact_mode_ = SOP_CHOL_BF16X3;
     bool any_tea_ = false, any_exact_ = false;
     bool use_graph_ = true;

@@ -29,6 +29,11 @@ struct StepShape {
 // are too short for less than eight rows per wavefront.
 constexpr int kRowsTwo = 4500, kRowsFour = 17000, kRowsEight = 34000, kRowsMaxLds = 90000, kRowsMaxGlobal = 220000;
 constexpr int kRowsShort = 28;
+// A block of steps in one launch (k_block_rows; measurements at
+// Engine::block_rows): beads of a job up to which it is possible, beads up to
+// which it pays for any number of jobs, jobs of the largest size (by rows)
+// from which it pays past that, and steps of one launch.
+constexpr int kBlockBeads = 256, kBlockShort = 32, kBlockJobs = 100, kBlockSteps = 250;
 // The autotuner tries split_rows only where the launch has at most this many
 // 64-row tiles.
 constexpr int kSplitMaxTiles = 1536;
@@ -76,6 +81,11 @@ hipError_t launch_read_coords(const DevJob* job, const DevJobState* st, int n, f
 hipError_t launch_job_advance(const DevJob* jobs, DevJobState* st, int njobs, int nsteps, hipStream_t stream);
 // Output / parity hooks.
 hipError_t launch_energies(const DevJob* jobs, const DevJobState* st, int job, int n, hipStream_t stream);
+// Steps state.step + kstep .. + nsteps - 1 of njobs jobs of at most `beads`
+// beads, R rows per wavefront (ceil(beads / R) <= 16), in one launch, which then
+// adds `advance` to the step counters.
+hipError_t launch_block_rows(const StepDesc* descs, DevJobState* st, int njobs, int beads, int R, int kstep, int nsteps,
+                             int advance, hipStream_t stream);
 // Forces only (the step kernels' force terms, no state change) of the jobs
 // of the given tiles / LDS plan, into out[bead] (one job per launch).
 hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,

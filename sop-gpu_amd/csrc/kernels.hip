@@ -297,21 +297,25 @@ __device__ __forceinline__ void step_head(const DevJob& J, int i, int r, int n, 
 // The per-bead state the tail reads and its noise, formed ahead by a caller
 // with latency to hide (which then also writes the RNG state back): the
 // Gaussian triple, the temperature accumulator and the fixed/pulled flag.
+// A caller that takes several steps says whether one starts a stride (due) and
+// gets T and the new coordinates c back.
 struct TailPre {
     float3 g;
     float T;
     int flag;
+    bool due;
+    float4 c;
 };
 
 // The rest of a bead's step, after the repulsive pairs: indentation walls,
 // then (FO) the forces written to cout, or the noise (of amplitude var), the
 // fixed/pulled rules and the Euler update written to `cout` in global memory.  Hydrodynamic
 // jobs stop after the forces.  pre: the state loaded ahead (null: loaded
-// here).
-template <bool FO, typename D>
+// here).  KEEP: T and the coordinates stay in *pre, nothing is written.
+template <bool FO, bool KEEP = false, typename D>
 __device__ __forceinline__ void step_tail(const D& J, const DevJobState& S, float var, long long s, int i, const float4 c,
                                           float fx, float fy, float fz, float4* __restrict__ cout,
-                                          const TailPre* pre = nullptr) {
+                                          TailPre* pre = nullptr) {
     // indentation tip and substrate plane (indentation_kernel.cu:71-128)
     if (J.flags & JF_INDENTATION) {
         float4 fin = J.tipF[i];
@@ -375,10 +379,16 @@ __device__ __forceinline__ void step_tail(const D& J, const DevJobState& S, floa
     cn.z += dz;
     // the temperature accumulator is cleared at updater passes that fall
     // on a multiple of nav (output_manager.cu:124-126)
-    const bool reset = (s % J.stride == 0) && (s % J.nav == 0);
+    const bool reset = (KEEP ? pre->due : s % J.stride == 0) && s % J.nav == 0;
     const float T0 = reset ? 0.0f : (pre ? pre->T : J.T[i]);
-    J.T[i] = T0 + J.tempNorm * (dx * dx + dy * dy + dz * dz);
-    cout[i] = cn;
+    const float T1 = T0 + J.tempNorm * (dx * dx + dy * dy + dz * dz);
+    if constexpr (KEEP) {
+        pre->T = T1;
+        pre->c = cn;
+    } else {
+        J.T[i] = T1;
+        cout[i] = cn;
+    }
 }
 
 // One bead's step: FENE, native and repulsive terms gathered from `cin`
@@ -492,10 +502,10 @@ __global__ __launch_bounds__(1024, PB <= 6 ? 8 : 4) void k_step_lds(const DevJob
 // dependent reads (tile, record, lists, partners) where rows are few, by VALU
 // issue from about 30,000 rows on; measured at Engine::effective_shape (18,000
 // beads: 58 us one bead per lane, 16 us here).
-template <int R>
+template <int R, bool BLK = false>
 struct RowsShape {
     static constexpr int P = 64 / R;              // positions of a row evaluated at a time
-    static constexpr int U = R <= 4 ? 4 : 8;      // terms per lane and chunk
+    static constexpr int U = R <= 4 || BLK ? 4 : 8;  // terms per lane and chunk
     static constexpr int K = P * U;               // terms of a row per chunk
     // row stride of the LDS rows: the R rows' P consecutive words (writes) and
     // 16-byte reads fall in distinct banks
@@ -569,10 +579,15 @@ __device__ __forceinline__ void rows_add(const float* __restrict__ t, int m, flo
 }
 
 // The rows of k_step_rows: R rows of one job by one wavefront, lists of IdxT.
-template <bool FO, int R, typename IdxT>
+// BLK (k_block_rows): nsteps steps, the coordinates in LDS (two buffers of
+// ldc beads from lc, the first filled), a workgroup barrier after each step;
+// what a step reads besides them stays in registers.
+template <bool FO, int R, typename IdxT, bool BLK = false>
 __device__ __forceinline__ void step_rows(const StepDesc& D, const DevJobState& S, float var, long long s, int row0,
-                                          float (*term)[R][RowsShape<R>::KP], float4* __restrict__ fout) {
-    constexpr int P = RowsShape<R>::P, U = RowsShape<R>::U, K = RowsShape<R>::K;
+                                          float (*term)[R][RowsShape<R, BLK>::KP], float4* __restrict__ fout,
+                                          float4* lc = nullptr, int ldc = 0, int nsteps = 1) {
+    using Shape = RowsShape<R, BLK>;
+    constexpr int P = Shape::P, U = Shape::U, K = Shape::K;
     const int lane = threadIdx.x & 63;
     const int n = D.n;
     const float4* const cin = (s & 1) ? D.coord[1] : D.coord[0];
@@ -603,7 +618,12 @@ __device__ __forceinline__ void step_rows(const StepDesc& D, const DevJobState& 
         nn = gmem(D.nat_cnt)[i];
     }
     const int col = D.b_cnt ? rc : i;
-    const float4 c = ldg_coord(cin, i);
+    const float4* lin = lc;  // BLK: the step's coordinates
+    auto coord = [&](int j) {
+        if constexpr (BLK) return lin[j];
+        else return ldg_coord(cin, j);
+    };
+    float4 c = coord(i);
     const bool noise = !FO && !(D.flags & JF_MINIMIZATION);
     TailPre pre;
     uint4 rng = make_uint4(0, 0, 0, 0);
@@ -640,7 +660,7 @@ __device__ __forceinline__ void step_rows(const StepDesc& D, const DevJobState& 
     float4 o[U];
     auto gather = [&](int b) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) o[u] = ldg_coord(cin, b + u * P + p < np ? (int)jn[u] : i);
+        for (int u = 0; u < U; ++u) o[u] = coord(b + u * P + p < np ? (int)jn[u] : i);
     };
     auto fetch = [&](int b) {
 #pragma unroll
@@ -655,103 +675,127 @@ __device__ __forceinline__ void step_rows(const StepDesc& D, const DevJobState& 
             if (b + u * P < nbm) f[u] = bonded_fetch<IdxT>(D, b + u * P + p, col, i, nc, nn);
     };
     bonded(0);
-    if (npm > 0) gather(0);
-    if (npm > K) fetch(K);
-    // lanes p = 0 and 1 draw the step's four numbers and form one Box-Muller
-    // pair each (gauss3's order; the second's cosine is not used)
-    if (noise) {
-        const uint32_t u0 = hybrid_taus(rng);
-        const uint32_t u1 = hybrid_taus(rng);
-        const uint32_t u2 = hybrid_taus(rng);
-        const uint32_t u3 = hybrid_taus(rng);
-        if (p == 0 && r < n) D.rng[i] = rng;
-        float sn, cs;
-        const float rr = sqrtf(-2.0f * logf_series(uint_to_unit(p == 0 ? u0 : u2)));
-        const float th = (float)(6.283185307179586 * (double)uint_to_unit(p == 0 ? u1 : u3));
-        sincosf_series(th, sn, cs);
-        const float gs = rr * sn;
-        pre.g = make_float3(gs, rr * cs, __shfl(gs, (lane + R) & 63));
-    }
-    // FENE and native terms
-    for (int b = 0; b < nbm; b += P * UB) {
-        if (b > 0) bonded(b);
+    int phase = BLK ? (int)(s % D.stride) : 0;  // of the step within the stride
+    for (int step = 0; step < (BLK ? nsteps : 1); ++step) {
+        if (BLK && step > 0) {
+            c = coord(i);
+            acc = 0.0f;
+            if (nbm > P * UB) bonded(0);
+            if (npm > K) fetch(0);
+        }
+        if (npm > 0) gather(0);
+        if (npm > K) fetch(K);
+        // lanes p = 0 and 1 draw the step's four numbers and form one Box-Muller
+        // pair each (gauss3's order; the second's cosine is not used)
+        if (noise) {
+            const uint32_t u0 = hybrid_taus(rng);
+            const uint32_t u1 = hybrid_taus(rng);
+            const uint32_t u2 = hybrid_taus(rng);
+            const uint32_t u3 = hybrid_taus(rng);
+            if (!BLK && p == 0 && r < n) D.rng[i] = rng;
+            float sn, cs;
+            const float rr = sqrtf(-2.0f * logf_series(uint_to_unit(p == 0 ? u0 : u2)));
+            const float th = (float)(6.283185307179586 * (double)uint_to_unit(p == 0 ? u1 : u3));
+            sincosf_series(th, sn, cs);
+            const float gs = rr * sn;
+            pre.g = make_float3(gs, rr * cs, __shfl(gs, (lane + R) & 63));
+        }
+        // FENE and native terms
+        for (int b = 0; b < nbm; b += P * UB) {
+            if (b > 0) bonded(b);
 #pragma unroll
-        for (int u = 0; u < UB; ++u)
-            if (b + u * P < nbm) {
-                const float4 w = ldg_coord(cin, f[u].j);
-                const float x = w.x - c.x, y = w.y - c.y, z = w.z - c.z;
-                float tx = -0.0f, ty = -0.0f, tz = -0.0f;
-                if (f[u].type == 0) {
-                    const float v = fene_w(D.ks, D.R2, x, y, z, f[u].par.x);
-                    tx = v * x;
-                    ty = v * y;
-                    tz = v * z;
-                } else if (f[u].type == 1) {
-                    const float v = native_q(x, y, z, f[u].par);
-                    tx = x * v;
-                    ty = y * v;
-                    tz = z * v;
+            for (int u = 0; u < UB; ++u)
+                if (b + u * P < nbm) {
+                    const float4 w = coord(f[u].j);
+                    const float x = w.x - c.x, y = w.y - c.y, z = w.z - c.z;
+                    float tx = -0.0f, ty = -0.0f, tz = -0.0f;
+                    if (f[u].type == 0) {
+                        const float v = fene_w(D.ks, D.R2, x, y, z, f[u].par.x);
+                        tx = v * x;
+                        ty = v * y;
+                        tz = v * z;
+                    } else if (f[u].type == 1) {
+                        const float v = native_q(x, y, z, f[u].par);
+                        tx = x * v;
+                        ty = y * v;
+                        tz = z * v;
+                    }
+                    term[0][q][u * P + p] = tx;
+                    term[1][q][u * P + p] = ty;
+                    term[2][q][u * P + p] = tz;
                 }
-                term[0][q][u * P + p] = tx;
-                term[1][q][u * P + p] = ty;
-                term[2][q][u * P + p] = tz;
-            }
-        wave_lds_order();
-        if (p < 3) rows_add(&term[p][q][0], min(P * UB, nbm - b), acc);
-        wave_lds_order();
-    }
-    // repulsive pairs: the next chunk's partners and the entries of the one
-    // after it are in flight while a chunk is added
-    const float rc2 = D.rc2, a2 = D.a2, m6 = D.m6;
-    const bool fast = div_fast_numerator(a2) && rc2 <= kDivFastMaxB;
-    // term u of the chunk from b into LDS; its factor by the short division,
-    // or (SLOW) by whichever the divisor admits
-    auto put = [&](int u, bool ok, float x, float y, float z, float w) {
-        term[0][q][u * P + p] = ok ? x * w : -0.0f;
-        term[1][q][u * P + p] = ok ? y * w : -0.0f;
-        term[2][q][u * P + p] = ok ? z * w : -0.0f;
-    };
-    for (int b = 0; b < npm; b += K) {
-        // straight-line code over the chunk's terms, so that their latencies
-        // overlap; a divisor outside the short division's range (beads almost
-        // on top of each other) sends the chunk through the general one
-        bool bad = !fast;
+            wave_lds_order();
+            if (p < 3) rows_add(&term[p][q][0], min(P * UB, nbm - b), acc);
+            wave_lds_order();
+        }
+        // repulsive pairs: the next chunk's partners and the entries of the one
+        // after it are in flight while a chunk is added
+        const float rc2 = D.rc2, a2 = D.a2, m6 = D.m6;
+        const bool fast = div_fast_numerator(a2) && rc2 <= kDivFastMaxB;
+        // term u of the chunk from b into LDS; its factor by the short division,
+        // or (SLOW) by whichever the divisor admits
+        auto put = [&](int u, bool ok, float x, float y, float z, float w) {
+            term[0][q][u * P + p] = ok ? x * w : -0.0f;
+            term[1][q][u * P + p] = ok ? y * w : -0.0f;
+            term[2][q][u * P + p] = ok ? z * w : -0.0f;
+        };
+        for (int b = 0; b < npm; b += K) {
+            // straight-line code over the chunk's terms, so that their latencies
+            // overlap; a divisor outside the short division's range (beads almost
+            // on top of each other) sends the chunk through the general one
+            bool bad = !fast;
 #pragma unroll
-        for (int h = 0; h < U; h += 4)
-            if (b + h * P < npm) {
+            for (int h = 0; h < U; h += 4)
+                if (b + h * P < npm) {
 #pragma unroll
-                for (int u = h; u < h + 4; ++u) {
-                    const float x = o[u].x - c.x, y = o[u].y - c.y, z = o[u].z - c.z;
+                    for (int u = h; u < h + 4; ++u) {
+                        const float x = o[u].x - c.x, y = o[u].y - c.y, z = o[u].z - c.z;
+                        const float d2 = x * x + y * y + z * z;
+                        const bool ok = (b + u * P + p < np) & (d2 < rc2);
+                        bad = bad | (ok & !(d2 >= kDivFastMinB));
+                        float w = div_rn_fast(a2, d2);
+                        w = w * w;
+                        put(u, ok, x, y, z, m6 * w * w);
+                    }
+                }
+            if (__builtin_amdgcn_ballot_w64(bad)) {
+                for (int u = 0; u < U && b + u * P < npm; ++u) {
+                    float4 w = o[0];  // the partner of term u (o is indexed by constants only)
+#pragma unroll
+                    for (int v = 1; v < U; ++v)
+                        if (v == u) w = o[v];
+                    const float x = w.x - c.x, y = w.y - c.y, z = w.z - c.z;
                     const float d2 = x * x + y * y + z * z;
                     const bool ok = (b + u * P + p < np) & (d2 < rc2);
-                    bad = bad | (ok & !(d2 >= kDivFastMinB));
-                    float w = div_rn_fast(a2, d2);
-                    w = w * w;
-                    put(u, ok, x, y, z, m6 * w * w);
+                    put(u, ok, x, y, z, ok ? pair_q(d2, a2, m6, fast) : 0.0f);
                 }
             }
-        if (__builtin_amdgcn_ballot_w64(bad)) {
-            for (int u = 0; u < U && b + u * P < npm; ++u) {
-                float4 w = o[0];  // the partner of term u (o is indexed by constants only)
-#pragma unroll
-                for (int v = 1; v < U; ++v)
-                    if (v == u) w = o[v];
-                const float x = w.x - c.x, y = w.y - c.y, z = w.z - c.z;
-                const float d2 = x * x + y * y + z * z;
-                const bool ok = (b + u * P + p < np) & (d2 < rc2);
-                put(u, ok, x, y, z, ok ? pair_q(d2, a2, m6, fast) : 0.0f);
-            }
+            if (b + K < npm) gather(b + K);
+            if (b + 2 * K < npm) fetch(b + 2 * K);
+            wave_lds_order();
+            if (p < 3) rows_add(&term[p][q][0], min(K, npm - b), acc);
+            wave_lds_order();
         }
-        if (b + K < npm) gather(b + K);
-        if (b + 2 * K < npm) fetch(b + 2 * K);
-        wave_lds_order();
-        if (p < 3) rows_add(&term[p][q][0], min(K, npm - b), acc);
-        wave_lds_order();
+        const float fy = __shfl(acc, (lane + R) & 63), fz = __shfl(acc, (lane + 2 * R) & 63);
+        if constexpr (BLK) {
+            if (p == 0 && r < n) {
+                pre.due = phase == 0;
+                step_tail<false, true>(D, S, var, s + step, i, c, acc, fy, fz, nullptr, &pre);
+                lc[((step + 1) & 1) * ldc + i] = pre.c;
+                // both buffers are left as one launch per step leaves them
+                if (step + 2 >= nsteps) (((s + step) & 1) ? D.coord[0] : D.coord[1])[i] = pre.c;
+            }
+            __syncthreads();
+            lin = lc + ((step + 1) & 1) * ldc;
+            if (++phase == D.stride) phase = 0;
+        } else if (p == 0 && r < n) {
+            float4* const cout = FO ? fout : (s & 1) ? D.coord[0] : D.coord[1];
+            step_tail<FO>(D, S, var, s, i, c, acc, fy, fz, cout, FO ? nullptr : &pre);
+        }
     }
-    const float fy = __shfl(acc, (lane + R) & 63), fz = __shfl(acc, (lane + 2 * R) & 63);
-    if (p == 0 && r < n) {
-        float4* const cout = FO ? fout : (s & 1) ? D.coord[0] : D.coord[1];
-        step_tail<FO>(D, S, var, s, i, c, acc, fy, fz, cout, FO ? nullptr : &pre);
+    if (BLK && p == 0 && r < n) {
+        D.T[i] = pre.T;
+        if (noise) D.rng[i] = rng;
     }
 }
 
@@ -787,6 +831,46 @@ __global__ __launch_bounds__(256, 4) void k_step_rows(const StepDesc* __restrict
         step_rows<FO, R, unsigned short>(D, st[td.x], var, s, row0, terms[w], fout);
     else
         step_rows<FO, R, int>(D, st[td.x], var, s, row0, terms[w], fout);
+}
+
+// The steps of a block in one launch, for launches of small jobs: one workgroup
+// per job, a wavefront per R of its rows (blockDim.x / 64 >= ceil(n / R)), the
+// coordinates in LDS and a barrier between steps in the place of a launch.  Of
+// k_step_rows' chain only the sums are left: lists and generators stay in
+// registers, partners come from LDS.  Bound by VALU issue, about 1,000
+// instructions a step and wavefront, at one wavefront a SIMD.  ldc: beads of
+// the launch's largest job; advance: what the block's last launch adds to the
+// step counters (in the place of k_job_advance), 0 for none.  350 peptides of
+// 22 beads, a block of ten steps: 37 us, 75 as ten launches of k_step_rows and
+// the gaps between them.
+template <int R>
+__global__ __launch_bounds__(1024) void k_block_rows(const StepDesc* __restrict__ descs,
+                                                     DevJobState* __restrict__ st, int ldc, int kstep, int nsteps,
+                                                     int advance) {
+    using Rows = float[3][R][RowsShape<R, true>::KP];
+    extern __shared__ float4 lds_coord[];
+    Rows* const terms = reinterpret_cast<Rows*>(lds_coord + 2 * ldc);
+    const StepDesc D = descs[blockIdx.x];
+    const long long s = st[blockIdx.x].step + kstep;
+    const float var = st[blockIdx.x].var;
+    asm volatile("" ::"s"(D.coord[0]), "s"(D.coord[1]), "s"(D.perm), "s"(D.pair_cnt), "s"(D.pair_j), "s"(D.b_cnt),
+                 "s"(D.cov_j), "s"(D.cov_r0), "s"(D.nat_j), "s"(D.nat_par), "s"(D.rng), "s"(D.T), "s"(D.bflag));
+    const int steps = (int)min((long long)nsteps, D.end_step - s);
+    if (steps <= 0) return;
+    const float4* const cin = (s & 1) ? D.coord[1] : D.coord[0];
+    for (int i = threadIdx.x; i < D.n; i += blockDim.x) lds_coord[i] = ldg_coord(cin, i);
+    __syncthreads();
+    const int w = wave_id(), row0 = R * w;
+    if (row0 >= D.n) {  // no rows: the barriers of the others' steps
+        for (int k = 0; k < steps; ++k) __syncthreads();
+    } else if (D.idx16) {
+        step_rows<false, R, unsigned short, true>(D, st[blockIdx.x], var, s, row0, terms[w], nullptr, lds_coord, ldc,
+                                                  steps);
+    } else {
+        step_rows<false, R, int, true>(D, st[blockIdx.x], var, s, row0, terms[w], nullptr, lds_coord, ldc, steps);
+    }
+    // every wavefront took the step before its first barrier
+    if (advance && threadIdx.x == 0) st[blockIdx.x].step = min(s - kstep + advance, D.end_step);
 }
 
 // ---------------------------------------------------------------------------
@@ -1859,6 +1943,23 @@ hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const DevJobSt
         else
             hipLaunchKernelGGL((k_step_lds<false, 6>), g, b, lds, stream, jobs, st, units, segs, nunits, kstep, nullptr);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_block_rows(const StepDesc* descs, DevJobState* st, int njobs, int beads, int R, int kstep, int nsteps,
+                             int advance, hipStream_t stream) {
+    const int waves = (beads + R - 1) / R;
+    if (waves > 16) return hipErrorInvalidValue;
+    const dim3 g(njobs), b(64 * waves);
+    auto lds = [&](int kp) { return (size_t)2 * beads * 16 + (size_t)waves * 3 * R * kp * 4; };
+    if (R == 2)
+        hipLaunchKernelGGL(k_block_rows<2>, g, b, lds(RowsShape<2, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
+    else if (R == 4)
+        hipLaunchKernelGGL(k_block_rows<4>, g, b, lds(RowsShape<4, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
+    else if (R == 8)
+        hipLaunchKernelGGL(k_block_rows<8>, g, b, lds(RowsShape<8, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
+    else
+        hipLaunchKernelGGL(k_block_rows<16>, g, b, lds(RowsShape<16, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
     return hipGetLastError();
 }
 

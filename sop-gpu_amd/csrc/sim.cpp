@@ -617,6 +617,7 @@ struct StepIntegrator : SOPIntegrator {  // LangevinIntegrator / TeaIntegrator
         }
         sim.check(sim.eng->stage_step(sim.substep++));
     }
+    void integrate_all(int n) { sim.check(sim.eng->stage_steps(n)); }
 };
 
 // ---- configuration -> sop_params (the plugins' PARAMETER()s) ---------------
@@ -889,12 +890,17 @@ static void run_sim(Sim& sim) {
     // of the topology's [ pairs ], so the step-0 energies use it (gsop.cu:126)
     for (size_t k = 0; k < sim.builtin_updaters; ++k)
         if (sim.updaters[k]->name == "Pairlist") sim.updaters[k]->update();
+    auto* const own_step = dynamic_cast<StepIntegrator*>(sim.integrator.get());
     for (long long b = sim.step / stride; b <= sim.numsteps / stride; ++b) {
         sim.substep = 0;
         for (auto& u : sim.updaters) u->update();
-        for (int j = 0; j < stride; ++j) {
-            for (auto& pot : sim.potentials) pot->compute();
-            sim.integrator->integrate();
+        if (own_step && !host_pot) {  // nothing on the host acts between the steps
+            own_step->integrate_all(stride);
+        } else {
+            for (int j = 0; j < stride; ++j) {
+                for (auto& pot : sim.potentials) pot->compute();
+                sim.integrator->integrate();
+            }
         }
         sim.check(sim.eng->stage_advance(stride));
         sim.step += stride;
