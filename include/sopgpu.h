@@ -148,7 +148,8 @@ int sop_engine_job_bytes(const sop_params* p, const sop_system* s, unsigned long
 
 /* Launch shape: max_blocks caps the persistent step grid (0: one
  * workgroup per 4 tiles); use_graph != 0 replays each block from a
- * captured hipGraph. */
+ * captured hipGraph (several at a time, once their launch sequence has come
+ * four times). */
 int sop_engine_set_tuning(sop_engine* e, int max_blocks, int use_graph);
 /* Possible-pairs builder (src/Updaters/possiblepairlist_kernel.cu:18-71
  * scans all same-trajectory pairs): jobs of min_beads beads and more admitted

@@ -157,7 +157,9 @@ class Engine {
     int launch_block(int slot_only);  // slot_only < 0: all jobs
     int lists_due(int slot_only) const;
     std::vector<long long> block_key() const;
-    int capture_graph(const std::vector<long long>& key);
+    int launch_blocks(int blocks);
+    int graph_blocks() const;
+    int capture_graph(const std::vector<long long>& key, int blocks);
     void drop_graph();
     int check(hipError_t e, const char* what);
     int read_state(int slot, DevJobState* out);
@@ -224,10 +226,13 @@ class Engine {
     int exact_mode_ = SOP_CHOL_BF16X3;
     bool any_tea_ = false, any_exact_ = false;
     bool use_graph_ = true;
-    // captured blocks by launch sequence (block_key()): the list kernels due
-    // and each exact-HI job's refactorisation steps; at most kMaxGraphs
-    static constexpr size_t kMaxGraphs = 32;
+    // captured blocks by launch sequence (block_key() of each): the list
+    // kernels due and each exact-HI job's refactorisation steps; at most
+    // kMaxGraphs.  came_: how often a sequence not captured has come
+    static constexpr size_t kMaxGraphs = 32, kMaxCame = 256;
+    static constexpr int kGraphSteps = 100, kGraphBlocks = 10, kGraphAfter = 4;
     std::map<std::vector<long long>, hipGraphExec_t> graphs_;
+    std::map<std::vector<long long>, int> came_;
     // profiling
     bool profiling_ = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev_pool_;
