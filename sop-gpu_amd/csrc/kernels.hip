@@ -1791,53 +1791,101 @@ __global__ __launch_bounds__(1024) void k_read_coords(const DevJob* __restrict__
 // ---------------------------------------------------------------------------
 // energies (output cadence only)
 // ---------------------------------------------------------------------------
+// A wavefront takes kEnergyRows Verlet rows, lane q + R p the terms p, p + P,
+// ... (P = 64 / R) of row q: four in flight, into LDS, where the row's first
+// lane adds them in list order (positions without a term hold -0.0, which
+// changes no sum).  FENE terms, few and subtracted in FP64, go round by lane
+// reads.  Bound by the gathers' latency where one lane per row walked the
+// ~1,000 entries one after another: 134 us for 18,000 beads, 21 here.
+constexpr int kEnergyRows = 4;
 __global__ __launch_bounds__(256) void k_energies(const DevJob* __restrict__ jobs, const DevJobState* __restrict__ st,
                                                   int job) {
+    constexpr int R = kEnergyRows, P = 64 / R, U = 4, K = P * U;
+    __shared__ __align__(16) float terms[4][R][K + 4];
     const DevJob& J = jobs[job];
-    const int n = J.n;
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;  // Verlet row of bead i
-    if (r >= n) return;
-    const int i = J.perm[r];
-    const long long s = st[job].step;
-    const float4* __restrict__ cur = J.coord[s & 1];
+    const int n = J.n, w = wave_id(), row0 = R * (4 * (int)blockIdx.x + w);
+    if (row0 >= n) return;
+    const int lane = threadIdx.x & 63, q = lane % R, p = lane / R;
+    const int r = row0 + q, rc = min(r, n - 1);
+    const CoordGlobal cur{J.coord[st[job].step & 1]};
+    const int i = gmem(J.perm)[rc];
     const float4 c = cur[i];
+    const bool own = r < n;
+    const int nc = own ? gmem(J.cov_cnt)[i] : 0, nn = own ? gmem(J.nat_cnt)[i] : 0, np = own ? gmem(J.pair_cnt)[rc] : 0;
+    int ncm = nc, nnm = nn, npm = np;  // the longest rows (every set of R lanes holds all rows)
+#pragma unroll
+    for (int o = R / 2; o > 0; o >>= 1) {
+        ncm = max(ncm, __shfl_xor(ncm, o));
+        nnm = max(nnm, __shfl_xor(nnm, o));
+        npm = max(npm, __shfl_xor(npm, o));
+    }
+    ncm = __builtin_amdgcn_readfirstlane(ncm);
+    nnm = __builtin_amdgcn_readfirstlane(nnm);
+    npm = __builtin_amdgcn_readfirstlane(npm);
     float pot = 0.0f;
-    for (int k = 0; k < J.cov_cnt[i]; ++k) {
-        const int j = J.cov_j[(size_t)k * n + i];
-        const float r0 = J.cov_r0[(size_t)k * n + i];
-        const float4 o = cur[j];
-        const float x = o.x - c.x, y = o.y - c.y, z = o.z - c.z;
-        float w = sqrtf(x * x + y * y + z * z);
-        w = w - r0;
-        pot = (float)((double)pot - ((double)J.ks / 2.0) * (double)J.R2 * (double)logf_series(1.0f - w * w / (J.R2)));
-    }
-    J.energies[i] = pot;
-    pot = 0.0f;
-    for (int k = 0; k < J.nat_cnt[i]; ++k) {
-        const int j = J.nat_j[(size_t)k * n + i];
-        const float2 par = J.nat_par[(size_t)k * n + i];
-        const float4 o = cur[j];
-        const float x = o.x - c.x, y = o.y - c.y, z = o.z - c.z;
-        const float q = par.x / (x * x + y * y + z * z);
-        float p6 = q * q * q;
-        const float p12 = p6 * p6;
-        p6 = -2.0f * p6;
-        const float eh = (float)((double)(-par.y * par.x) / 12.0);
-        pot += eh * (p6 + p12);
-    }
-    J.energies[n + i] = pot;
-    pot = 0.0f;
-    for (int k = 0; k < J.pair_cnt[r]; ++k) {
-        const int j = list_at(J.pair_j, J.idx16, (size_t)k * J.pair_ld + r);
-        const float4 o = cur[j];
-        const float x = o.x - c.x, y = o.y - c.y, z = o.z - c.z;
-        const float d2 = x * x + y * y + z * z;
-        if (d2 < J.rc2) {
-            const float q = J.a2 / d2;
-            pot += J.el * q * q * q;
+    for (int b = 0; b < ncm; b += P) {
+        double t = 0.0;
+        if (b + p < nc) {
+            const size_t e = (size_t)(b + p) * n + i;
+            const float4 o = cur[gmem(J.cov_j)[e]];
+            const float x = o.x - c.x, y = o.y - c.y, z = o.z - c.z;
+            float d = sqrtf(x * x + y * y + z * z);
+            d = d - gmem(J.cov_r0)[e];
+            t = ((double)J.ks / 2.0) * (double)J.R2 * (double)logf_series(1.0f - d * d / (J.R2));
+        }
+        for (int u = 0; u < min(P, ncm - b); ++u) {
+            const double v = __shfl(t, q + R * u);
+            if (b + u < nc) pot = (float)((double)pot - v);
         }
     }
-    J.energies[2 * n + i] = pot;
+    if (own && p == 0) J.energies[i] = pot;
+    pot = 0.0f;
+    for (int b = 0; b < nnm; b += K) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = b + u * P + p;
+            float t = -0.0f;
+            if (k < nn) {
+                const size_t e = (size_t)k * n + i;
+                const float4 o = cur[gmem(J.nat_j)[e]];
+                const float2 par = ldg2(J.nat_par, e);
+                const float x = o.x - c.x, y = o.y - c.y, z = o.z - c.z;
+                const float f = par.x / (x * x + y * y + z * z);
+                float p6 = f * f * f;
+                const float p12 = p6 * p6;
+                p6 = -2.0f * p6;
+                const float eh = (float)((double)(-par.y * par.x) / 12.0);
+                t = eh * (p6 + p12);
+            }
+            terms[w][q][u * P + p] = t;
+        }
+        wave_lds_order();
+        if (p == 0) rows_add(terms[w][q], min(K, nnm - b), pot);
+        wave_lds_order();
+    }
+    if (own && p == 0) J.energies[n + i] = pot;
+    pot = 0.0f;
+    for (int b = 0; b < npm; b += K) {
+        float4 o[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // positions past the row's entries gather its own bead
+            const int k = b + u * P + p;
+            const int j = list_at(J.pair_j, J.idx16, (size_t)min(k, max(np - 1, 0)) * J.pair_ld + rc);
+            o[u] = cur[k < np ? j : i];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float x = o[u].x - c.x, y = o[u].y - c.y, z = o[u].z - c.z;
+            const float d2 = x * x + y * y + z * z;
+            const float f = J.a2 / d2;
+            terms[w][q][u * P + p] = (b + u * P + p < np && d2 < J.rc2) ? J.el * f * f * f : -0.0f;
+        }
+        wave_lds_order();
+        if (p == 0) rows_add(terms[w][q], min(K, npm - b), pot);
+        wave_lds_order();
+    }
+    if (own && p == 0) J.energies[2 * n + i] = pot;
 }
 
 // Self-check of div_rn_fast against the IEEE division: every float bit
@@ -2050,7 +2098,7 @@ hipError_t launch_read_coords(const DevJob* job, const DevJobState* st, int n, f
 }
 
 hipError_t launch_energies(const DevJob* jobs, const DevJobState* st, int job, int n, hipStream_t stream) {
-    hipLaunchKernelGGL(k_energies, dim3((n + 255) / 256), dim3(256), 0, stream, jobs, st, job);
+    hipLaunchKernelGGL(k_energies, dim3((n + 4 * kEnergyRows - 1) / (4 * kEnergyRows)), dim3(256), 0, stream, jobs, st, job);
     return hipGetLastError();
 }
 
