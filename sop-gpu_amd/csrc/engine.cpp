@@ -793,7 +793,8 @@ int Engine::sync_tables() {
         cap_jobs_ = cap;
     }
     std::vector<DevJob> dj(nj);
-    std::vector<StepDesc> sd(nj);
+    std::vector<StepDesc>& sd = descs_;
+    sd.resize(nj);
     std::vector<DevJobState> ds(nj);
     std::vector<int2> tiles;
     int g = 0;
@@ -1124,11 +1125,13 @@ int Engine::launch_block(int slot_only) {
     const StepDesc* descs = d_descs_;
     DevJobState* st = d_state_;
     const int2* tiles = d_tiles_;
+    const StepDesc* one = one_job();
     int nj = (int)jobs_.size(), nt = ntiles_, L = L_;
     if (slot_only >= 0) {
         if (int rc = tiles_for_slot(slot_only, &nt)) return rc;
         jobs = d_jobs_ + slot_only;
         descs = d_descs_ + slot_only;
+        one = &descs_[slot_only];
         st = d_state_ + slot_only;
         tiles = d_tiles1_;
         nj = 1;
@@ -1195,10 +1198,10 @@ int Engine::launch_block(int slot_only) {
             : block ? launch_block_rows(descs, st, nj, beads, block, k, std::min(L - k, kBlockSteps),
                                       k + kBlockSteps >= L ? L : 0, stream_)
             : slot_only >= 0
-                ? launch_step(jobs, descs, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
+                ? launch_step(jobs, descs, one, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
                               jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, k, max_blocks_, stream_,
                               eff1_)
-                : launch_step(jobs, descs, st, tiles, nt, any_global_, d_sunits_, d_segs_, nsunits_, lds_beads_, k,
+                : launch_step(jobs, descs, one, st, tiles, nt, any_global_, d_sunits_, d_segs_, nsunits_, lds_beads_, k,
                               max_blocks_, stream_, eff_);
         if (int rc = check(e, "step")) return rc;
         if (prof_end) {
@@ -1308,8 +1311,8 @@ int Engine::stage_tea_update() {
 }
 int Engine::stage_step(int k) {
     if (int rc = sync_tables()) return rc;
-    if (int rc = check(launch_step(d_jobs_, d_descs_, d_state_, d_tiles_, ntiles_, any_global_, d_sunits_, d_segs_, nsunits_,
-                                   lds_beads_, k, max_blocks_, stream_, eff_),
+    if (int rc = check(launch_step(d_jobs_, d_descs_, one_job(), d_state_, d_tiles_, ntiles_, any_global_, d_sunits_,
+                                   d_segs_, nsunits_, lds_beads_, k, max_blocks_, stream_, eff_),
                        "step"))
         return rc;
     if (any_tea_)
@@ -1656,8 +1659,8 @@ int Engine::compute_forces(int id, float* out4) {
     int nt = 0;
     if (int rc = tiles_for_slot(slot, &nt)) return rc;
     const bool lds = hj.dj.lds_step != 0;
-    if (int rc = check(launch_forces(d_jobs_ + slot, d_descs_ + slot, d_state_ + slot, d_tiles1_, nt, !lds, d_sunits1_, d_segs1_,
-                                     lds ? nsunits1_ : 0, hj.n, d_scratch4_, stream_, eff1_),
+    if (int rc = check(launch_forces(d_jobs_ + slot, d_descs_ + slot, &descs_[slot], d_state_ + slot, d_tiles1_, nt, !lds,
+                                     d_sunits1_, d_segs1_, lds ? nsunits1_ : 0, hj.n, d_scratch4_, stream_, eff1_),
                        "forces"))
         return rc;
     if (int rc = synchronize()) return rc;

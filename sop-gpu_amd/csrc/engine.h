@@ -176,6 +176,8 @@ class Engine {
     // device tables
     DevJob* d_jobs_ = nullptr;
     StepDesc* d_descs_ = nullptr;
+    std::vector<StepDesc> descs_;  // the same on the host
+    const StepDesc* one_job() const { return descs_.size() == 1 ? descs_.data() : nullptr; }
     DevJobState* d_state_ = nullptr;
     int2* d_tiles_ = nullptr;
     int cap_jobs_ = 0, cap_tiles_ = 0, ntiles_ = 0;

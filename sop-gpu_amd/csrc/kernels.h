@@ -45,8 +45,10 @@ constexpr int kSplitMaxTiles = 1536;
 // in float4; lds_beads = the largest LDS use of a unit), the others by the
 // tile kernel (launched when any_global is set).  With shape.split_rows set
 // (split_global) the LDS-step (other) jobs are stepped by k_step_rows over the
-// tiles instead, from the step records `descs`.
-hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
+// tiles instead, from the step records `descs` (one: the record, in host
+// memory, where the launch has a single job; else null).
+hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const StepDesc* one, const DevJobState* st,
+                       const int2* tiles, int ntiles, int any_global,
                        const int2* units, const int4* segs, int nunits, int lds_beads, int kstep, int max_blocks,
                        hipStream_t stream, const StepShape& shape);
 // List rebuilds for jobs whose cadence is due (force != 0: rebuild all).
@@ -88,7 +90,8 @@ hipError_t launch_block_rows(const StepDesc* descs, DevJobState* st, int njobs, 
                              int advance, hipStream_t stream);
 // Forces only (the step kernels' force terms, no state change) of the jobs
 // of the given tiles / LDS plan, into out[bead] (one job per launch).
-hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const DevJobState* st, const int2* tiles, int ntiles, int any_global,
+hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const StepDesc* one, const DevJobState* st,
+                         const int2* tiles, int ntiles, int any_global,
                          const int2* units, const int4* segs, int nunits, int lds_beads, float4* out,
                          hipStream_t stream, const StepShape& shape);
 hipError_t launch_rng_probe(uint4* state, int n, int count, int gaussian, float* out, hipStream_t stream);

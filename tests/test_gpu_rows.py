@@ -64,3 +64,22 @@ def test_coincident_beads_take_the_general_division(gap):
     ref.build_possible()
     ref.build_verlet()
     np.testing.assert_array_equal(f, ref.forces32())
+
+
+# a launch of one job takes its record as an argument, and so does one job of
+# a batch run by itself; beside another job of its kind it reads the table
+@pytest.mark.parametrize("n", [63, 65, 1000, 5121])
+@pytest.mark.parametrize("rows", [4, 8, 16])
+def test_one_job_equals_the_same_job_in_a_batch(n, rows):
+    print("case: %d beads alone and in a batch, %d rows" % (n, rows), flush=True)
+    job, other = _job(n, 1300), _job(130, 1301)
+    shape = dict(split_rows=rows, split_global=rows)
+    alone, batch = _run([job], shape, 6), _run([job, other], shape, 6)[:4]
+    with S.Engine(0, 8 << 30) as e:
+        e.set_shape(**shape)
+        ids = [e.add_job(S.make_params(**kw), sysm, 50) for sysm, kw in (other, job)]
+        e.run_job(ids[1])
+        single = [e.coords(ids[1]), e.rng(ids[1]), e.temperature(ids[1]), e.forces(ids[1])]
+    for a, b, c in zip(alone, batch, single):
+        np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(a, c)
