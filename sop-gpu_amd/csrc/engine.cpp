@@ -931,8 +931,9 @@ StepShape Engine::effective_shape(long long lds_rows, long long global_rows, lon
 // Rows per wavefront of k_block_rows for jobs first .. first + count - 1, 0 where
 // their steps take a launch each: a shape that was set, a job past kBlockBeads
 // or with hydrodynamics, or few jobs whose rows the spread step divides over
-// more CUs than they have workgroups here.  Measured, us per step of a block of
-// 10, a launch per step | R = 8, 16 (the larger R where rows are many):
+// more CUs than they have workgroups here.  Measured with updaters and lists in
+// launches of their own, us per step of a block of 10, a launch per step | R =
+// 8, 16 (the larger R where rows are many):
 //   beads x jobs   22 x 1      64        256       512        1,000       6,000
 //                  6.7 | 5.0  7.1 | 5.1  8.1 | 5.8  10.2 | 7.4  17.0 | 10.4  64 | 55, 50
 //   100 x          7.3 | 8.3  8.3 | 8.8  14.7 | 10.9, 12.1  20.0 | 19.9, 16.3  45 | 40, 32
@@ -1137,7 +1138,14 @@ int Engine::launch_block(int slot_only) {
         nj = 1;
         L = jobs_[slot_only].dj.stride;
     }
-    if (int rc = check(launch_job_update(jobs, st, nj, stream_), "job update")) return rc;
+    // a block in one launch begins with the updaters (but for the tip) and the
+    // Verlet lists
+    int beads = 0;
+    const int block = slot_only >= 0 ? block_rows(slot_only, 1, &beads) : block_rows(0, nj, &beads);
+    bool tip = !block;
+    for (int k = 0; k < nj && !tip; ++k) tip = jobs_[slot_only >= 0 ? slot_only : k].dj.flags & JF_INDENTATION;
+    if (tip)
+        if (int rc = check(launch_job_update(jobs, st, nj, stream_, block ? 1 : 7), "job update")) return rc;
     const int due = lists_due(slot_only);
     if (due & 1) {
         const hipError_t e =
@@ -1152,13 +1160,16 @@ int Engine::launch_block(int slot_only) {
     }
     if (due & 2) {
         const bool sort = (due & 4) != 0;
+        const int sort1 = slot_only >= 0 && sort && jobs_[slot_only].dj.sort_rows
+                              ? (jobs_[slot_only].n + kLdsUnit - 1) / kLdsUnit
+                              : 0;
         const hipError_t e =
-            slot_only >= 0
+            block ? launch_sort_rows(jobs, st, slot_only >= 0 ? d_units1_ : d_units_,
+                                     slot_only >= 0 ? sort1 : sort ? nunits_ : 0, 0, stream_,
+                                     slot_only >= 0 ? eff1_ : eff_)
+            : slot_only >= 0
                 ? launch_verlet(jobs, st, tiles, nt, !jobs_[slot_only].dj.idx16, !jobs_[slot_only].dj.lds_step,
-                                d_units1_,
-                                sort && jobs_[slot_only].dj.sort_rows ? (jobs_[slot_only].n + kLdsUnit - 1) / kLdsUnit
-                                                                      : 0,
-                                d_sunits1_, d_segs1_, jobs_[slot_only].dj.lds_step ? nsunits1_ : 0,
+                                d_units1_, sort1, d_sunits1_, d_segs1_, jobs_[slot_only].dj.lds_step ? nsunits1_ : 0,
                                 jobs_[slot_only].n, 0, stream_, eff1_)
                 : launch_verlet(jobs, st, tiles, nt, any_idx32_, any_global_, d_units_, sort ? nunits_ : 0,
                                 d_sunits_, d_segs_, nsunits_, lds_beads_, 0, stream_, eff_);
@@ -1175,8 +1186,6 @@ int Engine::launch_block(int slot_only) {
     // profiling: HIP events around the step launches; when nothing else is
     // launched between them, one pair spans the block's L launches
     const bool span = !tea && !exact;
-    int beads = 0;
-    const int block = slot_only >= 0 ? block_rows(slot_only, 1, &beads) : block_rows(0, nj, &beads);
     for (int k = 0; k < L; ++k) {
         const bool prof = profiling_ && (!span || k == 0);
         const bool prof_end = profiling_ && (!span || k == L - 1);
@@ -1195,8 +1204,9 @@ int Engine::launch_block(int slot_only) {
         }
         const hipError_t e =
             block && k % kBlockSteps ? hipSuccess  // in the launch before
-            : block ? launch_block_rows(descs, st, nj, beads, block, k, std::min(L - k, kBlockSteps),
-                                      k + kBlockSteps >= L ? L : 0, stream_)
+            : block ? launch_block_rows(jobs, descs, st, nj, beads, block, k, std::min(L - k, kBlockSteps),
+                                        k + kBlockSteps >= L ? L : 0,
+                                        k == 0 ? BLOCK_UPDATE | (due & 2 ? BLOCK_VERLET : 0) : 0, stream_)
             : slot_only >= 0
                 ? launch_step(jobs, descs, one, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
                               jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, k, max_blocks_, stream_,
@@ -1334,8 +1344,8 @@ int Engine::stage_steps(int n) {
     int beads = 0;
     const int block = block_rows(0, (int)jobs_.size(), &beads);
     for (int k = 0; k < n; k += block ? kBlockSteps : 1)
-        if (int rc = block ? check(launch_block_rows(d_descs_, d_state_, (int)jobs_.size(), beads, block, k,
-                                                     std::min(n - k, kBlockSteps), 0, stream_),
+        if (int rc = block ? check(launch_block_rows(d_jobs_, d_descs_, d_state_, (int)jobs_.size(), beads, block,
+                                                     k, std::min(n - k, kBlockSteps), 0, 0, stream_),
                                    "steps")
                            : stage_step(k))
             return rc;

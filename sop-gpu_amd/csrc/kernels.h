@@ -61,6 +61,9 @@ hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const StepDesc
 hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int use_boxes,
                            int any_global, const int2* sunits, const int4* segs, int nsunits,
                            int lds_beads, int force, hipStream_t stream, const StepShape& shape);
+// The rows of units (job, first row) re-sorted by list length, where due.
+hipError_t launch_sort_rows(const DevJob* jobs, DevJobState* st, const int2* units, int nunits, int force,
+                            hipStream_t stream, const StepShape& shape);
 // any_idx32: some job of the launch stores its lists as int32 (n >= 65536).
 // units (job, first row) of the jobs whose rows are re-sorted first;
 // sunits/segs/nsunits/lds_beads: the LDS step plan (see launch_step), whose
@@ -85,9 +88,11 @@ hipError_t launch_job_advance(const DevJob* jobs, DevJobState* st, int njobs, in
 hipError_t launch_energies(const DevJob* jobs, const DevJobState* st, int job, int n, hipStream_t stream);
 // Steps state.step + kstep .. + nsteps - 1 of njobs jobs of at most `beads`
 // beads, R rows per wavefront (ceil(beads / R) <= 16), in one launch, which then
-// adds `advance` to the step counters.
-hipError_t launch_block_rows(const StepDesc* descs, DevJobState* st, int njobs, int beads, int R, int kstep, int nsteps,
-                             int advance, hipStream_t stream);
+// adds `advance` to the step counters.  begin: the launch starts with the
+// pulling and heating updaters and the Verlet lists of the jobs due.
+enum { BLOCK_UPDATE = 1, BLOCK_VERLET = 2 };
+hipError_t launch_block_rows(const DevJob* jobs, const StepDesc* descs, DevJobState* st, int njobs, int beads, int R,
+                             int kstep, int nsteps, int advance, int begin, hipStream_t stream);
 // Forces only (the step kernels' force terms, no state change) of the jobs
 // of the given tiles / LDS plan, into out[bead] (one job per launch).
 hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const StepDesc* one, const DevJobState* st,

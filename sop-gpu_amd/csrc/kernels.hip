@@ -859,46 +859,6 @@ __global__ __launch_bounds__(256, 4) void k_step_rows_one(const StepDesc D, cons
     step_rows_of<FO, R>(D, *st, kstep, 64 * at.x + at.y, terms[w], fout);
 }
 
-// The steps of a block in one launch, for launches of small jobs: one workgroup
-// per job, a wavefront per R of its rows (blockDim.x / 64 >= ceil(n / R)), the
-// coordinates in LDS and a barrier between steps in the place of a launch.  Of
-// k_step_rows' chain only the sums are left: lists and generators stay in
-// registers, partners come from LDS.  Bound by VALU issue, about 1,000
-// instructions a step and wavefront, at one wavefront a SIMD.  ldc: beads of
-// the launch's largest job; advance: what the block's last launch adds to the
-// step counters (in the place of k_job_advance), 0 for none.  350 peptides of
-// 22 beads, a block of ten steps: 37 us, 75 as ten launches of k_step_rows and
-// the gaps between them.
-template <int R>
-__global__ __launch_bounds__(1024) void k_block_rows(const StepDesc* __restrict__ descs,
-                                                     DevJobState* __restrict__ st, int ldc, int kstep, int nsteps,
-                                                     int advance) {
-    using Rows = float[3][R][RowsShape<R, true>::KP];
-    extern __shared__ float4 lds_coord[];
-    Rows* const terms = reinterpret_cast<Rows*>(lds_coord + 2 * ldc);
-    const StepDesc D = descs[blockIdx.x];
-    const long long s = st[blockIdx.x].step + kstep;
-    const float var = st[blockIdx.x].var;
-    asm volatile("" ::"s"(D.coord[0]), "s"(D.coord[1]), "s"(D.perm), "s"(D.pair_cnt), "s"(D.pair_j), "s"(D.b_cnt),
-                 "s"(D.cov_j), "s"(D.cov_r0), "s"(D.nat_j), "s"(D.nat_par), "s"(D.rng), "s"(D.T), "s"(D.bflag));
-    const int steps = (int)min((long long)nsteps, D.end_step - s);
-    if (steps <= 0) return;
-    const float4* const cin = (s & 1) ? D.coord[1] : D.coord[0];
-    for (int i = threadIdx.x; i < D.n; i += blockDim.x) lds_coord[i] = ldg_coord(cin, i);
-    __syncthreads();
-    const int w = wave_id(), row0 = R * w;
-    if (row0 >= D.n) {  // no rows: the barriers of the others' steps
-        for (int k = 0; k < steps; ++k) __syncthreads();
-    } else if (D.idx16) {
-        step_rows<false, R, unsigned short, true>(D, st[blockIdx.x], var, s, row0, terms[w], nullptr, lds_coord, ldc,
-                                                  steps);
-    } else {
-        step_rows<false, R, int, true>(D, st[blockIdx.x], var, s, row0, terms[w], nullptr, lds_coord, ldc, steps);
-    }
-    // every wavefront took the step before its first barrier
-    if (advance && threadIdx.x == 0) st[blockIdx.x].step = min(s - kstep + advance, D.end_step);
-}
-
 // ---------------------------------------------------------------------------
 // pairlists
 // ---------------------------------------------------------------------------
@@ -1777,6 +1737,16 @@ __device__ void pull_update(const DevJob& J, DevJobState& S, long long s) {
     }
 }
 
+// The updaters of one thread's work at step s (mask as k_job_update's).
+__device__ void job_update_scalar(const DevJob& J, DevJobState& S, long long s, int mask) {
+    if (s >= J.end_step || s % J.stride != 0) return;
+    if ((mask & 2) && (J.flags & JF_PULL_UPDATER)) pull_update(J, S, s);
+    if ((mask & 4) && (J.flags & JF_HEATING) && s % J.tempFreq == 0) {
+        const float temp = J.initialT + (float)(s / J.tempFreq) * J.deltaT;
+        S.var = sqrtf(2.0f * temp * J.zeta / J.h);
+    }
+}
+
 // mask: 1 indentation tip, 2 pulling cantilever, 4 heating schedule.
 // One 64-thread workgroup per job; lane 0 does the scalar work.
 __global__ __launch_bounds__(64) void k_job_update(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
@@ -1788,12 +1758,109 @@ __global__ __launch_bounds__(64) void k_job_update(const DevJob* __restrict__ jo
     const long long s = S.step;
     if (s >= J.end_step || s % J.stride != 0) return;
     if ((mask & 1) && (J.flags & JF_INDENTATION)) tip_update(J, S, s);
-    if (threadIdx.x != 0) return;
-    if ((mask & 2) && (J.flags & JF_PULL_UPDATER)) pull_update(J, S, s);
-    if ((mask & 4) && (J.flags & JF_HEATING) && s % J.tempFreq == 0) {
-        const float temp = J.initialT + (float)(s / J.tempFreq) * J.deltaT;
-        S.var = sqrtf(2.0f * temp * J.zeta / J.h);
+    if (threadIdx.x == 0) job_update_scalar(J, S, s, mask);
+}
+
+// Verlet lists of the R rows from row0 by one wavefront (k_verlet's filter, in
+// the same order), the job's coordinates in LDS: the rows' chunks of 64 possible
+// partners are loaded together, and the accepted ones, few, go to their slots
+// directly.
+template <int R>
+__device__ __forceinline__ void verlet_few(const DevJob& J, DevJobState& S, const float4* cur, int row0) {
+    const int lane = threadIdx.x & 63, nr = min(R, J.n - row0);
+    const int cap = J.pair_cap, ppcap = J.pp_cap, idx16 = J.idx16;
+    const float d2max = J.pl_d2;
+    const int bl = gmem(J.perm)[row0 + min(lane, nr - 1)];
+    const int cl = lane < nr ? gmem(J.pp_cnt)[bl] : 0;
+    int most = cl;
+#pragma unroll
+    for (int o = R / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
+    most = __builtin_amdgcn_readfirstlane(most);
+    int cnt[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) cnt[q] = 0;
+    for (int base = 0; base < most; base += 64) {
+        int j[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            j[q] = list_at(J.pp_j, idx16,
+                           (size_t)__builtin_amdgcn_readlane(bl, q) * J.pp_ld + min(base + lane, ppcap - 1));
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const bool in = base + lane < __builtin_amdgcn_readlane(cl, q);
+            const float4 o = cur[in ? j[q] : 0], c = cur[__builtin_amdgcn_readlane(bl, q)];
+            const float x = o.x - c.x, y = o.y - c.y, z = o.z - c.z;
+            const bool ok = in & (x * x + y * y + z * z <= d2max);
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
+            const int pos = (int)__builtin_amdgcn_mbcnt_hi(
+                (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)cnt[q]));
+            if (ok && pos < cap) list_put(J.pair_j, idx16, (size_t)pos * J.pair_ld + row0 + q, j[q]);
+            cnt[q] += __popcll(m);
+        }
     }
+    int total = cnt[0];
+#pragma unroll
+    for (int q = 1; q < R; ++q) total = lane == q ? cnt[q] : total;
+    if (lane < nr) {
+        J.pair_cnt[row0 + lane] = min(total, cap);
+        if (total > cap) atomicOr(&S.overflow, 2);
+    }
+}
+
+// The steps of a block in one launch, for launches of small jobs: one workgroup
+// per job, a wavefront per R of its rows (blockDim.x / 64 >= ceil(n / R)), the
+// coordinates in LDS and a barrier between steps in the place of a launch.  Of
+// k_step_rows' chain only the sums are left: lists and generators stay in
+// registers, partners come from LDS.  Bound by VALU issue, about 1,000
+// instructions a step and wavefront, at one wavefront a SIMD.  ldc: beads of
+// the launch's largest job; advance: what the block's last launch adds to the
+// step counters (in the place of k_job_advance), 0 for none.  350 peptides of
+// 22 beads, a block of ten steps: 37 us, 75 as ten launches of k_step_rows and
+// the gaps between them.  begin (BLOCK_*): what the block begins with here, in
+// the place of k_job_update (but for the tip) and k_verlet_split: 3 us more, for
+// the 12 of the two launches.
+template <int R>
+__global__ __launch_bounds__(1024) void k_block_rows(const DevJob* __restrict__ jobs,
+                                                     const StepDesc* __restrict__ descs,
+                                                     DevJobState* __restrict__ st, int ldc, int kstep, int nsteps,
+                                                     int advance, int begin) {
+    using Rows = float[3][R][RowsShape<R, true>::KP];
+    extern __shared__ float4 lds_coord[];
+    __shared__ float var_s;
+    Rows* const terms = reinterpret_cast<Rows*>(lds_coord + 2 * ldc);
+    const StepDesc D = descs[blockIdx.x];
+    const long long s = st[blockIdx.x].step + kstep;
+    float var = st[blockIdx.x].var;
+    asm volatile("" ::"s"(D.coord[0]), "s"(D.coord[1]), "s"(D.perm), "s"(D.pair_cnt), "s"(D.pair_j), "s"(D.b_cnt),
+                 "s"(D.cov_j), "s"(D.cov_r0), "s"(D.nat_j), "s"(D.nat_par), "s"(D.rng), "s"(D.T), "s"(D.bflag));
+    const int steps = (int)min((long long)nsteps, D.end_step - s);
+    if (steps <= 0) return;
+    const float4* const cin = (s & 1) ? D.coord[1] : D.coord[0];
+    for (int i = threadIdx.x; i < D.n; i += blockDim.x) lds_coord[i] = ldg_coord(cin, i);
+    const int w = wave_id(), row0 = R * w;
+    if (begin & BLOCK_UPDATE) {
+        if (threadIdx.x == 0) {
+            job_update_scalar(jobs[blockIdx.x], st[blockIdx.x], s, 6);
+            var_s = st[blockIdx.x].var;
+        }
+        __syncthreads();
+        var = var_s;
+    }
+    __syncthreads();
+    if ((begin & BLOCK_VERLET) && due(jobs[blockIdx.x], s, jobs[blockIdx.x].pairs_freq)) {
+        if (row0 < D.n) verlet_few<R>(jobs[blockIdx.x], st[blockIdx.x], lds_coord, row0);
+        __syncthreads();
+    }
+    if (row0 >= D.n) {  // no rows: the barriers of the others' steps
+        for (int k = 0; k < steps; ++k) __syncthreads();
+    } else if (D.idx16) {
+        step_rows<false, R, unsigned short, true>(D, st[blockIdx.x], var, s, row0, terms[w], nullptr, lds_coord, ldc,
+                                                  steps);
+    } else {
+        step_rows<false, R, int, true>(D, st[blockIdx.x], var, s, row0, terms[w], nullptr, lds_coord, ldc, steps);
+    }
+    // every wavefront took the step before its first barrier
+    if (advance && threadIdx.x == 0) st[blockIdx.x].step = min(s - kstep + advance, D.end_step);
 }
 
 __global__ void k_job_advance(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st, int njobs, int nsteps) {
@@ -2026,20 +2093,24 @@ hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const StepDesc
     return hipGetLastError();
 }
 
-hipError_t launch_block_rows(const StepDesc* descs, DevJobState* st, int njobs, int beads, int R, int kstep, int nsteps,
-                             int advance, hipStream_t stream) {
+hipError_t launch_block_rows(const DevJob* jobs, const StepDesc* descs, DevJobState* st, int njobs, int beads, int R,
+                             int kstep, int nsteps, int advance, int begin, hipStream_t stream) {
     const int waves = (beads + R - 1) / R;
     if (waves > 16) return hipErrorInvalidValue;
     const dim3 g(njobs), b(64 * waves);
     auto lds = [&](int kp) { return (size_t)2 * beads * 16 + (size_t)waves * 3 * R * kp * 4; };
     if (R == 2)
-        hipLaunchKernelGGL(k_block_rows<2>, g, b, lds(RowsShape<2, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
+        hipLaunchKernelGGL(k_block_rows<2>, g, b, lds(RowsShape<2, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
+                           begin);
     else if (R == 4)
-        hipLaunchKernelGGL(k_block_rows<4>, g, b, lds(RowsShape<4, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
+        hipLaunchKernelGGL(k_block_rows<4>, g, b, lds(RowsShape<4, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
+                           begin);
     else if (R == 8)
-        hipLaunchKernelGGL(k_block_rows<8>, g, b, lds(RowsShape<8, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
+        hipLaunchKernelGGL(k_block_rows<8>, g, b, lds(RowsShape<8, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
+                           begin);
     else
-        hipLaunchKernelGGL(k_block_rows<16>, g, b, lds(RowsShape<16, true>::KP), stream, descs, st, beads, kstep, nsteps, advance);
+        hipLaunchKernelGGL(k_block_rows<16>, g, b, lds(RowsShape<16, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
+                           begin);
     return hipGetLastError();
 }
 
@@ -2083,13 +2154,19 @@ hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tile
     return hipGetLastError();
 }
 
+hipError_t launch_sort_rows(const DevJob* jobs, DevJobState* st, const int2* units, int nunits, int force,
+                            hipStream_t stream, const StepShape& shape) {
+    if (nunits > 0)
+        hipLaunchKernelGGL(k_sort_rows, dim3(nunits), dim3(kLdsUnit), 0, stream, jobs, st, units, nunits,
+                           shape.sort_every, force);
+    return hipGetLastError();
+}
+
 hipError_t launch_verlet(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int any_idx32,
                          int any_global, const int2* units, int nunits, const int2* sunits, const int4* segs,
                          int nsunits, int lds_beads, int force, hipStream_t stream, const StepShape& shape) {
     if (ntiles <= 0) return hipSuccess;
-    if (nunits > 0)
-        hipLaunchKernelGGL(k_sort_rows, dim3(nunits), dim3(kLdsUnit), 0, stream, jobs, st, units, nunits,
-                           shape.sort_every, force);
+    if (const hipError_t e = launch_sort_rows(jobs, st, units, nunits, force, stream, shape)) return e;
     int blocks = ntiles;
     if (blocks >= 8) blocks = (blocks + 7) / 8 * 8;
     const size_t lds = any_idx32 ? 64 * VerletLds<int>::stride * sizeof(int)

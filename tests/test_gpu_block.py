@@ -1,7 +1,7 @@
 """A block of steps in one launch, for small jobs: coordinates, generators,
 temperatures and the forces after it are those of one launch per step, to the
 bit -- for the smallest jobs and the largest it takes, jobs of several sizes
-in one launch, ends inside a block, blocks longer than one launch, a tip and
+in one launch, ends inside a block, lists that overflow, heating, blocks longer than one launch, a tip and
 a plane, minimization, and one job of the batch run by itself."""
 import numpy as np
 import pytest
@@ -54,7 +54,9 @@ def test_sizes(sizes):
     (100, 6, dict(pulling=0, indentation=1, indTip=(0.0, 0.0, 80.0), indChip=(0.0, 0.0, 80.0),
                   indDirection=(0.0, 0.0, -1.0), indSurfR0=(0.0, 0.0, -60.0), indSurfN=(0.0, 0.0, 1.0), indTipR=20.0,
                   indKs=0.07, indDeltaX=0.01, indTipZeta=5000.0, indTipA=0.0, indTipB=1.0)),
-], ids=["end-inside", "long-block", "minimization", "tip"])
+    (100, 6, dict(max_pairs=4)),
+    (100, 9, dict(heating=1, initialT=0.3, deltaT=0.05, tempFreq=20)),
+], ids=["end-inside", "long-block", "minimization", "tip", "overflow", "heating"])
 def test_forms(steps, blocks, kw):
     print("case: %r" % (kw,), flush=True)
     _compare([_job(n, 2100 + n, **kw) for n in (30, 22, 7)], steps, blocks)
