@@ -896,8 +896,8 @@ int Engine::sync_tables() {
 // one set by set_shape or autotune, else the spread step (k_step_rows) up to
 // kRowsMaxLds and kRowsMaxGlobal rows and one bead per lane above.
 //
-// Rows per wavefront, measured per step launch with R = 2 / 4 / 8 / 16 and
-// one bead per lane (us):
+// Rows per wavefront, measured per step launch (the record from the table)
+// with R = 2 / 4 / 8 / 16 and one bead per lane (us):
 //   1,000 rows of one chain        7.7 / 8.5 /  11 /  15,  31
 //   3,186 of three chains          8.6 / 9.0 /  12 /  17
 //   9,558 of nine chains            16 /  11 /  13 /  17,  34

@@ -1117,10 +1117,32 @@ __device__ __forceinline__ void update_tile(float* __restrict__ M, size_t ld, in
         }
         __syncthreads();
     };
-    // kw is a multiple of 64: an even number of chunks
+    // kw is a multiple of 64: an even number of chunks.  The narrow tiles
+    // (registers to spare) sum kPart columns at a time and add the parts: one
+    // chain of 512 FP32 additions left the FP32 factor's error 8 to 30 % above
+    // that of the shorter chains of a step's wavefronts, in parts it is below
+    // (order 4,001: 1.29e-6, 1.22e-6 and 1.11e-6 of the factor's norm)
+    constexpr bool kParts = NI * NJ <= 8;
+    constexpr int kPart = 128;
+    f32x4 sum[NI][NJ];
     for (int k = 0; k < nch; k += 2) {
         chunk(k, v[0]);
         chunk(k + 1, v[D - 1]);
+        if (kParts && ((k + 2) % (kPart / 32) == 0 || k + 2 == nch)) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    sum[i][j] = k + 2 > kPart / 32 ? sum[i][j] + acc[i][j] : acc[i][j];
+                    acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    }
+    if constexpr (kParts) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i][j] = sum[i][j];
     }
     // C -= acc: D rows 4(l/16) + q, column l%16 of each 16x16 tile
     constexpr int NB_ = 32;  // elements of a lane at a time
@@ -1603,7 +1625,8 @@ hipError_t launch_hi_tea_step(const DevJob* jobs, const DevJobState* st, const i
 // The lower triangle's rows from s on, columns [s, s + cols) (cols < 0: all),
 // minus the panel copy's kw columns times their transpose.  The next panel's
 // columns (cols = 512): 128x64 tiles, which put 3,700 rows on 232 CUs, or
-// 128x128 from 8,000 rows on, where those fill two rounds of CUs.  Regions of
+// in split-BF16 128x128 from 8,000 rows on, where those fill two rounds of CUs
+// (in FP32 128x64, whose sums are taken in parts, update_tile).  Regions of
 // at least a round of 256x256 tiles take those, smaller ones 128x128.
 static constexpr int kTrailBigMinTiles = 256;
 template <int MODE>
@@ -1612,7 +1635,7 @@ static void trailing_update(float* M, size_t ld, int s, int mp, int cols, int kw
     if (s >= mp) return;
     const int nr = (mp - s + 127) / 128;
     const int ntr = (mp - s + BT - 1) / BT, ntile = ntr * (ntr + 1) / 2;
-    if (cols >= 0 && nr <= 62)
+    if (cols >= 0 && (nr <= 62 || MODE == SOP_CHOL_F32))
         hipLaunchKernelGGL((k_update<MODE, 128, 64>), dim3(nr, cols / 64), dim3(256), 0, stream, M, ld, s, mp, kw, pan);
     else if (cols < 0 && ntile >= kTrailBigMinTiles)
         hipLaunchKernelGGL((k_update_big<MODE>), dim3((ntile + kXcds - 1) / kXcds * kXcds), dim3(512), 0, stream, M, ld,
