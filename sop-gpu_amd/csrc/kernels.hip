@@ -499,8 +499,8 @@ __global__ __launch_bounds__(1024, PB <= 6 ? 8 : 4) void k_step_lds(const DevJob
 // launch of any number of rows.  Partners are gathered from global memory
 // (the coordinates of a job stay in L1/L2), so jobs on either side of the
 // LDS limit are stepped by the same launch.  Bound by the latency of its
-// dependent reads (tile, record, lists, partners) where rows are few, by VALU
-// issue from about 30,000 rows on; measured at Engine::effective_shape (18,000
+// dependent reads (tile, record, lists, partners) where rows are few, by those
+// and VALU issue (53 % of the cycles at 100,000 rows of a capsid) where many; measured at Engine::effective_shape (18,000
 // beads: 58 us one bead per lane, 16 us here).
 template <int R, bool BLK = false>
 struct RowsShape {
@@ -1811,9 +1811,9 @@ __device__ __forceinline__ void verlet_few(const DevJob& J, DevJobState& S, cons
 // per job, a wavefront per R of its rows (blockDim.x / 64 >= ceil(n / R)), the
 // coordinates in LDS and a barrier between steps in the place of a launch.  Of
 // k_step_rows' chain only the sums are left: lists and generators stay in
-// registers, partners come from LDS.  Bound by VALU issue, about 1,000
-// instructions a step and wavefront, at one wavefront a SIMD.  ldc: beads of
-// the launch's largest job; advance: what the block's last launch adds to the
+// registers, partners come from LDS.  Bound by the latency of its dependent
+// operations: 560 vector instructions a step and wavefront in ~9,000 cycles, at
+// one or two wavefronts a SIMD.  ldc: beads of the launch's largest job; advance: what the block's last launch adds to the
 // step counters (in the place of k_job_advance), 0 for none.  350 peptides of
 // 22 beads, a block of ten steps: 37 us, 75 as ten launches of k_step_rows and
 // the gaps between them.  begin (BLOCK_*): what the block begins with here, in
