@@ -87,7 +87,7 @@ hipError_t launch_job_advance(const DevJob* jobs, DevJobState* st, int njobs, in
 // Output / parity hooks.
 hipError_t launch_energies(const DevJob* jobs, const DevJobState* st, int job, int n, hipStream_t stream);
 // Steps state.step + kstep .. + nsteps - 1 of njobs jobs of at most `beads`
-// beads, R rows per wavefront (ceil(beads / R) <= 16), in one launch, which then
+// beads, R = 8 or 16 rows per wavefront (ceil(beads / R) <= 16), in one launch, which then
 // adds `advance` to the step counters.  begin: the launch starts with the
 // pulling and heating updaters and the Verlet lists of the jobs due.
 enum { BLOCK_UPDATE = 1, BLOCK_VERLET = 2 };

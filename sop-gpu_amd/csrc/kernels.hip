@@ -500,8 +500,9 @@ __global__ __launch_bounds__(1024, PB <= 6 ? 8 : 4) void k_step_lds(const DevJob
 // (the coordinates of a job stay in L1/L2), so jobs on either side of the
 // LDS limit are stepped by the same launch.  Bound by the latency of its
 // dependent reads (tile, record, lists, partners) where rows are few, by those
-// and VALU issue (53 % of the cycles at 100,000 rows of a capsid) where many; measured at Engine::effective_shape (18,000
-// beads: 58 us one bead per lane, 16 us here).
+// and VALU issue (53 % of the cycles at 100,000 rows of a capsid) where many;
+// measured at Engine::effective_shape (18,000 beads: 58 us one bead per lane, 16
+// us here).
 template <int R, bool BLK = false>
 struct RowsShape {
     static constexpr int P = 64 / R;              // positions of a row evaluated at a time
@@ -2096,16 +2097,10 @@ hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const StepDesc
 hipError_t launch_block_rows(const DevJob* jobs, const StepDesc* descs, DevJobState* st, int njobs, int beads, int R,
                              int kstep, int nsteps, int advance, int begin, hipStream_t stream) {
     const int waves = (beads + R - 1) / R;
-    if (waves > 16) return hipErrorInvalidValue;
+    if (waves > 16 || (R != 8 && R != 16)) return hipErrorInvalidValue;
     const dim3 g(njobs), b(64 * waves);
     auto lds = [&](int kp) { return (size_t)2 * beads * 16 + (size_t)waves * 3 * R * kp * 4; };
-    if (R == 2)
-        hipLaunchKernelGGL(k_block_rows<2>, g, b, lds(RowsShape<2, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
-                           begin);
-    else if (R == 4)
-        hipLaunchKernelGGL(k_block_rows<4>, g, b, lds(RowsShape<4, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
-                           begin);
-    else if (R == 8)
+    if (R == 8)
         hipLaunchKernelGGL(k_block_rows<8>, g, b, lds(RowsShape<8, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
                            begin);
     else
