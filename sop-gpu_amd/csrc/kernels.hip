@@ -704,26 +704,29 @@ __device__ __forceinline__ void step_rows(const StepDesc& D, const DevJobState& 
         // FENE and native terms
         for (int b = 0; b < nbm; b += P * UB) {
             if (b > 0) bonded(b);
+            // all the chunk's partners first (positions without a term have the
+            // row's own bead), and where both kinds of term occur, both formed
+            // side by side: behind a branch each, one waited for the other (350
+            // peptides 21.4 -> 21.0 ms; 100,000 beads, 400 steps 27.6 -> 27.2)
+            float4 w[UB];
+#pragma unroll
+            for (int u = 0; u < UB; ++u) w[u] = coord(b + u * P < nbm ? f[u].j : i);
 #pragma unroll
             for (int u = 0; u < UB; ++u)
                 if (b + u * P < nbm) {
-                    const float4 w = coord(f[u].j);
-                    const float x = w.x - c.x, y = w.y - c.y, z = w.z - c.z;
-                    float tx = -0.0f, ty = -0.0f, tz = -0.0f;
-                    if (f[u].type == 0) {
-                        const float v = fene_w(D.ks, D.R2, x, y, z, f[u].par.x);
-                        tx = v * x;
-                        ty = v * y;
-                        tz = v * z;
-                    } else if (f[u].type == 1) {
-                        const float v = native_q(x, y, z, f[u].par);
-                        tx = x * v;
-                        ty = y * v;
-                        tz = z * v;
+                    const float x = w[u].x - c.x, y = w[u].y - c.y, z = w[u].z - c.z;
+                    float v;
+                    if (__builtin_amdgcn_ballot_w64(f[u].type == 0)) {
+                        const float vf = fene_w(D.ks, D.R2, x, y, z, f[u].par.x);
+                        const float vn = native_q(x, y, z, f[u].par);
+                        v = f[u].type == 0 ? vf : vn;
+                    } else {
+                        v = native_q(x, y, z, f[u].par);
                     }
-                    term[0][q][u * P + p] = tx;
-                    term[1][q][u * P + p] = ty;
-                    term[2][q][u * P + p] = tz;
+                    const bool ok = f[u].type < 3;
+                    term[0][q][u * P + p] = ok ? x * v : -0.0f;
+                    term[1][q][u * P + p] = ok ? y * v : -0.0f;
+                    term[2][q][u * P + p] = ok ? z * v : -0.0f;
                 }
             wave_lds_order();
             if (p < 3) rows_add(&term[p][q][0], min(P * UB, nbm - b), acc);
