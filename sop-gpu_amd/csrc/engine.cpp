@@ -1709,8 +1709,8 @@ int Engine::rebuild_lists(int id, int mask) {
     int nt = 0;
     if (int rc = tiles_for_slot(slot, &nt)) return rc;
     if (mask & 1)
-        if (int rc = check(launch_possible(d_jobs_ + slot, d_state_ + slot, d_tiles1_, nt, boxes_of(jobs_[slot].dj), !jobs_[slot].dj.lds_step, d_sunits1_,
-                                           d_segs1_,
+        if (int rc = check(launch_possible(d_jobs_ + slot, d_state_ + slot, d_tiles1_, nt, boxes_of(jobs_[slot].dj),
+                                           !jobs_[slot].dj.lds_step, d_sunits1_, d_segs1_,
                                            jobs_[slot].dj.lds_step ? nsunits1_ : 0, jobs_[slot].n, 1, stream_,
                                            eff1_),
                            "possible pairs"))

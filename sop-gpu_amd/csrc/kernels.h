@@ -87,9 +87,9 @@ hipError_t launch_job_advance(const DevJob* jobs, DevJobState* st, int njobs, in
 // Output / parity hooks.
 hipError_t launch_energies(const DevJob* jobs, const DevJobState* st, int job, int n, hipStream_t stream);
 // Steps state.step + kstep .. + nsteps - 1 of njobs jobs of at most `beads`
-// beads, R = 8 or 16 rows per wavefront (ceil(beads / R) <= 16), in one launch, which then
-// adds `advance` to the step counters.  begin: the launch starts with the
-// pulling and heating updaters and the Verlet lists of the jobs due.
+// beads, R = 8 or 16 rows per wavefront (ceil(beads / R) <= 16), in one launch,
+// which then adds `advance` to the step counters.  begin: the launch starts with
+// the pulling and heating updaters and the Verlet lists of the jobs due.
 enum { BLOCK_UPDATE = 1, BLOCK_VERLET = 2 };
 hipError_t launch_block_rows(const DevJob* jobs, const StepDesc* descs, DevJobState* st, int njobs, int beads, int R,
                              int kstep, int nsteps, int advance, int begin, hipStream_t stream);

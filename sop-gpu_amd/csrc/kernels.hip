@@ -2104,11 +2104,11 @@ hipError_t launch_block_rows(const DevJob* jobs, const StepDesc* descs, DevJobSt
     const dim3 g(njobs), b(64 * waves);
     auto lds = [&](int kp) { return (size_t)2 * beads * 16 + (size_t)waves * 3 * R * kp * 4; };
     if (R == 8)
-        hipLaunchKernelGGL(k_block_rows<8>, g, b, lds(RowsShape<8, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
-                           begin);
+        hipLaunchKernelGGL(k_block_rows<8>, g, b, lds(RowsShape<8, true>::KP), stream, jobs, descs, st, beads, kstep,
+                           nsteps, advance, begin);
     else
-        hipLaunchKernelGGL(k_block_rows<16>, g, b, lds(RowsShape<16, true>::KP), stream, jobs, descs, st, beads, kstep, nsteps, advance,
-                           begin);
+        hipLaunchKernelGGL(k_block_rows<16>, g, b, lds(RowsShape<16, true>::KP), stream, jobs, descs, st, beads, kstep,
+                           nsteps, advance, begin);
     return hipGetLastError();
 }
 
