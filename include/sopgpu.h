@@ -285,8 +285,9 @@ int sop_rng_probe(int device, const uint32_t* seeds4, int n, int count, int gaus
  * d^2 lies in [2^-64, 2^62]; this counts, over every float bit pattern b in
  * [lo, hi) within that range and each numerator a[0..na) (each 0 or in
  * [2^-60, 2^60]), the quotients that differ from the IEEE division, and the
- * b whose short square root (the hydrodynamic pair terms') differs from the
- * IEEE one. */
+ * b whose reciprocal estimate after the Newton step, or whose short square
+ * root (both used by the hydrodynamic pair terms), differs from the IEEE
+ * one. */
 int sop_check_division(int device, unsigned int lo, unsigned int hi, const float* a, int na,
                        unsigned long long* mismatches);
 

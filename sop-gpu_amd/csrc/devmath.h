@@ -48,8 +48,11 @@ __device__ __forceinline__ float div_rn_fast(float a, float b) {
     const float q = a * y;
     return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
-// RN(1/b) as div_rn_fast forms it, and RN(a/b) from it, for several quotients
-// with one divisor.
+// RN(1/b) as div_rn_fast forms it (b in [kDivFastMinB, kDivFastMaxB]), and
+// RN(a/b) from it, for several quotients with one divisor.  The hydrodynamic
+// pair terms also use the reciprocal itself (2/b as twice RN(1/b)), so its
+// rounding is checked apart from the quotient, which the last FMA would
+// repair: sop_check_division compares it with the IEEE 1/b for every such b.
 __device__ __forceinline__ float recip_rn_fast(float b) {
     const float y0 = __builtin_amdgcn_rcpf(b);
     return __builtin_fmaf(__builtin_fmaf(-b, y0, 1.0f), y0, y0);

@@ -1987,14 +1987,15 @@ __global__ __launch_bounds__(256) void k_energies(const DevJob* __restrict__ job
 
 // Self-check of div_rn_fast against the IEEE division: every float bit
 // pattern b in [lo, hi) (inside the fast range) with each numerator a[k];
-// counts the results that differ, and the b whose sqrt_rn_fast is not the
-// IEEE square root.
+// counts the results that differ, and the b whose sqrt_rn_fast or
+// recip_rn_fast is not the IEEE square root or reciprocal.
 __global__ void k_division_check(unsigned lo, unsigned hi, const float* __restrict__ a, int na,
                                  unsigned long long* __restrict__ bad) {
     unsigned long long mine = 0;
     for (unsigned u = lo + blockIdx.x * blockDim.x + threadIdx.x; u < hi; u += gridDim.x * blockDim.x) {
         const float b = __uint_as_float(u);
         mine += __float_as_uint(sqrt_rn_fast(b)) != __float_as_uint(sqrtf(b)) ? 1ull : 0ull;
+        mine += __float_as_uint(recip_rn_fast(b)) != __float_as_uint(1.0f / b) ? 1ull : 0ull;
         for (int k = 0; k < na; ++k)
             mine += __float_as_uint(div_rn_fast(a[k], b)) != __float_as_uint(a[k] / b) ? 1ull : 0ull;
     }
