@@ -177,17 +177,21 @@ typedef struct sop_tuning {
     int sort_every;   /* Verlet rows re-sorted by length at every k-th Verlet rebuild */
     int split_rows;   /* 4, 8 or 16: the jobs of at most 5120 beads are stepped with each bead's force terms
                          spread over the lanes of a wavefront, that many beads per wavefront, and their lists
-                         built one wavefront per bead (the same results); 0: one bead per lane.  Until a shape
-                         is set or tuned, the engine chooses by the beads it steps. */
-    int split_global; /* the same step for the jobs above 5120 beads (partners gathered from global memory) */
+                         built one wavefront per bead (the same results; 4 takes two beads per wavefront in
+                         launches of at most 4500); 0: one bead per lane; -1 (the default): chosen by the
+                         beads of the launch, with whole blocks of steps in one launch for small jobs.
+                         unit_rows, shared_units, pair_batch and verlet_chunk act where a bead has a lane. */
+    int split_global; /* the same for the jobs above 5120 beads (partners gathered from global memory);
+                         max_blocks acts where a bead has a lane */
 } sop_tuning;
 int sop_engine_get_shape(sop_engine* e, sop_tuning* out);
 int sop_engine_set_shape(sop_engine* e, const sop_tuning* shape);
 /* Searches the shapes on the admitted jobs and keeps the fastest: each
  * candidate runs real blocks (whole periods of the jobs' list cadences)
  * from a device snapshot of every job, restored afterwards, so the jobs do
- * not advance.  Reports the chosen shape, the ms per step of the shape the
- * search started from and of the chosen one, and the candidates timed. */
+ * not advance.  Reports the chosen shape (which sop_engine_set_shape sets on
+ * another engine, too), the ms per step of the shape the search started from
+ * and of the chosen one, and the candidates timed. */
 int sop_engine_autotune(sop_engine* e, sop_tuning* best, double* ms_per_step_start, double* ms_per_step_best,
                         int* trials);
 

@@ -852,11 +852,8 @@ int Engine::sync_tables() {
     std::vector<int2> units;
     lds_beads_ = 0;
     any_global_ = 0;
-    long long lds_rows = 0, global_rows = 0, short_rows = 0;
     for (int k = 0; k < nj; ++k) {
         const DevJob& J = jobs_[k].dj;
-        (J.lds_step ? lds_rows : global_rows) += J.n;
-        if (J.n <= kRowsShort) short_rows += J.n;
         if (!J.lds_step) {
             any_global_ = 1;
             continue;
@@ -877,7 +874,7 @@ int Engine::sync_tables() {
                            "unit upload"))
             return rc;
     }
-    eff_ = effective_shape(lds_rows, global_rows, short_rows);
+    eff_ = effective_shape(0, nj);
     // LDS step plan
     std::vector<int2> su;
     std::vector<int4> sg;
@@ -891,10 +888,11 @@ int Engine::sync_tables() {
     return 0;
 }
 
-// The launch shape for so many rows (Verlet rows: beads) of LDS-step jobs and
-// of the others, short_rows of them of jobs of at most kRowsShort beads: the
-// one set by set_shape or autotune, else the spread step (k_step_rows) up to
-// kRowsMaxLds and kRowsMaxGlobal rows and one bead per lane above.
+// The launch shape of jobs first .. first + count - 1: for the LDS-step jobs and
+// the others each the rows per wavefront that were asked for, or (-1, the
+// default) chosen by the rows of the launch (Verlet rows: beads): the spread
+// step (k_step_rows) up to kRowsMaxLds and kRowsMaxGlobal rows and one bead per
+// lane above.
 //
 // Rows per wavefront, measured per step launch (the record from the table)
 // with R = 2 / 4 / 8 / 16 and one bead per lane (us):
@@ -911,27 +909,32 @@ int Engine::sync_tables() {
 // Few rows want many wavefronts; many rows want few instructions per row.
 // Lists as short as the peptides' leave most of a 4-row wavefront's positions
 // empty.
-StepShape Engine::effective_shape(long long lds_rows, long long global_rows, long long short_rows) const {
+StepShape Engine::effective_shape(int first, int count) const {
     StepShape e = shape_;
-    const bool set = shape_set_;
-    const bool l = lds_rows > 0 && (set ? e.split_rows > 0 : lds_rows <= kRowsMaxLds);
-    const bool g = global_rows > 0 && (set ? e.split_global > 0 : global_rows <= kRowsMaxGlobal);
+    long long lds_rows = 0, global_rows = 0, short_rows = 0;  // short_rows: of jobs of at most kRowsShort beads
+    for (int k = first; k < first + count; ++k) {
+        const DevJob& J = jobs_[k].dj;
+        (J.lds_step ? lds_rows : global_rows) += J.n;
+        if (J.n <= kRowsShort) short_rows += J.n;
+    }
+    const bool l = lds_rows > 0 && (e.split_rows < 0 ? lds_rows <= kRowsMaxLds : e.split_rows > 0);
+    const bool g = global_rows > 0 && (e.split_global < 0 ? global_rows <= kRowsMaxGlobal : e.split_global > 0);
     const long long rows = (l ? lds_rows : 0) + (g ? global_rows : 0);  // both classes in one launch
     const bool shorts = 2 * short_rows > rows, two = rows <= kRowsTwo && !shorts;
     auto rows_per_wave = [&](int asked) {
-        if (set) return asked == 4 && two ? 2 : asked;
+        if (asked >= 0) return asked == 4 && two ? 2 : asked;
         if (rows <= kRowsFour) return shorts ? 8 : two ? 2 : 4;
         return rows <= kRowsEight ? 8 : 16;
     };
-    if (l) e.split_rows = rows_per_wave(e.split_rows);
-    if (g) e.split_global = rows_per_wave(e.split_global);
+    e.split_rows = l ? rows_per_wave(e.split_rows) : 0;
+    e.split_global = g ? rows_per_wave(e.split_global) : 0;
     return e;
 }
 
 // Rows per wavefront of k_block_rows for jobs first .. first + count - 1, 0 where
-// their steps take a launch each: a shape that was set, a job past kBlockBeads
-// or with hydrodynamics, or few jobs whose rows the spread step divides over
-// more CUs than they have workgroups here.  Measured with updaters and lists in
+// their steps take a launch each: rows per wavefront that were asked for, a job
+// past kBlockBeads or with hydrodynamics, or few jobs whose rows the spread step
+// divides over more CUs than they have workgroups here.  Measured with updaters and lists in
 // launches of their own, us per step of a block of 10, a launch per step | R =
 // 8, 16 (the larger R where rows are many):
 //   beads x jobs   22 x 1      64        256       512        1,000       6,000
@@ -949,7 +952,7 @@ int Engine::block_rows(int first, int count, int* beads) const {
         most = std::max(most, J.n);
     }
     *beads = most;
-    if (shape_set_ || (most > kBlockShort && rows < (long long)kBlockJobs * most)) return 0;
+    if (shape_.split_rows >= 0 || (most > kBlockShort && rows < (long long)kBlockJobs * most)) return 0;
     return most <= 128 && rows <= kRowsEight ? 8 : 16;
 }
 
@@ -1249,8 +1252,7 @@ int Engine::tiles_for_slot(int slot, int* nt) {
     const int n = jobs_[slot].n;
     const int need = (n + 63) / 64;
     *nt = need;
-    const bool lds = jobs_[slot].dj.lds_step != 0;
-    eff1_ = effective_shape(lds ? n : 0, lds ? 0 : n, n <= kRowsShort ? n : 0);
+    eff1_ = effective_shape(slot, 1);
     if (tiles1_n_ == n && tiles1_rows_ == shape_.unit_rows) return 0;
     if (need > cap_tiles1_) {
         (void)hipFree(d_tiles1_);
@@ -1751,11 +1753,11 @@ Tuning Engine::tuning() const {
 }
 
 int Engine::set_shape(const Tuning& t) {
+    auto rows_ok = [](int r) { return r == -1 || r == 0 || r == 4 || r == 8 || r == 16; };
     const bool ok = t.max_blocks >= 0 && t.unit_rows >= 64 && t.unit_rows <= 1024 && t.unit_rows % 64 == 0 &&
                     (t.pair_batch == 4 || t.pair_batch == 6 || t.pair_batch == 8) &&
                     (t.verlet_chunk == 4 || t.verlet_chunk == 8) && t.sort_every >= 1 && t.sort_every <= 1000 &&
-                    (t.split_rows == 0 || t.split_rows == 4 || t.split_rows == 8 || t.split_rows == 16) &&
-                    (t.split_global == 0 || t.split_global == 4 || t.split_global == 8 || t.split_global == 16);
+                    rows_ok(t.split_rows) && rows_ok(t.split_global);
     if (!ok) return fail(SOP_E_ARG, "launch shape out of range");
     max_blocks_ = t.max_blocks;
     shape_.unit_rows = t.unit_rows;
@@ -1765,7 +1767,6 @@ int Engine::set_shape(const Tuning& t) {
     shape_.split_rows = t.split_rows;
     shape_.split_global = t.split_global;
     shared_units_ = t.shared_units != 0;
-    shape_set_ = true;
     tables_dirty_ = true;  // the unit plan depends on unit_rows and shared_units
     tiles1_n_ = -1;
     drop_graph();
@@ -1856,15 +1857,10 @@ int Engine::time_blocks(int nblocks, double* ms) {
 int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int* trials_out) {
     if (hipSetDevice(device_) != hipSuccess) return fail(SOP_E_HIP, "hipSetDevice failed");
     if (int rc = sync_tables()) return rc;
-    const bool was_set = shape_set_;
-    Tuning start = tuning();
+    const Tuning start = tuning();
     if (best_out) *best_out = start;
     if (trials_out) *trials_out = 0;
     if (jobs_.empty()) return 0;
-    if (!was_set) {  // the shape the jobs run in now (four rows per wavefront stand for two, too)
-        start.split_rows = eff_.split_rows == 2 ? 4 : eff_.split_rows;
-        start.split_global = eff_.split_global == 2 ? 4 : eff_.split_global;
-    }
     bool lds = false;
     long long window = L_;
     for (auto& j : jobs_) {
@@ -1882,17 +1878,31 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
     void* snap = nullptr;
     if (int rc = snapshot(&snap)) return rc;
     int trials = 0;
-    auto unset = [&] {  // the shape follows the rows again
-        shape_.split_rows = shape_.split_global = 0;
-        shape_set_ = false;
+    // whether small jobs take a block in one launch where their rows per
+    // wavefront are not asked for
+    auto under = [&](const Tuning& t, auto f) {  // f() with t's rows per wavefront
+        const StepShape now = shape_;
+        shape_.split_rows = t.split_rows;
+        shape_.split_global = t.split_global;
+        const int r = f();
+        shape_ = now;
+        return r;
     };
-    // a block in one launch is taken only where no shape is set: measured as
-    // such, and left so unless a set shape is faster
+    Tuning chosen = start;
+    chosen.split_rows = -1;
     int beads = 0;
-    bool block = block_rows(0, (int)jobs_.size(), &beads) > 0;
+    const bool block = under(chosen, [&] { return block_rows(0, (int)jobs_.size(), &beads); }) > 0;
+    // rows per wavefront of a class under t, beside the other class's, with -1
+    // as it is chosen (four stand for two, too)
+    auto rows_of = [&](const Tuning& t, int Tuning::*field) {
+        return under(t, [&] {
+            const StepShape e = effective_shape(0, (int)jobs_.size());
+            const int r = field == &Tuning::split_rows ? e.split_rows : e.split_global;
+            return r == 2 ? 4 : r;
+        });
+    };
     auto trial = [&](const Tuning& t, double* per_step) -> int {
         if (int rc = set_shape(t)) return rc;
-        if (block && trials == 0) unset();
         if (int rc = restore(snap, steps)) return rc;
         double ms = 0.0;
         if (int rc = time_blocks(nblocks, &ms)) return rc;
@@ -1911,14 +1921,19 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
         if (!rc && ms < best_ms * 0.995) {  // a real gain, beyond run-to-run noise
             best = t;
             best_ms = ms;
-            block = false;
+        }
+    };
+    // the other values of a class's rows per wavefront that launch something else
+    auto consider_rows = [&](int Tuning::*field, bool in_block) {
+        for (int v : {-1, 0, 16, 8, 4}) {
+            Tuning t = best;
+            t.*field = v;
+            if (v != best.*field && (in_block || rows_of(t, field) != rows_of(best, field))) consider(t);
         }
     };
     // each bead's terms spread over a wavefront, or one bead per lane
-    if (lds && ntiles_ <= kSplitMaxTiles)
-        for (int v : {0, 16, 8, 4})
-            if (v != best.split_rows) { Tuning t = best; t.split_rows = v; consider(t); }
-    if (lds && !best.split_rows) {
+    if (lds && ntiles_ <= kSplitMaxTiles) consider_rows(&Tuning::split_rows, block);
+    if (lds && rows_of(best, &Tuning::split_rows) == 0) {
         // smaller units spread a few small jobs over more CUs
         for (int v : {1024, 768, 512, 256, 128})
             if (v != best.unit_rows) { Tuning t = best; t.unit_rows = v; consider(t); }
@@ -1930,10 +1945,9 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
             if (v != best.sort_every) { Tuning t = best; t.sort_every = v; consider(t); }
     }
     if (any_global_) {
-        for (int v : {0, 16, 8, 4})
-            if (v != best.split_global) { Tuning t = best; t.split_global = v; consider(t); }
+        consider_rows(&Tuning::split_global, false);
         const int full = (ntiles_ + 3) / 4;
-        if (!best.split_global) {
+        if (rows_of(best, &Tuning::split_global) == 0) {
             for (int b : {256, 1024, 4096})
                 if (b < full && b != best.max_blocks) { Tuning t = best; t.max_blocks = b; consider(t); }
             if (best.max_blocks != 0) { Tuning t = best; t.max_blocks = 0; consider(t); }
@@ -1941,7 +1955,6 @@ int Engine::autotune(Tuning* best_out, double* ms_default, double* ms_best, int*
     }
     // the jobs as they were, under the chosen shape
     const int rc2 = set_shape(rc ? start : best);
-    if (block || (rc && !was_set)) unset();
     const int rc3 = restore(snap, steps);
     (void)hipFree(snap);
     use_graph_ = saved_graph;

@@ -77,7 +77,8 @@ struct Tuning {
     int pair_batch;    // Verlet entries fetched ahead per lane in the LDS step
     int verlet_chunk;  // 64-entry chunks in flight per row in the LDS Verlet build
     int sort_every;    // Verlet rows re-sorted at every k-th Verlet rebuild
-    int split_rows;    // 4, 8 or 16: LDS-step jobs stepped by k_step_rows, that many rows per wavefront (0: off)
+    int split_rows;    // 4, 8 or 16: LDS-step jobs stepped by k_step_rows, that many rows per wavefront (0: one
+                       // bead per lane; -1: chosen by the rows of the launch, or a block in one launch)
     int split_global;  // the same for the jobs above the LDS limit
 };
 
@@ -214,9 +215,8 @@ class Engine {
     int cap_sunits1_ = 0, cap_segs1_ = 0, nsunits1_ = 0;
     int tiles1_rows_ = 0;  // unit rows the single-job plan was built for
     StepShape shape_;
-    bool shape_set_ = false;  // by set_shape or autotune; else the spread step follows the rows (effective_shape)
-    StepShape eff_, eff1_;    // the shapes launched: of the admitted jobs, and of the single-job path's job
-    StepShape effective_shape(long long lds_rows, long long global_rows, long long short_rows) const;
+    StepShape eff_, eff1_;  // the shapes launched: of the admitted jobs, and of the single-job path's job
+    StepShape effective_shape(int first, int count) const;
     bool shared_units_ = true;
     // autotuner snapshot of the jobs' device arrays and state table
     int snapshot(void** buf);

@@ -12,17 +12,19 @@ namespace sop {
 // in flight per row in the Verlet build, and the row-sort cadence (every
 // k-th Verlet rebuild).  split_rows (4, 8 or 16; 0: off) steps the LDS-step
 // jobs by k_step_rows instead, that many rows per wavefront (two instead of
-// four in the smallest launches) with each row's force terms spread over its lanes, and builds their lists one wavefront
-// per row; split_global steps the jobs above the LDS limit the same way.
+// four in the smallest launches) with each row's force terms spread over its
+// lanes, and builds their lists one wavefront per row; split_global steps the
+// jobs above the LDS limit the same way.  -1 (not in a shape that is launched):
+// chosen by the rows of the launch.
 struct StepShape {
     int unit_rows = kLdsUnit;
     int pair_batch = 6;
     int verlet_chunk = 8;
     int sort_every = kSortEvery;
-    int split_rows = 0;
-    int split_global = 0;
+    int split_rows = -1;
+    int split_global = -1;
 };
-// The rule for the spread step where no shape was set (measurements at
+// The rule for the spread step where its rows are not asked for (measurements at
 // Engine::effective_shape): rows of the launch up to which a wavefront takes
 // two, four and eight rows (sixteen above), the rows of LDS-step jobs and of the
 // others up to which they are spread at all, and the beads of a job whose lists
