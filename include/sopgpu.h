@@ -147,9 +147,12 @@ int sop_engine_remove_job(sop_engine* e, int job_id);
 int sop_engine_job_bytes(const sop_params* p, const sop_system* s, unsigned long long* bytes);
 
 /* Launch shape: max_blocks caps the persistent step grid (0: one
- * workgroup per 4 tiles); use_graph != 0 replays each block from a
- * captured hipGraph (several at a time, once their launch sequence has come
- * four times). */
+ * workgroup per 4 tiles); use_graph != 0 replays blocks from captured
+ * hipGraphs, about 100 steps a graph, once their launch sequence has come
+ * four times.  The blocks that a call of run_blocks (or a server's pump) has
+ * over, or a shorter call's, are a graph of their own from 50 steps on and
+ * launched directly below (a graph of ten steps takes the GPU longer than its
+ * launches do), and always where a block of steps is one launch. */
 int sop_engine_set_tuning(sop_engine* e, int max_blocks, int use_graph);
 /* Possible-pairs builder (src/Updaters/possiblepairlist_kernel.cu:18-71
  * scans all same-trajectory pairs): jobs of min_beads beads and more admitted
@@ -362,7 +365,7 @@ int sop_sim_add_forces(sop_sim* s, int traj, const float* f4);
  * runs one system or identical replicas per process, src/sop-gpu.cpp:18-65).
  * submit copies the request and queues it; pump admits queued requests in
  * arrival order while the HBM budget has room, advances every admitted job
- * by nblocks blocks in one step kernel per step, and retires finished jobs
+ * by nblocks blocks (sop_engine_run_blocks), and retires finished jobs
  * (coordinates copied out, memory released).  Times are seconds since the
  * server was created; state: 0 queued, 1 running, 2 done, -1 failed. */
 typedef struct sop_server sop_server;

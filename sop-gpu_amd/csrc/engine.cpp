@@ -1399,48 +1399,65 @@ int Engine::capture_graph(const std::vector<long long>& key, int blocks) {
 // hydrodynamics: one, its factorisations are hundreds of launches.
 int Engine::graph_blocks() const { return any_exact_ ? 1 : (int)std::clamp(kGraphSteps / L_, 1, kGraphBlocks); }
 
+// Whether m blocks, fewer than graph_blocks(), are worth a graph: half of
+// kGraphSteps, where a step is a launch of its own.  A graph takes 20 us of the
+// host, whatever it holds, and up to 5 of the GPU; a launch takes 3 of the host.
+// Calls of m blocks of ten steps, us per block on the GPU and (the host), direct
+// | graph:
+//                 1,000 beads              18,000 beads               350 peptides (a block a launch)
+//   m = 1     81 (41) | 86 (20)      183 (45) | 190 (19)       39.3 (7.6) | 44.8 (22)
+//   m = 3     81 (40) | 80 (7.1)     182 (43) | 185 (6.6)      39.2 (6.8) | 41.3 (9.3)
+//   m = 5     81 (41) | 80 (4.2)     183 (44) | 184 (4.0)      39.3 (6.8) | 40.4 (6.9)
+bool Engine::graph_pays(int m) const {
+    int beads = 0;
+    return m * L_ >= kGraphSteps / 2 && block_rows(0, (int)jobs_.size(), &beads) == 0;
+}
+
 int Engine::run_blocks(int nblocks) {
     if (hipSetDevice(device_) != hipSuccess) return fail(SOP_E_HIP, "hipSetDevice failed");
     if (int rc = sync_tables()) return rc;
     if (jobs_.empty()) return 0;
-    // blocks are replayed, some at a time, from the graph captured for their
-    // launch sequence; a sequence is launched directly until it has come
+    // blocks are replayed, up to K at a time, from the graph captured for
+    // their launch sequence; a sequence is launched directly until it has come
     // kGraphAfter times, and captured behind the last of these while the GPU
     // works on it.  Past kMaxGraphs sequences (exact-HI jobs whose
     // refactorisation steps keep shifting against the block) the new ones are
-    // launched directly
+    // launched directly, and so are a call's last blocks, or a shorter call's,
+    // where graph_pays says so
     const int K = use_graph_ && !profiling_ ? graph_blocks() : 0;
     std::vector<long long> before(jobs_.size()), after(jobs_.size());
-    while (K > 0 && nblocks >= K) {
+    auto at = [&](const std::vector<long long>& steps) {
+        for (size_t q = 0; q < jobs_.size(); ++q) jobs_[q].step = steps[q];
+    };
+    for (; nblocks > 0; nblocks -= K) {
+        const int m = std::min(K, nblocks);
+        if (K == 0 || (m < K && !graph_pays(m))) return launch_blocks(nblocks);
         for (size_t q = 0; q < jobs_.size(); ++q) before[q] = jobs_[q].step;
-        std::vector<long long> key;
-        for (int b = 0; b < K; ++b) {
+        std::vector<long long> key;  // of each block, so of their number too
+        for (int b = 0; b < m; ++b) {
             const std::vector<long long> one = block_key();
             key.insert(key.end(), one.begin(), one.end());
             for (auto& j : jobs_) j.step = std::min(j.step + L_, j.end_step);
         }
         for (size_t q = 0; q < jobs_.size(); ++q) after[q] = jobs_[q].step;
+        at(before);  // on an error, the steps whose launches were accepted
         const auto it = graphs_.find(key);
         if (it != graphs_.end()) {
             if (int rc = check(hipGraphLaunch(it->second, stream_), "graph launch")) return rc;
         } else {
-            auto rewind = [&] {
-                for (size_t q = 0; q < jobs_.size(); ++q) jobs_[q].step = before[q];
-            };
-            rewind();
-            if (int rc = launch_blocks(K)) return rc;
+            if (int rc = launch_blocks(m)) return rc;
             if (graphs_.size() < kMaxGraphs && (came_.size() < kMaxCame || came_.count(key)) &&
                 ++came_[key] >= kGraphAfter) {
                 came_.erase(key);
-                rewind();
-                const int rc = capture_graph(key, K);
-                for (size_t q = 0; q < jobs_.size(); ++q) jobs_[q].step = after[q];
+                at(before);
+                const int rc = capture_graph(key, m);
+                at(after);
                 if (rc) return rc;
             }
         }
-        nblocks -= K;
+        at(after);
     }
-    return launch_blocks(nblocks);
+    return 0;
 }
 
 int Engine::run_job(int id) {

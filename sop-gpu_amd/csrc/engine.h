@@ -160,6 +160,7 @@ class Engine {
     std::vector<long long> block_key() const;
     int launch_blocks(int blocks);
     int graph_blocks() const;
+    bool graph_pays(int m) const;
     int capture_graph(const std::vector<long long>& key, int blocks);
     void drop_graph();
     int check(hipError_t e, const char* what);
