@@ -232,8 +232,9 @@ int sop_engine_compute_energies(sop_engine* e, int job_id, float* per_bead3n, fl
 /* Force a list rebuild now (mask: 1 possible, 2 Verlet). */
 int sop_engine_rebuild_lists(sop_engine* e, int job_id, int mask);
 
-/* Timing of the step kernel with HIP events on the engine's stream:
- * while enabled, each step-kernel launch is bracketed by events. */
+/* Timing of the steps with HIP events on the engine's stream: while enabled,
+ * the launches that step the jobs (and nothing else) are bracketed by events.
+ * *launches counts steps, whether a step is a launch or a block of them. */
 int sop_engine_profile(sop_engine* e, int enable);
 int sop_engine_profile_read(sop_engine* e, long long* launches, double* total_ms);
 /* Average list lengths over admitted jobs' beads (covalent, native,

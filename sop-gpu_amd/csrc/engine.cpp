@@ -1142,13 +1142,14 @@ int Engine::launch_block(int slot_only) {
         L = jobs_[slot_only].dj.stride;
     }
     // a block in one launch begins with the updaters (but for the tip) and the
-    // Verlet lists
+    // Verlet lists, except while the steps are timed
     int beads = 0;
     const int block = slot_only >= 0 ? block_rows(slot_only, 1, &beads) : block_rows(0, nj, &beads);
-    bool tip = !block;
-    for (int k = 0; k < nj && !tip; ++k) tip = jobs_[slot_only >= 0 ? slot_only : k].dj.flags & JF_INDENTATION;
-    if (tip)
-        if (int rc = check(launch_job_update(jobs, st, nj, stream_, block ? 1 : 7), "job update")) return rc;
+    const bool begins = block && !profiling_;
+    bool update = !begins;
+    for (int k = 0; k < nj && !update; ++k) update = jobs_[slot_only >= 0 ? slot_only : k].dj.flags & JF_INDENTATION;
+    if (update)
+        if (int rc = check(launch_job_update(jobs, st, nj, stream_, begins ? 1 : 7), "job update")) return rc;
     const int due = lists_due(slot_only);
     if (due & 1) {
         const hipError_t e =
@@ -1167,9 +1168,9 @@ int Engine::launch_block(int slot_only) {
                               ? (jobs_[slot_only].n + kLdsUnit - 1) / kLdsUnit
                               : 0;
         const hipError_t e =
-            block ? launch_sort_rows(jobs, st, slot_only >= 0 ? d_units1_ : d_units_,
-                                     slot_only >= 0 ? sort1 : sort ? nunits_ : 0, 0, stream_,
-                                     slot_only >= 0 ? eff1_ : eff_)
+            begins ? launch_sort_rows(jobs, st, slot_only >= 0 ? d_units1_ : d_units_,
+                                      slot_only >= 0 ? sort1 : sort ? nunits_ : 0, 0, stream_,
+                                      slot_only >= 0 ? eff1_ : eff_)
             : slot_only >= 0
                 ? launch_verlet(jobs, st, tiles, nt, !jobs_[slot_only].dj.idx16, !jobs_[slot_only].dj.lds_step,
                                 d_units1_, sort1, d_sunits1_, d_segs1_, jobs_[slot_only].dj.lds_step ? nsunits1_ : 0,
@@ -1187,7 +1188,7 @@ int Engine::launch_block(int slot_only) {
                            "TEA update"))
             return rc;
     // profiling: HIP events around the step launches; when nothing else is
-    // launched between them, one pair spans the block's L launches
+    // launched between them, one pair spans the block's L steps
     const bool span = !tea && !exact;
     for (int k = 0; k < L; ++k) {
         const bool prof = profiling_ && (!span || k == 0);
@@ -1209,7 +1210,7 @@ int Engine::launch_block(int slot_only) {
             block && k % kBlockSteps ? hipSuccess  // in the launch before
             : block ? launch_block_rows(jobs, descs, st, nj, beads, block, k, std::min(L - k, kBlockSteps),
                                         k + kBlockSteps >= L ? L : 0,
-                                        k == 0 ? BLOCK_UPDATE | (due & 2 ? BLOCK_VERLET : 0) : 0, stream_)
+                                        begins && k == 0 ? BLOCK_UPDATE | (due & 2 ? BLOCK_VERLET : 0) : 0, stream_)
             : slot_only >= 0
                 ? launch_step(jobs, descs, one, st, tiles, nt, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
                               jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, k, max_blocks_, stream_,
