@@ -1624,10 +1624,12 @@ hipError_t launch_hi_tea_step(const DevJob* jobs, const DevJobState* st, const i
 
 // The lower triangle's rows from s on, columns [s, s + cols) (cols < 0: all),
 // minus the panel copy's kw columns times their transpose.  The next panel's
-// columns (cols = 512): 128x64 tiles, which put 3,700 rows on 232 CUs, or
-// in split-BF16 128x128 from 8,000 rows on, where those fill two rounds of CUs
-// (in FP32 128x64, whose sums are taken in parts, update_tile).  Regions of
-// at least a round of 256x256 tiles take those, smaller ones 128x128.
+// columns (cols = 512): 128x64 tiles, which put 3,700 rows on 232 CUs and whose
+// sums are taken in parts (update_tile); 128x128 tiles, one sum per element, are
+// no faster from 8,000 rows on either (order 12,288 split-BF16 5.33 ms, 5.32 with
+// 128x64) and left the factor's error 0.1 % above that of sums in parts.  The
+// rest: regions of at least a round of 256x256 tiles take those, smaller ones
+// 128x128.
 static constexpr int kTrailBigMinTiles = 256;
 template <int MODE>
 static void trailing_update(float* M, size_t ld, int s, int mp, int cols, int kw, const char* pan,
@@ -1635,13 +1637,13 @@ static void trailing_update(float* M, size_t ld, int s, int mp, int cols, int kw
     if (s >= mp) return;
     const int nr = (mp - s + 127) / 128;
     const int ntr = (mp - s + BT - 1) / BT, ntile = ntr * (ntr + 1) / 2;
-    if (cols >= 0 && (nr <= 62 || MODE == SOP_CHOL_F32))
+    if (cols >= 0)
         hipLaunchKernelGGL((k_update<MODE, 128, 64>), dim3(nr, cols / 64), dim3(256), 0, stream, M, ld, s, mp, kw, pan);
-    else if (cols < 0 && ntile >= kTrailBigMinTiles)
+    else if (ntile >= kTrailBigMinTiles)
         hipLaunchKernelGGL((k_update_big<MODE>), dim3((ntile + kXcds - 1) / kXcds * kXcds), dim3(512), 0, stream, M, ld,
                            s, mp, kw, ntr, pan);
     else
-        hipLaunchKernelGGL((k_update<MODE, 128, 128>), dim3(nr, cols < 0 ? nr : cols / 128), dim3(256), 0, stream, M, ld,
+        hipLaunchKernelGGL((k_update<MODE, 128, 128>), dim3(nr, nr), dim3(256), 0, stream, M, ld,
                            s, mp, kw, pan);
 }
 
