@@ -158,8 +158,11 @@ int sop_engine_set_tuning(sop_engine* e, int max_blocks, int use_graph);
  * scans all same-trajectory pairs): jobs of min_beads beads and more admitted
  * after this call (default 8192; 0 keeps the threshold, < 0 none) get the
  * bounding boxes of their tiles of 64 beads and build the identical list, in
- * the identical order, from the tiles in reach of each bead.  enabled = 0
- * makes every job use the all-pairs scan again (the boxes stay allocated). */
+ * the identical order, from the tiles in reach of each bead, or from a cell
+ * grid where the beads are in no spatial order along the chain (jobs of more
+ * than 20480 beads; seen when a job is admitted, when its coordinates are set
+ * and when its state is read).  enabled = 0 makes every job use the all-pairs
+ * scan again (the boxes and the grid stay allocated). */
 int sop_engine_set_cells(sop_engine* e, int min_beads, int enabled);
 /* Step kernel variant (the reference's potentials + integrator,
  * src/gsop.cu:136-142): jobs of at most 5120 beads are stepped with their

@@ -497,6 +497,41 @@ static size_t nbytes(const std::vector<T>& v) {
 
 static unsigned long long round_up(unsigned long long x) { return (x + kAlign - 1) / kAlign * kAlign; }
 
+// Whether a job of n beads, if it has tile boxes, may take a cell grid: where it
+// has more tiles than kWideTiles, and its bitmap fits.
+static bool uses_grid(size_t n) { return n > (size_t)64 * kWideTiles && n <= (size_t)64 * kMaxCellWords; }
+
+// The tiles of 64 beads that a bead reaches (boxes within the threshold, d2max)
+// on average, from 32 beads and 32 tiles spread over the job (a few
+// microseconds, beside a copy of the coordinates).
+static double tiles_in_reach(const float4* c, int n, float d2max) {
+    constexpr int kSample = 32;
+    const int nt = (n + 63) / 64, S = std::min(nt, kSample);
+    if (S < 2) return nt;
+    float4 lo[kSample], hi[kSample], p[kSample];
+    auto lower = [](float x, float l) { return x < l ? x : l; };  // l where x is not a number
+    auto upper = [](float x, float h) { return x > h ? x : h; };
+    for (int k = 0; k < S; ++k) {
+        const int b = 64 * (int)((long long)k * nt / S), e = std::min(b + 64, n);
+        float4 l{INFINITY, INFINITY, INFINITY, 0.0f}, h{-INFINITY, -INFINITY, -INFINITY, 0.0f};
+        for (int i = b; i < e; ++i) {
+            l.x = lower(c[i].x, l.x), h.x = upper(c[i].x, h.x);
+            l.y = lower(c[i].y, l.y), h.y = upper(c[i].y, h.y);
+            l.z = lower(c[i].z, l.z), h.z = upper(c[i].z, h.z);
+        }
+        lo[k] = l, hi[k] = h, p[k] = c[std::min(b + 32, n - 1)];
+    }
+    int reached = 0;  // of the tiles but the bead's own
+    for (int k = 0; k < S; ++k)
+        for (int q = 0; q < S; ++q) {
+            const float x = upper(lo[q].x - p[k].x, upper(p[k].x - hi[q].x, 0.0f));
+            const float y = upper(lo[q].y - p[k].y, upper(p[k].y - hi[q].y, 0.0f));
+            const float z = upper(lo[q].z - p[k].z, upper(p[k].z - hi[q].z, 0.0f));
+            reached += (q != k) & (x * x + y * y + z * z <= d2max);
+        }
+    return 1.0 + (double)reached / ((double)S * (S - 1)) * (nt - 1);
+}
+
 static unsigned long long built_bytes(const BuiltJob& b, bool pulling, bool indentation) {
     const unsigned long long n = b.n;
     unsigned long long t = 0;
@@ -518,7 +553,9 @@ static unsigned long long built_bytes(const BuiltJob& b, bool pulling, bool inde
     t += round_up(std::max<size_t>(1, b.pulled.size()) * 4);
     t += round_up(n * 12);                // energies
     if (b.dj.flags & JF_EXTRA_FORCE) t += round_up(n * 16);  // forces of host potentials
-    if (n >= (unsigned long long)kBoxMinBeads) t += round_up((n + 63) / 64 * 32);  // tile boxes
+    if (n >= (unsigned long long)kBoxMinBeads)  // tile boxes, or the cell grid with the boxes in it
+        t += uses_grid(n) ? round_up((n + 64) * 4) + round_up((n + 65) * 4) + 3 * round_up(n * 4)
+                          : round_up((n + 63) / 64 * 32);
     if (b.dj.flags & JF_HI) {
         t += 3 * round_up(n * 16) + round_up(n * 4);  // rforce, mforce, ci, eps
         if (b.dj.flags & JF_HI_EXACT) {
@@ -596,7 +633,18 @@ int Engine::add_job(const sop_params& p, const sop_system& s, long long numsteps
     J.energies = (float*)A(n * 12);
     J.lds_step = use_lds_step_ && n <= (size_t)kLdsStepBeads ? 1 : 0;
     J.sort_rows = J.lds_step && J.rb_cnt ? 1 : 0;
-    if (uses_boxes(n)) J.tile_box = (float4*)A((n + 63) / 64 * 32);
+    if (uses_boxes(n) && uses_grid(n)) {
+        J.cell_cap = (int)n + 64;
+        J.cell_cnt = (int*)A((size_t)J.cell_cap * 4);
+        J.cell_start = (int*)A((size_t)(J.cell_cap + 1) * 4);
+        J.cell_beads = (int*)A(n * 4);
+        J.bead_cell = (int*)A(n * 4);
+        J.bead_slot = (int*)A(n * 4);
+        J.tile_box = (float4*)J.cell_beads;  // never both in use
+        J.wide = tiles_in_reach(b.coord.data(), b.n, J.pp_d2) > kWideTiles;
+    } else if (uses_boxes(n)) {
+        J.tile_box = (float4*)A((n + 63) / 64 * 32);
+    }
     HiExactWork hw{};
     if (J.flags & JF_HI) {
         J.rforce = (float4*)A(n * 16);
@@ -810,12 +858,13 @@ int Engine::sync_tables() {
     }
     L_ = g > 0 ? g : 1;
     any_tea_ = any_exact_ = false;
-    any_boxes_ = 0;
+    any_boxes_ = cell_words_ = 0;
     any_idx32_ = 0;
     std::vector<int2> tea_tiles;  // the tiles of the TEA jobs
     for (auto& j : jobs_) {
         if (!j.dj.idx16) any_idx32_ = 1;
         any_boxes_ |= boxes_of(j.dj);
+        if (j.dj.wide) cell_words_ = std::max(cell_words_, (j.n + 63) / 64);
         if ((j.dj.flags & JF_HI) && !(j.dj.flags & JF_HI_EXACT)) {
             any_tea_ = true;
             tea_tiles.insert(tea_tiles.end(), tiles.begin() + j.tile0, tiles.begin() + j.tile0 + j.ntile);
@@ -1029,7 +1078,28 @@ void Engine::drop_graph() {
 
 bool Engine::uses_boxes(size_t n) const { return box_min_ > 0 && n >= (size_t)box_min_; }
 
-int Engine::boxes_of(const DevJob& J) const { return use_boxes_ && J.tile_box; }
+int Engine::boxes_of(const DevJob& J) const {
+    return !use_boxes_ || !J.tile_box ? 0 : J.wide ? BOXES_WIDE : BOXES_NEAR;
+}
+
+void Engine::set_wide(HostJob& hj, bool wide) {
+    if (!hj.dj.cell_cnt || hj.dj.wide == (int)wide) return;
+    hj.dj.wide = wide;
+    tables_dirty_ = true;
+    drop_graph();
+}
+
+// Whether a job's beads have left their order, so that the boxes of its
+// tiles reach over most of it: from the tiles reached that the builds since the
+// last read of its state sampled.  A job stays with the grid until its
+// coordinates are set anew.
+void Engine::judge_wide(HostJob& hj, const DevJobState& s) {
+    const long long groups = (long long)(s.near_groups - hj.seen_groups);
+    const double tiles = (double)(long long)(s.near_tiles - hj.seen_tiles);
+    hj.seen_groups = s.near_groups;
+    hj.seen_tiles = s.near_tiles;
+    if (groups > 0 && tiles > (double)kWideTiles * groups) set_wide(hj, true);
+}
 
 void Engine::set_cells(int min_beads, int enabled) {
     if (min_beads != 0) box_min_ = min_beads;
@@ -1154,12 +1224,12 @@ int Engine::launch_block(int slot_only) {
     if (due & 1) {
         const hipError_t e =
             slot_only >= 0
-                ? launch_possible(jobs, st, tiles, nt, boxes_of(jobs_[slot_only].dj),
-                                  !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
+                ? launch_possible(jobs, st, tiles, nt, nj, boxes_of(jobs_[slot_only].dj),
+                                  (jobs_[slot_only].n + 63) / 64, !jobs_[slot_only].dj.lds_step, d_sunits1_, d_segs1_,
                                   jobs_[slot_only].dj.lds_step ? nsunits1_ : 0, jobs_[slot_only].n, 0, stream_,
                                   eff1_)
-                : launch_possible(jobs, st, tiles, nt, any_boxes_, any_global_, d_sunits_, d_segs_, nsunits_,
-                                  lds_beads_, 0, stream_, eff_);
+                : launch_possible(jobs, st, tiles, nt, nj, any_boxes_, cell_words_, any_global_, d_sunits_, d_segs_,
+                                  nsunits_, lds_beads_, 0, stream_, eff_);
         if (int rc = check(e, "possible pairs")) return rc;
     }
     if (due & 2) {
@@ -1303,8 +1373,8 @@ int Engine::stage_job_update(int mask) {
 int Engine::stage_possible() {
     if (int rc = sync_tables()) return rc;
     if (!(lists_due(-1) & 1)) return 0;
-    return check(launch_possible(d_jobs_, d_state_, d_tiles_, ntiles_, any_boxes_, any_global_, d_sunits_, d_segs_,
-                                 nsunits_, lds_beads_, 0, stream_, eff_),
+    return check(launch_possible(d_jobs_, d_state_, d_tiles_, ntiles_, (int)jobs_.size(), any_boxes_, cell_words_,
+                                 any_global_, d_sunits_, d_segs_, nsunits_, lds_beads_, 0, stream_, eff_),
                  "possible pairs");
 }
 int Engine::stage_verlet() {
@@ -1482,7 +1552,10 @@ int Engine::synchronize() {
 int Engine::read_state(int slot, DevJobState* out) {
     if (int rc = sync_tables()) return rc;
     if (int rc = synchronize()) return rc;
-    return check(hipMemcpy(out, d_state_ + slot, sizeof(DevJobState), hipMemcpyDeviceToHost), "state read");
+    if (int rc = check(hipMemcpy(out, d_state_ + slot, sizeof(DevJobState), hipMemcpyDeviceToHost), "state read"))
+        return rc;
+    judge_wide(jobs_[slot], *out);
+    return 0;
 }
 
 int Engine::job_status(int id, long long* step, long long* end, int* overflow) {
@@ -1562,7 +1635,9 @@ int Engine::set_coords(int id, const float* in4) {
     if (slot < 0) return fail(SOP_E_ARG, "no such job");
     DevJobState s;
     if (int rc = read_state(slot, &s)) return rc;
-    const HostJob& hj = jobs_[slot];
+    HostJob& hj = jobs_[slot];
+    if (hj.dj.cell_cnt)
+        set_wide(hj, tiles_in_reach(reinterpret_cast<const float4*>(in4), hj.n, hj.dj.pp_d2) > kWideTiles);
     return check(hipMemcpy(hj.dj.coord[s.step & 1], in4, (size_t)hj.n * 16, hipMemcpyHostToDevice), "coords write");
 }
 
@@ -1729,8 +1804,8 @@ int Engine::rebuild_lists(int id, int mask) {
     int nt = 0;
     if (int rc = tiles_for_slot(slot, &nt)) return rc;
     if (mask & 1)
-        if (int rc = check(launch_possible(d_jobs_ + slot, d_state_ + slot, d_tiles1_, nt, boxes_of(jobs_[slot].dj),
-                                           !jobs_[slot].dj.lds_step, d_sunits1_, d_segs1_,
+        if (int rc = check(launch_possible(d_jobs_ + slot, d_state_ + slot, d_tiles1_, nt, 1, boxes_of(jobs_[slot].dj),
+                                           (jobs_[slot].n + 63) / 64, !jobs_[slot].dj.lds_step, d_sunits1_, d_segs1_,
                                            jobs_[slot].dj.lds_step ? nsunits1_ : 0, jobs_[slot].n, 1, stream_,
                                            eff1_),
                            "possible pairs"))

@@ -67,6 +67,7 @@ struct HostJob {
     std::vector<size_t> sizes;  // bytes of each block (snapshots for the autotuner)
     HiExactWork hw{};      // exact-HI factorisation workspace (hw.M null otherwise)
     int tile0 = 0, ntile = 0;  // the job's range in the tile table
+    unsigned long long seen_tiles = 0, seen_groups = 0;  // DevJobState's near_* at the last read of the state
 };
 
 // Launch shapes the autotuner searches; none of them changes a result.
@@ -132,8 +133,9 @@ class Engine {
 
     void set_tuning(int max_blocks, int use_graph);
     // Possible-pairs tile boxes: jobs of min_beads beads and more admitted
-    // from now on get them (0 keeps the threshold, < 0 gives none); enabled = 0
-    // builds every list by the all-pairs scan.
+    // from now on get them (0 keeps the threshold, < 0 gives none), and a cell
+    // grid where their beads are in no spatial order; enabled = 0 builds every
+    // list by the all-pairs scan.
     void set_cells(int min_beads, int enabled);
     // Step jobs of at most kLdsStepBeads beads with their coordinates in
     // LDS (default) or, enabled = 0, all from global memory.
@@ -195,7 +197,9 @@ class Engine {
     int max_blocks_ = 0;
     int box_min_ = kBoxMinBeads;
     bool use_boxes_ = true;
-    int any_boxes_ = 0;
+    int any_boxes_ = 0, cell_words_ = 0;
+    void set_wide(HostJob& hj, bool wide);
+    void judge_wide(HostJob& hj, const DevJobState& s);
     float4* stage_ = nullptr;  // pinned host memory that k_read_coords writes: kStageBeads entries, its ticket
     unsigned ticket_ = 0;
     int any_idx32_ = 0;  // some job stores int32 list entries

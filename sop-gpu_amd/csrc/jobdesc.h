@@ -73,6 +73,17 @@ struct DevJob {
     // bounding boxes (lo, hi) of the tiles for the possible-pairs build, for
     // jobs of kBoxMinBeads beads and more (null otherwise)
     float4* tile_box;
+    // wide: the possible pairs come from a cell grid instead.  Jobs that may
+    // become so (uses_grid) have one: per-cell counts and exclusive starts, the
+    // beads grouped by cell (the boxes share this array), each bead's cell and
+    // slot within it
+    int wide;
+    int* cell_cnt;
+    int* cell_start;
+    int* cell_beads;
+    int* bead_cell;
+    int* bead_slot;
+    int cell_cap;
     int lds_step;   // stepped by k_step_lds (coordinates staged in LDS)
     int* pulled;    // bead indices of pulled beads
     float* energies; // 3n per-bead energies (output cadence)
@@ -165,6 +176,10 @@ struct DevJobState {
     float tipDr;      // |chip - tip| of the last tip update, before the tip moved
     float beta;       // TEA beta' (bdhitea.cu:162-170)
     double eps_traj;  // TEA epsilon of the last update
+    unsigned long long near_tiles, near_groups;  // tiles that sampled groups of beads reached, and the groups
+    float cell_org[3];  // possible-pairs cell grid of the last rebuild
+    float cell_inv;     // 1 / cell edge
+    int cell_dim[3];
 };
 
 inline StepDesc step_desc(const DevJob& J) {
@@ -227,6 +242,19 @@ inline StepDesc step_desc(const DevJob& J) {
 // tiles whose boxes are near instead of the all-pairs scan (same list, same
 // order).
 constexpr int kBoxMinBeads = 8192;
+// Such a job takes a cell grid where its beads reach more tiles than this on
+// average (beads in no spatial order along the chain).  A rebuild by boxes |
+// by the grid, us, beads of a shell in no order (every tile in reach) with
+// thresholds of 16, 24 and 32 A (80, 250 and 550 entries a bead):
+//   18,000 (282 tiles)      266 | 390       292 | 456       307 | 605
+//   30,000 (469)            624 | 456       685 | 546       729 | 737
+//   50,000 (782)          1,428 | 569     1,535 | 679     1,657 | 961
+//   100,000 (1,563)       4,692 | 1,390   4,938 | 1,634   5,243 | 2,319
+//   200,000 (3,125)      17,402 | 5,129  18,048 | 6,009  18,926 | 7,250
+// and in order along the chain 222 | 945, 290 | 1,468 and 367 | 2,382 for 100,000.
+// A bead and tile cost 30 to 50 ps by boxes, whatever the order, and the grid
+// as much per bead as 300 to 900 tiles.
+constexpr int kWideTiles = 320;
 // Jobs of at most this many beads are stepped with their coordinates staged
 // in LDS (16 bytes per bead: 80 KB, two workgroups per CU).
 constexpr int kLdsStepBeads = 5120;

@@ -54,15 +54,19 @@ hipError_t launch_step(const DevJob* jobs, const StepDesc* descs, const StepDesc
                        const int2* units, const int4* segs, int nunits, int lds_beads, int kstep, int max_blocks,
                        hipStream_t stream, const StepShape& shape);
 // List rebuilds for jobs whose cadence is due (force != 0: rebuild all).
-// use_boxes: jobs with tile boxes build their possible list by them (0: every
-// job by the all-pairs scan).
+// boxes: jobs with tile boxes build their possible list by them (BOXES_NEAR) or,
+// the wide ones, by their cell grid (BOXES_WIDE, cell_words bitmap words --
+// ceil(n/64) -- of the largest); 0: every job by the all-pairs scan.
 // sunits/segs/nsunits/lds_beads: the LDS step plan (see launch_step), whose
 // jobs get their possible lists scanned from LDS-staged coordinates
 // (nsunits = 0: all jobs by the tile kernels); any_global: some job is
 // outside that plan (the tile kernel is launched only then).
-hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int use_boxes,
-                           int any_global, const int2* sunits, const int4* segs, int nsunits,
+enum { BOXES_NEAR = 1, BOXES_WIDE = 2 };
+hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int njobs, int boxes,
+                           int cell_words, int any_global, const int2* sunits, const int4* segs, int nsunits,
                            int lds_beads, int force, hipStream_t stream, const StepShape& shape);
+// Largest cell_words launch_possible accepts (the LDS bitmap of one wavefront).
+constexpr int kMaxCellWords = 8192;
 // The rows of units (job, first row) re-sorted by list length, where due.
 hipError_t launch_sort_rows(const DevJob* jobs, DevJobState* st, const int2* units, int nunits, int force,
                             hipStream_t stream, const StepShape& shape);

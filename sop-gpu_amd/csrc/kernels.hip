@@ -9,7 +9,7 @@
 //              beads in LDS.  Reference bodies: src/Potentials/covalent_kernel.cu:28-51,
 //              native_kernel.cu:27-52, pairs_kernel.cu:33-59,
 //              indentation_kernel.cu:71-128, src/Integrators/langevin_kernel.cu:17-58.
-// k_possible, k_possible_lds, k_possible_boxes
+// k_possible, k_possible_lds, k_possible_boxes, k_possible_cells
 //              possible-pairs list: same-job beads j != i, ascending j, with
 //              sqrtf(d^2) < threshold, excluding covalent and native partners
 //              (src/Updaters/possiblepairlist_kernel.cu:18-71).
@@ -40,7 +40,6 @@
 namespace sop {
 
 static constexpr int kTilesPerBlock = 4;  // 256-thread workgroups
-
 
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
@@ -1132,7 +1131,7 @@ __global__ __launch_bounds__(256) void k_tile_boxes(const DevJob* __restrict__ j
     for (int t = tr.begin; t < tr.end; t += tr.step) {
         const int2 td = tiles[t];
         const DevJob& J = jobs[td.x];
-        if (!J.tile_box) continue;
+        if (!J.tile_box || J.wide) continue;
         const long long s = st[td.x].step;
         if (!force && !due(J, s, J.pp_freq)) continue;
         const CoordGlobal cur{J.coord[s & 1]};
@@ -1160,13 +1159,13 @@ __global__ __launch_bounds__(256) void k_tile_boxes(const DevJob* __restrict__ j
 // capsid shell (32 A threshold, ~1,000 entries a bead) and 340 us for 100,000;
 // eight take 108 and 345 (too few wavefronts for the smaller), two 76 and 380.
 // Taking the candidates bead by bead from a cell grid and sorting the accepted
-// ones through a bitmap of the job's beads took 947 and 2,283 us.  Beads in no
-// spatial order along the chain make every box span the job and the scan
-// k_possible's (a rebuild of 18,000: 313 us, 621 by the grid; of 100,000: 5,386
-// and 2,342).
+// ones through a bitmap of the job's beads takes 947 and 2,283 us.  Beads in no
+// spatial order along the chain make every box span the job: past kWideTiles
+// tiles in reach such jobs take the grid (k_possible_cells).
 constexpr int kBoxBeads = 4;
 constexpr int kBoxAhead = 4;
 constexpr int kBoxList = 256;  // collected tiles before they are worked off
+constexpr int kBoxSample = 8;  // one group of beads in so many tiles is sampled
 __global__ __launch_bounds__(256) void k_possible_boxes(const DevJob* __restrict__ jobs,
                                                         DevJobState* __restrict__ st,
                                                         const int2* __restrict__ tiles, int ntiles, int force) {
@@ -1182,7 +1181,7 @@ __global__ __launch_bounds__(256) void k_possible_boxes(const DevJob* __restrict
     for (int h = xcd * slice + 4 * (int)(blockIdx.x / nxcd) + wv; h < hend; h += 4 * (nb / nxcd)) {
         const int2 td = tiles[h / kUnits];
         const DevJob& J = jobs[td.x];
-        if (!J.tile_box) continue;
+        if (!J.tile_box || J.wide) continue;
         const long long s = st[td.x].step;
         if (!force && !due(J, s, J.pp_freq)) continue;
         const int n = J.n, nt = (n + 63) >> 6;
@@ -1259,7 +1258,7 @@ __global__ __launch_bounds__(256) void k_possible_boxes(const DevJob* __restrict
                 cnt[b] += __popcll(m);
             }
         };
-        int m = 0;  // collected tiles
+        int m = 0, reached = 0;  // collected tiles, and all of them
         for (int c0 = 0; c0 < nt; c0 += 64) {
             const int cn = min(c0 + 64 + lane, nt - 1);
             const float4 lon = box[2 * cn], hin = box[2 * cn + 1];
@@ -1278,6 +1277,7 @@ __global__ __launch_bounds__(256) void k_possible_boxes(const DevJob* __restrict
                                                __builtin_amdgcn_mbcnt_lo((unsigned)some, (unsigned)m))] =
                     (unsigned)(c0 + lane) << 8 | mask;
             m += __popcll(some);
+            reached += __popcll(some);
             lo = lon;
             hi = hin;
             if (m == 0 || (m < kBoxList && c0 + 64 < nt)) continue;
@@ -1308,9 +1308,336 @@ __global__ __launch_bounds__(256) void k_possible_boxes(const DevJob* __restrict
         int total = cnt[0];
 #pragma unroll
         for (int b = 1; b < kBoxBeads; ++b) total = lane == b ? cnt[b] : total;
+        // a sample of the tiles that a group reaches, for the host's choice of the
+        // jobs that take the cell grid (Engine::judge_wide)
+        if (h % (kBoxSample * kUnits) == 0 && lane == 0) {
+            atomicAdd(&st[td.x].near_tiles, (unsigned long long)reached);
+            atomicAdd(&st[td.x].near_groups, 1ull);
+        }
         if (lane < nbead) {
             J.pp_cnt[i0 + lane] = min(total, cap);
             if (total > cap) atomicOr(&st[td.x].overflow, 1);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// possible pairs by a cell grid (large jobs of beads in no spatial order)
+// ---------------------------------------------------------------------------
+// The list of k_possible -- the same predicate on the same operands, the
+// same ascending-j order -- from the candidates in the 27 cells around the
+// bead, for the jobs whose beads lie in no spatial order along the chain
+// (J.wide): every box of 64 consecutive beads then spans the job, and
+// k_possible_boxes scans all pairs.  Cells are cubes of edge thr*(1+1e-4) +
+// 0.01 A + 2^-20 of the job's extent: a pair with sqrtf(d^2) < thr has every
+// |coordinate difference| within thr*(1 + 2^-21), and the cell index
+// (x - x0) / edge is computed with an error below the margin, so such a pair
+// always lies in adjacent cells.  Accepted j are set in a per-wave LDS bitmap
+// over the job's beads, the bead's exclusions cleared, and the bitmap read back
+// in index order with a wave prefix sum of popcounts.  Bound by the two LDS
+// atomics per accepted pair.  Measurements beside kWideTiles.
+
+__device__ __forceinline__ int cell_axis(float x, float org, float inv, int dim) {
+    const float q = (x - org) * inv;
+    if (!(q >= 0.0f)) return 0;  // below the grid, or NaN
+    if (q >= (float)dim) return dim - 1;
+    return min((int)q, dim - 1);
+}
+
+__device__ __forceinline__ int wave_min(int v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
+    return v;
+}
+__device__ __forceinline__ int wave_max(int v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
+    return v;
+}
+__device__ __forceinline__ int wave_inclusive_sum(int v, int lane) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(v, o);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
+// Per job (one 1024-thread block each): bounding box of the coordinates,
+// the grid (edge grown until the cell count fits cell_cap), zeroed counts.
+__global__ __launch_bounds__(1024) void k_cells_setup(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
+                                                      int njobs, int force) {
+    const int jb = blockIdx.x;
+    if (jb >= njobs) return;
+    const DevJob& J = jobs[jb];
+    if (!J.wide) return;
+    DevJobState& S = st[jb];
+    const long long s = S.step;
+    if (!force && !due(J, s, J.pp_freq)) return;
+    const float4* __restrict__ cur = J.coord[s & 1];
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int i = threadIdx.x; i < J.n; i += blockDim.x) {
+        const float4 r = cur[i];
+        lo[0] = fminf(lo[0], r.x), hi[0] = fmaxf(hi[0], r.x);
+        lo[1] = fminf(lo[1], r.y), hi[1] = fmaxf(hi[1], r.y);
+        lo[2] = fminf(lo[2], r.z), hi[2] = fmaxf(hi[2], r.z);
+    }
+    __shared__ float red[6][16];
+    __shared__ int dims[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        float a = lo[d], b = hi[d];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            a = fminf(a, __shfl_xor(a, o));
+            b = fmaxf(b, __shfl_xor(b, o));
+        }
+        if (lane == 0) {
+            red[d][w] = a;
+            red[3 + d][w] = b;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int nw = blockDim.x >> 6;
+        float org[3], ext[3];
+        for (int d = 0; d < 3; ++d) {
+            float a = red[d][0], b = red[3 + d][0];
+            for (int k = 1; k < nw; ++k) a = fminf(a, red[d][k]), b = fmaxf(b, red[3 + d][k]);
+            org[d] = a;
+            ext[d] = b - a;
+        }
+        int dm[3] = {1, 1, 1};
+        const bool finite = isfinite(ext[0]) && isfinite(ext[1]) && isfinite(ext[2]);
+        // the last term covers the rounding of x - x0 and of its product
+        float edge = J.pp_thr * 1.0001f + 0.01f + 0x1p-20f * fmaxf(fmaxf(ext[0], ext[1]), ext[2]);
+        if (finite) {
+            for (int it = 0; it < 200; ++it) {
+                double cells = 1.0;
+                for (int d = 0; d < 3; ++d) cells *= floor((double)ext[d] / edge) + 1.0;
+                if (cells <= (double)J.cell_cap) break;
+                edge *= 1.1f;
+            }
+            for (int d = 0; d < 3; ++d) dm[d] = (int)floor((double)ext[d] / edge) + 1;
+            if ((long long)dm[0] * dm[1] * dm[2] > J.cell_cap) dm[0] = dm[1] = dm[2] = 1;
+        } else {
+            org[0] = org[1] = org[2] = 0.0f;
+        }
+        for (int d = 0; d < 3; ++d) {
+            S.cell_org[d] = org[d];
+            S.cell_dim[d] = dm[d];
+        }
+        S.cell_inv = 1.0f / edge;
+        dims[0] = dm[0] * dm[1] * dm[2];
+    }
+    __syncthreads();
+    const int nc = dims[0];
+    for (int c = threadIdx.x; c < nc; c += blockDim.x) J.cell_cnt[c] = 0;
+}
+
+// Each bead's cell and its slot there (the order within a cell is free:
+// the bitmap restores index order).
+__global__ __launch_bounds__(256) void k_cells_count(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
+                                                     const int2* __restrict__ tiles, int ntiles, int force) {
+    const int lane = threadIdx.x & 63;
+    const TileRange tr = xcd_tiles(ntiles);
+    for (int t = tr.begin; t < tr.end; t += tr.step) {
+        const int2 td = tiles[t];
+        const DevJob& J = jobs[td.x];
+        if (!J.wide) continue;
+        const DevJobState& S = st[td.x];
+        const long long s = S.step;
+        if (!force && !due(J, s, J.pp_freq)) continue;
+        const int i = td.y + lane;
+        if (i >= J.n) continue;
+        const float4 r = J.coord[s & 1][i];
+        const int cx = cell_axis(r.x, S.cell_org[0], S.cell_inv, S.cell_dim[0]);
+        const int cy = cell_axis(r.y, S.cell_org[1], S.cell_inv, S.cell_dim[1]);
+        const int cz = cell_axis(r.z, S.cell_org[2], S.cell_inv, S.cell_dim[2]);
+        const int c = (cz * S.cell_dim[1] + cy) * S.cell_dim[0] + cx;
+        J.bead_cell[i] = c;
+        J.bead_slot[i] = atomicAdd(&J.cell_cnt[c], 1);
+    }
+}
+
+// Exclusive scan of the cell counts (one 1024-thread block per job).
+__global__ __launch_bounds__(1024) void k_cells_scan(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
+                                                     int njobs, int force) {
+    const int jb = blockIdx.x;
+    if (jb >= njobs) return;
+    const DevJob& J = jobs[jb];
+    if (!J.wide) return;
+    const DevJobState& S = st[jb];
+    if (!force && !due(J, S.step, J.pp_freq)) return;
+    const int nc = S.cell_dim[0] * S.cell_dim[1] * S.cell_dim[2];
+    const int per = (nc + blockDim.x - 1) / blockDim.x;
+    const int b = threadIdx.x * per, e = min(b + per, nc);
+    int sum = 0;
+    for (int c = b; c < e; ++c) sum += J.cell_cnt[c];
+    __shared__ int part[1024];
+    part[threadIdx.x] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int acc = 0;
+        for (int k = 0; k < (int)blockDim.x; ++k) {
+            const int v = part[k];
+            part[k] = acc;
+            acc += v;
+        }
+    }
+    __syncthreads();
+    int acc = part[threadIdx.x];
+    for (int c = b; c < e; ++c) {
+        J.cell_start[c] = acc;
+        acc += J.cell_cnt[c];
+    }
+    if (threadIdx.x == 0) J.cell_start[nc] = J.n;
+}
+
+__global__ __launch_bounds__(256) void k_cells_fill(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
+                                                    const int2* __restrict__ tiles, int ntiles, int force) {
+    const int lane = threadIdx.x & 63;
+    const TileRange tr = xcd_tiles(ntiles);
+    for (int t = tr.begin; t < tr.end; t += tr.step) {
+        const int2 td = tiles[t];
+        const DevJob& J = jobs[td.x];
+        if (!J.wide) continue;
+        if (!force && !due(J, st[td.x].step, J.pp_freq)) continue;
+        const int i = td.y + lane;
+        if (i >= J.n) continue;
+        J.cell_beads[J.cell_start[J.bead_cell[i]] + J.bead_slot[i]] = i;
+    }
+}
+
+// One 64-thread workgroup (one wavefront) per tile; dynamic LDS holds the
+// bitmap of ceil(n/64) words for the largest cell-binned job.
+// One wavefront per half tile (32 beads), its beads one after another.  A bead's
+// candidates (the 3 x 3 rows of three x-adjacent cells, each row one
+// contiguous range of cell_beads) are read eight 64-entry chunks at a time,
+// all index loads and then all coordinate gathers in flight together; the
+// next bead's coordinates and first 64 exclusions are loaded while this one
+// is scanned.  Accepted j set bit j of the LDS bitmap bm and bit j / 64 of
+// bm2, so the read-back in index order visits only the 64-word blocks of bm
+// that hold an entry.
+constexpr int kCellChunks = 8;
+__global__ __launch_bounds__(64) void k_possible_cells(const DevJob* __restrict__ jobs, DevJobState* __restrict__ st,
+                                                       const int2* __restrict__ tiles, int ntiles, int force,
+                                                       int cell_words) {
+    extern __shared__ unsigned long long bm[];
+    unsigned long long* const bm2 = bm + cell_words;  // one bit per word of bm
+    const int lane = threadIdx.x;
+    const int nb = gridDim.x, nxcd = nb >= 8 ? 8 : 1;
+    const int nhalf = 2 * ntiles;  // work units: the two halves of every tile
+    const int slice = (nhalf + nxcd - 1) / nxcd;
+    const int xcd = blockIdx.x % nxcd;
+    const int hend = min((xcd + 1) * slice, nhalf);
+    for (int h = xcd * slice + blockIdx.x / nxcd; h < hend; h += nb / nxcd) {
+        const int2 td = tiles[h >> 1];
+        const DevJob& J = jobs[td.x];
+        if (!J.wide) continue;
+        const DevJobState& S = st[td.x];
+        const long long s = S.step;
+        if (!force && !due(J, s, J.pp_freq)) continue;
+        const int n = J.n;
+        const int i0 = td.y + 32 * (h & 1);
+        if (i0 >= n) continue;
+        const int nwords = (n + 63) >> 6;
+        for (int w = lane; w < nwords; w += 64) bm[w] = 0ull;
+        for (int w = lane; w < (nwords + 63) >> 6; w += 64) bm2[w] = 0ull;
+        __syncthreads();
+        const CoordGlobal cur{J.coord[s & 1]};
+        const auto cbeads = gmem(J.cell_beads);
+        const auto cstart = gmem(J.cell_start);
+        const auto ecnt = gmem(J.excl_cnt);
+        const auto ej = gmem(J.excl_j);
+        const float d2max = J.pp_d2;
+        const int cap = J.pp_cap, ecap = J.excl_cap;
+        const int dx = S.cell_dim[0], dy = S.cell_dim[1], dz = S.cell_dim[2];
+        const int iend = min(i0 + 32, n);
+        float4 r1n = cur[i0];
+        int nen = ecnt[i0];
+        int evn = ej[(size_t)min(lane, ecap - 1) * n + i0];
+        for (int i = i0; i < iend; ++i) {
+            const float4 r1 = r1n;
+            const int ne = nen, ev = evn;
+            if (i + 1 < iend) {
+                r1n = cur[i + 1];
+                nen = ecnt[i + 1];
+                evn = ej[(size_t)min(lane, ecap - 1) * n + i + 1];
+            }
+            const int cx = cell_axis(r1.x, S.cell_org[0], S.cell_inv, dx);
+            const int cy = cell_axis(r1.y, S.cell_org[1], S.cell_inv, dy);
+            const int cz = cell_axis(r1.z, S.cell_org[2], S.cell_inv, dz);
+            int jlo = INT_MAX, jhi = -1;
+            for (int z = max(cz - 1, 0); z <= min(cz + 1, dz - 1); ++z)
+                for (int y = max(cy - 1, 0); y <= min(cy + 1, dy - 1); ++y) {
+                    const int row = (z * dy + y) * dx;
+                    // the cells x-1..x+1 of one row are contiguous in cell_beads
+                    const int b = cstart[row + max(cx - 1, 0)];
+                    const int e = cstart[row + min(cx + 1, dx - 1) + 1];
+                    for (int k0 = b; k0 < e; k0 += 64 * kCellChunks) {
+                        int jj[kCellChunks];
+#pragma unroll
+                        for (int u = 0; u < kCellChunks; ++u) {
+                            const int k = k0 + 64 * u + lane;
+                            jj[u] = k < e ? cbeads[k] : i;  // past the range: the bead itself, skipped
+                        }
+                        float4 r2[kCellChunks];
+#pragma unroll
+                        for (int u = 0; u < kCellChunks; ++u) r2[u] = cur[jj[u]];
+#pragma unroll
+                        for (int u = 0; u < kCellChunks; ++u) {
+                            const int j = jj[u];
+                            const float x = r2[u].x - r1.x, y2 = r2[u].y - r1.y, z2 = r2[u].z - r1.z;
+                            if (j != i && x * x + y2 * y2 + z2 * z2 <= d2max) {
+                                atomicOr(&bm[j >> 6], 1ull << (j & 63));
+                                atomicOr(&bm2[j >> 12], 1ull << ((j >> 6) & 63));
+                                jlo = min(jlo, j);
+                                jhi = max(jhi, j);
+                            }
+                        }
+                    }
+                }
+            __syncthreads();
+            for (int k = lane; k < ne; k += 64) {
+                const int e = k < 64 ? ev : ej[(size_t)k * n + i];
+                atomicAnd(&bm[e >> 6], ~(1ull << (e & 63)));
+            }
+            __syncthreads();
+            jlo = wave_min(jlo);
+            jhi = wave_max(jhi);
+            int cnt = 0;
+            const size_t rowp = (size_t)i * J.pp_ld;
+            if (jhi >= 0) {
+                const int wlo = jlo >> 6, whi = jhi >> 6;
+                for (int wb = wlo & ~63; wb <= whi; wb += 64) {
+                    const unsigned long long m2 = bm2[wb >> 6];
+                    if (m2 == 0ull) continue;  // no entry in these 64 words
+                    const int w = wb + lane;
+                    unsigned long long word = 0ull;
+                    if ((m2 >> lane) & 1ull) {
+                        word = bm[w];
+                        bm[w] = 0ull;
+                    }
+                    const int pc = __popcll(word);
+                    const int incl = wave_inclusive_sum(pc, lane);
+                    int pos = cnt + incl - pc;
+                    while (word) {
+                        const int j = (w << 6) + __builtin_ctzll(word);
+                        if (pos < cap) list_put(J.pp_j, J.idx16, rowp + pos, j);
+                        ++pos;
+                        word &= word - 1ull;
+                    }
+                    cnt += __shfl(incl, 63);
+                    if (lane == 0) bm2[wb >> 6] = 0ull;
+                }
+            }
+            __syncthreads();
+            if (lane == 0) {
+                J.pp_cnt[i] = cnt < cap ? cnt : cap;
+                if (cnt > cap) atomicOr(&st[td.x].overflow, 1);
+            }
         }
     }
 }
@@ -2131,10 +2458,11 @@ hipError_t launch_forces(const DevJob* jobs, const StepDesc* descs, const StepDe
     return hipGetLastError();
 }
 
-hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int use_boxes,
-                           int any_global, const int2* sunits, const int4* segs, int nsunits,
+hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tiles, int ntiles, int njobs, int boxes,
+                           int cell_words, int any_global, const int2* sunits, const int4* segs, int nsunits,
                            int lds_beads, int force, hipStream_t stream, const StepShape& shape) {
     if (ntiles <= 0) return hipSuccess;
+    const int use_boxes = boxes != 0;
     if (any_global || nsunits <= 0)
         hipLaunchKernelGGL(k_possible, dim3(grid_for(ntiles, 0)), dim3(256), 0, stream, jobs, st, tiles, ntiles,
                            force, use_boxes, nsunits > 0);
@@ -2144,11 +2472,22 @@ hipError_t launch_possible(const DevJob* jobs, DevJobState* st, const int2* tile
     else if (nsunits > 0)
         hipLaunchKernelGGL(k_possible_lds, dim3(nsunits), dim3(kLdsUnit), (size_t)lds_beads * sizeof(float4), stream,
                            jobs, st, sunits, segs, nsunits, force, use_boxes);
-    if (use_boxes) {
+    auto of_xcds = [](int blocks) { return blocks >= 8 ? (blocks + 7) / 8 * 8 : blocks; };
+    if (boxes & BOXES_NEAR) {
         hipLaunchKernelGGL(k_tile_boxes, dim3(grid_for(ntiles, 0)), dim3(256), 0, stream, jobs, st, tiles, ntiles, force);
-        int blocks = 64 / kBoxBeads / 4 * ntiles;
-        if (blocks >= 8) blocks = (blocks + 7) / 8 * 8;
-        hipLaunchKernelGGL(k_possible_boxes, dim3(blocks), dim3(256), 0, stream, jobs, st, tiles, ntiles, force);
+        hipLaunchKernelGGL(k_possible_boxes, dim3(of_xcds(64 / kBoxBeads / 4 * ntiles)), dim3(256), 0, stream, jobs, st,
+                           tiles, ntiles, force);
+    }
+    if (boxes & BOXES_WIDE) {
+        const dim3 g(grid_for(ntiles, 0)), b(256);
+        hipLaunchKernelGGL(k_cells_setup, dim3(njobs), dim3(1024), 0, stream, jobs, st, njobs, force);
+        hipLaunchKernelGGL(k_cells_count, g, b, 0, stream, jobs, st, tiles, ntiles, force);
+        hipLaunchKernelGGL(k_cells_scan, dim3(njobs), dim3(1024), 0, stream, jobs, st, njobs, force);
+        hipLaunchKernelGGL(k_cells_fill, g, b, 0, stream, jobs, st, tiles, ntiles, force);
+        // one wavefront per half tile
+        hipLaunchKernelGGL(k_possible_cells, dim3(of_xcds(2 * ntiles)), dim3(64),
+                           (size_t)(cell_words + (cell_words + 63) / 64) * 8, stream, jobs, st, tiles, ntiles, force,
+                           cell_words);
     }
     return hipGetLastError();
 }

@@ -1,0 +1,171 @@
+"""Possible pairs of large jobs whose beads are in no spatial order along the
+chain, where the boxes of 64 consecutive beads span the job: taken from a cell
+grid (the list itself: src/Updaters/possiblepairlist_kernel.cu:18-71).
+Entries, order, counts and the overflow flag are the all-pairs scan's, at the
+smallest such job, for coordinates that are not finite or far apart, beside
+jobs of both other kinds and as the order of a job changes; and a rebuild
+takes a fraction of the all-pairs scan's time, also where the job's beads
+were in order when it was admitted."""
+import time
+
+import numpy as np
+import pytest
+
+import sopgpu as S
+from helpers import c0_params
+
+pytestmark = pytest.mark.gpu
+
+KW = dict(pairs_threshold=16.0, pairs_cutoff=16.0, pairlist_cutoff=16.0, max_possiblePairs=512)
+
+
+def _shell(n, shuffled=True, seed=5):
+    chains = -(-n // 500)
+    sysm = S.synth_shell(chains, 500, seed=seed, radius=140.0 * (chains * 500 / 1e5) ** 0.5)
+    if shuffled:
+        sysm.coords = np.ascontiguousarray(sysm.coords[np.random.default_rng(seed).permutation(sysm.n)])
+    return sysm
+
+
+def _list(e, j):
+    e.rebuild(j, 3)
+    cnt, ent = e.list(j, 3)
+    m = int(cnt.max())
+    return e.status(j)[2], cnt, np.where(np.arange(m)[:, None] < cnt[None, :], ent[:m], -1)
+
+
+def _equal(a, b):
+    assert a[0] == b[0]
+    np.testing.assert_array_equal(a[1], b[1])
+    np.testing.assert_array_equal(a[2], b[2])
+
+
+def _both(sysm, **kw):
+    with S.Engine(0, 16 << 30) as e:
+        j = e.add_job(S.make_params(**c0_params(**dict(KW, **kw))), sysm, 0)
+        a = _list(e, j)
+    with S.Engine(0, 16 << 30) as e:
+        e.set_cells(enabled=False)
+        j = e.add_job(S.make_params(**c0_params(**dict(KW, **kw))), sysm, 0)
+        _equal(a, _list(e, j))
+    return a
+
+
+@pytest.mark.parametrize("n,kw", [(20500, {}), (30000, dict(pairs_threshold=32.0, max_possiblePairs=1024)),
+                                  (70000, {}), (24000, dict(max_possiblePairs=64))],
+                         ids=["20500", "30000-32A", "70000-int32", "overflow"])
+def test_lists(n, kw):
+    print("case: %d beads in no order, %r" % (n, kw), flush=True)
+    flag, cnt, _ = _both(_shell(n), **kw)
+    assert (flag & 1) == (kw.get("max_possiblePairs") == 64) and cnt.max() > 40
+
+
+@pytest.mark.parametrize("what", ["nan", "inf", "far", "stretched"])
+def test_coordinates(what):
+    sysm = _shell(24000)
+    c = sysm.coords
+    if what == "far":
+        c[5, 0] = 1e7
+        c[700, :3] = (-3e6, 1e5, 2e7)
+    elif what == "stretched":  # cells of the last bits of the coordinates: 3e6 A long
+        c[:, 0] += np.float32(3e6 / sysm.n) * np.random.default_rng(1).permutation(sysm.n).astype(np.float32)
+        c[: sysm.n // 2, 0] = c[sysm.n // 2:, 0] + np.float32(15.75)
+        c[:, 1:3] = 0.0
+    else:
+        c[70, 0] = float(what)
+        c[128:192, 1] = float(what)
+    print("case: coordinates %s" % what, flush=True)
+    _both(sysm)
+
+
+def _renumbered(sysm, seed):
+    """The same system with its beads numbered in no order."""
+    inv = np.random.default_rng(seed).permutation(sysm.n).astype(np.int32)  # bead i becomes inv[i]
+    c = np.empty_like(sysm.coords)
+    c[inv] = sysm.coords
+    sysm.coords, sysm.bonds, sysm.natives = c, inv[sysm.bonds], inv[sysm.natives]
+    return sysm
+
+
+def test_beside_other_jobs():
+    """A job in no order, one in order and a small one, batched, then the
+    first alone."""
+    out = []
+    for on in (True, False):
+        systems = [_renumbered(_shell(21000, False, 7), 1), _shell(21000, False, 8), S.synth_chain(300, seed=9)]
+        with S.Engine(0, 30 << 30) as e:
+            e.set_cells(enabled=on)
+            ids = [e.add_job(S.make_params(**c0_params(seed=40 + k, temperature=0.6, **KW)), s, 290)
+                   for k, s in enumerate(systems)]
+            print("case: three jobs, boxes %s" % on, flush=True)
+            e.run_blocks(21)
+            got = [x for j in ids for x in (e.coords(j), np.array(e.status(j)))] + [_list(e, j)[2] for j in ids]
+            print("case: the first alone, boxes %s" % on, flush=True)
+            e.run_job(ids[0])
+            out.append(got + [e.coords(ids[0]), np.array(e.status(ids[0]))])
+    assert np.isfinite(out[0][0]).all()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_as_the_order_changes():
+    """Coordinates set in no order and in order again, in two jobs by turns."""
+    order = _shell(21000, False).coords
+    none = np.ascontiguousarray(order[np.random.default_rng(2).permutation(len(order))])
+    out = []
+    for on in (True, False):
+        with S.Engine(0, 30 << 30) as e:
+            e.set_cells(enabled=on)
+            ids = [e.add_job(S.make_params(**c0_params(**KW)), _shell(21000, sh), 0) for sh in (False, True)]
+            got = []
+            for k, pair in enumerate([(order, none), (none, none), (none, order), (order, order), (none, none)]):
+                print("case: change %d, boxes %s" % (k, on), flush=True)
+                for j, c in zip(ids, pair):
+                    e.set_coords(j, c)
+                got += [_list(e, j) for j in ids]
+            out.append(got)
+    for a, b in zip(*out):
+        _equal(a, b)
+
+
+def _time(e, j):
+    e.rebuild(j, 1)
+    best = 1e9
+    for _ in range(5):
+        a = time.perf_counter()
+        e.rebuild(j, 1)
+        best = min(best, time.perf_counter() - a)
+    return best
+
+
+def test_rebuild_time():
+    """60,000 beads: 0.57 ms of the all-pairs scan's 8.1; every box in reach,
+    1.9 ms.  The line is 15 %."""
+    with S.Engine(0, 16 << 30) as e:
+        j = e.add_job(S.make_params(**c0_params(**KW)), _shell(60000), 0)
+        grid = _time(e, j)
+        e.set_cells(enabled=False)
+        pairs = _time(e, j)
+    print("case: rebuild %.0f us, all pairs %.0f" % (grid * 1e6, pairs * 1e6), flush=True)
+    assert grid < 0.15 * pairs
+
+
+def test_order_lost_unseen_by_the_host():
+    """The tiles that the host looks at when the job is admitted are small
+    clusters apart, all the others in no order: the first build shows the tiles
+    really reached, the read of the state acts on it."""
+    sysm = _shell(60000)
+    nt = (sysm.n + 63) // 64
+    for k in range(32):
+        b = 64 * (k * nt // 32)
+        sysm.coords[b:b + 64, :3] = np.random.default_rng(k).normal(size=(64, 3)) * 4.0 + (600.0 + 60.0 * k, 0.0, 0.0)
+    with S.Engine(0, 16 << 30) as e:
+        j = e.add_job(S.make_params(**c0_params(**KW)), sysm, 0)
+        first = _time(e, j)
+        a = _list(e, j)  # reads the state
+        then = _time(e, j)
+        _equal(a, _list(e, j))
+        e.set_cells(enabled=False)
+        _equal(a, _list(e, j))
+    print("case: rebuild %.0f us, then %.0f" % (first * 1e6, then * 1e6), flush=True)
+    assert then < 0.6 * first
