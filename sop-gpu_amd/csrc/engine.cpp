@@ -1759,8 +1759,9 @@ int Engine::compute_forces(int id, float* out4) {
         if (int rc = check(hipMalloc(&d_scratch4_, (size_t)hj.n * 16), "scratch")) return rc;
         scratch4_n_ = hj.n;
     }
-    // the step kernel the job is stepped by (LDS or global gathers), in its
-    // forces-only instantiation, over the job's own tiles / units
+    // the step kernel of the job by itself (run_job's; in a batch the job may
+    // be stepped by another, with the same bits), in its forces-only
+    // instantiation, over the job's own tiles / units
     int nt = 0;
     if (int rc = tiles_for_slot(slot, &nt)) return rc;
     const bool lds = hj.dj.lds_step != 0;

@@ -288,9 +288,6 @@ struct HiPairBase {
     const float4* __restrict__ cur;
     float4 c[2];
     float a;
-    struct Src {
-        float4 r;
-    };
     __device__ __forceinline__ void sep(int k, const float4 r, float& x, float& y, float& z) const {
         x = r.x - c[k].x;
         y = r.y - c[k].y;
@@ -393,7 +390,7 @@ __global__ __launch_bounds__(64 * B) void k_hi_eps(const DevJob* __restrict__ jo
         J.eps[d] = sum.w;
         return;
     }
-    // unlisted: lanes 16c + b of wavefront 0 sum component c of bead dbase + b
+    // unlisted: lanes B c + b of wavefront 0 sum component c of bead dbase + b
     const int dbase = td.y + B * q;
     int bb[2];
     hi_beads<B>(dbase, n, bb);
@@ -404,7 +401,7 @@ __global__ __launch_bounds__(64 * B) void k_hi_eps(const DevJob* __restrict__ jo
     pair.c[1] = ld4(cur, bb[1]);
     float acc = 0.f;
     hi_ordered_sums<B, C, 4>(eterm, n, bb, pair, acc);
-    // component c of bead dbase + b is in lane 16c + b of wavefront 0
+    // component c of bead dbase + b is in lane B c + b of wavefront 0
     const float sy = __shfl(acc, lane + B), sz = __shfl(acc, lane + 2 * B), sw = __shfl(acc, (lane + 3 * B) & 63);
     if (w == 0 && lane < B && dbase + lane < n) {
         J.ci[dbase + lane] = make_float4(acc, sy, sz, sw);
@@ -586,7 +583,7 @@ __global__ __launch_bounds__(64 * B) void k_hi_tea(const DevJob* __restrict__ jo
         return;
     }
     // unlisted: the wavefront's two beads with their ci (uniform over the
-    // wavefront); lanes 16c + b of wavefront 0 sum component c of bead dbase + b
+    // wavefront); lanes B c + b of wavefront 0 sum component c of bead dbase + b
     // from its starting value
     const int dbase = td.y + B * q, ds = dbase + lane % B;
     int bd[2];
@@ -606,7 +603,7 @@ __global__ __launch_bounds__(64 * B) void k_hi_tea(const DevJob* __restrict__ jo
         pair.c[k] = ld4(cur, bd[k]);
     }
     float acc = 0.f;
-    if (w == 0 && lane < 3 * B && ds < n) {  // the bead's starting value, component lane / 16
+    if (w == 0 && lane < 3 * B && ds < n) {  // the bead's starting value, component lane / B
         const float4 cs = J.ci[ds], f0 = J.mforce[ds], df = J.rforce[ds];
         const float bb = S.beta * S.beta;
         const int k = lane / B;
@@ -767,8 +764,7 @@ static constexpr int NB2 = kCholPanel;  // outer panel: depth of the trailing up
 // another -- 32 floats (FP32), or 32 bf16 hi parts followed by the 32 lo
 // parts (split-BF16).  A wavefront that reads 16 rows of a chunk reads 2 KB on
 // end; from rows a kilobyte or a matrix row apart the same operands came from
-// a few L2 channels at a quarter of the rate (the row blocks' update of 960
-// columns: 19 us).
+// a few L2 channels at a quarter of the rate (an update of 960 columns: 19 us).
 __device__ __forceinline__ size_t panel_rec(size_t mp, int chunk, size_t row) {
     return ((size_t)chunk * mp + row) * kCholRecord;
 }
@@ -1199,12 +1195,12 @@ __global__ __launch_bounds__(256, 2) void k_update(float* __restrict__ M, size_t
 // diagonal block):
 //  (1) for j >= 1, each row block's solve against column block j-1:
 //      X_g = B_g Li^T with B_g the block as the previous step left it and
-//      Li^T the inverse of L_{j-1,j-1} (FP64 accumulation), written to M and,
-//      split-BF16 mode, to the panel copy;
+//      Li^T the inverse of L_{j-1,j-1} (accumulated in CholReal), written to M
+//      and to the panel copy;
 //  (2) for j < nb, column block j of each row block minus the products of
 //      this panel's columns 0 .. 64j-1, on MFMA:
 //      B_g = A_gj - sum_k X_gk X_dk^T.  Workgroup 0 (g = d) factors B in
-//      FP64 into L_jj and its inverse; the others store B for step j+1.
+//      CholReal into L_jj and its inverse; the others store B for step j+1.
 // Every workgroup forms X_d for (2) itself (the diagonal row block's solve,
 // the same arithmetic as workgroup 0's), so no workgroup waits for another.
 // Lookahead: the diagonal workgroup's chain (solve, update, factor, inverse)
@@ -1427,7 +1423,7 @@ __device__ __forceinline__ void mfma_lds(f32x4 (&acc)[2], const float* __restric
             for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[t], acc[t], 0, 0, 0);
         }
     } else {
-        const int lg = l >> 4;  // k = kc+4g .. kc+4g+3, as in mfma_rows
+        const int lg = l >> 4;  // k = kc+4g .. kc+4g+3
 #pragma unroll
         for (int kc = 0; kc < NB; kc += 16) {
             const float4 a = *reinterpret_cast<const float4*>(Xg + (16 * w + lr) * XS + kc + 4 * lg);
@@ -1446,9 +1442,10 @@ __device__ __forceinline__ void mfma_lds(f32x4 (&acc)[2], const float* __restric
     }
 }
 
-// Eight wavefronts: with four, one per SIMD, the row blocks' long update (up
-// to 960 columns) waited for its operands and outlasted the diagonal
-// workgroup's chain (row blocks 20-25 us a step, the diagonal 18).
+// Eight wavefronts: with four, one per SIMD, the row blocks' long update
+// waited for its operands and outlasted the diagonal workgroup's chain (row
+// blocks 20-25 us a step, the diagonal 18, while the update still reached over
+// the panel before as well, up to 960 columns; now it is at most 384).
 template <int MODE>
 __global__ __launch_bounds__(kCholThreads) void k_chol_step(CholStep a) {
     using R = CholReal<MODE>;

@@ -9,6 +9,12 @@
 //              beads in LDS.  Reference bodies: src/Potentials/covalent_kernel.cu:28-51,
 //              native_kernel.cu:27-52, pairs_kernel.cu:33-59,
 //              indentation_kernel.cu:71-128, src/Integrators/langevin_kernel.cu:17-58.
+// k_step_rows, k_step_rows_one
+//              the same step with each bead's force terms spread over the lanes
+//              of a wavefront, for launches of too few beads for one per lane;
+//              the latter for launches of a single job.
+// k_block_rows the steps of a block of small jobs in one launch, a workgroup
+//              per job, with the updaters and Verlet lists it begins with.
 // k_possible, k_possible_lds, k_possible_boxes, k_possible_cells
 //              possible-pairs list: same-job beads j != i, ascending j, with
 //              sqrtf(d^2) < threshold, excluding covalent and native partners
@@ -204,9 +210,6 @@ __device__ __forceinline__ void ext_rules_flag(const D& J, int i, int f, float& 
         const float4 e = J.ext[i];
         fx += e.x; fy += e.y; fz += e.z;
     }
-}
-__device__ __forceinline__ void ext_rules(const DevJob& J, int i, float& fx, float& fy, float& fz) {
-    ext_rules_flag(J, i, J.bflag[i], fx, fy, fz);
 }
 
 // FENE (covalent_kernel.cu:36-48) and native LJ 12-6 (native_kernel.cu:36-49)
@@ -2144,12 +2147,13 @@ __device__ __forceinline__ void verlet_few(const DevJob& J, DevJobState& S, cons
 // k_step_rows' chain only the sums are left: lists and generators stay in
 // registers, partners come from LDS.  Bound by the latency of its dependent
 // operations: 560 vector instructions a step and wavefront in ~9,000 cycles, at
-// one or two wavefronts a SIMD.  ldc: beads of the launch's largest job; advance: what the block's last launch adds to the
-// step counters (in the place of k_job_advance), 0 for none.  350 peptides of
-// 22 beads, a block of ten steps: 37 us, 75 as ten launches of k_step_rows and
-// the gaps between them.  begin (BLOCK_*): what the block begins with here, in
-// the place of k_job_update (but for the tip) and k_verlet_split: 3 us more, for
-// the 12 of the two launches.
+// one or two wavefronts a SIMD.  ldc: beads of the launch's largest job;
+// advance: what the block's last launch adds to the step counters (in the place
+// of k_job_advance), 0 for none.  350 peptides of 22 beads, a block of ten
+// steps: 37 us, 75 as ten launches of k_step_rows and the gaps between them.
+// begin (BLOCK_*): what the block begins with here, in the place of k_job_update
+// (but for the tip) and k_verlet_split: 3 us more, for the 12 of the two
+// launches.
 template <int R>
 __global__ __launch_bounds__(1024) void k_block_rows(const DevJob* __restrict__ jobs,
                                                      const StepDesc* __restrict__ descs,

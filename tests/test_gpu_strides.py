@@ -27,7 +27,8 @@ HEAT = dict(heating=1, initialT=0.3, deltaT=0.05)
 
 # block lengths 5, 1 and (longer than one launch) 300
 @pytest.mark.parametrize("jobs,L", [
-    ([(22, 10, 100, dict(HEAT, tempFreq=20)), (30, 15, 200, {}), (7, 10, 60, {}), (25, 35, 280, dict(HEAT, tempFreq=35))], 5),
+    ([(22, 10, 100, dict(HEAT, tempFreq=20)), (30, 15, 200, {}), (7, 10, 60, {}),
+      (25, 35, 280, dict(HEAT, tempFreq=35))], 5),
     ([(22, 7, 70, dict(HEAT, tempFreq=14)), (9, 10, 120, {})], 1),
     ([(22, 300, 900, {}), (12, 600, 1200, dict(HEAT, tempFreq=600))], 300),
 ], ids=["5", "1", "300"])
