@@ -957,7 +957,10 @@ int Engine::sync_tables() {
 //   7,700 of peptides (22 beads)    11 /  10 / 7.9 / 7.8,  21
 // Few rows want many wavefronts; many rows want few instructions per row.
 // Lists as short as the peptides' leave most of a 4-row wavefront's positions
-// empty.
+// empty.  Around kRowsShort (28 beads), us per step of whole blocks, R = 4 | 8:
+//   beads x jobs   24 x 99     24 x 350    29 x 99     40 x 99     64 x 99     64 x 350
+//                  6.1 | 6.3   11.2 | 8.4  8.0 | 6.5   8.2 | 6.8   7.0 | 7.7   12.9 | 10.7
+// (jobs of up to kBlockShort beads take these only beside larger ones).
 StepShape Engine::effective_shape(int first, int count) const {
     StepShape e = shape_;
     long long lds_rows = 0, global_rows = 0, short_rows = 0;  // short_rows: of jobs of at most kRowsShort beads
@@ -991,6 +994,14 @@ StepShape Engine::effective_shape(int first, int count) const {
 //   100 x          7.3 | 8.3  8.3 | 8.8  14.7 | 10.9, 12.1  20.0 | 19.9, 16.3  45 | 40, 32
 //   150 x 8        7.6 | -, 11.1   128: 13.4 | -, 12.8   512: 32.7 | -, 26.9
 //   250 x 32       9.5 | -, 15.2   128: 17.6 | -, 17.5   512: 59.4 | -, 41.5
+// Around kBlockShort (32 beads) and kBlockJobs, whole blocks, the best launch
+// per step | the block:
+//   beads x jobs   1             20            99            350           1,000
+//   28             5.1 | 3.5     5.5 | 3.6     6.2 | 3.7     8.5 | 4.5     12.4 | 7.0
+//   33             5.3 | 3.9     6.0 | 4.0     6.9 | 4.1     9.0 | 5.4     14.5 | 14.0
+//   40             5.4 | 3.9     6.1 | 4.1     6.8 | 4.2     9.3 | 5.8     15.6 | 8.3
+//   64             5.8 | 5.8     6.1 | 6.0     7.0 | 6.2     10.7 | 8.8    20.6 | 12.8
+//   99             6.2 | 7.3     7.1 | 7.6     9.5 | 7.9     17.0 | 11.3   38.6 | 23.1
 int Engine::block_rows(int first, int count, int* beads) const {
     long long rows = 0;
     int most = 0;
