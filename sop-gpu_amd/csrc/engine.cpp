@@ -503,31 +503,37 @@ static bool uses_grid(size_t n) { return n > (size_t)64 * kWideTiles && n <= (si
 
 // The tiles of 64 beads that a bead reaches (boxes within the threshold, d2max)
 // on average, from 32 beads and 32 tiles spread over the job (a few
-// microseconds, beside a copy of the coordinates).
-static double tiles_in_reach(const float4* c, int n, float d2max) {
+// microseconds, beside a copy of the coordinates).  c: four floats a bead, a
+// caller's, aligned as floats are.
+static double tiles_in_reach(const float* c, int n, float d2max) {
     constexpr int kSample = 32;
     const int nt = (n + 63) / 64, S = std::min(nt, kSample);
     if (S < 2) return nt;
-    float4 lo[kSample], hi[kSample], p[kSample];
+    float lo[kSample][3], hi[kSample][3], p[kSample][3];
     auto lower = [](float x, float l) { return x < l ? x : l; };  // l where x is not a number
     auto upper = [](float x, float h) { return x > h ? x : h; };
     for (int k = 0; k < S; ++k) {
         const int b = 64 * (int)((long long)k * nt / S), e = std::min(b + 64, n);
-        float4 l{INFINITY, INFINITY, INFINITY, 0.0f}, h{-INFINITY, -INFINITY, -INFINITY, 0.0f};
-        for (int i = b; i < e; ++i) {
-            l.x = lower(c[i].x, l.x), h.x = upper(c[i].x, h.x);
-            l.y = lower(c[i].y, l.y), h.y = upper(c[i].y, h.y);
-            l.z = lower(c[i].z, l.z), h.z = upper(c[i].z, h.z);
+        for (int d = 0; d < 3; ++d) {
+            lo[k][d] = INFINITY, hi[k][d] = -INFINITY;
+            p[k][d] = c[4 * (size_t)std::min(b + 32, n - 1) + d];
         }
-        lo[k] = l, hi[k] = h, p[k] = c[std::min(b + 32, n - 1)];
+        for (int i = b; i < e; ++i)
+            for (int d = 0; d < 3; ++d) {
+                const float x = c[4 * (size_t)i + d];
+                lo[k][d] = lower(x, lo[k][d]);
+                hi[k][d] = upper(x, hi[k][d]);
+            }
     }
     int reached = 0;  // of the tiles but the bead's own
     for (int k = 0; k < S; ++k)
         for (int q = 0; q < S; ++q) {
-            const float x = upper(lo[q].x - p[k].x, upper(p[k].x - hi[q].x, 0.0f));
-            const float y = upper(lo[q].y - p[k].y, upper(p[k].y - hi[q].y, 0.0f));
-            const float z = upper(lo[q].z - p[k].z, upper(p[k].z - hi[q].z, 0.0f));
-            reached += (q != k) & (x * x + y * y + z * z <= d2max);
+            float d2 = 0.0f;
+            for (int d = 0; d < 3; ++d) {
+                const float x = upper(lo[q][d] - p[k][d], upper(p[k][d] - hi[q][d], 0.0f));
+                d2 += x * x;
+            }
+            reached += (q != k) & (d2 <= d2max);
         }
     return 1.0 + (double)reached / ((double)S * (S - 1)) * (nt - 1);
 }
@@ -641,7 +647,7 @@ int Engine::add_job(const sop_params& p, const sop_system& s, long long numsteps
         J.bead_cell = (int*)A(n * 4);
         J.bead_slot = (int*)A(n * 4);
         J.tile_box = (float4*)J.cell_beads;  // never both in use
-        J.wide = tiles_in_reach(b.coord.data(), b.n, J.pp_d2) > kWideTiles;
+        J.wide = tiles_in_reach(&b.coord[0].x, b.n, J.pp_d2) > kWideTiles;
     } else if (uses_boxes(n)) {
         J.tile_box = (float4*)A((n + 63) / 64 * 32);
     }
@@ -986,9 +992,9 @@ StepShape Engine::effective_shape(int first, int count) const {
 // Rows per wavefront of k_block_rows for jobs first .. first + count - 1, 0 where
 // their steps take a launch each: rows per wavefront that were asked for, a job
 // past kBlockBeads or with hydrodynamics, or few jobs whose rows the spread step
-// divides over more CUs than they have workgroups here.  Measured with updaters and lists in
-// launches of their own, us per step of a block of 10, a launch per step | R =
-// 8, 16 (the larger R where rows are many):
+// divides over more CUs than they have workgroups here.  Measured with updaters
+// and lists in launches of their own, us per step of a block of 10, a launch per
+// step | R = 8, 16 (the larger R where rows are many):
 //   beads x jobs   22 x 1      64        256       512        1,000       6,000
 //                  6.7 | 5.0  7.1 | 5.1  8.1 | 5.8  10.2 | 7.4  17.0 | 10.4  64 | 55, 50
 //   100 x          7.3 | 8.3  8.3 | 8.8  14.7 | 10.9, 12.1  20.0 | 19.9, 16.3  45 | 40, 32
@@ -1648,7 +1654,7 @@ int Engine::set_coords(int id, const float* in4) {
     if (int rc = read_state(slot, &s)) return rc;
     HostJob& hj = jobs_[slot];
     if (hj.dj.cell_cnt)
-        set_wide(hj, tiles_in_reach(reinterpret_cast<const float4*>(in4), hj.n, hj.dj.pp_d2) > kWideTiles);
+        set_wide(hj, tiles_in_reach(in4, hj.n, hj.dj.pp_d2) > kWideTiles);
     return check(hipMemcpy(hj.dj.coord[s.step & 1], in4, (size_t)hj.n * 16, hipMemcpyHostToDevice), "coords write");
 }
 

@@ -169,3 +169,21 @@ def test_order_lost_unseen_by_the_host():
         _equal(a, _list(e, j))
     print("case: rebuild %.0f us, then %.0f" % (first * 1e6, then * 1e6), flush=True)
     assert then < 0.6 * first
+
+
+@pytest.mark.parametrize("offset", [4, 8, 12])
+def test_coordinates_set_from_any_float_address(offset):
+    """Coordinates handed in at an address that only floats are aligned to."""
+    sysm = _shell(21000)
+    buf = np.empty(16 * sysm.n + 32, np.uint8)
+    start = (-buf.ctypes.data) % 16 + offset
+    c = buf[start:start + 16 * sysm.n].view(np.float32).reshape(sysm.n, 4)
+    c[:] = sysm.coords[::-1]
+    print("case: %d bytes past a 16-byte boundary" % offset, flush=True)
+    with S.Engine(0, 8 << 30) as e:
+        j = e.add_job(S.make_params(**c0_params(**KW)), sysm, 0)
+        e.set_coords(j, c)
+        np.testing.assert_array_equal(e.coords(j), c)
+        a = _list(e, j)
+        e.set_cells(enabled=False)
+        _equal(a, _list(e, j))
